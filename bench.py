@@ -829,7 +829,7 @@ def main():
         if args.only == "apply":
             a = extra["apply"]
             out.update({"value": a["mixed_GBps"], "unit": "GB/s", "ms_per_step": a["mixed_ms"],
-                        "dtype": "c64/fp32+TwoSum", "config": {"workload": a["workload"]}})
+                        "dtype": "c64/fp64", "config": {"workload": a["workload"]}})
     if args.only in (None, "batch") and not args.no_extra:
         extra["batch"] = bench_batch(args, torch, qa)
     if args.only in (None, "large") and not args.no_extra:

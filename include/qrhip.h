@@ -291,9 +291,9 @@ int qr_mm_read_close(qr_mm_reader *reader);
  *   y_v[r] = sum_g D_g(r) * x_v[r ^ x_g],  D_g(r) = sum_{t in g} (-1)^popcount(r&z_t) c'_t
  * for nvec state vectors stored one after another (x_v at offset v*2^n).
  *   QR_PREC_FP64  : x, y complex128; FP64 throughout.
- *   QR_PREC_MIXED : x, y complex64; D_g(r) merged in FP64 and rounded to FP32,
- *                   products and the sum over groups in FP32 with TwoSum
- *                   compensation; <x|y> reduced in FP64.
+ *   QR_PREC_MIXED : x, y complex64; coefficients, products and sums in FP64,
+ *                   y rounded to complex64 when it is written; <x|y> reduced
+ *                   in FP64 from the unrounded y.
  * d_expect (optional, may be NULL): 2*nvec doubles (device) receiving
  * <x_v | y_v> = sum_r conj(x_v[r]) y_v[r] in FP64.
  * d_y may be NULL when d_expect is given: then only <x|H|x> is produced and
@@ -308,8 +308,10 @@ int qr_mm_read_close(qr_mm_reader *reader);
  * The library picks one from the operator's masks and the state size; the
  * environment variable QR_APPLY_FORM=1 (gather) or 2 (staged) forces it.
  * QR_PREC_MIXED takes tiles of 2^11 rows, or of 2^10 when the launch would
- * otherwise have fewer than 4 tiles per CU (results again equal within
- * rounding); QR_APPLY_SMALL=0 or 1 forces the larger or the smaller.
+ * otherwise have fewer than 2 tiles per CU (results again equal within
+ * rounding); QR_APPLY_SMALL=0 or 1 forces the larger or the smaller.  Launches
+ * of few tiles share a tile's groups among 2 or 4 thread groups per block
+ * (QR_APPLY_SPLIT=1, 2 or 4 forces the number).
  * ---------------------------------------------------------------------- */
 enum qr_precision { QR_PREC_FP64 = 0, QR_PREC_MIXED = 1 };
 
@@ -325,7 +327,7 @@ int qr_pauli_apply(const qr_op *op, int32_t precision, uint32_t nvec, const void
  *    device (2^19 doubles): 2 * nvec * (2^n >> L) doubles must fit, with
  *    L = 11 (QR_PREC_MIXED) or 10 (QR_PREC_FP64) -- e.g. 8 states of 24
  *    qubits, or one of 28 -- else QR_ERR_SIZE (complex64 launches of fewer
- *    than 4 tiles per CU take tiles of 2^10 rows, whose partials always fit);
+ *    than 2 tiles per CU take tiles of 2^10 rows, whose partials always fit);
  *  - the operator's device tables for this precision must already be on the
  *    device: one qr_pauli_apply call of the same operator and precision on
  *    that device uploads them (QR_ERR_ARG otherwise).  Complex64 has tables

@@ -22,8 +22,8 @@ SOURCES = ["qr_api.cpp", "qr_csr.hip", "qr_apply.hip", "qr_batch.hip", "qr_group
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-x", "hip", "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
-    # no fused multiply-add unless written as fma(): TwoSum and the bit-exact
-    # CSR values depend on it
+    # no fused multiply-add unless written as fma(): the bit-exact CSR values
+    # depend on it
     "-ffp-contract=off",
     # packed FP32 instructions are kept out of every kernel
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

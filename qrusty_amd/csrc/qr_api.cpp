@@ -99,142 +99,241 @@ static void build_rank_lists(const std::vector<uint64_t> &gx, std::vector<uint32
     for (size_t j = 0; j < G; ++j) out.insert(out.end(), lists[j].begin(), lists[j].end());
 }
 
+static void free_patterns(DeviceTables::Patterns &pt);
+
 void free_tables(DeviceTables &t) {
     void *ptrs[] = {t.gx, t.gterm, t.tz, t.tc, t.rl_ptr, t.rl, t.gkind, t.heavy, t.leaf_heavy, t.ttz, t.ttc};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
-    for (auto &pt : t.pat) {
-        void *pp[] = {pt.grp, pt.chunk, pt.run, pt.ug, pt.pzl, pt.ptptr, pt.ptz, pt.ptc};
-        for (void *p : pp)
-            if (p) (void)hipFree(p);
-    }
+    for (auto &pt : t.pat) free_patterns(pt);
     t = DeviceTables{};
 }
+
+// A part under construction: patterns whose zl span at most kPartRank
+// dimensions.  basis[j]: the zl that raised the rank to j + 1; red: the same
+// span in echelon form, leading bits descending, comb[i] = red[i]'s
+// coordinates in the basis.
+struct PartBuild {
+    uint64_t basis[kPartRank] = {}, red[kPartRank] = {};
+    uint32_t comb[kPartRank] = {};
+    int rank = 0;
+    std::vector<size_t> pats;
+    std::vector<uint32_t> code;  // coordinates of each pattern's zl
+    // v minus its component in the span; the component's coordinates in *c
+    uint64_t reduce(uint64_t v, uint32_t *c) const {
+        *c = 0;
+        for (int i = 0; i < rank; ++i)
+            if ((v >> (63 - __builtin_clzll(red[i]))) & 1) {
+                v ^= red[i];
+                *c ^= comb[i];
+            }
+        return v;
+    }
+    bool add(size_t p, uint64_t zl) {
+        uint32_t c;
+        const uint64_t rest = reduce(zl, &c);
+        if (rest) {
+            if (rank == kPartRank) return false;
+            basis[rank] = zl;
+            c ^= 1u << rank;  // rest in the basis
+            int at = rank;
+            while (at > 0 && red[at - 1] < rest) {
+                red[at] = red[at - 1];
+                comb[at] = comb[at - 1];
+                --at;
+            }
+            red[at] = rest;
+            comb[at] = c;
+            c = 1u << rank;  // zl in the basis
+            ++rank;
+        }
+        pats.push_back(p);
+        code.push_back(c);
+        return true;
+    }
+    // table index bits of row bit i
+    uint32_t col(int i) const {
+        uint32_t c = 0;
+        for (int j = 0; j < rank; ++j) c |= uint32_t((basis[j] >> i) & 1) << j;
+        return c;
+    }
+};
 
 // Patterns: inside a tile of 2^L rows (fixed high bits h, low bits l), term t
 // of group g contributes (-1)^popcount(h & z_t) * c'_t * (-1)^popcount(l & zl_t)
 // with zl_t = z_t & (2^L - 1).  Terms of a group that share zl_t therefore
-// merge, per tile, into one coefficient.  The kernel splits l into tb
-// thread-index bits and the row-index bits above them; a pattern whose zl
-// lies in the thread bits costs once per thread, one whose zl lies in the
-// row bits once per block (a small per-tile table), and only the straddling
-// ones cost per row.  Terms keep input order inside a pattern.  With `pairs`
-// the low bits are taken in the paired-row order (pair_row_bits).
-void build_patterns(const qr_op *op, int L, int tb, uint32_t pcap, uint32_t ucap, bool staged,
-                    bool pairs, HostPatterns &out) {
+// merge, per tile, into one coefficient.  A group's patterns, by ascending zl,
+// go to the first part whose span holds their zl, else to the last part while
+// its rank is below kPartRank, else to a new one; the kernel tabulates each
+// part per tile (ApplyPart) and a row looks its value up.  Ascending zl keeps
+// the patterns of neighbouring bits together: the diagonal of a spin ring (two
+// patterns per bit) takes one part per three or four bits.  Terms keep input
+// order inside a pattern.  With `pairs` the low bits are taken in the
+// paired-row order (pair_row_bits).
+void build_patterns(const qr_op *op, const PatternShape &shape, const std::vector<uint8_t> &pass, uint8_t id,
+                    HostPatterns &out) {
+    const int L = shape.L, tb = shape.tb;
+    const bool staged = shape.staged, pairs = shape.pairs;
     const uint64_t mask = L >= 64 ? ~uint64_t(0) : ((uint64_t(1) << L) - 1);
-    const uint64_t tmask = (uint64_t(1) << tb) - 1;
+    // a mask's bits in the tile's row order (window passes: bits [0, f) and
+    // [s, s + L - f); the others are not part of the tile)
+    const ApplyWindow win = shape.win;
+    auto tile_bits = [&](uint64_t v) {
+        if (!win.s) return v & mask;
+        const uint64_t low = (uint64_t(1) << win.f) - 1;
+        return ((v & low) | ((v >> win.s) << win.f)) & mask;
+    };
     out = HostPatterns{};
-    out.ptptr.push_back(0);
     ApplyChunk cur{};
+    uint32_t cur_bytes = 0;  // table bytes of the chunk
+    std::vector<uint8_t> gcls;  // class of each group of the chunk, without the far bit
+    for (uint64_t g = 0; g < op->G; ++g) {
+        if (!pass.empty() && pass[g] != id) continue;
+        for (uint32_t i = op->gterm[g]; i < op->gterm[g + 1]; ++i) out.cplx = out.cplx || op->tc[2 * i + 1] != 0.0;
+    }
+    const int lg = out.cplx ? 4 : 3;  // log2 bytes of a table entry
     const uint64_t far_mask = ~mask;
     // closes the chunk: its groups are reordered by class, or (staged) by
-    // partner tile and then class (patterns stay where they are; the table
-    // rows follow their groups)
-    auto close_chunk = [&out, &cur, far_mask, staged, pairs]() {
-        const uint32_t g0 = cur.cg[0], g1 = uint32_t(out.grp.size());
-        cur.p1 = uint32_t(out.pzl.size());
-        cur.u1 = uint32_t(out.ug.size());
+    // partner tile and then class
+    auto close_chunk = [&]() {
+        const uint32_t g0 = cur.cg[0], g1 = uint32_t(out.grp.size()), n = g1 - g0;
+        cur.t1 = uint32_t(out.tab.size());
         cur.r0 = cur.r1 = uint32_t(out.run.size());
-        if (g1 > g0) {
-            auto cls = [far_mask, pairs](const ApplyGroup &a) {
-                return ((a.m & far_mask) ? 1u : 0u) | ((a.u >= 0 || a.ps != a.pk) ? 2u : 0u) |
-                       ((a.flags & kGroupReal) ? 0u : 4u) | ((pairs && (a.m & 1)) ? 8u : 0u);
-            };
+        if (n) {
+            std::vector<uint32_t> order(n);
+            std::iota(order.begin(), order.end(), 0u);
+            const std::vector<ApplyGroup> was(out.grp.begin() + g0, out.grp.end());
+            auto cls = [&](uint32_t i) { return ((was[i].m & far_mask) ? 2u : 0u) | gcls[i]; };
+            auto hi = [&](uint32_t i) { return was[i].m & far_mask; };
+            if (!staged)
+                std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return cls(a) < cls(b); });
+            else
+                std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return hi(a) > hi(b); });
+            for (uint32_t i = 0; i < n; ++i) out.grp[g0 + i] = was[order[i]];
             if (!staged) {
-                std::stable_sort(out.grp.begin() + g0, out.grp.end(),
-                                 [&cls](const ApplyGroup &a, const ApplyGroup &b) { return cls(a) < cls(b); });
                 uint32_t c = 0;
-                for (uint32_t g = g0; g <= g1; ++g) {
-                    const uint32_t cg = g < g1 ? cls(out.grp[g]) : uint32_t(kApplyClasses);
-                    while (c <= cg && c <= uint32_t(kApplyClasses)) cur.cg[c++] = g;
+                for (uint32_t i = 0; i <= n; ++i) {
+                    const uint32_t cg = i < n ? cls(order[i]) : uint32_t(kApplyClasses);
+                    while (c <= cg && c <= uint32_t(kApplyClasses)) cur.cg[c++] = g0 + i;
                 }
             } else {
-                // run class: bit 0 row-varying, bit 1 complex (cls without the
-                // far bit; the staged form has no paired rows)
-                auto key = [&cls, far_mask](const ApplyGroup &a) {
-                    return std::make_pair(a.m & far_mask, (cls(a) >> 1) & 3u);
-                };
-                std::stable_sort(out.grp.begin() + g0, out.grp.end(),
-                                 [&key](const ApplyGroup &a, const ApplyGroup &b) { return key(a) < key(b); });
-                for (uint32_t g = g0; g < g1;) {
+                for (uint32_t i = 0; i < n; ++i) {
+                    if (i + 1 < n && hi(order[i + 1]) == hi(order[i])) continue;
                     ApplyRun r{};
-                    r.hi = out.grp[g].m & far_mask;
-                    uint32_t e = g;
-                    while (e < g1 && (out.grp[e].m & far_mask) == r.hi) ++e;
-                    uint32_t c = 0;
-                    for (uint32_t k = g; k <= e; ++k) {
-                        const uint32_t ck = k < e ? key(out.grp[k]).second : uint32_t(kRunClasses);
-                        while (c <= ck && c <= uint32_t(kRunClasses)) r.g[c++] = k;
-                    }
+                    r.hi = hi(order[i]);
+                    r.g1 = g0 + i + 1;
                     out.run.push_back(r);
-                    g = e;
                 }
                 cur.r1 = uint32_t(out.run.size());
                 for (uint32_t c = 0; c <= uint32_t(kApplyClasses); ++c) cur.cg[c] = g0;
                 cur.cg[kApplyClasses] = g1;
             }
-            for (uint32_t g = g0; g < g1; ++g) {
-                if (out.grp[g].u >= 0) out.ug[cur.u0 + uint32_t(out.grp[g].u)] = g;
-                if (out.grp[g].m & far_mask) ++out.nfar;
-            }
+            for (uint32_t i = 0; i < n; ++i)
+                if (was[i].m & far_mask) ++out.nfar;
             out.chunk.push_back(cur);
-            out.max_p = std::max(out.max_p, cur.p1 - cur.p0);
-            out.max_u = std::max(out.max_u, cur.u1 - cur.u0);
+            out.max_tab = std::max(out.max_tab, cur_bytes);
         }
         cur = ApplyChunk{};
         cur.cg[0] = g1;
-        cur.p0 = uint32_t(out.pzl.size());
-        cur.u0 = uint32_t(out.ug.size());
+        cur.t0 = uint32_t(out.tab.size());
+        cur_bytes = 0;
+        gcls.clear();
     };
-    auto cls = [tmask](uint64_t zl) {
-        if ((zl & ~tmask) == 0) return 0;  // thread bits only (or zl == 0)
-        if ((zl & tmask) == 0) return 2;   // row-index bits only
-        return 1;                          // straddling
-    };
-    for (uint64_t g = 0; g < op->G; ++g) {
-        std::vector<uint64_t> zls;
-        std::vector<std::vector<uint32_t>> members;
-        for (uint32_t i = op->gterm[g]; i < op->gterm[g + 1]; ++i) {
-            const uint64_t zl = pairs ? pair_row_bits(op->tz[i] & mask, tb) : op->tz[i] & mask;
-            size_t k = 0;
-            while (k < zls.size() && zls[k] != zl) ++k;
-            if (k == zls.size()) { zls.push_back(zl); members.emplace_back(); }
-            members[k].push_back(i);
-        }
-        std::vector<size_t> order;  // patterns by class, first-seen order inside a class
-        for (int c = 0; c < 3; ++c)
-            for (size_t k = 0; k < zls.size(); ++k)
-                if (cls(zls[k]) == c) order.push_back(k);
-        for (size_t s0 = 0; s0 < order.size(); s0 += pcap) {
-            const size_t s1 = std::min(order.size(), s0 + pcap);
-            uint32_t ncls[3] = {0, 0, 0};
-            for (size_t s = s0; s < s1; ++s) ++ncls[cls(zls[order[s]])];
-            const uint32_t n = uint32_t(s1 - s0), has_u = ncls[2] ? 1u : 0u;
-            if ((uint32_t(out.pzl.size()) - cur.p0) + n > pcap ||
-                (uint32_t(out.ug.size()) - cur.u0) + has_u > ucap)
-                close_chunk();
-            ApplyGroup a{};
-            a.m = op->gx[g];
-            a.p0 = uint32_t(out.pzl.size()) - cur.p0;
-            a.ps = a.p0 + ncls[0];
-            a.pk = a.ps + ncls[1];
-            a.p1 = a.pk + ncls[2];
-            bool real = true;
+    for (uint64_t k = 0; k < op->G; ++k) {
+        const uint64_t g = staged ? op->G - 1 - k : k;
+        if (!pass.empty() && pass[g] != id) continue;
+        // window passes keep the mask in the tile's row order
+        const uint64_t gm = win.s ? tile_bits(op->gx[g]) : op->gx[g];
+        std::vector<std::pair<uint64_t, uint32_t>> zt;  // (zl, term) by zl, terms in input order
+        for (uint32_t i = op->gterm[g]; i < op->gterm[g + 1]; ++i)
+            zt.emplace_back(pairs ? pair_row_bits(tile_bits(op->tz[i]), tb) : tile_bits(op->tz[i]), i);
+        std::stable_sort(zt.begin(), zt.end(),
+                         [](const auto &a, const auto &b) { return a.first < b.first; });
+        std::vector<size_t> heads;  // first term of each pattern
+        for (size_t i = 0; i < zt.size(); ++i)
+            if (i == 0 || zt[i].first != zt[i - 1].first) heads.push_back(i);
+        heads.push_back(zt.size());
+        const size_t npat = heads.size() - 1;
+        for (size_t s0 = 0; s0 < npat; s0 += shape.psplit) {
+            const size_t s1 = std::min(npat, s0 + shape.psplit);
+            std::vector<PartBuild> parts;
             for (size_t s = s0; s < s1; ++s) {
-                const size_t k = order[s];
-                out.pzl.push_back(uint32_t(zls[k]));
-                for (uint32_t i : members[k]) {
-                    out.ptz.push_back(op->tz[i]);
-                    out.ptc.push_back(op->tc[2 * i]);
-                    out.ptc.push_back(op->tc[2 * i + 1]);
-                    real = real && op->tc[2 * i + 1] == 0.0;
+                const uint64_t zl = zt[heads[s]].first;
+                bool placed = false;
+                uint32_t c;
+                for (size_t k = 0; k < parts.size() && !placed; ++k)
+                    if (k + 1 == parts.size() || parts[k].reduce(zl, &c) == 0) placed = parts[k].add(s, zl);
+                if (!placed) {
+                    parts.emplace_back();
+                    parts.back().add(s, zl);
                 }
-                out.ptptr.push_back(uint32_t(out.ptz.size()));
             }
-            a.u = has_u ? int32_t(uint32_t(out.ug.size()) - cur.u0) : -1;
-            if (has_u) out.ug.push_back(uint32_t(out.grp.size()));
-            a.flags = real ? kGroupReal : 0u;
+            bool real = true;
+            for (size_t i = heads[s0]; i < heads[s1]; ++i) real = real && op->tc[2 * zt[i].second + 1] == 0.0;
+            // each table aligned to its size
+            auto place = [&](uint32_t at, std::vector<uint32_t> *where) {
+                for (const PartBuild &p : parts) {
+                    const uint32_t size = 1u << (p.rank + lg);
+                    at = (at + size - 1) & ~(size - 1);
+                    if (where) where->push_back(at);
+                    at += size;
+                }
+                return at;
+            };
+            if (place(cur_bytes, nullptr) > shape.tcap) close_chunk();
+            std::vector<uint32_t> where;
+            cur_bytes = place(cur_bytes, &where);
+            ApplyGroup a{};
+            a.m = gm;
+            bool rowvar = false;
+            for (size_t k = 0; k < parts.size(); ++k) {
+                const PartBuild &p = parts[k];
+                auto span = [&p](int bit0, int nbits, uint32_t v) {  // index of bits [bit0, bit0 + nbits) = v
+                    uint32_t c = 0;
+                    for (int i = 0; i < nbits; ++i)
+                        if ((v >> i) & 1) c ^= p.col(bit0 + i);
+                    return c;
+                };
+                ApplyPart ap{};
+                for (uint32_t v = 0; v < 8; ++v) {
+                    ap.w0 |= span(0, 3, v) << (4 * v);
+                    ap.w1 |= span(3, 3, v) << (4 * v);
+                    ap.rc |= uint64_t(span(tb, 3, v) << lg) << (8 * v);
+                }
+                for (uint32_t v = 0; v < 4; ++v) ap.w2 |= (span(6, 2, v) << lg) << (8 * v);
+                ap.tab = (shape.tab0 + where[k]) / 4;
+                rowvar = rowvar || ap.rc;
+                if (parts.size() == 1) {
+                    a.w0 = ap.w0;
+                    a.w1 = ap.w1;
+                    a.w2 = ap.w2;
+                    a.rc = ap.rc;
+                    a.tab_n = ap.tab | (1u << 16);
+                } else {
+                    if (k == 0) {
+                        a.w0 = uint32_t(out.part.size());
+                        a.tab_n = uint32_t(parts.size()) << 16;
+                    }
+                    out.part.push_back(ap);
+                }
+                std::vector<size_t> by_code(16, npat);
+                for (size_t i = 0; i < p.pats.size(); ++i) by_code[p.code[i]] = p.pats[i];
+                for (uint32_t c = 0; c < 16; ++c) {
+                    ApplyRange pr{uint32_t(out.ptz.size()), 0};
+                    for (size_t q = by_code[c] < npat ? heads[by_code[c]] : 0;
+                         by_code[c] < npat && q < heads[by_code[c] + 1]; ++q) {
+                        const uint32_t t = zt[q].second;
+                        out.ptz.push_back(op->tz[t]);
+                        out.ptc.push_back(op->tc[2 * t]);
+                        out.ptc.push_back(op->tc[2 * t + 1]);
+                    }
+                    pr.t1 = uint32_t(out.ptz.size());
+                    out.pat.push_back(pr);
+                }
+                out.tab.push_back(ap.tab | (1u << (16 + p.rank)));
+            }
+            a.tab_n |= (rowvar ? kGroupRowvar : 0u) | (real ? 0u : kGroupCplx);
+            gcls.push_back(uint8_t(pairs ? a.m & 1 : 0));
             out.grp.push_back(a);
         }
     }
@@ -295,38 +394,129 @@ bool tables_ready(const qr_op *op, const DeviceTables *t, int slot, int L) {
     return t->pat[slot].L == L;
 }
 
-int device_patterns(const qr_op *op, DeviceTables *t, int slot, int L, int tb, uint32_t pcap,
-                    uint32_t ucap, bool staged, bool pairs, bool noalloc) {
-    std::lock_guard<std::mutex> lock(op->mu);
-    DeviceTables::Patterns &pt = t->pat[slot];
-    if (pt.L == L) return QR_OK;
-    if (noalloc)
-        return fail(QR_ERR_ARG, "apply_noalloc: the operator's apply tables for this precision "
-                                "are not on this device (one qr_pauli_apply of it with this "
-                                "precision on this device uploads them)");
-    for (void *p : {(void *)pt.grp, (void *)pt.chunk, (void *)pt.run, (void *)pt.ug, (void *)pt.pzl,
-                    (void *)pt.ptptr, (void *)pt.ptz, (void *)pt.ptc})
-        if (p) (void)hipFree(p);
-    pt = DeviceTables::Patterns{};
-    HostPatterns hp;
-    build_patterns(op, L, tb, pcap, ucap, staged, pairs, hp);
+// Which groups run in window passes.  In the pass over tiles of consecutive
+// rows, every distinct value of the mask bits above the tile is a partner tile
+// that each tile reads; those whose mask stays within about 2^17 complex128
+// (2^18 complex64) rows find it in the XCD's 4 MB L2, the others read it past
+// L2, at the 6.2-7 TB/s that HBM and the MALL deliver (L2: 31 TB/s).  A window
+// pass reads x once, and y once and writes it once more, whatever the number
+// of masks it holds: three streams of the state.  So the windows [s, s + w)
+// that save the most partner streams are taken in turn while they save at
+// least kWindowMinSaved (a partner stream is saved when all groups that share
+// it move).  Up to the MALL's 256 MB that is done for FP64 if together they
+// save half of the partners past L2 (the return value): nearest-neighbour
+// rings and chains, whose masks are a few adjacent bits.  Measured, one state
+// / 8 states, without and with: 24-qubit ring 432 -> 301 us / 3.49 -> 2.91 ms,
+// 22 qubits 107 -> 78 / 697 -> 633 us; k-local and molecular operators, where
+// windows save a sixth of the partners, lost 1-5% with them, and so did
+// complex64 rings, whose arithmetic takes as long as the streams.  For states
+// past the MALL every partner is read from HBM: 28-qubit k-local, complex64,
+// 242 -> 235 ms.
+constexpr uint32_t kWindowMinSaved = 5;
+constexpr int kWindowMinStateLog2 = 25, kMallLog2 = 28;  // bytes of one state
+bool choose_windows(const qr_op *op, int L, int elem_log2, std::vector<ApplyWindow> &wins,
+                    std::vector<uint8_t> &pass) {
+    wins.clear();
+    pass.assign(op->G, 0);
+    const int n = int(op->nq);
+    const bool past_mall = n + elem_log2 > kMallLog2;
+    if (!past_mall && (elem_log2 != 4 || n + elem_log2 < kWindowMinStateLog2)) return false;
+    const int f = 7 - elem_log2;  // 128-byte segments
+    const int w = L - f, near = 21 - elem_log2;
+    // gx ascends: the groups of one partner are adjacent
+    struct Partner { uint64_t g0, g1, bits; };
+    std::vector<Partner> far;
+    for (uint64_t g = 0; g < op->G;) {
+        uint64_t e = g, bits = 0;
+        while (e < op->G && (op->gx[e] >> L) == (op->gx[g] >> L)) bits |= op->gx[e++];
+        if (op->gx[e - 1] >> near) far.push_back({g, e, bits});
+        g = e;
+    }
+    while (int(wins.size()) < kMaxWindows) {
+        uint32_t best = 0;
+        int best_s = 0;
+        auto inside = [&](const Partner &p, int s) {
+            const uint64_t tile = ((uint64_t(1) << f) - 1) | (((uint64_t(1) << w) - 1) << s);
+            return pass[p.g0] == 0 && (p.bits & ~tile) == 0;
+        };
+        for (int s = n - w; s >= f + 1; --s) {
+            uint32_t saved = 0;
+            for (const Partner &p : far) saved += inside(p, s) ? 1u : 0u;
+            if (saved > best) {
+                best = saved;
+                best_s = s;
+            }
+        }
+        if (best < kWindowMinSaved) break;
+        wins.push_back({uint32_t(f), uint32_t(best_s)});
+        for (const Partner &p : far)
+            if (inside(p, best_s))
+                for (uint64_t g = p.g0; g < p.g1; ++g) pass[g] = uint8_t(wins.size());
+    }
+    size_t moved = 0;
+    for (const Partner &p : far) moved += pass[p.g0] != 0;
+    const bool most = !wins.empty() && 2 * moved >= far.size();
+    if (!most && !past_mall) {
+        wins.clear();
+        pass.assign(op->G, 0);
+    }
+    return most;
+}
+
+static int upload_patterns(DeviceTables::Patterns &pt, const HostPatterns &hp, const PatternShape &shape) {
     std::vector<double2> c2(hp.ptz.size());
     for (size_t i = 0; i < c2.size(); ++i) c2[i] = make_double2(hp.ptc[2 * i], hp.ptc[2 * i + 1]);
     int rc;
     if ((rc = upload(&pt.grp, hp.grp)) || (rc = upload(&pt.chunk, hp.chunk)) ||
-        (staged && (rc = upload(&pt.run, hp.run))) ||
-        (rc = upload(&pt.ug, hp.ug)) || (rc = upload(&pt.pzl, hp.pzl)) ||
-        (rc = upload(&pt.ptptr, hp.ptptr)) || (rc = upload(&pt.ptz, hp.ptz)) ||
-        (rc = upload(&pt.ptc, c2)))
+        (shape.staged && (rc = upload(&pt.run, hp.run))) ||
+        (rc = upload(&pt.part, hp.part)) || (rc = upload(&pt.tab, hp.tab)) ||
+        (rc = upload(&pt.pat, hp.pat)) ||
+        (rc = upload(&pt.ptz, hp.ptz)) || (rc = upload(&pt.ptc, c2)))
         return rc;
-    pt.P = uint32_t(hp.pzl.size());
     pt.ngrp = uint32_t(hp.grp.size());
     pt.nchunk = uint32_t(hp.chunk.size());
     pt.nrun = uint32_t(hp.run.size());
     pt.nfar = hp.nfar;
-    pt.max_p = hp.max_p;
-    pt.max_u = hp.max_u;
-    pt.L = L;
+    pt.max_tab = hp.max_tab;
+    pt.cplx = hp.cplx;
+    pt.win = shape.win;
+    return QR_OK;
+}
+
+static void free_patterns(DeviceTables::Patterns &pt) {
+    for (void *p : {(void *)pt.grp, (void *)pt.chunk, (void *)pt.run, (void *)pt.part, (void *)pt.tab,
+                    (void *)pt.pat, (void *)pt.ptz, (void *)pt.ptc})
+        if (p) (void)hipFree(p);
+    pt = DeviceTables::Patterns{};
+}
+
+int device_patterns(const qr_op *op, DeviceTables *t, int slot, const PatternShape &shape,
+                    const PatternShape &win_shape, int elem_log2, bool noalloc) {
+    std::lock_guard<std::mutex> lock(op->mu);
+    DeviceTables::Patterns &pt = t->pat[slot];
+    if (pt.L == shape.L) return QR_OK;
+    if (noalloc)
+        return fail(QR_ERR_ARG, "apply_noalloc: the operator's apply tables for this precision "
+                                "are not on this device (one qr_pauli_apply of it with this "
+                                "precision on this device uploads them)");
+    for (int k = 0; k <= kMaxWindows; ++k) free_patterns(t->pat[slot + kApplySlots * k]);
+    std::vector<ApplyWindow> wins;
+    std::vector<uint8_t> pass;
+    if (win_shape.L) choose_windows(op, win_shape.L, elem_log2, wins, pass);
+    HostPatterns hp;
+    int rc;
+    for (size_t k = 0; k < wins.size(); ++k) {
+        PatternShape ws = win_shape;
+        ws.win = wins[k];
+        build_patterns(op, ws, pass, uint8_t(k + 1), hp);
+        DeviceTables::Patterns &pw = t->pat[slot + kApplySlots * int(k + 1)];
+        if ((rc = upload_patterns(pw, hp, ws))) return rc;
+        pw.L = ws.L;
+    }
+    build_patterns(op, shape, pass, 0, hp);
+    if ((rc = upload_patterns(pt, hp, shape))) return rc;
+    pt.nwin = uint32_t(wins.size());
+    pt.L = shape.L;
     return QR_OK;
 }
 

@@ -7,45 +7,57 @@
 // entries: D_g(r) is the CSR value of group g in row r, x[r ^ x_g] the gather
 // of its column.
 //
-// Work decomposition (one block of 256 threads = one tile of 2^L consecutive
-// rows of one state vector; four blocks share a CU, so that some compute
-// while others wait at a barrier or on their loads):
-//  * The tile's slice of x is staged in LDS (coalesced); groups whose x mask
-//    is below 2^L gather from LDS, the others ("far" groups) gather the
-//    partner tile t ^ (x_g >> L) from global memory (coalesced, permuted
-//    inside a line).
+// Work decomposition (one block = one tile of 2^L consecutive rows of one
+// state vector: 256 threads, or 2 or 4 times as many that share the tile's
+// groups, see apply_split; at most 40 KB of LDS, so that four blocks share a
+// CU and some compute while others wait at a barrier or on their loads):
+//  * The tile's slice of x is staged in LDS (LDS-DMA); groups whose x mask is
+//    below 2^L gather from LDS, the others ("far" groups) gather the partner
+//    tile t ^ (x_g >> L) from global memory (coalesced, permuted inside a
+//    line).
 //  * Blocks are ordered vector-major, and each XCD receives one contiguous
 //    range of tiles of the vector: the far partners of nearby tiles are read
 //    through the same L2, and one complex64 vector (128 MiB at 24 qubits)
 //    stays resident in the 256 MB MALL while the chip works on it.
 //  * Row r = h + l (h = tile base, l < 2^L):  (-1)^popcount(r & z) =
-//    (-1)^popcount(h & z) * (-1)^popcount(l & zl).  The host merges the terms
-//    of a group that share zl into "patterns"; per tile each pattern's
-//    coefficient A_p = sum (-1)^popcount(h & z_t) c'_t is formed once (wave-
-//    uniform), and per row only patterns with zl != 0 cost a sign.  The block
-//    forms all its patterns' coefficients in parallel at the start of the
-//    tile and keeps them in LDS next to the x tile.  Thread `tid` owns rows
-//    l = tid + 256*k: the sign splits again into a per-thread part (bits of
-//    tid) and a per-k part (wave-uniform), so each pattern costs one FMA per
-//    row.  The gather form on full complex64 tiles owns row pairs instead,
-//    l = 2*tid + (k & 1) + 512*(k >> 1), so that one 16-byte load gathers
-//    both partners of a pair and one 16-byte store writes both results; the
-//    patterns' low z bits are permuted to match (row bit 0 counts with k).
+//    (-1)^popcount(h & z) * (-1)^popcount(l & zl), zl = z & (2^L - 1).  The
+//    host merges the terms of a group that share zl into "patterns" and cuts
+//    the patterns into parts whose zl span at most four dimensions.  Over the
+//    tile a part's sum takes at most 16 values, which the block tabulates in
+//    LDS (chunk_tables); the index of a row's value is linear in the bits of
+//    l, so a thread finds it with a few shifts and XORs of two words of the
+//    group's descriptor (ApplyPart) whatever the number of terms.  Summing the
+//    signed coefficients per thread instead took 5-6 vector instructions per
+//    pattern: 103 per group and 8 rows on the 28-qubit k-local operator (now
+//    70), 90 per group and 4 rows on a 20-qubit molecule (now 30); molecules
+//    of 12 / 16 / 20 / 22 qubits, FP64, one state: 290 / 556 / 1633 / 10100 ->
+//    35 / 114 / 912 / 5120 us, 20 qubits and 2000 random terms 1590 -> 1100.
+//    What bounds them now is the chain of descriptor loads, lookups and
+//    gathers of each group (vector ALU about half busy).
+//  * Thread `tid` owns rows l = tid + 256*k.  The gather form on full
+//    complex64 tiles owns row pairs instead, l = 2*tid + (k & 1) + 512*(k >>
+//    1), so that one 16-byte load gathers both partners of a pair and one
+//    16-byte store writes both results; the patterns' low z bits are permuted
+//    to match (row bit 0 counts with k).
 //  * Partner-staged form (k_apply_staged): when many far groups share a
 //    partner tile (their masks agree above the tile), the groups are ordered
 //    by partner and each partner tile is loaded into LDS once, double-
 //    buffered, instead of being gathered once per group.
+//  * Window passes (ApplyWindow): groups whose partner tiles would be
+//    read past L2 are applied in a second pass over tiles made of the low bits
+//    and a window of high ones, where their masks stay inside the tile.
 //
 // Precision modes
-//   FP64 : complex128 state, FP64 FMAs (tile 2^10 rows, 4 rows per thread).
-//   MIXED: complex64 state (tile 2^11 rows, 8 rows per thread).  D_g(r) is
-//          merged in FP64 -- where terms sharing an x mask cancel -- and then
-//          rounded to FP32.  Products and the sum over groups run in FP32:
-//          products are accumulated into a block partial over up to
-//          kCompBlock groups, and block partials are added to the running sum
-//          with TwoSum (s + e == a + b exactly); the error e starts the next
-//          block partial, so y = s + b at the end.  <x|y> is reduced in FP64
-//          from s + b.
+//   FP64 : complex128 state (tile 2^10 rows, 4 rows per thread).
+//   MIXED: complex64 state (tile 2^11 rows, 8 rows per thread), rounded to
+//          complex64 once, when y is written.
+// In both, D_g(r), the products and the sum over groups are FP64.  For the
+// complex64 state that is also the cheapest arithmetic: FP64 FMAs and
+// FP32 -> FP64 conversions issue at the rate of FP32 ones here (packed FP32 is
+// off; measured 4.7-5.2 cycles per wave instruction and SIMD, all of them), so
+// a row and group takes 2 conversions and 2 FMAs against 2 FMAs and the 3
+// additions of a compensated FP32 sum (TwoSum every 4 groups) -- and its error
+// is the rounding of y: 3.5e-8 against 4.7e-8 on the 24-qubit ring.
 // <x|y> is reduced deterministically: per thread, per block (fixed tree),
 // then one pass over the block partials of each vector.
 #include "qr_internal.h"
@@ -68,65 +80,45 @@ namespace qr {
 // 72-88 VGPRs, 5-7 waves per SIMD) measured 1.84 / 3.59 ms and 278 / 436 ms
 // against 1.63 / 3.50 and 238 / 401 with 256 threads (block partials summed
 // in FP64 in both): the per-group work of a thread is shared by fewer rows.
-// Forcing 5 or 6 waves per SIMD on 256 threads spills 120-330 registers.
+// (All of these before the coefficients were tabulated.)
 constexpr int kApplyThreads = 256;
 constexpr int kApplyThreadBits = 8;
-// Groups per FP32 block partial between TwoSum steps.  Measured on the same
-// 24-qubit Heisenberg case (8 states, psi rounded to complex64; error of
-// <psi|H|psi> relative to the FP64 value on the rounded state, max over
-// states), by block size: 1: 2.6e-7, 2.16 ms; 4: 2.8e-7, 1.69 ms;
-// 16: 5.9e-7, 1.62 ms; 32: 6.6e-7, 1.62 ms.  4 keeps the whole-call error of
-// <psi|H|psi> (rounding of psi included) near 5e-7.  Those figures are
-// with the TwoSum errors collected in a separate compensation c; feeding
-// each error into the next block partial instead saves the compensation's
-// adds, zeroing and 16 registers (113 -> 95 VGPRs, 5 waves per SIMD): 1.651
-// -> 1.583 ms, E 5.05e-7 -> 5.22e-7 end to end, y unchanged.  Adding the
-// block partials into FP64 running sums gave 1.63 ms; the accumulation stays
-// FP32 with TwoSum compensation, FP64 being kept to the merging of
-// coefficients and the <x|y> reduction.
-constexpr int kCompBlock = 4;
 constexpr size_t kApplyMaxLDS = 40 * 1024;  // LDS of one block
+// of an operator with a group that needs more than a chunk's share of it
+constexpr size_t kApplyLDSLimit = 160 * 1024;
+// dynamic LDS that a launch may ask for without raising the kernel's limit
+constexpr size_t kDefaultLDS = 64 * 1024;
 
 // Tile of 2^L rows (x tile in LDS: 16 KB in both precisions at the default
 // L; 8 KB for the small complex64 tiles), R rows per thread, and the LDS left
-// for one chunk of pattern coefficients (20 B each) and the row-bit table
-// (R x 16 B per row, plus a zero row).
+// for one chunk of tables.
 //
-// Small complex64 tiles (2^10 rows, 4 per thread) serve launches that would
-// leave CUs short of blocks with 2^11-row tiles: the block keeps the latency
-// of its LDS and gather round trips hidden only with others beside it.
-// Measured, one state (20 qubits, 14251 terms in 2536 groups; 512 blocks of
-// 2^11 rows, two per CU): 2.29 -> 1.70 ms.  Where the default tiles fill the
-// chip they are 20-27% slower (22- and 24-qubit operators of 811-3792
-// groups, the 20-qubit one with 4 states, 24-qubit Heisenberg with 8).
+// Small complex64 tiles (2^10 rows, 4 per thread) serve launches of fewer than
+// two 2^11-row tiles per CU, with four thread groups per block (apply_split):
+// one state, 2^11-row tiles and two thread groups / small tiles and four:
+// molecules 12 / 16 / 18 qubits 64 / 200 / 321 -> 36 / 110 / 183 us.  From two
+// tiles per CU on the larger ones win: 20 qubits 804 / 915, random 761 / 1009.
 constexpr int kMixedSmallL = 10;
 template <bool kMixed, int kL = kMixed ? 11 : 10>
 struct ApplyShape {
     static constexpr int L = kL;
     static constexpr int R = (1 << L) / kApplyThreads;
     static constexpr size_t kTile = (size_t(1) << L) * (kMixed ? 8 : 16);
-    // LDS after the x tile: 5/8 for patterns, 3/8 for the row-bit table
-    static constexpr size_t kRest = kApplyMaxLDS - kTile - 1024;
-    static constexpr uint32_t kPatChunk = uint32_t(kRest * 5 / 8 / 20) < 2048u ? uint32_t(kRest * 5 / 8 / 20) : 2048u;
-    static constexpr uint32_t kTableRows = uint32_t(kRest * 3 / 8 / (R * 16)) - 1;
-    // partner-staged form: two tile buffers, the rest split the same way
-    static constexpr size_t kRestS = kApplyMaxLDS - 2 * kTile - 1024;
-    static constexpr uint32_t kPatChunkS = uint32_t(kRestS * 5 / 8 / 20);
-    static constexpr uint32_t kTableRowsS = uint32_t(kRestS * 3 / 8 / (R * 16)) - 1;
+    // LDS for adding up the sums of `split` thread groups (merge_splits)
+    static constexpr size_t merge_bytes(int split) { return size_t(split / 2) * R * kApplyThreads * 16; }
+    // table bytes of one chunk, in the LDS after the x tile (gather form) or
+    // after two tile buffers (partner-staged form); a group of more than
+    // kPatSplit patterns is split, one that needs more than a chunk takes a
+    // larger chunk of its own
+    static constexpr uint32_t kPatSplit = 736, kPatSplitS = 224;
+    static constexpr uint32_t kTabChunk = uint32_t(kApplyMaxLDS - kTile - 1024);
+    static constexpr uint32_t kTabChunkS = uint32_t(kApplyMaxLDS - 2 * kTile - 1024);
 };
 
 template <bool kNarrow>
 __device__ __forceinline__ uint32_t parity_of(uint64_t a, uint64_t b) {
     if (kNarrow) return __popc(uint32_t(a) & uint32_t(b)) & 1u;
     return __popcll(a & b) & 1u;
-}
-
-// Knuth's TwoSum: s + e == a + b exactly (round-to-nearest, no reassociation).
-__device__ __forceinline__ void two_sum(float a, float b, float &s, float &e) {
-    s = a + b;
-    const float bp = s - a;
-    const float ap = s - bp;
-    e = (a - ap) + (b - bp);
 }
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -145,241 +137,261 @@ __device__ __forceinline__ double flip_sign(double a, uint32_t flip) {
 // format; offsets are bounds-checked against num_records bytes.
 constexpr int kBufferWord3 = 0x00020000;
 
-// Gathers of x[r ^ m] for the R rows of a thread: from the LDS x tile, or --
-// for masks above the tile -- from the partner tile in global memory, with
-// one uniform base pointer per row block and the thread's offset shared.
+// Complex elements as builtin vectors: they load, store and copy across
+// address spaces as one 8- or 16-byte access.
+typedef float fvec2 __attribute__((ext_vector_type(2)));
+typedef float fvec4 __attribute__((ext_vector_type(4)));
+typedef double dvec2 __attribute__((ext_vector_type(2)));
+
+typedef __attribute__((address_space(3))) unsigned char lds_byte;
+
+// LDS by absolute byte address.  The tile buffers and tables are aligned to
+// their sizes, so places in them are formed with XOR.
+template <typename T>
+__device__ __forceinline__ T lds_load(uint32_t at) {
+    return *(const __attribute__((address_space(3))) T *)(at);
+}
+
+// Gathers of x[r ^ m] for the R rows of a thread: from the LDS x tile (at
+// LDS address xt), or -- for masks above the tile -- from the partner tile in
+// global memory, with one uniform base pointer per row block and the
+// thread's offset shared.
 // With kPairs (complex64, full tiles) the thread's rows k = 2j, 2j+1 are the
 // adjacent rows (2 tid, 2 tid + 1) + 2^9 j: their partners r ^ m form one
 // aligned pair, read with one 16-byte load.  When bit 0 of m is set, row k's
-// partner is xg[k ^ 1]: such groups form classes of their own, whose
-// accumulation reads the pair crosswise (no data is moved).
+// partner is xg[k ^ 1]: such groups form classes of their own, whose products
+// read the pair crosswise (no data is moved).
 template <bool kFar, bool kFull, bool kPairs, int R, typename cT>
 __device__ __forceinline__ void gather(uint64_t m, uint32_t tid, uint64_t tile_rows, uint64_t base,
-                                       const cT *xt, const cT *__restrict__ xv, cT (&xg)[R]) {
-    const uint64_t mlo = m & (tile_rows - 1), mhi = m & ~(tile_rows - 1);
+                                       uint32_t xt, const cT *__restrict__ xv, cT (&xg)[R]) {
+    const uint64_t mhi = m & ~(tile_rows - 1);
+    const uint32_t mlo = uint32_t(m & (tile_rows - 1));
+    constexpr uint32_t kS = sizeof(cT);
     if constexpr (kPairs) {
         static_assert(sizeof(cT) == 8 && kFull && R % 2 == 0, "pairs: complex64, full tiles");
         constexpr int kJ = kApplyThreadBits + 1;  // row bit of the pair index j
-        const uint32_t tq = tid ^ uint32_t((mlo >> 1) & (kApplyThreads - 1));
-        const uint32_t jm = uint32_t(mlo >> kJ);
-        float4 pr[R / 2];
+        const uint32_t tq = tid ^ ((mlo >> 1) & (kApplyThreads - 1));
+        fvec4 pr[R / 2];
         if (kFar) {
             const cT *far = xv + (base ^ mhi);
             const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<cT *>(far), 0, int(tile_rows * sizeof(cT)), kBufferWord3);
-            const uint32_t voff = tq * uint32_t(2 * sizeof(cT));
+                const_cast<cT *>(far), 0, int(tile_rows * kS), kBufferWord3);
+            const uint32_t jm = mlo >> kJ;
 #pragma unroll
             for (int j = 0; j < R / 2; ++j) {
-                const uint32_t soff = ((uint32_t(j) ^ jm) << kJ) * uint32_t(sizeof(cT));
-                pr[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 0));
+                const uint32_t soff = ((uint32_t(j) ^ jm) << kJ) * kS;
+                pr[j] = __builtin_bit_cast(fvec4, __builtin_amdgcn_raw_buffer_load_b128(rs, tq * 2 * kS, soff, 0));
             }
         } else {
-            const float4 *xrow = reinterpret_cast<const float4 *>(xt) + tq;
+            const uint32_t at = xt + tq * 2 * kS + ((mlo >> kJ) << kJ) * kS;
 #pragma unroll
-            for (int j = 0; j < R / 2; ++j) pr[j] = xrow[(uint32_t(j) ^ jm) << kApplyThreadBits];
+            for (int j = 0; j < R / 2; ++j) pr[j] = lds_load<fvec4>(at ^ ((uint32_t(j) << kJ) * kS));
         }
 #pragma unroll
         for (int j = 0; j < R / 2; ++j) {
-            xg[2 * j] = make_float2(pr[j].x, pr[j].y);
-            xg[2 * j + 1] = make_float2(pr[j].z, pr[j].w);
+            xg[2 * j] = fvec2{pr[j].x, pr[j].y};
+            xg[2 * j + 1] = fvec2{pr[j].z, pr[j].w};
         }
         return;
     }
-    const uint32_t tx = tid ^ uint32_t(mlo & (kApplyThreads - 1));
-    const uint32_t mk = uint32_t(mlo >> kApplyThreadBits);
+    const uint32_t tx = tid ^ (mlo & (kApplyThreads - 1));
+    const uint32_t mk = mlo >> kApplyThreadBits;
     if (kFar) {
         // the partner tile through a buffer resource: the row block's offset
         // is a scalar, the thread's offset one VGPR shared by the R loads
         const cT *far = xv + (base ^ mhi);
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<cT *>(far), 0, int(tile_rows * sizeof(cT)), kBufferWord3);
-        const uint32_t voff = tx * uint32_t(sizeof(cT));
+            const_cast<cT *>(far), 0, int(tile_rows * kS), kBufferWord3);
 #pragma unroll
         for (int k = 0; k < R; ++k) {
             if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
-            const uint32_t soff = ((uint32_t(k) ^ mk) << kApplyThreadBits) * uint32_t(sizeof(cT));
+            const uint32_t soff = ((uint32_t(k) ^ mk) << kApplyThreadBits) * kS;
             if constexpr (sizeof(cT) == 8)
-                xg[k] = __builtin_bit_cast(cT, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 0));
+                xg[k] = __builtin_bit_cast(cT, __builtin_amdgcn_raw_buffer_load_b64(rs, tx * kS, soff, 0));
             else
-                xg[k] = __builtin_bit_cast(cT, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 0));
+                xg[k] = __builtin_bit_cast(cT, __builtin_amdgcn_raw_buffer_load_b128(rs, tx * kS, soff, 0));
         }
     } else {
-        // the thread's column in the LDS tile once, then a uniform row offset
-        const cT *xrow = xt + tx;
+        const uint32_t at = xt + tx * kS + (mk << kApplyThreadBits) * kS;
 #pragma unroll
         for (int k = 0; k < R; ++k) {
             if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
-            xg[k] = xrow[(uint32_t(k) ^ mk) << kApplyThreadBits];
+            xg[k] = lds_load<cT>(at ^ ((uint32_t(k) << kApplyThreadBits) * kS));
         }
     }
 }
 
-// y += D_g(r) x[r ^ m] for the R rows of a thread.  fetch() gathers x into
-// xg (row k's partner in xg[k], or in xg[k ^ 1] with kSwap): first thing for
-// groups with one D per thread, so that the loads fly during the pattern
-// loop; after the per-row D for row-varying groups, so that the gathered
-// registers and the coefficient temporaries are not live together.  D_g is
-// formed from the chunk's pattern coefficients: thread-bit patterns once per
-// thread, then -- for row-varying groups (kRowvar) -- per row the row-bit
-// table entry sU[urow*R + k] and the straddling patterns.  Products go to the
-// FP64 accumulators ar/ai, or (mixed) to the FP32 block partials br/bi; those
-// with Im D only for complex groups (kCplx).
-template <bool kMixed, bool kFull, bool kRowvar, bool kCplx, bool kSwap, int R, typename cT, typename Fetch>
-__device__ __forceinline__ void accumulate(const ApplyGroup &gd, uint32_t tid, uint64_t tile_rows,
-                                           uint32_t zero_row, const double2 *sA, const uint32_t *sZ,
-                                           const double2 *sU, cT (&xg)[R], Fetch fetch, double (&ar)[R],
-                                           double (&ai)[R], float (&br)[R], float (&bi)[R]) {
-    constexpr bool cplx = kCplx;
-    if (!kRowvar) fetch();
-    double cr = 0.0, ci = 0.0;
-    uint32_t p = gd.p0;
-    for (; p + 1 < gd.ps; p += 2) {  // two patterns per step: loads in flight together
-        const double2 a0 = sA[p], a1 = sA[p + 1];
-        const uint32_t f0 = uint32_t(__popc(tid & sZ[p])) << 31;
-        const uint32_t f1 = uint32_t(__popc(tid & sZ[p + 1])) << 31;
-        cr += flip_sign(a0.x, f0);
-        cr += flip_sign(a1.x, f1);
-        if (cplx) {
-            ci += flip_sign(a0.y, f0);
-            ci += flip_sign(a1.y, f1);
-        }
-    }
-    if (p < gd.ps) {
-        const double2 a = sA[p];
-        const uint32_t flip = uint32_t(__popc(tid & sZ[p])) << 31;
-        cr += flip_sign(a.x, flip);
-        if (cplx) ci += flip_sign(a.y, flip);
-    }
-    if (!kRowvar) {
-        // D is the same for the R rows of this thread
-        if (kMixed) {
-            const float fr = float(cr), fi = float(ci);
+// The thread's places in the index words of a part (ApplyPart): nibble shifts
+// of its thread bits 0-2 and 3-5, byte shift of its wave.
+struct TabView {
+    uint32_t sh0, sh1, shw;
+};
+
+__device__ __forceinline__ TabView tab_view(uint32_t tid) {
+    const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
+    return {(tid & 7u) * 4u, ((tid >> 3) & 7u) * 4u, wave * 8u};
+}
+
+// LDS address of the thread's value (row index 0) in a part's table of
+// elements of 2^kLg bytes; row k's is the same XOR byte k of rc.
+template <int kLg>
+__device__ __forceinline__ uint32_t tab_place(const TabView &tv, uint32_t w0, uint32_t w1, uint32_t w2,
+                                              uint32_t tab) {
+    const uint32_t t = ((w0 >> tv.sh0) ^ (w1 >> tv.sh1)) & 15u;
+    return ((t << kLg) + (tab << 2)) ^ ((w2 >> tv.shw) & 0xffu);
+}
+
+// y += D_g(r) x[r ^ m] for the R rows of a thread, in FP64.  fetch() gathers
+// x into xg (row k's partner in xg[k], or in xg[k ^ 1] with kSwap).  D_g is
+// read from the chunk's tables: one value per row, or -- groups without a
+// row-index bit in their patterns -- one per thread; groups of several parts
+// add their parts' values.  kCplx: complex tables; groups with real
+// coefficients skip the products with Im D.  next() loads the next group's
+// descriptor once this one's LDS reads have returned (scalar loads share
+// their counter and return out of order), ahead of the products.
+template <bool kFull, bool kCplx, bool kSwap, int R, typename cT, typename Fetch, typename Next>
+__device__ __forceinline__ void accumulate(const ApplyGroup &gd, const ApplyPart *__restrict__ part,
+                                           uint32_t tid, uint64_t tile_rows, const TabView &tv, cT (&xg)[R],
+                                           Fetch fetch, Next next, double (&ar)[R], double (&ai)[R]) {
+    constexpr int kLg = 3 + int(kCplx);
+    using dT = typename std::conditional<kCplx, dvec2, double>::type;
+    fetch();
+    dT d[R];
+    if (gd.nparts() == 1) {
+        const uint32_t at = tab_place<kLg>(tv, gd.w0, gd.w1, gd.w2, gd.tab());
+        d[0] = lds_load<dT>(at);
+        if (gd.tab_n & kGroupRowvar) {
 #pragma unroll
-            for (int k = 0; k < R; ++k) {
-                if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
-                br[k] = fmaf(fr, xg[k ^ int(kSwap)].x, br[k]);
-                bi[k] = fmaf(fr, xg[k ^ int(kSwap)].y, bi[k]);
-            }
-            if (cplx) {
-#pragma unroll
-                for (int k = 0; k < R; ++k) {
-                    if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
-                    br[k] = fmaf(-fi, xg[k ^ int(kSwap)].y, br[k]);
-                    bi[k] = fmaf(fi, xg[k ^ int(kSwap)].x, bi[k]);
-                }
-            }
+            for (int k = 1; k < R; ++k) d[k] = lds_load<dT>(at ^ uint32_t((gd.rc >> (8 * k)) & 0xffu));
         } else {
 #pragma unroll
-            for (int k = 0; k < R; ++k) {
-                if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
-                ar[k] = fma(cr, xg[k ^ int(kSwap)].x, ar[k]);
-                ai[k] = fma(cr, xg[k ^ int(kSwap)].y, ai[k]);
-            }
-            if (cplx) {
-#pragma unroll
-                for (int k = 0; k < R; ++k) {
-                    if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
-                    ar[k] = fma(-ci, xg[k ^ int(kSwap)].y, ar[k]);
-                    ai[k] = fma(ci, xg[k ^ int(kSwap)].x, ai[k]);
-                }
-            }
+            for (int k = 1; k < R; ++k) d[k] = d[0];
         }
-        return;
-    }
-    // D per row for the row-varying groups (rounded to FP32 in mixed mode),
-    // formed by one of the paths below; a single block of products follows,
-    // so that every path leaves the accumulators in the same registers
-    using dT = typename std::conditional<kMixed, float, double>::type;
-    dT dre[R], dim[R];
-    if (!kFull) {
-#pragma unroll
-        for (int k = 0; k < R; ++k) dre[k] = dim[k] = dT(0);
-    }
-    const double2 *su = sU + (gd.u >= 0 ? uint32_t(gd.u) : zero_row) * R;
-    const uint32_t nst = gd.pk - gd.ps;
-    if (nst <= 2) {
-        // at most two straddling patterns: each one's per-thread coefficient
-        // (the sign of the thread bits applied) is formed once, and per row
-        // only the wave-uniform sign of the row-index bits flips it
-        auto rows = [&](auto nst_t) {
-            constexpr uint32_t kN = decltype(nst_t)::value;
-            double2 aq[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
-            uint32_t zh[2] = {0u, 0u};
-#pragma unroll
-            for (uint32_t j = 0; j < kN; ++j) {
-                const double2 a = sA[gd.ps + j];
-                const uint32_t zl = uint32_t(__builtin_amdgcn_readfirstlane(int(sZ[gd.ps + j])));
-                const uint32_t f = uint32_t(__popc(tid & zl)) << 31;
-                aq[j] = make_double2(flip_sign(a.x, f), flip_sign(a.y, f));
-                zh[j] = zl >> kApplyThreadBits;
-            }
-#pragma unroll
-            for (int k = 0; k < R; ++k) {
-                if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
-                const double2 uk = su[k];
-                double dr = cr + uk.x, di = cplx ? ci + uk.y : 0.0;
-#pragma unroll
-                for (uint32_t j = 0; j < kN; ++j) {
-                    // the row sign is wave-uniform: fma(+-1, a, d) rounds d +- a
-                    // exactly as the add does, with the sign in scalar registers
-                    const double sg = (__popc(uint32_t(k) & zh[j]) & 1u) ? -1.0 : 1.0;
-                    dr = fma(sg, aq[j].x, dr);
-                    if (cplx) di = fma(sg, aq[j].y, di);
-                }
-                dre[k] = dT(dr);
-                if (cplx) dim[k] = dT(di);
-            }
-        };
-        if (nst == 0) rows(std::integral_constant<uint32_t, 0>{});
-        else if (nst == 1) rows(std::integral_constant<uint32_t, 1>{});
-        else rows(std::integral_constant<uint32_t, 2>{});
     } else {
 #pragma unroll
-        for (int k = 0; k < R; ++k) {
-            if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
-            const double2 uk = su[k];
-            double dr = cr + uk.x, di = cplx ? ci + uk.y : 0.0;
-            for (uint32_t q = gd.ps; q < gd.pk; ++q) {
-                const double2 a = sA[q];
-                const uint32_t zl = uint32_t(__builtin_amdgcn_readfirstlane(int(sZ[q])));
-                const uint32_t flip =
-                    uint32_t(__popc(tid & zl) + __popc(uint32_t(k) & (zl >> kApplyThreadBits))) << 31;
-                dr += flip_sign(a.x, flip);
-                if (cplx) di += flip_sign(a.y, flip);
-            }
-            dre[k] = dT(dr);
-            if (cplx) dim[k] = dT(di);
+        for (int k = 0; k < R; ++k) d[k] = dT(0.0);
+        const uint32_t q1 = gd.w0 + gd.nparts();
+        for (uint32_t q = gd.w0; q < q1; ++q) {
+            const ApplyPart ap = part[q];
+            const uint32_t at = tab_place<kLg>(tv, ap.w0, ap.w1, ap.w2, ap.tab);
+#pragma unroll
+            for (int k = 0; k < R; ++k) d[k] += lds_load<dT>(at ^ uint32_t((ap.rc >> (8 * k)) & 0xffu));
         }
     }
-    fetch();
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    next();
+    // (keeps the compiler from sinking the load back to its use)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int k = 0; k < R; ++k) {
         if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
         const cT xb = xg[k ^ int(kSwap)];
-        if (!kMixed) {
-            ar[k] = fma(double(dre[k]), xb.x, ar[k]);
-            ai[k] = fma(double(dre[k]), xb.y, ai[k]);
-            if (cplx) {
-                ar[k] = fma(-double(dim[k]), xb.y, ar[k]);
-                ai[k] = fma(double(dim[k]), xb.x, ai[k]);
-            }
-        } else {
-            br[k] = fmaf(float(dre[k]), xb.x, br[k]);
-            bi[k] = fmaf(float(dre[k]), xb.y, bi[k]);
-            if (cplx) {
-                br[k] = fmaf(-float(dim[k]), xb.y, br[k]);
-                bi[k] = fmaf(float(dim[k]), xb.x, bi[k]);
+        double dr;
+        if constexpr (kCplx) dr = d[k].x;
+        else dr = d[k];
+        ar[k] = fma(dr, double(xb.x), ar[k]);
+        ai[k] = fma(dr, double(xb.y), ai[k]);
+    }
+    if constexpr (kCplx) {
+        if (gd.tab_n & kGroupCplx) {
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                if (!kFull && tid + uint64_t(k) * kApplyThreads >= tile_rows) break;
+                const cT xb = xg[k ^ int(kSwap)];
+                ar[k] = fma(-d[k].y, double(xb.y), ar[k]);
+                ai[k] = fma(d[k].y, double(xb.x), ai[k]);
             }
         }
     }
 }
 
-// y is written once and not read again by the kernel: nontemporal stores, so
-// they do not displace x (which the partner tiles still gather) from the caches.
-template <typename cT>
-__device__ __forceinline__ void store_y(cT *p, cT v) {
-    __builtin_nontemporal_store(v.x, &p->x);
-    __builtin_nontemporal_store(v.y, &p->y);
+// Sum of the kSplit thread groups' accumulators, in thread group 0: a fixed
+// tree, through LDS (kSplit / 2 x R x 256 values at `area`; the block's other
+// uses of it are over).
+template <int kSplit, int R>
+__device__ __forceinline__ void merge_splits(dvec2 *area, uint32_t tid, uint32_t sub, double (&ar)[R],
+                                             double (&ai)[R]) {
+#pragma unroll
+    for (int h = kSplit / 2; h >= 1; h /= 2) {
+        __syncthreads();
+        if (sub >= uint32_t(h) && sub < uint32_t(2 * h)) {
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+                area[(uint32_t(sub - h) * R + k) * kApplyThreads + tid] = dvec2{ar[k], ai[k]};
+        }
+        __syncthreads();
+        if (sub < uint32_t(h)) {
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const dvec2 v = area[(sub * R + k) * kApplyThreads + tid];
+                ar[k] += v.x;
+                ai[k] += v.y;
+            }
+        }
+    }
+}
+
+// The end of a tile: y of the thread's rows, and the block's <x|y> partial.  y is written once and not read again by the
+// kernel: nontemporal stores, so that it does not displace x, which the
+// partner tiles still gather, from the caches.
+// row(l) is the state's row of the tile's row l, x(l) its element.  kAdd: y
+// and the partial are added to (a window pass).
+template <bool kFull, bool kPairs, bool kAdd, int kSplit, int R, typename cT, typename Row, typename X>
+__device__ __forceinline__ void finish_tile(uint32_t tid, uint32_t sub, uint64_t tile_rows, Row row, X x,
+                                            cT *__restrict__ yv, double *__restrict__ partials, double *red, const double (&ar)[R],
+                                            const double (&ai)[R]) {
+    double er = 0.0, ei = 0.0;
+    if (kSplit == 1 || sub == 0) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const uint64_t l = kPairs ? ((uint64_t(tid) << 1) | uint64_t(k & 1) |
+                                         (uint64_t(k >> 1) << (kApplyThreadBits + 1)))
+                                      : tid + uint64_t(k) * kApplyThreads;
+            if (!kFull && l >= tile_rows) break;
+            using eT = decltype(cT{}.x + cT{}.x);
+            if (yv) {
+                if constexpr (kPairs) {
+                    // the pair's two rows in one 16-byte store, at the odd row
+                    if (k & 1) {
+                        fvec4 *at = reinterpret_cast<fvec4 *>(yv + row(l - 1));
+                        fvec4 was = {0.0f, 0.0f, 0.0f, 0.0f};
+                        if (kAdd) was = __builtin_nontemporal_load(at);
+                        __builtin_nontemporal_store(
+                            fvec4{float(ar[k - 1] + was.x), float(ai[k - 1] + was.y), float(ar[k] + was.z),
+                                  float(ai[k] + was.w)}, at);
+                    }
+                } else {
+                    cT *at = yv + row(l);
+                    cT was = {0, 0};
+                    if (kAdd) was = __builtin_nontemporal_load(at);
+                    __builtin_nontemporal_store(cT{eT(ar[k] + was.x), eT(ai[k] + was.y)}, at);
+                }
+            }
+            if (partials) {
+                const cT xr = x(l);
+                const double xa = xr.x, xb = xr.y;
+                er = fma(xa, ar[k], er); er = fma(xb, ai[k], er);
+                ei = fma(xa, ai[k], ei); ei = fma(-xb, ar[k], ei);
+            }
+        }
+    }
+    if (partials) {
+        __syncthreads();  // red shares LDS with the tables
+        const double a = wave_sum(er), b = wave_sum(ei);
+        if (sub == 0 && (tid & 63) == 0) {
+            red[2 * (tid / 64)] = a;
+            red[2 * (tid / 64) + 1] = b;
+        }
+        __syncthreads();
+        if (sub == 0 && tid == 0) {
+            double s0 = 0.0, s1 = 0.0;
+            for (int w = 0; w < kApplyThreads / 64; ++w) { s0 += red[2 * w]; s1 += red[2 * w + 1]; }
+            double *at = partials + 2 * uint64_t(blockIdx.x);
+            at[0] = kAdd ? at[0] + s0 : s0;
+            at[1] = kAdd ? at[1] + s1 : s1;
+        }
+    }
 }
 
 // A_p = sum_t (-1)^popcount(base & z_t) c'_t over the pattern's terms
@@ -413,228 +425,12 @@ __device__ __forceinline__ double2 pattern_coeff(uint64_t base, uint32_t t0, uin
     return make_double2(a_r, a_i);
 }
 
-// LDS layout of k_apply_tiled: x tile | sA[max_p] | sZ[max_p] | sU[max_u * R]
-template <typename cT>
-__host__ __device__ inline size_t apply_lds_offsets(uint64_t tile_rows, uint32_t max_p, uint32_t R,
-                                                    uint32_t max_u, size_t *oA, size_t *oZ,
-                                                    size_t *oU) {
-    const size_t a = (size_t(tile_rows) * sizeof(cT) + 15) & ~size_t(15);
-    const size_t z = a + size_t(max_p) * sizeof(double2);
-    const size_t u = (z + size_t(max_p) * sizeof(uint32_t) + 15) & ~size_t(15);
-    if (oA) *oA = a;
-    if (oZ) *oZ = z;
-    if (oU) *oU = u;
-    return u + size_t(max_u) * R * sizeof(double2);
+// LDS: x tile (gather form) or two tile buffers (partner-staged form) |
+// tables; at the end the split's sums and the <x|y> partials take it over.
+__host__ __device__ inline size_t apply_lds_bytes(size_t tiles, uint32_t max_tab, size_t merge) {
+    const size_t all = tiles + ((size_t(max_tab) + 15) & ~size_t(15));
+    return all > merge + 64 ? all : merge + 64;
 }
-
-// Per-chunk LDS tables of a tile: the pattern coefficients
-// sA[p] = A_p = sum_t (-1)^popcount(base & z_t) c'_t with their low z bits
-// sZ[p], then the row-bit table sU[u*R + k] = sum over the row-bit patterns of
-// the group of (-1)^popcount(k & (zl >> thread bits)) * A_p; row zero_row
-// stays zero for groups without such patterns.  Ends with a barrier.
-template <bool kNarrow, int R>
-__device__ __forceinline__ void chunk_tables(const ApplyChunk &ch, uint32_t tid, uint64_t base,
-                                             uint32_t zero_row, const ApplyGroup *__restrict__ grp,
-                                             const uint32_t *__restrict__ ug,
-                                             const uint32_t *__restrict__ pzl,
-                                             const uint32_t *__restrict__ ptptr,
-                                             const uint64_t *__restrict__ ptz,
-                                             const double2 *__restrict__ ptc, double2 *sA,
-                                             uint32_t *sZ, double2 *sU) {
-    for (uint32_t p = tid; p < ch.p1 - ch.p0; p += kApplyThreads) {
-        const uint32_t pa = ch.p0 + p;
-        sA[p] = pattern_coeff<kNarrow>(base, ptptr[pa], ptptr[pa + 1], ptz, ptc);
-        sZ[p] = pzl[pa];
-    }
-    __syncthreads();
-    for (uint32_t i = tid; i < (ch.u1 - ch.u0 + 1) * R; i += kApplyThreads) {
-        const uint32_t u = i / R, k = i % R;
-        double s_r = 0.0, s_i = 0.0;
-        if (u < ch.u1 - ch.u0) {
-            const ApplyGroup &gg = grp[ug[ch.u0 + u]];
-            for (uint32_t p = gg.pk; p < gg.p1; ++p) {
-                const double2 a = sA[p];
-                if (__popc(k & (sZ[p] >> kApplyThreadBits)) & 1u) { s_r -= a.x; s_i -= a.y; }
-                else { s_r += a.x; s_i += a.y; }
-            }
-        }
-        sU[(u < ch.u1 - ch.u0 ? u : zero_row) * R + k] = make_double2(s_r, s_i);
-    }
-    __syncthreads();
-}
-
-template <bool kMixed, bool kNarrow, bool kFull, int kL>
-__global__ __launch_bounds__(kApplyThreads) void k_apply_tiled(
-    uint64_t N, uint32_t ntiles, uint32_t tiles_per_xcd, uint32_t ngrp, uint32_t nchunk,
-    uint32_t max_p, uint32_t zero_row, const ApplyGroup *__restrict__ grp, const ApplyChunk *__restrict__ chunks,
-    const uint32_t *__restrict__ ug, const uint32_t *__restrict__ pzl,
-    const uint32_t *__restrict__ ptptr, const uint64_t *__restrict__ ptz,
-    const double2 *__restrict__ ptc, const void *__restrict__ xin, void *__restrict__ yout,
-    double *__restrict__ partials) {
-    using Shape = ApplyShape<kMixed, kL>;
-    constexpr int L = Shape::L, R = Shape::R;
-    // complex64 full tiles: paired rows (see gather); the patterns are built
-    // in the paired-row bit order to match
-    constexpr bool kPairs = kMixed && kFull;
-    using cT = typename std::conditional<kMixed, float2, double2>::type;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-
-    const uint32_t tid = threadIdx.x;
-    const uint32_t v = blockIdx.x / ntiles;
-    uint32_t tile = blockIdx.x % ntiles;
-    if (tiles_per_xcd) tile = (tile % 8) * tiles_per_xcd + tile / 8;
-    const uint64_t tile_rows = kFull ? (uint64_t(1) << L) : (N < (uint64_t(1) << L) ? N : (uint64_t(1) << L));
-    const uint64_t base = uint64_t(tile) * tile_rows;
-    const cT *__restrict__ xv = reinterpret_cast<const cT *>(xin) + uint64_t(v) * N;
-
-    size_t oA, oZ, oU;
-    apply_lds_offsets<cT>(tile_rows, max_p, R, 0, &oA, &oZ, &oU);
-    cT *xt = reinterpret_cast<cT *>(smem_raw);
-    double2 *sA = reinterpret_cast<double2 *>(smem_raw + oA);
-    uint32_t *sZ = reinterpret_cast<uint32_t *>(smem_raw + oZ);
-    double2 *sU = reinterpret_cast<double2 *>(smem_raw + oU);
-
-    for (uint64_t i = tid; i < tile_rows; i += kApplyThreads) xt[i] = xv[base + i];
-
-    // accumulators: FP64 (ar, ai) or FP32 running sum s, compensation c, block partial b
-    double ar[R], ai[R];
-    float sr[R], si[R], br[R], bi[R];
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        ar[k] = ai[k] = 0.0;
-        sr[k] = si[k] = br[k] = bi[k] = 0.0f;
-    }
-
-    uint32_t since_flush = 0;  // groups in the FP32 block partials
-    // add the FP32 block partials into the running sums with TwoSum
-    auto flush = [&]() {
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            float e, f;
-            two_sum(sr[k], br[k], sr[k], e);
-            two_sum(si[k], bi[k], si[k], f);
-            br[k] = e;  // the rounding error starts the next block partial
-            bi[k] = f;
-        }
-    };
-    cT xg[R];
-    for (uint32_t c = 0; c < nchunk; ++c) {
-        const ApplyChunk ch = chunks[c];
-        if (c) __syncthreads();  // the previous chunk's tables are no longer read
-        chunk_tables<kNarrow, R>(ch, tid, base, zero_row, grp, ug, pzl, ptptr, ptz, ptc, sA, sZ, sU);
-        // one loop per group class, each with a single straight path, in
-        // blocks of at most kCompBlock groups flushed after each block
-        auto run_class = [&](auto far_t, auto rowvar_t, auto cplx_t, auto swap_t, uint32_t g0, uint32_t g1) {
-            constexpr bool kFar = decltype(far_t)::value, kRowvar = decltype(rowvar_t)::value;
-            constexpr bool kCplx = decltype(cplx_t)::value, kSwap = decltype(swap_t)::value;
-            for (uint32_t gb = g0; gb < g1;) {
-                // up to the next flush point, counted over all classes
-                const uint32_t room = uint32_t(kCompBlock) - since_flush;
-                const uint32_t ge = g1 - gb > room ? gb + room : g1;
-                for (uint32_t g = gb; g < ge; ++g) {
-                    const ApplyGroup gd = grp[g];
-                    // all descriptor fields in SGPRs before the gathers are issued,
-                    // so that no later scalar-load wait also waits for them
-                    asm volatile("" ::"s"(gd.p0), "s"(gd.ps), "s"(gd.pk), "s"(gd.p1), "s"(gd.u),
-                                 "s"(gd.flags));
-                    const auto fetch = [&]() {
-                        gather<kFar, kFull, kPairs, R>(gd.m, tid, tile_rows, base, xt, xv, xg);
-                    };
-                    accumulate<kMixed, kFull, kRowvar, kCplx, kSwap, R>(gd, tid, tile_rows, zero_row, sA, sZ,
-                                                                        sU, xg, fetch, ar, ai, br, bi);
-                }
-                since_flush += ge - gb;
-                gb = ge;
-                // reset in both precisions: room must stay >= 1 for the loop to advance
-                if (since_flush == uint32_t(kCompBlock)) {
-                    if (kMixed) flush();
-                    since_flush = 0;
-                }
-            }
-        };
-        using F = std::false_type;
-        using T = std::true_type;
-        run_class(F{}, F{}, F{}, F{}, ch.cg[0], ch.cg[1]);
-        run_class(T{}, F{}, F{}, F{}, ch.cg[1], ch.cg[2]);
-        run_class(F{}, T{}, F{}, F{}, ch.cg[2], ch.cg[3]);
-        run_class(T{}, T{}, F{}, F{}, ch.cg[3], ch.cg[4]);
-        run_class(F{}, F{}, T{}, F{}, ch.cg[4], ch.cg[5]);
-        run_class(T{}, F{}, T{}, F{}, ch.cg[5], ch.cg[6]);
-        run_class(F{}, T{}, T{}, F{}, ch.cg[6], ch.cg[7]);
-        run_class(T{}, T{}, T{}, F{}, ch.cg[7], ch.cg[8]);
-        if constexpr (kPairs) {
-            // masks with row bit 0: each row's partner is the other half of its pair
-            run_class(F{}, F{}, F{}, T{}, ch.cg[8], ch.cg[9]);
-            run_class(T{}, F{}, F{}, T{}, ch.cg[9], ch.cg[10]);
-            run_class(F{}, T{}, F{}, T{}, ch.cg[10], ch.cg[11]);
-            run_class(T{}, T{}, F{}, T{}, ch.cg[11], ch.cg[12]);
-            run_class(F{}, F{}, T{}, T{}, ch.cg[12], ch.cg[13]);
-            run_class(T{}, F{}, T{}, T{}, ch.cg[13], ch.cg[14]);
-            run_class(F{}, T{}, T{}, T{}, ch.cg[14], ch.cg[15]);
-            run_class(T{}, T{}, T{}, T{}, ch.cg[15], ch.cg[16]);
-        }
-    }
-
-    if (kMixed && since_flush) flush();
-    double er = 0.0, ei = 0.0;
-    cT *__restrict__ yv = yout ? reinterpret_cast<cT *>(yout) + uint64_t(v) * N : nullptr;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const uint64_t l = kPairs ? ((uint64_t(tid) << 1) | uint64_t(k & 1) |
-                                     (uint64_t(k >> 1) << (kApplyThreadBits + 1)))
-                                  : tid + uint64_t(k) * kApplyThreads;
-        if (!kFull && l >= tile_rows) break;
-        double yr, yi;
-        if (!kMixed) {
-            yr = ar[k];
-            yi = ai[k];
-            if (yv) store_y(reinterpret_cast<double2 *>(yv) + base + l, make_double2(yr, yi));
-        } else {
-            yr = double(sr[k]) + double(br[k]);
-            yi = double(si[k]) + double(bi[k]);
-            if (yv) {
-                if constexpr (kPairs) {
-                    // the pair's two rows in one 16-byte store, at the odd row
-                    if (k & 1) {
-                        typedef float f4v __attribute__((ext_vector_type(4)));
-                        const f4v pv = {sr[k - 1] + br[k - 1], si[k - 1] + bi[k - 1],
-                                        sr[k] + br[k], si[k] + bi[k]};
-                        __builtin_nontemporal_store(
-                            pv, reinterpret_cast<f4v *>(reinterpret_cast<float2 *>(yv) + base + l - 1));
-                    }
-                } else {
-                    store_y(reinterpret_cast<float2 *>(yv) + base + l,
-                            make_float2(sr[k] + br[k], si[k] + bi[k]));
-                }
-            }
-        }
-        if (partials) {
-            const cT xr = xt[l];
-            const double xa = xr.x, xb = xr.y;
-            er = fma(xa, yr, er); er = fma(xb, yi, er);
-            ei = fma(xa, yi, ei); ei = fma(-xb, yr, ei);
-        }
-    }
-    if (partials) {
-        __shared__ double red[kApplyThreads / 64][2];
-        const double a = wave_sum(er), b = wave_sum(ei);
-        if ((tid & 63) == 0) { red[tid / 64][0] = a; red[tid / 64][1] = b; }
-        __syncthreads();
-        if (tid == 0) {
-            double s0 = 0.0, s1 = 0.0;
-            for (int w = 0; w < kApplyThreads / 64; ++w) { s0 += red[w][0]; s1 += red[w][1]; }
-            partials[2 * uint64_t(blockIdx.x)] = s0;
-            partials[2 * uint64_t(blockIdx.x) + 1] = s1;
-        }
-    }
-}
-
-// Partner-staged form of k_apply_tiled (full tiles only).  Instead of one
-// tile of x in LDS and far gathers from global memory, two tile buffers take
-// the partner tiles t ^ hi in turn, one per run of groups sharing hi (hi = 0:
-// the tile itself), so a partner tile is read once per chunk however many
-// groups use it.  The load of run r + 1 (LDS-DMA: global memory straight into
-// LDS, no registers) is in flight while run r is computed.
 
 // One LDS-DMA load: each lane reads the 16 bytes at its `src`, and the wave
 // writes them to LDS at lds + lane * 16 (lds: LDS byte address, wave-uniform,
@@ -660,110 +456,231 @@ __device__ __forceinline__ void lds_dma16(const void *src, uint32_t lds) {
         : "memory");
 }
 
-typedef __attribute__((address_space(3))) unsigned char lds_byte;
+// v of the lane whose number differs in bit `kBit` of the 16 lanes of a DPP
+// row: XOR 1 and 2 are quad permutations, XOR 4 and 8 a mirror (XOR 7 of 8
+// lanes, 15 of 16) undone on the lower bits.
+template <int kBit>
+__device__ __forceinline__ double row_xor(double v) {
+    auto dpp = [](int w) {
+        auto mov = [](int x, auto ctrl) {
+            return __builtin_amdgcn_update_dpp(0, x, decltype(ctrl)::value, 0xf, 0xf, true);
+        };
+        using Xor1 = std::integral_constant<int, 0xB1>;    // quad_perm [1, 0, 3, 2]
+        using Xor2 = std::integral_constant<int, 0x4E>;    // quad_perm [2, 3, 0, 1]
+        using Xor3 = std::integral_constant<int, 0x1B>;    // quad_perm [3, 2, 1, 0]
+        using Xor15 = std::integral_constant<int, 0x140>;  // row_mirror
+        using Xor7 = std::integral_constant<int, 0x141>;   // row_half_mirror
+        if constexpr (kBit == 1) return mov(w, Xor1{});
+        else if constexpr (kBit == 2) return mov(w, Xor2{});
+        else if constexpr (kBit == 4) return mov(mov(w, Xor7{}), Xor3{});
+        else return mov(mov(w, Xor15{}), Xor7{});
+    };
+    return __hiloint2double(dpp(__double2hiint(v)), dpp(__double2loint(v)));
+}
 
-template <bool kMixed, bool kNarrow, int kL>
-__global__ __launch_bounds__(kApplyThreads) void k_apply_staged(
-    uint64_t N, uint32_t ntiles, uint32_t tiles_per_xcd, uint32_t nchunk, uint32_t nrun,
-    uint32_t max_p, uint32_t zero_row, const ApplyGroup *__restrict__ grp,
-    const ApplyChunk *__restrict__ chunks, const ApplyRun *__restrict__ runs,
-    const uint32_t *__restrict__ ug, const uint32_t *__restrict__ pzl,
-    const uint32_t *__restrict__ ptptr, const uint64_t *__restrict__ ptz,
+// Per-chunk LDS tables of a tile, 16 lanes per part: lane c forms
+// A_c = sum_t (-1)^popcount(base & z_t) c'_t of the part's pattern of code c,
+// and a Walsh-Hadamard transform over the lanes turns the A_c into the
+// table's entries, entry e = sum_c (-1)^popcount(e & c) A_c.  Ends with a wait
+// for the wave's own global loads and a barrier.
+template <bool kNarrow, bool kCplx, uint32_t kThreads>
+__device__ __forceinline__ void chunk_tables(const ApplyChunk &ch, uint32_t t, uint64_t base,
+                                             const uint32_t *__restrict__ tab,
+                                             const ApplyRange *__restrict__ pat,
+                                             const uint64_t *__restrict__ ptz,
+                                             const double2 *__restrict__ ptc, unsigned char *smem) {
+    const uint32_t c = t & 15u;
+    // (the lanes of a part stay in the loop together)
+    for (uint32_t i = ch.t0 + t / 16u; i < ch.t1; i += kThreads / 16) {
+        const ApplyRange pr = pat[16 * uint64_t(i) + c];
+        const uint32_t place = tab[i];
+        double2 v = pattern_coeff<kNarrow>(base, pr.t0, pr.t1, ptz, ptc);
+        auto stage = [&](auto bit_t) {
+            constexpr int kBit = decltype(bit_t)::value;
+            const double ox = row_xor<kBit>(v.x);
+            v.x = ox + ((c & kBit) ? -v.x : v.x);
+            if (kCplx) {
+                const double oy = row_xor<kBit>(v.y);
+                v.y = oy + ((c & kBit) ? -v.y : v.y);
+            }
+        };
+        stage(std::integral_constant<int, 1>{});
+        stage(std::integral_constant<int, 2>{});
+        stage(std::integral_constant<int, 4>{});
+        stage(std::integral_constant<int, 8>{});
+        if (c < (place >> 16)) {
+            unsigned char *at = smem + 4u * (place & 0xffffu);
+            if (!kCplx) reinterpret_cast<double *>(at)[c] = v.x;
+            else reinterpret_cast<double2 *>(at)[c] = v;
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): LDS-DMA of the caller's tile
+    __syncthreads();
+}
+
+// kWin: a window pass (ApplyWindow), whose groups all gather inside the tile.
+template <bool kMixed, bool kNarrow, bool kCplx, bool kFull, int kL, int kSplit, bool kWin>
+__global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
+    uint64_t N, ApplyWindow win, uint32_t ntiles, uint32_t tiles_per_xcd, uint32_t nchunk,
+    const ApplyGroup *__restrict__ grp, const ApplyChunk *__restrict__ chunks,
+    const ApplyPart *__restrict__ part, const uint32_t *__restrict__ tab,
+    const ApplyRange *__restrict__ pat, const uint64_t *__restrict__ ptz,
     const double2 *__restrict__ ptc, const void *__restrict__ xin, void *__restrict__ yout,
     double *__restrict__ partials) {
     using Shape = ApplyShape<kMixed, kL>;
     constexpr int L = Shape::L, R = Shape::R;
-    using cT = typename std::conditional<kMixed, float2, double2>::type;
-    constexpr uint64_t tile_rows = uint64_t(1) << L;
-    constexpr uint32_t kStageTileBytes = uint32_t(Shape::kTile);  // one stage buffer: one tile
-    constexpr uint32_t kLoads = kStageTileBytes / (16u * kApplyThreads);  // 16-byte loads per thread
-    static_assert(tile_rows * sizeof(cT) == kStageTileBytes, "a tile fills one stage buffer");
-    static_assert(kStageTileBytes % (16u * kApplyThreads) == 0, "tile must split into 16-byte loads");
-    __shared__ __align__(16) unsigned char bufs[2 * kStageTileBytes];
-    extern __shared__ __align__(16) unsigned char smem_raw[];
+    // complex64 full tiles: paired rows (see gather); the patterns are built
+    // in the paired-row bit order to match
+    constexpr bool kPairs = kMixed && kFull;
+    using cT = typename std::conditional<kMixed, fvec2, dvec2>::type;
+    extern __shared__ __align__(256) unsigned char smem_raw[];
 
-    const uint32_t tid = threadIdx.x;
-    const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid / 64)));
+    const uint32_t tid = threadIdx.x % kApplyThreads;
+    const uint32_t sub =
+        kSplit == 1 ? 0u : uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x / kApplyThreads)));
+    const uint32_t v = blockIdx.x / ntiles;
+    uint32_t tile = blockIdx.x % ntiles;
+    if (tiles_per_xcd) tile = (tile % 8) * tiles_per_xcd + tile / 8;
+    const uint64_t tile_rows = kFull ? (uint64_t(1) << L) : (N < (uint64_t(1) << L) ? N : (uint64_t(1) << L));
+    // the tile's row 0, and row l of it
+    uint64_t base = uint64_t(tile) * tile_rows;
+    if (kWin) {
+        const uint32_t mid = win.s - win.f;  // tile index bits below the window
+        base = (uint64_t(tile & ((1u << mid) - 1u)) << win.f) | (uint64_t(tile >> mid) << (win.s + L - win.f));
+    }
+    auto row = [&](uint64_t l) {
+        return kWin ? base + ((l & ((1u << win.f) - 1u)) | ((l >> win.f) << win.s)) : base + l;
+    };
+    const cT *__restrict__ xv = reinterpret_cast<const cT *>(xin) + uint64_t(v) * N;
+
+    cT *xt = reinterpret_cast<cT *>(smem_raw);
+    const uint32_t lds0 = uint32_t(uintptr_t((lds_byte *)smem_raw));
+    const TabView tv = tab_view(tid);
+
+    // the tile: straight into LDS, 16 bytes per lane, in flight while the
+    // first chunk's tables are formed
+    if constexpr (kFull) {
+        constexpr uint32_t kThreads = kApplyThreads * kSplit, kPer = 16 / sizeof(cT);
+        const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x / 64)));
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t(Shape::kTile) - 1) / (16 * kThreads) + 1; ++i) {
+            const uint32_t off = (i * kThreads + wave * 64u) * 16u;
+            if (Shape::kTile % (16u * kThreads) != 0 && off >= Shape::kTile) break;
+            lds_dma16(xv + row((off / 16u + threadIdx.x % 64u) * kPer), lds0 + off);
+        }
+    } else {
+        for (uint64_t i = threadIdx.x; i < tile_rows; i += kApplyThreads * kSplit) xt[i] = xv[row(i)];
+    }
+
+    double ar[R], ai[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) ar[k] = ai[k] = 0.0;
+    cT xg[R];
+    for (uint32_t c = 0; c < nchunk; ++c) {
+        const ApplyChunk ch = chunks[c];
+        if (c) __syncthreads();  // the previous chunk's tables are no longer read
+        chunk_tables<kNarrow, kCplx, kApplyThreads * kSplit>(ch, threadIdx.x, base, tab, pat, ptz, ptc,
+                                                             smem_raw);
+        auto run_class = [&](auto far_t, auto swap_t, int cls) {
+            constexpr bool kFar = decltype(far_t)::value, kSwap = decltype(swap_t)::value;
+            const uint32_t g1 = ch.cg[cls + 1];
+            // thread group `sub` takes every kSplit-th group of the chunk
+            uint32_t g = ch.cg[cls] + (kSplit == 1 ? 0u : (sub - (ch.cg[cls] - ch.cg[0])) % kSplit);
+            if (g >= g1) return;
+            ApplyGroup nx = grp[g];
+            do {
+                const ApplyGroup gd = nx;
+                // all descriptor fields in SGPRs before the gathers are issued,
+                // so that no later scalar-load wait also waits for them
+                asm volatile("" ::"s"(gd.m), "s"(gd.w0), "s"(gd.w1), "s"(gd.w2), "s"(gd.tab_n), "s"(gd.rc));
+                g += kSplit;
+                const auto fetch = [&]() {
+                    gather<kFar, kFull, kPairs, R>(gd.m, tid, tile_rows, base, lds0, xv, xg);
+                };
+                const auto next = [&]() { nx = grp[g < g1 ? g : g1 - 1]; };
+                accumulate<kFull, kCplx, kSwap, R>(gd, part, tid, tile_rows, tv, xg, fetch, next, ar, ai);
+            } while (g < g1);
+        };
+        using F = std::false_type;
+        using T = std::true_type;
+        run_class(F{}, F{}, 0);
+        if constexpr (kPairs) run_class(F{}, T{}, 1);
+        if constexpr (!kWin) {
+            run_class(T{}, F{}, 2);
+            if constexpr (kPairs) run_class(T{}, T{}, 3);
+        }
+    }
+    if (kSplit > 1) merge_splits<kSplit, R>(reinterpret_cast<dvec2 *>(smem_raw), tid, sub, ar, ai);
+    // x from the tile in LDS, or from global memory where the merge used it
+    const auto x = [&](uint64_t l) { return kSplit == 1 ? xt[l] : xv[row(l)]; };
+    finish_tile<kFull, kPairs, kWin, kSplit, R, cT>(tid, sub, tile_rows, row, x,
+                                              yout ? reinterpret_cast<cT *>(yout) + uint64_t(v) * N : nullptr,
+                                              partials, reinterpret_cast<double *>(smem_raw), ar, ai);
+}
+
+// Partner-staged form of k_apply_tiled (full tiles only).  Instead of one
+// tile of x in LDS and far gathers from global memory, two tile buffers take
+// the partner tiles t ^ hi in turn, one per run of groups sharing hi (hi = 0:
+// the tile itself), so a partner tile is read once per chunk however many
+// groups use it.  The load of run r + 1 (LDS-DMA: global memory straight into
+// LDS, no registers) is in flight while run r is computed.
+
+template <bool kMixed, bool kNarrow, bool kCplx, int kL, int kSplit>
+__global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_staged(
+    uint64_t N, uint32_t ntiles, uint32_t tiles_per_xcd, uint32_t nchunk, uint32_t nrun,
+    const ApplyGroup *__restrict__ grp,
+    const ApplyChunk *__restrict__ chunks, const ApplyRun *__restrict__ runs,
+    const ApplyPart *__restrict__ part, const uint32_t *__restrict__ tab,
+    const ApplyRange *__restrict__ pat, const uint64_t *__restrict__ ptz,
+    const double2 *__restrict__ ptc, const void *__restrict__ xin, void *__restrict__ yout,
+    double *__restrict__ partials) {
+    using Shape = ApplyShape<kMixed, kL>;
+    constexpr int L = Shape::L, R = Shape::R;
+    using cT = typename std::conditional<kMixed, fvec2, dvec2>::type;
+    constexpr uint64_t tile_rows = uint64_t(1) << L;
+    constexpr uint32_t kThreads = kApplyThreads * kSplit;
+    constexpr uint32_t kStageTileBytes = uint32_t(Shape::kTile);  // one stage buffer: one tile
+    constexpr uint32_t kLoads = (kStageTileBytes - 1) / (16u * kThreads) + 1;  // 16-byte loads per thread
+    static_assert(tile_rows * sizeof(cT) == kStageTileBytes, "a tile fills one stage buffer");
+    static_assert(kStageTileBytes % 1024 == 0, "tile must split into the waves' 16-byte loads");
+    extern __shared__ __align__(256) unsigned char smem_raw[];
+
+    const uint32_t tid = threadIdx.x % kApplyThreads;
+    const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x / 64)));
+    const uint32_t sub = kSplit == 1 ? 0u : wave / (kApplyThreads / 64);
     const uint32_t v = blockIdx.x / ntiles;
     uint32_t tile = blockIdx.x % ntiles;
     if (tiles_per_xcd) tile = (tile % 8) * tiles_per_xcd + tile / 8;
     const uint64_t base = uint64_t(tile) * tile_rows;
     const cT *__restrict__ xv = reinterpret_cast<const cT *>(xin) + uint64_t(v) * N;
 
-    size_t oA, oZ, oU;
-    apply_lds_offsets<cT>(0, max_p, R, 0, &oA, &oZ, &oU);
-    double2 *sA = reinterpret_cast<double2 *>(smem_raw + oA);
-    uint32_t *sZ = reinterpret_cast<uint32_t *>(smem_raw + oZ);
-    double2 *sU = reinterpret_cast<double2 *>(smem_raw + oU);
+    const uint32_t lds0 = uint32_t(uintptr_t((lds_byte *)smem_raw));
+    const TabView tv = tab_view(tid);
 
     // partner tile base ^ hi into buffer b: each wave fills 1 KB per load,
     // lane i the 16 bytes at i * 16
-    const uint32_t lds_bufs = uint32_t(uintptr_t((lds_byte *)bufs));  // LDS address of bufs
     auto stage = [&](uint64_t hi, uint32_t b) {
         const unsigned char *src = reinterpret_cast<const unsigned char *>(xv + (base ^ hi));
 #pragma unroll
         for (uint32_t j = 0; j < kLoads; ++j) {
-            const uint32_t off = (j * kApplyThreads + wave * 64u) * 16u;
-            lds_dma16(src + off + (tid % 64u) * 16u, lds_bufs + b * kStageTileBytes + off);
+            const uint32_t off = (j * kThreads + wave * 64u) * 16u;
+            if (kStageTileBytes % (16u * kThreads) != 0 && off >= kStageTileBytes) break;
+            lds_dma16(src + off + (threadIdx.x % 64u) * 16u, lds0 + b * kStageTileBytes + off);
         }
     };
 
     double ar[R], ai[R];
-    float sr[R], si[R], br[R], bi[R];
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-        ar[k] = ai[k] = 0.0;
-        sr[k] = si[k] = br[k] = bi[k] = 0.0f;
-    }
-    uint32_t since_flush = 0;
-    auto flush = [&]() {
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            float e, f;
-            two_sum(sr[k], br[k], sr[k], e);
-            two_sum(si[k], bi[k], si[k], f);
-            br[k] = e;  // the rounding error starts the next block partial
-            bi[k] = f;
-        }
-    };
+    for (int k = 0; k < R; ++k) ar[k] = ai[k] = 0.0;
     cT xg[R];
-    // the groups of one run, all gathering from the tile in `xt`
-    auto run_groups = [&](const ApplyRun &run, const cT *xt) {
-        auto run_class = [&](auto rowvar_t, auto cplx_t, uint32_t g0, uint32_t g1) {
-            constexpr bool kRowvar = decltype(rowvar_t)::value;
-            constexpr bool kCplx = decltype(cplx_t)::value;
-            for (uint32_t gb = g0; gb < g1;) {
-                const uint32_t room = uint32_t(kCompBlock) - since_flush;
-                const uint32_t ge = g1 - gb > room ? gb + room : g1;
-                for (uint32_t g = gb; g < ge; ++g) {
-                    const ApplyGroup gd = grp[g];
-                    asm volatile("" ::"s"(gd.p0), "s"(gd.ps), "s"(gd.pk), "s"(gd.p1), "s"(gd.u),
-                                 "s"(gd.flags));
-                    const auto fetch = [&]() { gather<false, true, false, R>(gd.m, tid, tile_rows, base, xt, xv, xg); };
-                    accumulate<kMixed, true, kRowvar, kCplx, false, R>(gd, tid, tile_rows, zero_row, sA, sZ,
-                                                                       sU, xg, fetch, ar, ai, br, bi);
-                }
-                since_flush += ge - gb;
-                gb = ge;
-                if (since_flush == uint32_t(kCompBlock)) {
-                    if (kMixed) flush();
-                    since_flush = 0;
-                }
-            }
-        };
-        using F = std::false_type;
-        using T = std::true_type;
-        run_class(F{}, F{}, run.g[0], run.g[1]);
-        run_class(T{}, F{}, run.g[1], run.g[2]);
-        run_class(F{}, T{}, run.g[2], run.g[3]);
-        run_class(T{}, T{}, run.g[3], run.g[4]);
-    };
     if (nrun) stage(runs[0].hi, 0);
-    uint32_t r = 0;
+    uint32_t r = 0, g = sub;
+    const uint32_t glast = nrun ? runs[nrun - 1].g1 - 1 : 0;
+    ApplyGroup nx = grp[g < glast ? g : glast];
     for (uint32_t c = 0; c < nchunk; ++c) {
         const ApplyChunk ch = chunks[c];
         if (c) __syncthreads();  // the previous chunk's tables are no longer read
-        chunk_tables<kNarrow, R>(ch, tid, base, zero_row, grp, ug, pzl, ptptr, ptz, ptc, sA, sZ, sU);
+        chunk_tables<kNarrow, kCplx, kThreads>(ch, threadIdx.x, base, tab, pat, ptz, ptc, smem_raw);
         for (; r < ch.r1; ++r) {
             // run r's tile has landed (each wave waits for its own loads, the
             // barrier for all of them), and no wave still reads run r - 1's
@@ -771,49 +688,27 @@ __global__ __launch_bounds__(kApplyThreads) void k_apply_staged(
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
             __syncthreads();
             if (r + 1 < nrun) stage(runs[r + 1].hi, (r + 1) & 1u);
-            run_groups(runs[r], reinterpret_cast<const cT *>(bufs + (r & 1u) * kStageTileBytes));
+            // the run's groups (every kSplit-th), gathering from that tile
+            const uint32_t g1 = runs[r].g1, xt = lds0 + (r & 1u) * kStageTileBytes;
+            while (g < g1) {
+                const ApplyGroup gd = nx;
+                asm volatile("" ::"s"(gd.m), "s"(gd.w0), "s"(gd.w1), "s"(gd.w2), "s"(gd.tab_n), "s"(gd.rc));
+                g += kSplit;
+                const auto fetch = [&]() {
+                    gather<false, true, false, R>(gd.m, tid, tile_rows, base, xt, xv, xg);
+                };
+                const auto next = [&]() { nx = grp[g < glast ? g : glast]; };
+                accumulate<true, kCplx, false, R>(gd, part, tid, tile_rows, tv, xg, fetch, next, ar, ai);
+            }
         }
     }
-    if (kMixed && since_flush) flush();
-
-    // y, and <x|y> with x of the thread's rows read from global memory (the
-    // buffers hold partner tiles)
-    constexpr bool kFull = true;
-    double er = 0.0, ei = 0.0;
-    cT *__restrict__ yv = yout ? reinterpret_cast<cT *>(yout) + uint64_t(v) * N : nullptr;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const uint64_t l = tid + uint64_t(k) * kApplyThreads;
-        if (!kFull && l >= tile_rows) break;
-        double yr, yi;
-        if (!kMixed) {
-            yr = ar[k];
-            yi = ai[k];
-            if (yv) store_y(reinterpret_cast<double2 *>(yv) + base + l, make_double2(yr, yi));
-        } else {
-            yr = double(sr[k]) + double(br[k]);
-            yi = double(si[k]) + double(bi[k]);
-            if (yv) store_y(reinterpret_cast<float2 *>(yv) + base + l, make_float2(sr[k] + br[k], si[k] + bi[k]));
-        }
-        if (partials) {
-            const cT xr = xv[base + l];
-            const double xa = xr.x, xb = xr.y;
-            er = fma(xa, yr, er); er = fma(xb, yi, er);
-            ei = fma(xa, yi, ei); ei = fma(-xb, yr, ei);
-        }
-    }
-    if (partials) {
-        __shared__ double red[kApplyThreads / 64][2];
-        const double a = wave_sum(er), b = wave_sum(ei);
-        if ((tid & 63) == 0) { red[tid / 64][0] = a; red[tid / 64][1] = b; }
-        __syncthreads();
-        if (tid == 0) {
-            double s0 = 0.0, s1 = 0.0;
-            for (int w = 0; w < kApplyThreads / 64; ++w) { s0 += red[w][0]; s1 += red[w][1]; }
-            partials[2 * uint64_t(blockIdx.x)] = s0;
-            partials[2 * uint64_t(blockIdx.x) + 1] = s1;
-        }
-    }
+    if (kSplit > 1) merge_splits<kSplit, R>(reinterpret_cast<dvec2 *>(smem_raw), tid, sub, ar, ai);
+    const auto row = [base](uint64_t l) { return base + l; };
+    // (the buffers hold partner tiles)
+    const auto x = [&](uint64_t l) { return xv[base + l]; };
+    finish_tile<true, false, false, kSplit, R, cT>(tid, sub, tile_rows, row, x,
+                                            yout ? reinterpret_cast<cT *>(yout) + uint64_t(v) * N : nullptr,
+                                            partials, reinterpret_cast<double *>(smem_raw), ar, ai);
 }
 
 // out[2v], out[2v+1] = sum of the ntiles block partials of vector v
@@ -840,102 +735,109 @@ __global__ __launch_bounds__(256) void k_reduce_partials(uint32_t ntiles,
     if (threadIdx.x == 0) { out[2 * v] = ra[0]; out[2 * v + 1] = rb[0]; }
 }
 
-template <bool kMixed, bool kNarrow, int kL>
+template <bool kMixed, bool kNarrow, int kL, int kSplit, bool kWin = false>
 static int launch_tiled(const qr_op *op, DeviceTables *t, int slot, uint32_t nvec, const void *d_x,
                         void *d_y, double *partials, uint32_t ntiles, hipStream_t s) {
     using Shape = ApplyShape<kMixed, kL>;
-    using cT = typename std::conditional<kMixed, float2, double2>::type;
     const uint64_t N = uint64_t(1) << op->nq;
     const uint64_t tile_rows = N < (uint64_t(1) << Shape::L) ? N : (uint64_t(1) << Shape::L);
     const DeviceTables::Patterns &pt = t->pat[slot];
-    // the row-bit table holds max_u rows plus one zero row
-    const size_t shmem = apply_lds_offsets<cT>(tile_rows, pt.max_p, Shape::R, pt.max_u + 1,
-                                               nullptr, nullptr, nullptr);
-    if (shmem > kApplyMaxLDS) return fail(QR_ERR_SIZE, "apply: LDS stage too large");
+    const size_t shmem = apply_lds_bytes(Shape::kTile, pt.max_tab, Shape::merge_bytes(kSplit));
+    if (shmem > kApplyLDSLimit) return fail(QR_ERR_SIZE, "apply: LDS stage too large");
     const uint32_t tpx = (ntiles % 8 == 0) ? ntiles / 8 : 0;
     const bool full = tile_rows == (uint64_t(1) << Shape::L);
-    auto kern = full ? k_apply_tiled<kMixed, kNarrow, true, kL> : k_apply_tiled<kMixed, kNarrow, false, kL>;
-    QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
+    auto pick = [&](auto cplx_t) {
+        constexpr bool kC = decltype(cplx_t)::value;
+        return full ? k_apply_tiled<kMixed, kNarrow, kC, true, kL, kSplit, kWin>
+                    : k_apply_tiled<kMixed, kNarrow, kC, false, kL, kSplit, false>;
+    };
+    auto kern = pt.cplx ? pick(std::true_type{}) : pick(std::false_type{});
+    if (kWin && !full) return fail(QR_ERR_ARG, "apply: a window pass of partial tiles");
+    if (shmem > kDefaultLDS)
+        QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
     const uint64_t nblocks = uint64_t(ntiles) * nvec;
     if (nblocks > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "apply grid too large");
-    hipLaunchKernelGGL(kern, dim3(unsigned(nblocks)), dim3(kApplyThreads), shmem, s, N, ntiles,
-                       tpx, pt.ngrp, pt.nchunk, pt.max_p, pt.max_u, pt.grp, pt.chunk, pt.ug, pt.pzl, pt.ptptr, pt.ptz,
-                       pt.ptc, d_x, d_y, partials);
+    hipLaunchKernelGGL(kern, dim3(unsigned(nblocks)), dim3(kApplyThreads * kSplit), shmem, s, N, pt.win, ntiles,
+                       tpx, pt.nchunk, pt.grp, pt.chunk, pt.part, pt.tab, pt.pat,
+                       pt.ptz, pt.ptc, d_x, d_y, partials);
     QR_HIP_CHECK(hipGetLastError());
     return QR_OK;
 }
 
-template <bool kMixed, bool kNarrow, int kL>
+template <bool kMixed, bool kNarrow, int kL, int kSplit>
 static int launch_staged(const qr_op *op, DeviceTables *t, int slot, uint32_t nvec, const void *d_x,
                          void *d_y, double *partials, uint32_t ntiles, hipStream_t s) {
     using Shape = ApplyShape<kMixed, kL>;
-    using cT = typename std::conditional<kMixed, float2, double2>::type;
     const uint64_t N = uint64_t(1) << op->nq;
     const DeviceTables::Patterns &pt = t->pat[slot];
-    // dynamic LDS holds the tables; the two tile buffers are static
-    const size_t shmem = apply_lds_offsets<cT>(0, pt.max_p, Shape::R, pt.max_u + 1, nullptr,
-                                               nullptr, nullptr);
-    if (shmem + 2 * Shape::kTile + 1024 > kApplyMaxLDS)
-        return fail(QR_ERR_SIZE, "apply: LDS stage too large");
+    const size_t shmem = apply_lds_bytes(2 * Shape::kTile, pt.max_tab, Shape::merge_bytes(kSplit));
+    if (shmem > kApplyLDSLimit) return fail(QR_ERR_SIZE, "apply: LDS stage too large");
     const uint32_t tpx = (ntiles % 8 == 0) ? ntiles / 8 : 0;
-    auto kern = k_apply_staged<kMixed, kNarrow, kL>;
-    QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
+    auto kern = pt.cplx ? k_apply_staged<kMixed, kNarrow, true, kL, kSplit>
+                        : k_apply_staged<kMixed, kNarrow, false, kL, kSplit>;
+    if (shmem > kDefaultLDS)
+        QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
     const uint64_t nblocks = uint64_t(ntiles) * nvec;
     if (nblocks > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "apply grid too large");
-    hipLaunchKernelGGL(kern, dim3(unsigned(nblocks)), dim3(kApplyThreads), shmem, s, N, ntiles, tpx,
-                       pt.nchunk, pt.nrun, pt.max_p, pt.max_u, pt.grp, pt.chunk, pt.run, pt.ug, pt.pzl,
-                       pt.ptptr, pt.ptz, pt.ptc, d_x, d_y, partials);
+    hipLaunchKernelGGL(kern, dim3(unsigned(nblocks)), dim3(kApplyThreads * kSplit), shmem, s, N, ntiles, tpx,
+                       pt.nchunk, pt.nrun, pt.grp, pt.chunk, pt.run, pt.part, pt.tab, pt.pat, pt.ptz, pt.ptc, d_x, d_y, partials);
     QR_HIP_CHECK(hipGetLastError());
     return QR_OK;
 }
 
-// Which form applies the operator.  The partner-staged kernel needs full
-// tiles, and pays off when far groups share partner tiles: it loads a partner
-// tile once per run instead of gathering it once per group, but the load of a
-// one-group run is not hidden behind much work, and while the state is small
-// enough to stay in the caches the per-group gathers are cheap.  Measured
-// with the tiles above (F far groups on D distinct partner offsets; time of
-// the staged form against the gather form):
-//   mixed (2^11-row tiles):
-//     24-qubit k-local, 100..3000 terms: F/D 1.8..4.1, 1.24..1.46x faster;
-//     28-qubit k-local, 10000 terms: 1.40x faster;
-//     Heisenberg ring, 22 and 24 qubits: F/D 1, 0.96..1.01x;
-//     20-qubit random (8 MB state): F/D 1.05..1.24 -> 0.80..1.00x,
-//     2.3 -> 1.06x, 4.0 -> 1.12x;
-//   FP64 (2^10-row tiles): faster in every case measured -- k-local
-//     1.29..1.86x, 28-qubit k-local 1.40x, Heisenberg ring 1.07..1.10x,
-//     20-qubit random (F/D 1.0..2.3) 1.11..1.36x.
-//   small complex64 tiles (2^10 rows; only launches of at most four tiles
-//   per CU take them: at most 16 MiB of state on 256 CUs): the gather form, faster in
-//   every case measured -- 20 qubits, one state, gather / staged: the
-//   reference's H10 1.58 / 1.64 ms, random 2000 terms 1.19 / 1.45, random
-//   300 terms 0.20 / 0.28, k-local 3000 terms 0.43 / 0.46, k-local 500
-//   terms 0.13 / 0.15, Heisenberg ring 0.026 / 0.029.
-// Hence: FP64 staged whenever a group reaches outside the tile; mixed on
-// small tiles gathered; mixed on default tiles staged when F >= 1.5 D for
-// states of at least 32 MiB per vector, F >= 2 D below that.  The
-// environment variable QR_APPLY_FORM (1 gather, 2 staged) overrides the
+// Which form applies the operator (of the state's size, not of the number of
+// states, so that every call finds the same tables).  F groups reach outside
+// the tile, on D partner tiles.
+constexpr int kFormGather = 0;       // F gathers from memory
+constexpr int kFormStaged = 1;       // D partner tiles through LDS
+constexpr int kFormStagedDense = 2;  // the same with F >= 8 D
+// Measured (us, one state, gather / partner-staged):
+//   FP64: reference's molecules (F/D 9..), 16 / 20 / 22 qubits 134 / 113,
+//     1360 / 928, 7750 / 5050; k-local 24 qubits, 3000 terms (F/D 3.6) 7784 /
+//     7436, 300 terms, two states (1.4) 4140 / 3340, 20 qubits 459 / 400;
+//     random 20 qubits, 2000 terms (2.3) 1123 / 1104, 300 terms (1.1) 185 /
+//     203; below 2^20 rows, where x stays in L2,
+//     gathers win up to F/D 8: 18 qubits, 100 terms 50 / 60, k-local 16
+//     qubits 28 / 33.  Operators with window passes keep only partners that
+//     the L2 holds: 24-qubit ring 300 / 321.
+//   complex64 (2^11-row tiles): molecule 20 qubits 804 / 883, random 20 qubits
+//     762 / 840, k-local 24 qubits, 3000 terms 4940 / 5160, ring 24 qubits 183
+//     / 199; a state past the 256 MB MALL: k-local 28 qubits 236 / 229 ms.
+//   small complex64 tiles: gathers in all cases, within 5% at the worst.
+// The environment variable QR_APPLY_FORM (1 gather, 2 staged) overrides the
 // choice, for tests and measurement.
-static bool prefer_staged(const qr_op *op, int L, size_t elem_bytes, bool small_tiles) {
+static int apply_form(const qr_op *op, int kind, int L, const PatternShape &win_shape) {
     const char *e = getenv("QR_APPLY_FORM");
-    if (e && atoi(e) == 1) return false;
-    if (e && atoi(e) == 2) return true;
-    if (small_tiles) return false;
-    // gx ascends, so groups with equal bits above the tile are adjacent
-    uint64_t far = 0, distinct = 0, prev = 0;
-    for (uint64_t g = 0; g < op->G; ++g) {
-        const uint64_t hi = op->gx[g] >> L;
-        if (!hi) continue;
-        ++far;
-        if (distinct == 0 || hi != prev) ++distinct;
-        prev = hi;
+    if (e && atoi(e) == 1) return kFormGather;
+    int form = op->form[kind].load(std::memory_order_relaxed) - 1;
+    if (form < 0) {
+        const int elem_log2 = kind == 0 ? 4 : 3;
+        // gx ascends, so groups with equal bits above the tile are adjacent
+        uint64_t far = 0, distinct = 0, prev = 0;
+        for (uint64_t g = 0; g < op->G; ++g) {
+            const uint64_t hi = op->gx[g] >> L;
+            if (!hi) continue;
+            ++far;
+            if (distinct == 0 || hi != prev) ++distinct;
+            prev = hi;
+        }
+        std::vector<ApplyWindow> wins;
+        std::vector<uint8_t> pass;
+        // (then the partners left are mostly in L2)
+        const bool windows = win_shape.L && choose_windows(op, win_shape.L, elem_log2, wins, pass);
+        const bool dense = far >= 8 * distinct;
+        const int state_log2 = int(op->nq) + elem_log2;
+        bool staged = far > 0 && kind != 2 && !windows;
+        if (kind == 0)
+            staged = staged && (dense || state_log2 >= 26 || (state_log2 >= 24 && 2 * far >= 3 * distinct));
+        else staged = staged && state_log2 >= 28 && 2 * far >= 3 * distinct;
+        form = !staged ? kFormGather : dense ? kFormStagedDense : kFormStaged;
+        op->form[kind].store(form + 1, std::memory_order_relaxed);
     }
-    if (far == 0) return false;
-    if (elem_bytes == 16) return true;
-    const bool big = (uint64_t(1) << op->nq) * elem_bytes >= (uint64_t(32) << 20);
-    return big ? 2 * far >= 3 * distinct : far >= 2 * distinct;
+    if (e && atoi(e) == 2) return form == kFormStagedDense ? form : kFormStaged;
+    return form;
 }
 
 // One memory pool per device for the per-launch <x|y> workspaces.  Its
@@ -1012,9 +914,10 @@ static int apply_cus(int *out) {
 // slot that holds its tables (2 * kind + staged; kind 0: FP64, 1: complex64,
 // 2: small complex64 tiles).
 struct ApplyPlan {
-    int L = 0, slot = 0;
-    bool staged = false, pairs = false, small = false;
-    uint32_t pcap = 0, ucap = 0;
+    int L = 0, slot = 0, form = kFormGather;
+    bool small = false;
+    PatternShape shape = {}, win_shape = {};
+    int elem_log2 = 4;
 };
 
 template <bool kMixed, int kL>
@@ -1022,14 +925,37 @@ static ApplyPlan make_plan(const qr_op *op, int kind) {
     using Shape = ApplyShape<kMixed, kL>;
     ApplyPlan p;
     p.L = int(op->nq) < kL ? int(op->nq) : kL;
-    p.staged = p.L == kL && prefer_staged(op, p.L, kMixed ? 8 : 16, kind == 2);
-    p.pcap = p.staged ? Shape::kPatChunkS : Shape::kPatChunk;
-    p.ucap = p.staged ? Shape::kTableRowsS : Shape::kTableRows;
+    p.elem_log2 = kMixed ? 3 : 4;
+    if (p.L == kL)
+        p.win_shape = {p.L, kApplyThreadBits, Shape::kPatSplit, Shape::kTabChunk,
+                       uint32_t(Shape::kTile), false, kMixed, {}};
+    p.form = p.L == kL ? apply_form(op, kind, p.L, p.win_shape) : kFormGather;
+    const bool staged = p.form != kFormGather;
     // the gather form on full complex64 tiles runs the paired-row layout
-    p.pairs = kMixed && !p.staged && p.L == kL;
+    const bool pairs = kMixed && !staged && p.L == kL;
+    p.shape = {p.L, kApplyThreadBits, staged ? Shape::kPatSplitS : Shape::kPatSplit,
+               staged ? Shape::kTabChunkS : Shape::kTabChunk,
+               uint32_t(staged ? 2 * Shape::kTile : Shape::kTile), staged, pairs, {}};
     p.small = kind == 2;
-    p.slot = 2 * kind + (p.staged ? 1 : 0);
+    p.slot = 2 * kind + (staged ? 1 : 0);
     return p;
+}
+
+// Thread groups of 256 per block.  Several share a tile's groups (each takes
+// every split-th), so that a launch of few tiles still fills the CUs' wave
+// slots: the loop over the groups is a chain of scalar loads, table lookups
+// and gathers, which only other waves hide.  Measured (us, split 1 / 2 / 4):
+// FP64 molecules, 12 qubits 86 / 50 / 35, 16: 272 / 161 / 113, 18 (256 tiles):
+// 613 / 371 / 235, 20 (1024 tiles, staged, F/D 9): 1007 / 928 / 989, 22: 6020
+// / 5050 / 5570; k-local 20 qubits, 3000 terms (staged, F/D 5): 400 / 486 /
+// 716; ring 24 qubits (gather) 320 / 300 / 358.  Complex64, 2^11-row tiles:
+// molecule 20 qubits (512 tiles) 1085 / 804, k-local 24 qubits (8192 tiles)
+// 4940 / 5250; 2^10-row tiles: molecule 18 qubits (256 tiles) 439 / 256 / 183,
+// random 18 qubits, 3 states (768 tiles) 47 / 36 / 41.
+static int apply_split(const ApplyPlan &p, bool mixed, uint64_t blocks, int cus) {
+    if ((!mixed || p.small) && blocks <= uint64_t(2) * cus) return 4;
+    if (!mixed) return p.form == kFormStaged ? 1 : 2;
+    return p.small || blocks < uint64_t(4) * cus ? 2 : 1;
 }
 
 int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint32_t nvec,
@@ -1042,19 +968,18 @@ int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint
     const bool mixed = precision == QR_PREC_MIXED, narrow = op->nq <= 32 && !force_wide;
     const uint64_t N = uint64_t(1) << op->nq;
     if (nvec == 0) return fail(QR_ERR_SIZE, "apply: nvec == 0");
-    int rc;
+    int rc, cus = 0;
+    if ((rc = apply_cus(&cus))) return rc;
     ApplyPlan plan;
     if (!mixed) {
         plan = make_plan<false, ApplyShape<false>::L>(op, 0);
     } else {
-        // small complex64 tiles when the default ones give fewer than four
-        // blocks per CU (the blocks one CU holds at once); QR_APPLY_SMALL
-        // (0 never, 1 always where the state has more rows than a small
-        // tile) overrides the choice, for tests and measurement
-        int cus = 0;
-        if ((rc = apply_cus(&cus))) return rc;
+        // small complex64 tiles when the default ones give fewer than two
+        // blocks per CU; QR_APPLY_SMALL (0 never, 1 always where the state
+        // has more rows than a small tile) overrides the choice, for tests
+        // and measurement
         const bool can_small = int(op->nq) > kMixedSmallL;
-        bool small = can_small && (N >> ApplyShape<true>::L) * nvec < uint64_t(4) * uint64_t(cus);
+        bool small = can_small && (N >> ApplyShape<true>::L) * nvec < uint64_t(2) * uint64_t(cus);
         const char *small_env = getenv("QR_APPLY_SMALL");
         if (small_env) small = can_small && atoi(small_env) == 1;
         plan = small ? make_plan<true, kMixedSmallL>(op, 2) : make_plan<true, ApplyShape<true>::L>(op, 1);
@@ -1067,11 +992,9 @@ int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint
                 plan = other;
         }
     }
-    rc = device_patterns(op, t, plan.slot, plan.L, kApplyThreadBits, plan.pcap, plan.ucap,
-                         plan.staged, plan.pairs, noalloc);
+    rc = device_patterns(op, t, plan.slot, plan.shape, plan.win_shape, plan.elem_log2, noalloc);
     if (rc) return rc;
     const int L = plan.L;
-    const bool staged = plan.staged;
     if ((N >> L) * uint64_t(nvec) > 0x7FFFFFFFull)
         return fail(QR_ERR_SIZE, "apply: state too large for one launch");
     const uint32_t ntiles = uint32_t(N >> L);
@@ -1094,28 +1017,54 @@ int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint
         QR_HIP_CHECK(hipMallocFromPoolAsync(reinterpret_cast<void **>(&partials),
                                             size_t(ntiles) * nvec * 2 * sizeof(double), pool, s));
     }
-    constexpr int kLm = ApplyShape<true>::L, kLd = ApplyShape<false>::L, kLs = kMixedSmallL;
-    const int sl = plan.slot;
-    if (staged) {
-        if (mixed && plan.small)
-            rc = narrow ? launch_staged<true, true, kLs>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s)
-                        : launch_staged<true, false, kLs>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s);
-        else if (mixed)
-            rc = narrow ? launch_staged<true, true, kLm>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s)
-                        : launch_staged<true, false, kLm>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s);
-        else
-            rc = narrow ? launch_staged<false, true, kLd>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s)
-                        : launch_staged<false, false, kLd>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s);
-    } else if (mixed && plan.small) {
-        rc = narrow ? launch_tiled<true, true, kLs>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s)
-                    : launch_tiled<true, false, kLs>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s);
-    } else if (mixed) {
-        rc = narrow ? launch_tiled<true, true, kLm>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s)
-                    : launch_tiled<true, false, kLm>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s);
-    } else {
-        rc = narrow ? launch_tiled<false, true, kLd>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s)
-                    : launch_tiled<false, false, kLd>(op, t, sl, nvec, d_x, d_y, partials, ntiles, s);
-    }
+    // QR_APPLY_SPLIT (1, 2, 4) overrides the number of thread groups, for
+    // tests and measurement
+    const char *split_env = getenv("QR_APPLY_SPLIT");
+    const int split = split_env ? atoi(split_env) : apply_split(plan, mixed, uint64_t(ntiles) * nvec, cus);
+    const uint32_t nwin = t->pat[plan.slot].nwin;
+    auto launch = [&](auto mixed_t, auto l_t, auto split_t) {
+        constexpr bool kMixed = decltype(mixed_t)::value;
+        constexpr int kL = decltype(l_t)::value, kSplit = decltype(split_t)::value;
+        // all states in one launch; with window passes up to 128 MB of them
+        // at a time through all passes, so that the later ones find x and y in
+        // the 256 MB MALL
+        const uint64_t some = (uint64_t(1) << 27) / (N << plan.elem_log2);
+        const uint32_t step = nwin ? uint32_t(some ? some : 1) : nvec;
+        for (uint32_t v = 0; v < nvec; v += step) {
+            const uint32_t nv = nvec - v < step ? nvec - v : step;
+            const size_t off = size_t(v) * (N << plan.elem_log2);
+            const void *x = static_cast<const unsigned char *>(d_x) + off;
+            void *y = d_y ? static_cast<unsigned char *>(d_y) + off : nullptr;
+            double *e = partials ? partials + 2 * uint64_t(ntiles) * v : nullptr;
+            int r;
+            if (plan.form != kFormGather)
+                r = narrow ? launch_staged<kMixed, true, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s)
+                           : launch_staged<kMixed, false, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s);
+            else
+                r = narrow ? launch_tiled<kMixed, true, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s)
+                           : launch_tiled<kMixed, false, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s);
+            for (uint32_t k = 0; !r && k < nwin; ++k) {
+                const int sl = plan.slot + kApplySlots * int(k + 1);
+                r = narrow ? launch_tiled<kMixed, true, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s)
+                           : launch_tiled<kMixed, false, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s);
+            }
+            if (r) return r;
+        }
+        return int(QR_OK);
+    };
+    auto launch_split = [&](auto mixed_t, auto l_t) {
+        // (2^11-row tiles: four thread groups would not fit the registers)
+        constexpr int kMost = decltype(l_t)::value == kMixedSmallL ? 4 : 2;
+        if (split >= 4 && kMost == 4) return launch(mixed_t, l_t, std::integral_constant<int, kMost>{});
+        if (split >= 2) return launch(mixed_t, l_t, std::integral_constant<int, 2>{});
+        return launch(mixed_t, l_t, std::integral_constant<int, 1>{});
+    };
+    using MixedL = std::integral_constant<int, ApplyShape<true>::L>;
+    using SmallL = std::integral_constant<int, kMixedSmallL>;
+    using Fp64L = std::integral_constant<int, ApplyShape<false>::L>;
+    if (!mixed) rc = launch_split(std::false_type{}, Fp64L{});
+    else if (plan.small) rc = launch_split(std::true_type{}, SmallL{});
+    else rc = launch_split(std::true_type{}, MixedL{});
     if (!rc && d_expect) {
         hipLaunchKernelGGL(k_reduce_partials, dim3(nvec), dim3(256), 0, s, ntiles, partials,
                            d_expect);

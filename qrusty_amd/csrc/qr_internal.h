@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include <string>
@@ -60,46 +61,79 @@ struct RankEntry {
     int32_t sigma;
 };
 
-// One (sub)group of the matrix-free apply: x mask, its pattern range split by
-// class -- [p0, ps) z bits among the thread-index bits only, [ps, pk)
-// straddling, [pk, p1) row-index bits only -- and its row in the chunk's
-// per-tile table (-1 if it has no row-index patterns).  Pattern indices are
-// relative to the chunk.  32 bytes, read with one scalar load.
+// Matrix-free apply: D_g(r) by table.  Inside a tile, D_g is a sum of
+// "patterns" A_p (-1)^popcount(l & zl_p) (see build_patterns).  The patterns
+// of a group are cut into parts whose zl span at most kPartRank dimensions:
+// with a basis b_j of the part's zl, the part's sum depends on the row only
+// through the index whose bit j is parity(l & b_j), so the block tabulates it
+// once per tile (at most 16 values) and a row reads its value.  The index is
+// linear in the bits of l, so it is the XOR of the indices of the thread bits
+// 0-2 (nibble tid & 7 of w0), 3-5 (nibble of w1), of the wave (byte of w2)
+// and of the row index k (byte of rc).  w2 and rc are scaled to bytes of the
+// part's table, which starts at `tab` (in 4-byte units) of the block's LDS,
+// aligned to its size.
+constexpr int kPartRank = 4;
+struct ApplyPart {
+    uint32_t w0, w1, w2, tab;
+    uint64_t rc;
+};
+// One (sub)group: its x mask and its first part, or, with more than one part
+// (nparts > 1), the index of its parts in the part array in w0.  32 bytes,
+// read with one scalar load.
 struct ApplyGroup {
     uint64_t m;
-    uint32_t p0, ps, pk, p1;
-    int32_t u;
-    uint32_t flags;  // kGroupReal
+    uint32_t w0, w1, w2;
+    uint32_t tab_n;  // tab | nparts << 16 | flags
+    uint64_t rc;
+    __host__ __device__ uint32_t tab() const { return tab_n & 0xffffu; }
+    __host__ __device__ uint32_t nparts() const { return (tab_n >> 16) & 0xfffu; }
 };
-constexpr uint32_t kGroupReal = 1;  // every coefficient of the group is real
+constexpr uint32_t kGroupRowvar = 1u << 28;  // D varies with the row index: rc is not 0
+constexpr uint32_t kGroupCplx = 1u << 29;    // a coefficient with an imaginary part
+// The patterns of table i of the slot: entry 16 i + c is the term range of
+// its pattern of code c (whose zl is the sum of the basis vectors in c), empty
+// if it has none.  tab[i] is the table's place (4-byte units) | 2^rank << 16.
+// Table entries are FP64, complex unless every coefficient of the operator
+// (pass) is real.
+struct ApplyRange {
+    uint32_t t0, t1;
+};
 
-// Groups whose patterns [p0, p1) and table rows [u0, u1) are staged in LDS
-// together.  Inside a chunk the groups are ordered by class -- bit 0: the mask
-// reaches outside the tile ("far"), bit 1: D varies by row (row-bit or
-// straddling patterns), bit 2: complex coefficients, bit 3 (paired-row layout
-// only): row bit 0 of the mask set, so that each row's partner is the other
-// half of the gathered pair -- and class c holds the groups [cg[c], cg[c+1]).
-// For the partner-staged kernel the groups are ordered by partner tile
-// instead, in runs [r0, r1) (ApplyRun).
-constexpr int kApplyClasses = 16;
+// Groups whose tables [t0, t1) are formed in LDS together.  Inside a chunk the
+// groups are ordered by class -- bit 0 (the paired-row layout): row bit 0 of
+// the mask set, so that the rows of a pair exchange partners; bit 1: the mask
+// reaches outside the tile ("far") -- and class c holds the groups
+// [cg[c], cg[c+1]).  Masks ascend: the near groups come first, while the
+// neighbouring blocks load the tiles that the far ones read from L2 (24-qubit
+// ring, complex64, 8 states: 1.47 ms, 1.77 the other way round).  For the
+// partner-staged kernel the groups are ordered by partner tile instead, in
+// runs [r0, r1), the tile itself last (28-qubit k-local 236 -> 226 ms, 20-qubit
+// molecule 927 -> 891 us against the tile itself first).
+constexpr int kApplyClasses = 4;
 struct ApplyChunk {
     uint32_t cg[kApplyClasses + 1];
-    uint32_t p0, p1, u0, u1;
+    uint32_t t0, t1;
     uint32_t r0, r1;
-    uint32_t pad;
 };
 
 // Partner-staged apply: the groups of a chunk whose masks share the bits
 // above the tile (`hi`, a row offset) gather from the same partner tile,
-// which is loaded into LDS once for all of them.  Inside a run the groups are
-// ordered by class -- bit 0: D varies by row, bit 1: complex coefficients --
-// and class c holds the groups [g[c], g[c+1]).
-constexpr int kRunClasses = 4;
+// which is loaded into LDS once for all of them: the groups up to g1.
 struct ApplyRun {
     uint64_t hi;
-    uint32_t g[kRunClasses + 1];
-    uint32_t pad;
+    uint32_t g1, pad;
 };
+
+// Window pass of the apply: tiles of 2^L rows whose index bits are the
+// state's bits [0, f) and [s, s + L - f).  The groups whose masks lie in those
+// bits gather inside the tile there, where tiles of consecutive rows would
+// read a partner tile each; y is added to.  s = 0: no window.
+struct ApplyWindow {
+    uint32_t f = 0, s = 0;
+};
+constexpr int kMaxWindows = 3;
+
+constexpr int kApplySlots = 6;
 
 // Device copies of an operator's tables (one set per device that used it).
 struct DeviceTables {
@@ -119,34 +153,49 @@ struct DeviceTables {
     uint32_t *leaf_heavy = nullptr;  // qr_op::leaf_heavy
     // matrix-free apply tables, one set per tile kind and form (slot =
     // 2 * kind + staged; kind 0: FP64, 1: complex64, 2: small complex64 tiles)
+    // and pass (slot + kApplySlots * (k + 1): window pass k)
     struct Patterns {
         int L = -1;
-        uint32_t P = 0, ngrp = 0, nchunk = 0, nrun = 0, max_p = 0, max_u = 0;
+        uint32_t ngrp = 0, nchunk = 0, nrun = 0, max_tab = 0;
         uint32_t nfar = 0;  // groups whose mask reaches outside the tile
         ApplyGroup *grp = nullptr;    // [ngrp]
         ApplyChunk *chunk = nullptr;  // [nchunk]
         ApplyRun *run = nullptr;      // [nrun] (staged form only)
-        uint32_t *ug = nullptr;     // [U]   group (index into grp) of each table row
-        uint32_t *pzl = nullptr;    // [P]   z & (2^L - 1) of the pattern
-        uint32_t *ptptr = nullptr;  // [P+1] term range of each pattern
+        ApplyPart *part = nullptr;  // parts of the groups that have more than one
+        uint32_t *tab = nullptr;    // every part's table, by chunk
+        ApplyRange *pat = nullptr;  // [16 * tables] term range of each pattern
         uint64_t *ptz = nullptr;    // [T]   z masks in pattern order
         double2 *ptc = nullptr;     // [T]   c' in pattern order
-    } pat[6];
+        bool cplx = false;          // complex tables
+        uint32_t nwin = 0;          // window passes after this one
+        ApplyWindow win;            // (of a window pass)
+    } pat[kApplySlots * (1 + kMaxWindows)];
 };
 
-// Host build of the apply tables for tile size L, tb thread-index bits, at
-// most pcap patterns and ucap table rows per chunk (see qr_apply.hip).  A
-// group with more than pcap patterns is split into several ApplyGroups with
-// the same mask.  `staged` orders each chunk by partner tile (ApplyRun)
-// instead of by class.
+// Host build of the apply tables for tile size L, tb thread-index bits, of
+// the groups g with pass[g] == id (pass empty: all).  A
+// chunk takes up to tcap bytes of tables; a group that needs more has a chunk
+// of its own, and one of more than psplit patterns is split into several
+// ApplyGroups with the same mask.  The table area starts at byte
+// tab0 of the block's LDS.  `staged` orders each chunk by partner tile
+// (ApplyRun) instead of by class.
+struct PatternShape {
+    int L, tb;
+    uint32_t psplit, tcap, tab0;
+    bool staged, pairs;
+    ApplyWindow win;  // {}: tiles of consecutive rows
+};
 struct HostPatterns {
     std::vector<ApplyGroup> grp;
     std::vector<ApplyChunk> chunk;
-    std::vector<uint32_t> ug, pzl, ptptr;
+    std::vector<ApplyPart> part;
+    std::vector<uint32_t> tab;
+    std::vector<ApplyRange> pat;
     std::vector<uint64_t> ptz;
     std::vector<double> ptc;  // 2 per term
     std::vector<ApplyRun> run;  // staged form only
-    uint32_t max_p = 0, max_u = 0, nfar = 0;
+    uint32_t max_tab = 0, nfar = 0;
+    bool cplx = false;
 };
 // Paired-row layout of the mixed gather form: thread t owns the row pairs
 // (2t, 2t+1) + 2^(tb+1) j, so row-bit 0 counts with the row index (bit 0 of
@@ -156,14 +205,20 @@ inline uint64_t pair_row_bits(uint64_t zl, int tb) {
     const uint64_t tmask = (uint64_t(1) << tb) - 1;
     return ((zl >> 1) & tmask) | ((zl & 1) << tb) | (zl & ~((tmask << 1) | 1));
 }
-void build_patterns(const qr_op *op, int L, int tb, uint32_t pcap, uint32_t ucap, bool staged,
-                    bool pairs, HostPatterns &out);
+void build_patterns(const qr_op *op, const PatternShape &shape, const std::vector<uint8_t> &pass, uint8_t id,
+                    HostPatterns &out);
+// The window passes of an operator: pass[g] = 0 for the groups of the pass
+// over tiles of consecutive rows, k + 1 for those of wins[k] (see qr_api.cpp).
+// Returns whether they hold most of the masks that reach past L2.
+bool choose_windows(const qr_op *op, int L, int elem_log2, std::vector<ApplyWindow> &wins,
+                    std::vector<uint8_t> &pass);
 // Whether slot `slot` holds the apply tables for tile size L.
 bool tables_ready(const qr_op *op, const DeviceTables *t, int slot, int L);
-// With `noalloc` the tables must already be on the device (QR_ERR_ARG if not):
-// nothing is allocated or uploaded.
-int device_patterns(const qr_op *op, DeviceTables *t, int slot, int L, int tb, uint32_t pcap,
-                    uint32_t ucap, bool staged, bool pairs, bool noalloc = false);
+// The tables of slot `slot` and of its window passes (win_shape.L = 0: none
+// wanted).  With `noalloc` they must already be on the device (QR_ERR_ARG if
+// not): nothing is allocated or uploaded.
+int device_patterns(const qr_op *op, DeviceTables *t, int slot, const PatternShape &shape,
+                    const PatternShape &win_shape, int elem_log2, bool noalloc = false);
 
 }  // namespace qr
 
@@ -200,6 +255,9 @@ struct qr_op {
     uint32_t ntail = 0;
     std::vector<uint64_t> ttz;
     std::vector<double> ttc;  // 2 * ntail * G
+    // the matrix-free apply's form by tile kind (apply_form in qr_apply.hip)
+    // plus one, 0: not chosen yet
+    mutable std::atomic<int> form[qr::kApplySlots / 2] = {};
     // device state
     mutable std::mutex mu;
     mutable qr::DeviceTables dev[qr::kMaxDevices];
