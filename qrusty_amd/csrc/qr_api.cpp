@@ -9,6 +9,7 @@
 #include "qr_internal.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <numeric>
 #include <utility>
@@ -102,7 +103,7 @@ static void build_rank_lists(const std::vector<uint64_t> &gx, std::vector<uint32
 static void free_patterns(DeviceTables::Patterns &pt);
 
 void free_tables(DeviceTables &t) {
-    void *ptrs[] = {t.gx, t.gterm, t.tz, t.tc, t.rl_ptr, t.rl, t.gkind, t.heavy, t.leaf_heavy, t.ttz, t.ttc};
+    void *ptrs[] = {t.gx, t.gterm, t.tz, t.tc, t.rl_ptr, t.rl, t.gkind, t.heavy, t.leaf_heavy, t.real_heavy, t.real_ptr, t.real_terms, t.ttz, t.ttc};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (auto &pt : t.pat) free_patterns(pt);
@@ -349,11 +350,18 @@ static int upload(T **dst, const std::vector<T> &src) {
     return QR_OK;
 }
 
-int upload_tail(const qr_op *op, DeviceTables &t) {
+int upload_heavy(const qr_op *op, DeviceTables &t) {
+    int rc;
+    if ((!op->heavy.empty() && (rc = upload(&t.heavy, op->heavy))) ||
+        (!op->leaf_heavy.empty() && (rc = upload(&t.leaf_heavy, op->leaf_heavy))) ||
+        (!op->real_heavy.empty() && (rc = upload(&t.real_heavy, op->real_heavy))) ||
+        (!op->real_terms.empty() && ((rc = upload(&t.real_ptr, op->real_ptr)) ||
+                                     (rc = upload(&t.real_terms, op->real_terms)))))
+        return rc;
+    t.nheavy = uint32_t(op->heavy.size());
     if (!op->ntail) return QR_OK;
     std::vector<double2> c2(op->ttz.size());
     for (size_t i = 0; i < c2.size(); ++i) c2[i] = make_double2(op->ttc[2 * i], op->ttc[2 * i + 1]);
-    int rc;
     if ((rc = upload(&t.ttz, op->ttz)) || (rc = upload(&t.ttc, c2))) return rc;
     t.ntail = op->ntail;
     return QR_OK;
@@ -376,13 +384,10 @@ int device_tables(const qr_op *op, DeviceTables **out, bool noalloc) {
             (rc = upload(&t.tz, op->tz)) || (rc = upload(&t.tc, tc2)) ||
             (rc = upload(&t.rl_ptr, op->rl_ptr)) || (rc = upload(&t.rl, op->rl)) ||
             (rc = upload(&t.gkind, op->gkind)) ||
-            (!op->heavy.empty() && (rc = upload(&t.heavy, op->heavy))) ||
-            (!op->leaf_heavy.empty() && (rc = upload(&t.leaf_heavy, op->leaf_heavy))) ||
-            (rc = upload_tail(op, t))) {
+            (rc = upload_heavy(op, t))) {
             free_tables(t);
             return rc;
         }
-        t.nheavy = uint32_t(op->heavy.size());
         t.ready = true;
     }
     *out = &t;
@@ -523,15 +528,16 @@ int device_patterns(const qr_op *op, DeviceTables *t, int slot, const PatternSha
 // The parts of an operator derived from its grouped tables (gx, gterm):
 // the sub-operators (subtrees of at most kSubMaxG groups) and heavy groups.
 void finish_op(qr_op *op) {
-    // subtrees of at most kSubMaxG groups, split where build_rank_lists splits
-    if (op->G > kSubMaxG) {
+    // subtrees of at most `most` groups, split where build_rank_lists splits
+    auto cut = [op](uint32_t most, std::vector<qr_op::SubLeaf> &leaves) {
+        if (op->G <= most) return;
         struct Node { uint32_t lo, hi, depth; };
         std::vector<Node> stack{{0, uint32_t(op->G), 0}};
         while (!stack.empty()) {
             const Node nd = stack.back();
             stack.pop_back();
-            if (nd.hi - nd.lo <= kSubMaxG) {
-                op->leaves.push_back({nd.lo, nd.hi, nd.depth, 0, 0});
+            if (nd.hi - nd.lo <= most) {
+                leaves.push_back({nd.lo, nd.hi, nd.depth, 0, 0});
                 continue;
             }
             const uint64_t bit = uint64_t(1) << (63 - __builtin_clzll(op->gx[nd.lo] ^ op->gx[nd.hi - 1]));
@@ -542,7 +548,11 @@ void finish_op(qr_op *op) {
             stack.push_back({m, nd.hi, nd.depth + 1});
             stack.push_back({nd.lo, m, nd.depth + 1});
         }
-    }
+    };
+    cut(kSubMaxG, op->leaves);
+    op->real = true;
+    for (uint64_t i = 0; i < op->T; ++i) op->real = op->real && op->tc[2 * i + 1] == 0.0;
+    if (op->real) cut(kRealMaxG, op->real_leaves);
     // heavy groups: at least 8 terms and 4x the mean, the largest kMaxHeavy
     {
         const double mean = double(op->T) / double(op->G);
@@ -558,11 +568,28 @@ void finish_op(qr_op *op) {
         for (const auto &c : cand) op->heavy.push_back(c.second);
         std::sort(op->heavy.begin(), op->heavy.end());
         // each sub-operator's heavy groups, in its own (leaf-local) indices
-        for (auto &lf : op->leaves) {
-            lf.hoff = uint32_t(op->leaf_heavy.size());
-            for (uint32_t g : op->heavy)
-                if (g >= lf.s0 && g < lf.s1) op->leaf_heavy.push_back(g - lf.s0);
-            lf.hcnt = uint32_t(op->leaf_heavy.size()) - lf.hoff;
+        auto split = [op](std::vector<qr_op::SubLeaf> &leaves, std::vector<uint32_t> &heavy) {
+            for (auto &lf : leaves) {
+                lf.hoff = uint32_t(heavy.size());
+                for (uint32_t g : op->heavy)
+                    if (g >= lf.s0 && g < lf.s1) heavy.push_back(g - lf.s0);
+                lf.hcnt = uint32_t(heavy.size()) - lf.hoff;
+            }
+        };
+        split(op->leaves, op->leaf_heavy);
+        split(op->real_leaves, op->real_heavy);
+        if (op->real && op->nq <= 32 && !op->heavy.empty()) {
+            auto list = [op](uint32_t g0, const uint32_t *heavy, uint32_t n) {
+                op->real_ptr.push_back(uint32_t(op->real_terms.size()));
+                for (uint32_t k = 0; k < n; ++k) {
+                    for (uint32_t i = op->gterm[g0 + heavy[k]]; i < op->gterm[g0 + heavy[k] + 1]; ++i)
+                        op->real_terms.push_back({op->tc[2 * i], uint32_t(op->tz[i]),
+                                                  std::signbit(op->tc[2 * i + 1]) ? 0x80000000u : 0u});
+                    op->real_ptr.push_back(uint32_t(op->real_terms.size()));
+                }
+            };
+            if (op->real_leaves.empty()) list(0, op->heavy.data(), uint32_t(op->heavy.size()));
+            for (const auto &lf : op->real_leaves) list(lf.s0, op->real_heavy.data() + lf.hoff, lf.hcnt);
         }
     }
     // tail table: operators with heavy groups, whose other groups also run

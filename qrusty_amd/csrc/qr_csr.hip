@@ -33,6 +33,19 @@
 
 namespace qr {
 
+// Tile of a block: each of the 8 XCDs (blocks go to them round-robin) builds
+// one contiguous range of tiles, so that the lines at the ends of
+// neighbouring rows, which two blocks write parts of, meet in one L2, and an
+// XCD touches an eighth of the output's pages.  Launch order / this one (ms,
+// two output buffers each; their place moves the rate by up to 20%): 20 qubits
+// and 2000 random terms 9.42, 9.35 / 9.24, 8.55; 300 terms 1.39 / 1.23, 1.12;
+// 22 qubits, 60 terms 1.10, 0.96 / 1.01, 0.86; 20-qubit molecule 15.7, 12.5 /
+// 12.1, 11.4.  A grid that is no multiple of 8 keeps the launch order.
+__device__ __forceinline__ uint32_t xcd_tile() {
+    const uint32_t b = blockIdx.x, n = gridDim.x;
+    return n % 8u == 0 ? (b % 8u) * (n / 8u) + b / 8u : b;
+}
+
 // LDS-staged build: one block per tile of the shared tile builder
 // (qr_tile.h), without the fused matvec; the heavy-group instances of
 // fold_tiles run 2^op.fold_log2 consecutive tiles per block, folding the
@@ -44,12 +57,12 @@ __global__ __launch_bounds__(kStageThreads) void k_csr_build_staged(TileOp op) {
         const uint32_t tile_log2 = 10u - op.jw_log2 + 4u;
         const uint32_t k = 1u << op.fold_log2;
         for (uint32_t s = 0; s < k; ++s) {
-            const uint64_t tile = uint64_t(blockIdx.x) * k + s;
+            const uint64_t tile = uint64_t(xcd_tile()) * k + s;
             if ((((op.row_begin >> tile_log2) + tile) << tile_log2) >= op.row_end) break;
             build_tile_staged<kNarrow, kChunks, false, kMode>(op, tile, smem_raw, s);
         }
     } else {
-        build_tile_staged<kNarrow, kChunks, false, kMode>(op, blockIdx.x, smem_raw);
+        build_tile_staged<kNarrow, kChunks, false, kMode>(op, xcd_tile(), smem_raw);
     }
 }
 
@@ -59,13 +72,354 @@ __global__ __launch_bounds__(kStageThreads) void k_csr_build_staged(TileOp op) {
 template <bool kNarrow, int kChunks, int kMode>
 __global__ __launch_bounds__(kStageThreads, 8) void k_csr_build_sub(TileOp op) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    build_tile_staged<kNarrow, kChunks, false, kMode>(op, blockIdx.x, smem_raw);
+    build_tile_staged<kNarrow, kChunks, false, kMode>(op, xcd_tile(), smem_raw);
+}
+
+// CSR build of operators whose coefficients c' are all real (molecular and spin
+// Hamiltonians), masks in 32 bits: one group per thread, and per row three
+// vector instructions per term.  Thread layout as in qr_tile.h (kT = RS rows x
+// JW lanes, the rows of a tile in M = 2^m_log2 batches of RS), but
+//  * the sign of a term over the tile's M rows is one 32-bit word, the parity
+//    of r & z for batch m in bit 31 - m (the parity is linear in r: the fixed
+//    bits give all or none, each of the five batch bits an alternating
+//    pattern).  It carries the coefficient's own sign, is shifted up once per
+//    batch and its top bit goes straight into the coefficient's sign bit: a
+//    shift, a bit-field insert and an addition per term, against mask, count,
+//    compare, selects and two additions (the imaginary part of a real
+//    coefficient is a signed zero, and a sum of signed zeros is -0 only if
+//    all are: one word per group, the AND of its terms');
+//  * absent terms are -0.0, which every sum absorbs unchanged, so all lanes
+//    run the same six additions (two or four where no lane of the wave has
+//    more terms; terms past the sixth come from memory);
+//  * a row's slot moves by one addition per batch (the sigma of the bits that
+//    the step flips, qr_tile.h);
+//  * 64 VGPRs: two 1024-thread blocks per CU, one copying out while the other
+//    computes, and two stages per block, one barrier per batch.
+// Groups of many terms (op.heavy) are folded by a pass of their own at the
+// start of the tile, one thread per (group, row).  The additions are the same,
+// in the same order, as build_tile_staged's, so the values are bit-identical.
+// Operators of more than kRealMaxG groups are built as sub-operators of at
+// most that many (kSub), each with the power of two of threads that holds it.
+// What bounds it: the stores (4.6-6.4 TB/s of 24 B per entry, by the place of
+// the output).  The builder of qr_tile.h / this one, us: molecules of 12 / 16 /
+// 18 / 20 qubits 139 / 510 / 4031 / 28360 -> 28 / 326 / 2020-2160 / 11500-13850;
+// 14-qubit ring 24.5 -> 10.5, 24 qubits 2147 -> 1560-1790.  Not used for more
+// than kRealMaxG groups of mostly one term, which two group chunks per thread
+// build faster (17 qubits, 2516 groups 1800 / 1954).
+constexpr int kRealHold = 6;      // terms of a group held in registers
+constexpr int kRealMaxLog2 = 5;   // batches per tile (log2)
+constexpr size_t kRealLDS = 80 * 1024;  // of one block: two per CU
+
+// Sign words of the batch bits: bit b of m set <=> the bits of kSignWord[b]
+__device__ __forceinline__ uint32_t sign_word(uint32_t parity, uint32_t zm) {
+    uint32_t w = 0u - (parity & 1u);
+    w ^= (zm & 1u) ? 0x55555555u : 0u;
+    w ^= (zm & 2u) ? 0x33333333u : 0u;
+    w ^= (zm & 4u) ? 0x0F0F0F0Fu : 0u;
+    w ^= (zm & 8u) ? 0x00FF00FFu : 0u;
+    w ^= (zm & 16u) ? 0x0000FFFFu : 0u;
+    return w;
+}
+
+// |c| with the sign in bit 31 of w
+__device__ __forceinline__ double with_sign(double c, uint32_t w) {
+    return __hiloint2double(int((uint32_t(__double2hiint(c)) & 0x7fffffffu) | (w & 0x80000000u)), __double2loint(c));
+}
+__device__ __forceinline__ uint32_t sign_of(double c) { return uint32_t(__double2hiint(c)) & 0x80000000u; }
+
+// Term-order fold in row r of the terms [t, t1) in LDS, four loaded ahead of
+// their additions.
+__device__ __forceinline__ double2 fold_real(const RealTerm *terms, uint32_t t, uint32_t t1, uint32_t r) {
+    uint32_t im = 0x80000000u;
+    auto term = [&](const RealTerm &a) {
+        const uint32_t s = uint32_t(__popc(r & a.z)) << 31;
+        im &= a.im ^ s;
+        return __hiloint2double(__double2hiint(a.c) ^ int(s), __double2loint(a.c));
+    };
+    double v = term(terms[t]);
+    ++t;
+    constexpr uint32_t kF = 4;
+    for (; t + kF <= t1; t += kF) {
+        RealTerm a[kF];
+#pragma unroll
+        for (uint32_t u = 0; u < kF; ++u) a[u] = terms[t + u];
+#pragma unroll
+        for (uint32_t u = 0; u < kF; ++u) v = v + term(a[u]);
+    }
+    for (; t < t1; ++t) v = v + term(terms[t]);
+    return make_double2(v, __hiloint2double(int(im), 0));
+}
+
+// The heavy groups' terms of one build (qr_op::real_ptr, real_terms), and the
+// LDS bytes before their values (two stages, which the terms use first).
+struct RealHeavy {
+    const uint32_t *ptr;
+    const RealTerm *terms;
+    uint32_t hv_at;
+};
+
+template <bool kSub, int kT>
+__global__ __launch_bounds__(kT, 8) void k_csr_build_real(TileOp op, RealHeavy rh, uint32_t m_log2) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const TileMem mem = tile_mem(op);
+    const uint32_t G = op.G, jw_log2 = op.jw_log2;
+    const uint32_t rs_log2 = kSub ? 0u : uint32_t(__builtin_ctz(kT)) - jw_log2;
+    const uint32_t tile_log2 = rs_log2 + m_log2, M = 1u << m_log2;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = kSub ? tid : tid & ((1u << jw_log2) - 1u);
+    const uint32_t ro = kSub ? 0u : tid >> jw_log2;
+    const uint64_t row_begin = op.row_begin, row_end = op.row_end;
+    const uint64_t tile_base = ((row_begin >> tile_log2) + xcd_tile()) << tile_log2;
+    const uint32_t rfix = uint32_t(tile_base) | ro;  // at most 32 bits of row
+    const uint32_t batch_pad = ((G << rs_log2) + 1u) & ~1u;
+    const uint32_t stage_b = batch_pad * 24u;
+    double2 *hv = reinterpret_cast<double2 *>(smem_raw + rh.hv_at);
+
+    // heavy groups first, before the lanes' own terms take registers: their
+    // terms into LDS, then one thread per (group, row)
+    if (op.nheavy) {
+        const auto hptr = as_global(rh.ptr);
+        const uint32_t h0 = hptr[0];
+        uint4 *to = reinterpret_cast<uint4 *>(smem_raw);
+        const uint4 *from = reinterpret_cast<const uint4 *>(rh.terms + h0);
+        for (uint32_t i = tid; i < hptr[op.nheavy] - h0; i += kT) to[i] = from[i];
+        __syncthreads();
+        const uint32_t tr = 1u << tile_log2;
+        for (uint32_t i = tid; i < op.nheavy << tile_log2; i += kT) {
+            const uint32_t g = i >> tile_log2, r = uint32_t(tile_base) + (i & (tr - 1u));
+            hv[i] = fold_real(reinterpret_cast<const RealTerm *>(smem_raw), hptr[g] - h0, hptr[g + 1] - h0, r);
+        }
+        // (the barrier after the lanes' setup, which overlaps the long groups)
+    }
+
+    // slot of the lane's group in row rfix, and its change when the batch
+    // index goes from m to m + 1 with t = ctz(m + 1): sigma of bit t minus
+    // those of the bits below, which turn off
+    int32_t sig[kRealMaxLog2] = {0, 0, 0, 0, 0};
+    int32_t slot = int32_t(kSub ? op.gbase + lane : ro * G + lane);
+    auto take = [&](const RankEntry &en, int32_t sign, int32_t &at) {
+        const uint32_t b = uint32_t(en.bit), q = b - rs_log2;  // wraps for b < rs_log2
+        if (q >= m_log2) at += (rfix >> b) & 1u ? sign * en.sigma : 0;
+#pragma unroll
+        for (uint32_t k = 0; k < uint32_t(kRealMaxLog2); ++k)
+            if (q == k && q < m_log2) sig[k] += sign * en.sigma;
+    };
+    int32_t off = 0, osig[kRealMaxLog2] = {0, 0, 0, 0, 0};
+    if (kSub) {
+        // the sub-operator's first rank (qr_tile.h)
+        off = int32_t(op.gbase);
+        for (uint32_t e = 0; e < op.nanc; ++e) {
+            const RankEntry en = ld_rank(mem.rl + mem.rl_ptr[0] + e);
+            const uint32_t b = uint32_t(en.bit);
+            if (b >= m_log2) off += (rfix >> b) & 1u ? en.sigma : 0;
+#pragma unroll
+            for (uint32_t k = 0; k < uint32_t(kRealMaxLog2); ++k)
+                if (b == k && b < m_log2) osig[k] += en.sigma;
+        }
+    }
+    const bool valid = lane < G;
+    int32_t hs = -1;
+    uint32_t xj = 0, n = 0, tf = 0, wi = 0xffffffffu;
+    uint32_t w[kRealHold];
+    double c[kRealHold];
+#pragma unroll
+    for (int u = 0; u < kRealHold; ++u) {
+        w[u] = 0xffffffffu;  // -0.0
+        c[u] = 0.0;
+    }
+    if (valid) {
+        const uint32_t e1 = mem.rl_ptr[lane + 1];
+        for (uint32_t e = mem.rl_ptr[lane]; e < e1; ++e) take(ld_rank(mem.rl + e), 1, slot);
+        uint32_t lo = 0, hi = op.nheavy;  // heavy groups ascend
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (mem.heavy[mid] < lane) lo = mid + 1;
+            else hi = mid;
+        }
+        if (lo < op.nheavy && mem.heavy[lo] == lane) hs = int32_t(lo);
+        xj = uint32_t(mem.gx[lane]);
+        tf = mem.gterm[lane];
+        if (hs < 0) {
+            n = mem.gterm[lane + 1] - tf;
+#pragma unroll
+            for (int u = 0; u < kRealHold; ++u) {
+                if (uint32_t(u) >= n) break;
+                // terms past the second from the tail table (coalesced)
+                const bool tail = u >= 2 && uint32_t(u - 2) < op.ntail;
+                const uint32_t at = tail ? uint32_t(u - 2) * op.gstride + lane : tf + uint32_t(u);
+                const uint32_t z = uint32_t(tail ? mem.ttz[at] : mem.tz[at]);
+                const double2 cc = ld2((tail ? mem.ttc : mem.tc) + at);
+                const uint32_t s = sign_word(__popc(rfix & z), (z >> rs_log2) & (M - 1u));
+                w[u] = s ^ (sign_of(cc.x) ? 0xffffffffu : 0u);
+                wi &= s ^ (sign_of(cc.y) ? 0xffffffffu : 0u);
+                c[u] = cc.x;
+            }
+        }
+    }
+    slot -= off;
+    int32_t step[kRealMaxLog2];
+    {
+        int32_t below = 0;
+#pragma unroll
+        for (int k = 0; k < kRealMaxLog2; ++k) {
+            const int32_t s = sig[k] - osig[k];
+            step[k] = s - below;
+            below += s;
+        }
+    }
+    if (op.nheavy) __syncthreads();
+    // the wave's longest group, in registers and past them
+    const bool more2 = __any(n > 2), more4 = __any(n > 4), past = __any(n > uint32_t(kRealHold));
+
+    // the batch's entries, in LDS: written at the lane's slot, copied out by
+    // consecutive threads (a batch has at most kT of them)
+    const uint32_t stage_entries = G << rs_log2;
+    const bool whole = tile_base >= row_begin && tile_base + (uint64_t(M) << rs_log2) <= row_end;
+    // output place of the batch's first row (before row_begin: not used)
+    uint64_t dst = (tile_base - row_begin) * (kSub ? op.gstride : G);
+    if (kSub) dst += uint64_t(int64_t(off));
+    const uint64_t dst_step = uint64_t(kSub ? op.gstride : G) << rs_log2;
+    int32_t ostep[kRealMaxLog2];
+    {
+        int32_t below = 0;
+#pragma unroll
+        for (int k = 0; k < kRealMaxLog2; ++k) {
+            ostep[k] = osig[k] - below;
+            below += osig[k];
+        }
+    }
+    auto batch = [&](uint32_t m, uint32_t buf) {
+        uint64_t *si = reinterpret_cast<uint64_t *>(smem_raw + buf * stage_b);
+        double2 *sd = reinterpret_cast<double2 *>(si + batch_pad);
+        const uint32_t r = rfix + (m << rs_log2);
+        if (valid && (whole || (uint64_t(r) >= row_begin && uint64_t(r) < row_end))) {
+            double v = with_sign(c[0], w[0]);
+            v = v + with_sign(c[1], w[1]);
+            if (more2) {
+                v = v + with_sign(c[2], w[2]);
+                v = v + with_sign(c[3], w[3]);
+            }
+            if (more4) {
+                v = v + with_sign(c[4], w[4]);
+                v = v + with_sign(c[5], w[5]);
+            }
+            uint32_t im = wi;
+            if (past) {
+                for (uint32_t u = kRealHold; u < n; ++u) {
+                    const bool tail = u - 2 < op.ntail;
+                    const uint32_t at = tail ? (u - 2) * op.gstride + lane : tf + u;
+                    const double2 cc = ld2((tail ? mem.ttc : mem.tc) + at);
+                    const uint32_t s = uint32_t(__popc(r & uint32_t(tail ? mem.ttz[at] : mem.tz[at]))) << 31;
+                    v = v + __hiloint2double(__double2hiint(cc.x) ^ int(s), __double2loint(cc.x));
+                    im &= sign_of(cc.y) ^ s;
+                }
+            }
+            double2 e = make_double2(v, __hiloint2double(int(im & 0x80000000u), 0));
+            if (hs >= 0) e = hv[(uint32_t(hs) << tile_log2) | (m << rs_log2) | ro];
+            si[slot] = r ^ xj;
+            sd[slot] = e;
+        }
+#pragma unroll
+        for (int u = 0; u < kRealHold; ++u) w[u] <<= 1;
+        wi <<= 1;
+        __syncthreads();
+        bool mine = tid < stage_entries;
+        if (!whole) {
+            const uint64_t b0 = tile_base + (uint64_t(m) << rs_log2);
+            const uint64_t row = b0 + (kSub ? 0u : tid / G);
+            mine = mine && row >= row_begin && row < row_end;
+        }
+        if (mine) {
+            mem.indices[dst + tid] = si[tid];
+            const double2 dv = sd[tid];
+            mem.data[dst + tid] = dvec2{dv.x, dv.y};
+        }
+    };
+    auto advance = [&](int t) {
+        slot += step[t];
+        dst += dst_step;
+        if (kSub) dst += uint64_t(int64_t(ostep[t]));
+    };
+#pragma unroll 1
+    for (uint32_t m = 0; m < M; m += 4) {  // M is at least 4
+        batch(m, 0);
+        advance(0);
+        batch(m + 1, 1);
+        advance(1);
+        batch(m + 2, 0);
+        advance(0);
+        batch(m + 3, 1);
+        const uint32_t t = uint32_t(__builtin_ctz(m + 4u));  // 2 to 5 (the end)
+        if (t == 2) advance(2);
+        else if (t == 3) advance(3);
+        else advance(4);
+    }
 }
 
 __global__ __launch_bounds__(256) void k_indptr(uint64_t row_begin, uint64_t nrows, uint64_t G,
                                                 uint64_t *__restrict__ indptr) {
     uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
     if (i <= nrows) indptr[i] = (row_begin + i) * G;
+}
+
+// Builds of real operators (k_csr_build_real): the whole operator, or one
+// launch per sub-operator of op->real_leaves.
+static int launch_build_real(const qr_op *op, const DeviceTables *t, uint64_t row_begin, uint64_t row_end,
+                             uint64_t *d_indices, double *d_data, hipStream_t s) {
+    const uint32_t G = uint32_t(op->G);
+    auto run = [&](auto sub_t, auto threads_t, TileOp top, uint32_t rs_log2, size_t at) {
+        constexpr bool kSub = decltype(sub_t)::value;
+        constexpr int kT = decltype(threads_t)::value;
+        // batches per tile: as many as leave the launch four blocks per CU
+        uint32_t ml = kRealMaxLog2;
+        while (ml > 2 && ((row_end - row_begin) >> (rs_log2 + ml)) < 1024) --ml;
+        const uint32_t tl = rs_log2 + ml;
+        const uint64_t nt = ((row_end - 1) >> tl) - (row_begin >> tl) + 1;
+        if (nt > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "CSR build grid too large");
+        // heavy groups (their terms first in the stages' place, their values
+        // behind) as LDS allows with two blocks per CU; the rest run term by
+        // term
+        const size_t stage = size_t(((top.G << rs_log2) + 1u) & ~1u) * 24 * 2, each = size_t(16) << tl;
+        const uint32_t *ptr = top.nheavy ? op->real_ptr.data() + at : nullptr;
+        auto front = [&](uint32_t n) {
+            const size_t terms = n ? size_t(ptr[n] - ptr[0]) * sizeof(RealTerm) : 0;
+            return std::max(stage, terms);
+        };
+        while (top.nheavy && front(top.nheavy) + top.nheavy * each > kRealLDS) --top.nheavy;
+        const RealHeavy rh{t->real_ptr + at, t->real_terms, uint32_t(front(top.nheavy))};
+        const size_t shmem = rh.hv_at + top.nheavy * each;
+        auto kern = k_csr_build_real<kSub, kT>;
+        QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
+        hipLaunchKernelGGL(kern, dim3(unsigned(nt)), dim3(kT), shmem, s, top, rh, ml);
+        QR_HIP_CHECK(hipGetLastError());
+        return int(QR_OK);
+    };
+    using T = std::true_type;
+    using F = std::false_type;
+    using T256 = std::integral_constant<int, 256>;
+    using T512 = std::integral_constant<int, 512>;
+    using T1024 = std::integral_constant<int, 1024>;
+    auto tile_op = [&](uint32_t g0, uint32_t g, uint32_t depth, const uint32_t *heavy, uint32_t nheavy, uint32_t jw) {
+        return TileOp{t->gx + g0, t->gterm + g0, t->tz, t->tc, t->rl_ptr + g0, t->rl, d_indices,
+                      reinterpret_cast<double2 *>(d_data), nullptr, nullptr, nullptr, row_begin, row_end, g, jw, 1,
+                      1, heavy, nheavy, g0, depth, G, t->ntail ? t->ttz + g0 : nullptr,
+                      t->ntail ? t->ttc + g0 : nullptr, t->ntail, 0};
+    };
+    if (op->real_leaves.empty()) {
+        const uint32_t jw = stage_jw_log2(G);
+        return run(F{}, T1024{}, tile_op(0, G, 0, t->heavy, t->nheavy, jw), 10u - jw, 0);
+    }
+    for (size_t k = 0; k < op->real_leaves.size(); ++k) {
+        const auto &lf = op->real_leaves[k];
+        const uint32_t g = lf.s1 - lf.s0;
+        const TileOp top = tile_op(lf.s0, g, lf.depth, t->real_heavy + lf.hoff, lf.hcnt, 0);
+        const int rc = g <= 256   ? run(T{}, T256{}, top, 0, lf.hoff + k)
+                       : g <= 512 ? run(T{}, T512{}, top, 0, lf.hoff + k)
+                                  : run(T{}, T1024{}, top, 0, lf.hoff + k);
+        if (rc) return rc;
+    }
+    return QR_OK;
 }
 
 int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin, uint64_t row_end,
@@ -81,6 +435,8 @@ int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin,
     }
     if (nrows == 0) return QR_OK;
     const bool narrow = op->nq <= 32;
+    if (op->real && narrow && (G <= kRealMaxG || 4 * op->T >= 5 * op->G))
+        return launch_build_real(op, t, row_begin, row_end, d_indices, d_data, s);
     if (!op->leaves.empty()) {
         // one sub-operator per subtree of the mask trie, each <= kSubMaxG
         // groups with one row per batch (JW = 1024): the fast 1- and 2-chunk

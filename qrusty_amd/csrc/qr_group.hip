@@ -480,20 +480,11 @@ int group_terms_device(const char *const *labels, const double *coeffs, uint64_t
     for (void *p : {(void *)d_gx, (void *)d_gterm, (void *)d_tz, (void *)d_tc, (void *)d_rlptr,
                     (void *)d_rl, (void *)d_gkind})
         B.release(p);
-    auto put = [&](auto **dst, const auto &v) -> int {
-        using T_ = typename std::decay<decltype(v[0])>::type;
-        QR_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(dst), std::max<size_t>(v.size(), 1) * sizeof(T_)));
-        QR_HIP_CHECK(hipMemcpy(*dst, v.data(), v.size() * sizeof(T_), hipMemcpyHostToDevice));
-        return QR_OK;
-    };
-    if ((!op->heavy.empty() && (rc = put(&t.heavy, op->heavy))) ||
-        (!op->leaf_heavy.empty() && (rc = put(&t.leaf_heavy, op->leaf_heavy))) ||
-        (rc = upload_tail(op, t))) {
+    if ((rc = upload_heavy(op, t))) {
         free_tables(t);
         delete op;
         return rc;
     }
-    t.nheavy = uint32_t(op->heavy.size());
     t.ready = true;
     *out = op;
     return QR_OK;

@@ -50,6 +50,7 @@ constexpr uint32_t kMaxHeavy = 128;
 constexpr uint32_t kMaxTail = 16;
 constexpr uint64_t kMaxTailSlots = uint64_t(1) << 22;
 constexpr uint32_t kSubMaxG = 2048;  // groups of one CSR-build sub-operator
+constexpr uint32_t kRealMaxG = 1024;  // the same, operators of real coefficients
 // CSR matvecs load the CSR stream nontemporally from this many entries per
 // row on (measured crossover; qr_csr.hip)
 constexpr uint64_t kMvNontemporalMinRow = 256;
@@ -135,6 +136,13 @@ constexpr int kMaxWindows = 3;
 
 constexpr int kApplySlots = 6;
 
+// A term of an operator with real coefficients and masks of 32 bits: Re c',
+// z, and the sign of Im c' (a signed zero) in bit 31.
+struct RealTerm {
+    double c;
+    uint32_t z, im;
+};
+
 // Device copies of an operator's tables (one set per device that used it).
 struct DeviceTables {
     bool ready = false;
@@ -151,6 +159,9 @@ struct DeviceTables {
     double2 *ttc = nullptr;
     uint32_t ntail = 0;
     uint32_t *leaf_heavy = nullptr;  // qr_op::leaf_heavy
+    uint32_t *real_heavy = nullptr;  // qr_op::real_heavy, real_ptr, real_terms
+    uint32_t *real_ptr = nullptr;
+    RealTerm *real_terms = nullptr;
     // matrix-free apply tables, one set per tile kind and form (slot =
     // 2 * kind + staged; kind 0: FP64, 1: complex64, 2: small complex64 tiles)
     // and pass (slot + kApplySlots * (k + 1): window pass k)
@@ -248,6 +259,16 @@ struct qr_op {
     };
     std::vector<SubLeaf> leaves;
     std::vector<uint32_t> leaf_heavy;  // heavy groups of each leaf, leaf-local
+    // every coefficient c' is real: the builder of k_csr_build_real, on
+    // sub-operators of at most kRealMaxG groups
+    bool real = false;
+    std::vector<SubLeaf> real_leaves;
+    std::vector<uint32_t> real_heavy;
+    // the terms of the heavy groups, one list per real_leaves entry (or one
+    // for the whole operator): group k of list i has the terms
+    // real_terms[real_ptr[hoff + i + k] .. real_ptr[hoff + i + k + 1])
+    std::vector<uint32_t> real_ptr;
+    std::vector<qr::RealTerm> real_terms;
     // operators with heavy groups: the terms past each group's second,
     // transposed (slot u * G + g holds term gterm[g] + 2 + u, zero where the
     // group is shorter), so that the lanes of a batch -- one group each --
@@ -274,8 +295,8 @@ int group_terms_device(const char *const *labels, const double *coeffs, uint64_t
 // Sub-operators, heavy groups and tail table of an op whose grouped tables
 // are set.
 void finish_op(qr_op *op);
-// Uploads the op's tail table (if it has one) into t.
-int upload_tail(const qr_op *op, DeviceTables &t);
+// Uploads the op's heavy groups and tail table (where it has them) into t.
+int upload_heavy(const qr_op *op, DeviceTables &t);
 // Frees one device's tables of an op.
 void free_tables(DeviceTables &t);
 

@@ -1,0 +1,93 @@
+"""CSR builds of operators with real coefficients (k_csr_build_real): bit-exact
+against the oracle's rows at the edges of its layout -- groups of 1 to past 6
+terms, zero coefficients of both signs, one and many rows per batch,
+sub-operators, more heavy groups than LDS holds, and row windows that begin
+and end inside a tile."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import qrusty_amd  # noqa: F401
+    yield
+    torch.cuda.synchronize()
+
+
+def _op(labels, coeffs):
+    import qrusty_amd as qa
+    return qa.SparsePauliOp([qa.Pauli(s) for s in labels], coeffs)
+
+
+def _label(n, xm, zm):
+    return "".join("IXZY"[((xm >> q) & 1) | (((zm >> q) & 1) << 1)] for q in reversed(range(n)))
+
+
+def _real_operator(n, groups, sizes, seed):
+    """`groups` masks of sizes[k % len(sizes)] terms each, in shuffled order,
+    every c' real (an even number of Y, or an odd one with an imaginary
+    coefficient), some coefficients 0.0 or -0.0."""
+    rng = np.random.default_rng(seed)
+    masks = rng.choice(1 << n, size=min(groups, 1 << n), replace=False)
+    labels, coeffs = [], []
+    for k, xm in enumerate(masks):
+        for _ in range(sizes[k % len(sizes)]):
+            zm = int(rng.integers(0, 1 << n))
+            c = float(rng.choice([0.0, -0.0, rng.normal()], p=[0.05, 0.05, 0.9]))
+            odd = bin(int(xm) & zm).count("1") % 2
+            labels.append(_label(n, int(xm), zm))
+            coeffs.append(complex(0.0, c) if odd else complex(c, rng.choice([0.0, -0.0])))
+    order = rng.permutation(len(labels))
+    return [labels[i] for i in order], [coeffs[i] for i in order]
+
+
+CASES = [(3, 1, [1]), (5, 7, [1, 2]), (9, 25, [2, 2, 2, 48]), (8, 200, [1, 2, 3, 4, 5, 6, 7, 8]),
+         (11, 500, [4, 4, 6]), (11, 1024, [3]), (11, 1025, [2, 5]), (12, 2600, [4, 4, 4, 6, 9]),
+         (12, 90, [40] * 60 + [2] * 30), (10, 130, [12])]
+
+
+@pytest.mark.parametrize("n,groups,sizes", CASES)
+def test_whole(n, groups, sizes):
+    labels, coeffs = _real_operator(n, groups, sizes, 10 * n + groups)
+    p = orc.Params(labels, coeffs)
+    assert np.all(p.cp.view(np.float64)[1::2] == 0.0)
+    print(f"[gpu] real build n={n} groups={groups} T={len(labels)}", flush=True)
+    ip, ind, dat = orc.build_csr(p)
+    _, data, indices, indptr = _op(labels, coeffs).to_matrix_mode("RowwiseUnsafeChunked/100").export()
+    assert indptr.tobytes() == ip.tobytes()
+    assert indices.tobytes() == ind.tobytes()
+    assert data.tobytes() == dat.tobytes()
+
+
+@pytest.mark.parametrize("n,groups,sizes", [(13, 300, [2, 4, 30]), (13, 1500, [4, 6]), (13, 20, [2, 2, 50])])
+def test_row_windows(n, groups, sizes):
+    from qrusty_amd import _lib as L
+    labels, coeffs = _real_operator(n, groups, sizes, n + groups)
+    p, op = orc.Params(labels, coeffs), _op(labels, coeffs)
+    h = op._handle(L.QR_PHASE_ROWWISE)
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for r0, r1 in [(0, 1), (5, 9), (31, 33), (100, 4500), (4097, 8192), (8191, 8192)]:
+        nnz = (r1 - r0) * h.G
+        # a guard entry on both sides
+        ix = torch.full((nnz + 2,), -7, dtype=torch.int64, device="cuda")
+        d = torch.full((nnz + 2,), 7.0, dtype=torch.complex128, device="cuda")
+        print(f"[gpu] real build rows {r0}..{r1} of n={n} groups={groups}", flush=True)
+        L.check(L.lib.qr_csr_build_rows(h.h, r0, r1, ctypes.c_void_p(ix.data_ptr() + 8),
+                                        ctypes.c_void_p(d.data_ptr() + 16), s))
+        ih, dh = ix.cpu().numpy(), d.cpu().numpy()
+        assert ih[0] == ih[-1] == -7 and dh[0] == dh[-1] == 7.0
+        for r in sorted({r0, (r0 + r1) // 2, r1 - 1}):
+            cols, vals = orc.make_row(p, r)
+            a = 1 + (r - r0) * h.G
+            assert np.array_equal(ih[a:a + h.G].view(np.uint64), cols)
+            assert dh[a:a + h.G].tobytes() == vals.tobytes()
