@@ -9,7 +9,6 @@
 #include "qr_internal.h"
 
 #include <algorithm>
-#include <cmath>
 #include <cstring>
 #include <numeric>
 #include <utility>
@@ -103,7 +102,7 @@ static void build_rank_lists(const std::vector<uint64_t> &gx, std::vector<uint32
 static void free_patterns(DeviceTables::Patterns &pt);
 
 void free_tables(DeviceTables &t) {
-    void *ptrs[] = {t.gx, t.gterm, t.tz, t.tc, t.rl_ptr, t.rl, t.gkind, t.heavy, t.leaf_heavy, t.real_heavy, t.real_ptr, t.real_terms, t.ttz, t.ttc};
+    void *ptrs[] = {t.gx, t.gterm, t.tz, t.tc, t.rl_ptr, t.rl, t.gkind, t.heavy, t.leaf_heavy, t.word_leaves, t.word_groups, t.word_rank, t.word_ptr, t.word_terms, t.ttz, t.ttc};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (auto &pt : t.pat) free_patterns(pt);
@@ -353,11 +352,23 @@ static int upload(T **dst, const std::vector<T> &src) {
 int upload_heavy(const qr_op *op, DeviceTables &t) {
     int rc;
     if ((!op->heavy.empty() && (rc = upload(&t.heavy, op->heavy))) ||
-        (!op->leaf_heavy.empty() && (rc = upload(&t.leaf_heavy, op->leaf_heavy))) ||
-        (!op->real_heavy.empty() && (rc = upload(&t.real_heavy, op->real_heavy))) ||
-        (!op->real_terms.empty() && ((rc = upload(&t.real_ptr, op->real_ptr)) ||
-                                     (rc = upload(&t.real_terms, op->real_terms)))))
+        (!op->leaf_heavy.empty() && (rc = upload(&t.leaf_heavy, op->leaf_heavy))) )
         return rc;
+    if (!op->word_leaves.empty()) {
+        // rank lists by bit, without the sub-operators' ancestors
+        std::vector<int32_t> rank(uint64_t(op->nq) * op->G, 0);
+        for (const auto &lf : op->word_leaves) {
+            uint32_t depth = 0;
+            for (int32_t v : lf.off) depth += v != 0;
+            for (uint32_t g = lf.s0; g < lf.s0 + lf.g; ++g)
+                for (uint32_t e = op->rl_ptr[g] + depth; e < op->rl_ptr[g + 1]; ++e)
+                    rank[uint64_t(op->rl[e].bit) * op->G + g] = op->rl[e].sigma;
+        }
+        if ((rc = upload(&t.word_leaves, op->word_leaves)) || (rc = upload(&t.word_groups, op->word_groups)) ||
+            (rc = upload(&t.word_rank, rank)) || (rc = upload(&t.word_ptr, op->word_ptr)) ||
+            (!op->word_terms.empty() && (rc = upload(&t.word_terms, op->word_terms))))
+            return rc;
+    }
     t.nheavy = uint32_t(op->heavy.size());
     if (!op->ntail) return QR_OK;
     std::vector<double2> c2(op->ttz.size());
@@ -550,9 +561,6 @@ void finish_op(qr_op *op) {
         }
     };
     cut(kSubMaxG, op->leaves);
-    op->real = true;
-    for (uint64_t i = 0; i < op->T; ++i) op->real = op->real && op->tc[2 * i + 1] == 0.0;
-    if (op->real) cut(kRealMaxG, op->real_leaves);
     // heavy groups: at least 8 terms and 4x the mean, the largest kMaxHeavy
     {
         const double mean = double(op->T) / double(op->G);
@@ -577,24 +585,47 @@ void finish_op(qr_op *op) {
             }
         };
         split(op->leaves, op->leaf_heavy);
-        split(op->real_leaves, op->real_heavy);
-        if (op->real && op->nq <= 32 && !op->heavy.empty()) {
-            auto list = [op](uint32_t g0, const uint32_t *heavy, uint32_t n) {
-                op->real_ptr.push_back(uint32_t(op->real_terms.size()));
-                for (uint32_t k = 0; k < n; ++k) {
-                    for (uint32_t i = op->gterm[g0 + heavy[k]]; i < op->gterm[g0 + heavy[k] + 1]; ++i)
-                        op->real_terms.push_back({op->tc[2 * i], uint32_t(op->tz[i]),
-                                                  std::signbit(op->tc[2 * i + 1]) ? 0x80000000u : 0u});
-                    op->real_ptr.push_back(uint32_t(op->real_terms.size()));
-                }
-            };
-            if (op->real_leaves.empty()) list(0, op->heavy.data(), uint32_t(op->heavy.size()));
-            for (const auto &lf : op->real_leaves) list(lf.s0, op->real_heavy.data() + lf.hoff, lf.hcnt);
+    }
+    if (op->nq <= 32) {
+        std::vector<qr_op::SubLeaf> leaves;
+        cut(kWordMaxG, leaves);
+        if (leaves.empty()) leaves.push_back({0, uint32_t(op->G), 0, 0, 0});
+        std::stable_sort(leaves.begin(), leaves.end(), [](const auto &a, const auto &b) {
+            auto threads = [](const auto &l) { return l.s1 - l.s0 <= 256 ? 0 : l.s1 - l.s0 <= 512 ? 1 : 2; };
+            return threads(a) < threads(b);
+        });
+        op->word_groups.resize(op->G);
+        for (const auto &l : leaves) {
+            WordLeaf lf{l.s0, l.s1 - l.s0, 0, uint32_t(op->word_ptr.size()), {}};
+            for (uint32_t e = op->rl_ptr[l.s0]; e < op->rl_ptr[l.s0] + l.depth; ++e) lf.off[op->rl[e].bit] = op->rl[e].sigma;
+            for (uint32_t g = l.s0; g < l.s1; ++g) {
+                const uint32_t t0 = op->gterm[g], t1 = op->gterm[g + 1];
+                op->word_groups[g] = {uint32_t(op->gx[g]), t0, t1 - t0, -1};
+                if (!std::binary_search(op->heavy.begin(), op->heavy.end(), g)) continue;
+                op->word_groups[g].heavy = int32_t(lf.hcnt++);
+                op->word_ptr.push_back(uint32_t(op->word_terms.size()));
+                for (uint32_t i = t0; i < t1; ++i)
+                    op->word_terms.push_back({op->tc[2 * i], op->tc[2 * i + 1], uint32_t(op->tz[i]), 0});
+            }
+            op->word_ptr.push_back(uint32_t(op->word_terms.size()));
+            op->word_leaves.push_back(lf);
         }
     }
+    // the form of the sign-word builder: terms past those it holds are loaded
+    // again for every row, so they have to be few
+    bool real = true;
+    for (uint64_t i = 0; i < op->T; ++i) real = real && op->tc[2 * i + 1] == 0.0;
+    uint64_t past = 0;
+    for (uint64_t g = 0; g < op->G; ++g) {
+        const uint64_t n = op->gterm[g + 1] - op->gterm[g];
+        if (n > kWordHold && !std::binary_search(op->heavy.begin(), op->heavy.end(), uint32_t(g)))
+            past += n - kWordHold;
+    }
+    op->word_real = real && 16 * past <= op->G;
     // tail table: operators with heavy groups, whose other groups also run
-    // past two terms (the molecular Hamiltonians: 4 and 6)
-    if (!op->heavy.empty()) {
+    // past two terms (the molecular Hamiltonians: 4 and 6), and those of many
+    // terms per group
+    if (!op->heavy.empty() || op->T >= 2 * op->G) {
         uint32_t nt = 0;
         for (uint64_t g = 0; g < op->G; ++g) {
             const uint32_t n = op->gterm[g + 1] - op->gterm[g];

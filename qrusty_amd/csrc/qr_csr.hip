@@ -15,9 +15,9 @@
 // which is exactly the reference's stable-sort-then-fold result, so indices
 // and values are bit-identical.  The kernel is bound by HBM writes (24 B per
 // nnz).  Rows are staged in LDS by the tile builder (qr_tile.h) and copied out
-// coalesced; an operator with more than kSubMaxG groups is built as
-// sub-operators, subtrees of the mask trie that fill a contiguous segment of
-// every row (qr_tile.h TileOp::gbase).
+// coalesced; an operator with more than kWordMaxG groups (kSubMaxG past 32
+// qubits) is built as sub-operators, subtrees of the mask trie that fill a
+// contiguous segment of every row.
 //
 // CSR matvec (replaces accel::rowwise::spmat_dot_densevec, accel.rs:338-370):
 // a power-of-two team of lanes per row streams the row's indices/values with
@@ -38,9 +38,10 @@ namespace qr {
 // neighbouring rows, which two blocks write parts of, meet in one L2, and an
 // XCD touches an eighth of the output's pages.  Launch order / this one (ms,
 // two output buffers each; their place moves the rate by up to 20%): 20 qubits
-// and 2000 random terms 9.42, 9.35 / 9.24, 8.55; 300 terms 1.39 / 1.23, 1.12;
-// 22 qubits, 60 terms 1.10, 0.96 / 1.01, 0.86; 20-qubit molecule 15.7, 12.5 /
-// 12.1, 11.4.  A grid that is no multiple of 8 keeps the launch order.
+// and 2000 random terms 10.5, 8.6 / 7.9, 7.4; 300 terms 1.34, 1.11 / 1.25,
+// 1.08; 24-qubit ring 1.79, 1.52 / 1.76, 1.46; 20-qubit molecule 13.3, 11.8 /
+// 11.0, 10.2.  Windows of 8 times 8 to 512 tiles lie between.  A grid that is
+// no multiple of 8 keeps the launch order.
 __device__ __forceinline__ uint32_t xcd_tile() {
     const uint32_t b = blockIdx.x, n = gridDim.x;
     return n % 8u == 0 ? (b % 8u) * (n / 8u) + b / 8u : b;
@@ -50,7 +51,7 @@ __device__ __forceinline__ uint32_t xcd_tile() {
 // (qr_tile.h), without the fused matvec; the heavy-group instances of
 // fold_tiles run 2^op.fold_log2 consecutive tiles per block, folding the
 // heavy groups once for all of them.
-template <bool kNarrow, int kChunks, int kMode>
+template <int kChunks, int kMode>
 __global__ __launch_bounds__(kStageThreads) void k_csr_build_staged(TileOp op) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     if constexpr (fold_tiles<kChunks, kMode>()) {
@@ -59,56 +60,62 @@ __global__ __launch_bounds__(kStageThreads) void k_csr_build_staged(TileOp op) {
         for (uint32_t s = 0; s < k; ++s) {
             const uint64_t tile = uint64_t(xcd_tile()) * k + s;
             if ((((op.row_begin >> tile_log2) + tile) << tile_log2) >= op.row_end) break;
-            build_tile_staged<kNarrow, kChunks, false, kMode>(op, tile, smem_raw, s);
+            build_tile_staged<false, kChunks, false, kMode>(op, tile, smem_raw, s);
         }
     } else {
-        build_tile_staged<kNarrow, kChunks, false, kMode>(op, xcd_tile(), smem_raw);
+        build_tile_staged<false, kChunks, false, kMode>(op, xcd_tile(), smem_raw);
     }
 }
 
-// Sub-operators of at most 32 qubits (at most 2048 groups, a 48 KB stage):
-// held to 64 VGPRs, i.e. 8 waves per SIMD, so that two 1024-thread blocks
-// share a CU
-template <bool kNarrow, int kChunks, int kMode>
-__global__ __launch_bounds__(kStageThreads, 8) void k_csr_build_sub(TileOp op) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    build_tile_staged<kNarrow, kChunks, false, kMode>(op, xcd_tile(), smem_raw);
-}
-
-// CSR build of operators whose coefficients c' are all real (molecular and spin
-// Hamiltonians), masks in 32 bits: one group per thread, and per row three
-// vector instructions per term.  Thread layout as in qr_tile.h (kT = RS rows x
-// JW lanes, the rows of a tile in M = 2^m_log2 batches of RS), but
-//  * the sign of a term over the tile's M rows is one 32-bit word, the parity
-//    of r & z for batch m in bit 31 - m (the parity is linear in r: the fixed
-//    bits give all or none, each of the five batch bits an alternating
-//    pattern).  It carries the coefficient's own sign, is shifted up once per
-//    batch and its top bit goes straight into the coefficient's sign bit: a
-//    shift, a bit-field insert and an addition per term, against mask, count,
-//    compare, selects and two additions (the imaginary part of a real
-//    coefficient is a signed zero, and a sum of signed zeros is -0 only if
-//    all are: one word per group, the AND of its terms');
+// The sign-word builder (operators of at most 32 qubits): one group per thread
+// and few vector instructions per term and row.  Thread layout as in qr_tile.h
+// (kT = RS rows x JW lanes, the rows of a tile in M = 2^m_log2 batches of RS),
+// but
+//  * kReal, for operators whose coefficients c' are all real and whose groups
+//    have few terms past kWordHold (molecular and spin Hamiltonians): a lane
+//    holds its group's terms.  The sign of a term over the tile's M rows is one
+//    32-bit word, the parity of r & z for batch m in bit 31 - m (the parity is
+//    linear in r: the fixed bits give all or none, each of the five batch bits
+//    an alternating pattern), shifted up once per batch; its top bit goes
+//    straight into the coefficient's sign bit: a shift, a bit-field insert and
+//    an addition per term, against mask, count, compare, selects and two
+//    additions.  (The imaginary part of a real coefficient is a signed zero,
+//    and a sum of signed zeros is -0 only if all are: one word per group, the
+//    AND of its terms'.)  Terms past those held come from memory;
+//  * otherwise every term is loaded once per four batches, whose rows differ
+//    in two bits and so in two sign flips, and added to four sums;
 //  * absent terms are -0.0, which every sum absorbs unchanged, so all lanes
-//    run the same six additions (two or four where no lane of the wave has
-//    more terms; terms past the sixth come from memory);
-//  * a row's slot moves by one addition per batch (the sigma of the bits that
-//    the step flips, qr_tile.h);
+//    run the same additions;
+//  * a lane's first slot comes from a table by row bit (word_rank), all its
+//    loads at once, where a walk along its rank list is a chain of them that a
+//    tile of 32 rows did not hide (20-qubit molecule 11.5 -> 10.2 ms, 16 qubits
+//    and 24069 groups 7.3 -> 5.9);
+//  * a row's slot moves by one addition per batch (what the bits that the step
+//    flips add, qr_tile.h);
 //  * 64 VGPRs: two 1024-thread blocks per CU, one copying out while the other
-//    computes, and two stages per block, one barrier per batch.
-// Groups of many terms (op.heavy) are folded by a pass of their own at the
-// start of the tile, one thread per (group, row).  The additions are the same,
-// in the same order, as build_tile_staged's, so the values are bit-identical.
-// Operators of more than kRealMaxG groups are built as sub-operators of at
-// most that many (kSub), each with the power of two of threads that holds it.
-// What bounds it: the stores (4.6-6.4 TB/s of 24 B per entry, by the place of
-// the output).  The builder of qr_tile.h / this one, us: molecules of 12 / 16 /
-// 18 / 20 qubits 139 / 510 / 4031 / 28360 -> 28 / 326 / 2020-2160 / 11500-13850;
-// 14-qubit ring 24.5 -> 10.5, 24 qubits 2147 -> 1560-1790.  Not used for more
-// than kRealMaxG groups of mostly one term, which two group chunks per thread
-// build faster (17 qubits, 2516 groups 1800 / 1954).
-constexpr int kRealHold = 6;      // terms of a group held in registers
-constexpr int kRealMaxLog2 = 5;   // batches per tile (log2)
-constexpr size_t kRealLDS = 80 * 1024;  // of one block: two per CU
+//    computes, and two stages per block, one barrier per batch;
+//  * M is chosen so that small operators still fill the chip.
+// Groups of many terms are folded by a pass of their own at the start of the
+// tile, one thread per (group, row), their terms in LDS.  The additions are
+// the same, in the same order, as build_tile_staged's, so the values are
+// bit-identical.  Operators of more than kWordMaxG groups are built as
+// sub-operators of at most that many (kSub), each with the power of two of
+// threads that holds it, consecutive blocks building the same rows.
+// What bounds it: the stores (5.2 or 6.5 TB/s of 24 B per entry, by the place
+// of the output in memory; fills reach 6.65), and from about five terms per
+// group on the additions and the loads of the terms.  The two-group-chunk
+// builder that it replaced / this one, us: molecules of 12 / 16 / 18 / 20
+// qubits 139 / 510 / 4030 / 28100 -> 20 / 290 / 1820-2430 / 10200-12500; rings
+// of 14 / 24 qubits 24.5 / 2160 -> 7.6 / 1480-1780; one-term groups, 12 qubits
+// (195 groups) 29 -> 7.9, 20 qubits (1999) 9000-9400 -> 7400-8900, 18 qubits
+// (4948) 7000 -> 4500-5600, 16 qubits (24069) 10010 -> 6200; terms of weight 1
+// to 4, 16 qubits (332 groups of 3.0 terms) 196 -> 104, 20 qubits (610 of 3.3)
+// 6350 -> 2900, 18 qubits (1208 of 6.6) 8790 -> 2580.  Holding four complex
+// terms per lane instead of loading them for every four batches: 600 groups of
+// 4 terms 688 against 775, but of 8 3620 against 1060, and a wave waits for
+// its longest group.
+constexpr int kWordMaxLog2 = 5;   // batches per tile (log2)
+constexpr uint32_t kWordLDS = 80 * 1024;  // of one block: two per CU
 
 // Sign words of the batch bits: bit b of m set <=> the bits of kSignWord[b]
 __device__ __forceinline__ uint32_t sign_word(uint32_t parity, uint32_t zm) {
@@ -127,200 +134,267 @@ __device__ __forceinline__ double with_sign(double c, uint32_t w) {
 }
 __device__ __forceinline__ uint32_t sign_of(double c) { return uint32_t(__double2hiint(c)) & 0x80000000u; }
 
-// Term-order fold in row r of the terms [t, t1) in LDS, four loaded ahead of
-// their additions.
-__device__ __forceinline__ double2 fold_real(const RealTerm *terms, uint32_t t, uint32_t t1, uint32_t r) {
-    uint32_t im = 0x80000000u;
-    auto term = [&](const RealTerm &a) {
-        const uint32_t s = uint32_t(__popc(r & a.z)) << 31;
-        im &= a.im ^ s;
-        return __hiloint2double(__double2hiint(a.c) ^ int(s), __double2loint(a.c));
-    };
-    double v = term(terms[t]);
-    ++t;
-    constexpr uint32_t kF = 4;
-    for (; t + kF <= t1; t += kF) {
-        RealTerm a[kF];
-#pragma unroll
-        for (uint32_t u = 0; u < kF; ++u) a[u] = terms[t + u];
-#pragma unroll
-        for (uint32_t u = 0; u < kF; ++u) v = v + term(a[u]);
-    }
-    for (; t < t1; ++t) v = v + term(terms[t]);
-    return make_double2(v, __hiloint2double(int(im), 0));
+__device__ __forceinline__ double flip(double c, uint32_t sign) {
+    return __hiloint2double(__double2hiint(c) ^ int(sign), __double2loint(c));
 }
 
-// The heavy groups' terms of one build (qr_op::real_ptr, real_terms), and the
-// LDS bytes before their values (two stages, which the terms use first).
-struct RealHeavy {
-    const uint32_t *ptr;
-    const RealTerm *terms;
-    uint32_t hv_at;
+// A heavy group's term in LDS, a broadcast read or two for a wave: the real
+// form's 16 bytes (re, z and the sign of im), the other's double2 and z apart.
+struct RealTerm {
+    double re;
+    uint32_t z, im;
+};
+template <bool kReal>
+struct HeavyTerms {
+    unsigned char *at;
+    uint32_t most;  // terms that fit
+    __device__ HeavyTerms(unsigned char *a, uint32_t bytes) : at(a), most(bytes / (kReal ? 16u : 20u)) {}
+    __device__ uint32_t *z() const { return reinterpret_cast<uint32_t *>(at + 16u * most); }
+    __device__ void put(uint32_t i, const WordTerm &t) const {
+        if constexpr (kReal) {
+            reinterpret_cast<RealTerm *>(at)[i] = RealTerm{t.re, t.z, sign_of(t.im)};
+        } else {
+            reinterpret_cast<double2 *>(at)[i] = make_double2(t.re, t.im);
+            z()[i] = t.z;
+        }
+    }
+    __device__ WordTerm get(uint32_t i) const {
+        if constexpr (kReal) {
+            const RealTerm t = reinterpret_cast<const RealTerm *>(at)[i];
+            return WordTerm{t.re, __hiloint2double(int(t.im), 0), t.z, 0};
+        } else {
+            const double2 c = reinterpret_cast<const double2 *>(at)[i];
+            return WordTerm{c.x, c.y, z()[i], 0};
+        }
+    }
 };
 
-template <bool kSub, int kT>
-__global__ __launch_bounds__(kT, 8) void k_csr_build_real(TileOp op, RealHeavy rh, uint32_t m_log2) {
+// v plus, in term order, the terms [t, t1) in row r, four loaded ahead of
+// their additions.
+template <bool kReal>
+__device__ __forceinline__ double2 fold_words(double2 v, const HeavyTerms<kReal> &terms, uint32_t t, uint32_t t1,
+                                              uint32_t r) {
+    uint32_t im = sign_of(v.y);
+    auto add = [&](const WordTerm &e) {
+        const uint32_t s = uint32_t(__popc(r & e.z)) << 31;
+        v.x = v.x + flip(e.re, s);
+        if (kReal) im &= sign_of(e.im) ^ s;
+        else v.y = v.y + flip(e.im, s);
+    };
+    constexpr uint32_t kF = 4;
+    for (; t + kF <= t1; t += kF) {
+        WordTerm e[kF];
+#pragma unroll
+        for (uint32_t u = 0; u < kF; ++u) e[u] = terms.get(t + u);
+#pragma unroll
+        for (uint32_t u = 0; u < kF; ++u) add(e[u]);
+    }
+    for (; t < t1; ++t) add(terms.get(t));
+    if (kReal) v.y = __hiloint2double(int(im), 0);
+    return v;
+}
+
+// What the builder runs on: the operator's tables, the sub-operators of this
+// launch (one: the whole operator, if !kSub), and its outputs (indptr null:
+// not this launch).
+struct WordOp {
+    const WordLeaf *leaves;
+    const WordGroup *groups;
+    const int32_t *rank;
+    const uint64_t *tz, *ttz;  // terms, and the tail table (qr_op::ttz, ttc)
+    const double2 *tc, *ttc;
+    const uint32_t *ptr;       // heavy groups' terms
+    const WordTerm *terms;
+    uint64_t *indptr, *indices;
+    double2 *data;
+    uint64_t row_begin, row_end;
+    uint32_t G, nq, nleaves, ntail, jw_log2, m_log2;
+};
+
+// LDS of a block: two stages, whose place the heavy groups' terms take first
+// (in turns of that size), and those groups' values: as many of them as leave
+// two blocks to a CU; the rest run term by term.
+struct WordLds {
+    uint32_t nheavy, hv_at, total;
+    __host__ __device__ WordLds(uint32_t g, uint32_t rs_log2, uint32_t tile_log2, uint32_t hcnt, const uint32_t *ptr) {
+        const uint32_t stage = (((g << rs_log2) + 1u) & ~1u) * 48u, each = 16u << tile_log2;
+        const uint32_t fit = (kWordLDS - stage) / each;
+        nheavy = hcnt < fit ? hcnt : fit;
+        hv_at = stage;
+        if (nheavy) {
+            const uint32_t room = kWordLDS - nheavy * each, n = ptr[nheavy] - ptr[0];
+            const uint32_t want = n < room / 20u ? (20u * n + 15u) & ~15u : room;
+            if (want > hv_at) hv_at = want;
+        }
+        total = hv_at + nheavy * each;
+    }
+};
+
+template <bool kReal, bool kSub, int kT>
+__global__ __launch_bounds__(kT, 8) void k_csr_build_words(WordOp op) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const TileMem mem = tile_mem(op);
-    const uint32_t G = op.G, jw_log2 = op.jw_log2;
+    const uint32_t block = xcd_tile(), tile = kSub ? block / op.nleaves : block;
+    const WordLeaf &lf = op.leaves[kSub ? block - tile * op.nleaves : 0u];
+    const uint32_t G = lf.g, s0 = lf.s0, hcnt = lf.hcnt, at = lf.at, jw_log2 = op.jw_log2;
     const uint32_t rs_log2 = kSub ? 0u : uint32_t(__builtin_ctz(kT)) - jw_log2;
-    const uint32_t tile_log2 = rs_log2 + m_log2, M = 1u << m_log2;
+    const uint32_t m_log2 = op.m_log2, tile_log2 = rs_log2 + m_log2, M = 1u << m_log2;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = kSub ? tid : tid & ((1u << jw_log2) - 1u);
     const uint32_t ro = kSub ? 0u : tid >> jw_log2;
     const uint64_t row_begin = op.row_begin, row_end = op.row_end;
-    const uint64_t tile_base = ((row_begin >> tile_log2) + xcd_tile()) << tile_log2;
+    const uint64_t tile_base = ((row_begin >> tile_log2) + tile) << tile_log2;
     const uint32_t rfix = uint32_t(tile_base) | ro;  // at most 32 bits of row
     const uint32_t batch_pad = ((G << rs_log2) + 1u) & ~1u;
     const uint32_t stage_b = batch_pad * 24u;
-    double2 *hv = reinterpret_cast<double2 *>(smem_raw + rh.hv_at);
+    const WordLds lds(G, rs_log2, tile_log2, hcnt, op.ptr + at);
+    const uint32_t nheavy = lds.nheavy;
+    double2 *hv = reinterpret_cast<double2 *>(smem_raw + lds.hv_at);
+
+    if (op.indptr && (!kSub || block == tile * op.nleaves)) {
+        const uint64_t r0 = max(row_begin, tile_base), r1 = min(row_end, tile_base + (1ull << tile_log2));
+        const uint64_t g = op.G;
+        for (uint64_t r = r0 + tid; r < r1 + (r1 == row_end); r += kT) op.indptr[r - row_begin] = r * g;
+    }
 
     // heavy groups first, before the lanes' own terms take registers: their
     // terms into LDS, then one thread per (group, row)
-    if (op.nheavy) {
-        const auto hptr = as_global(rh.ptr);
-        const uint32_t h0 = hptr[0];
-        uint4 *to = reinterpret_cast<uint4 *>(smem_raw);
-        const uint4 *from = reinterpret_cast<const uint4 *>(rh.terms + h0);
-        for (uint32_t i = tid; i < hptr[op.nheavy] - h0; i += kT) to[i] = from[i];
-        __syncthreads();
-        const uint32_t tr = 1u << tile_log2;
-        for (uint32_t i = tid; i < op.nheavy << tile_log2; i += kT) {
-            const uint32_t g = i >> tile_log2, r = uint32_t(tile_base) + (i & (tr - 1u));
-            hv[i] = fold_real(reinterpret_cast<const RealTerm *>(smem_raw), hptr[g] - h0, hptr[g + 1] - h0, r);
+    if (nheavy) {
+        const auto hptr = as_global(op.ptr) + at;
+        const HeavyTerms<kReal> terms(smem_raw, lds.hv_at);
+        const uint32_t h0 = hptr[0], nt = hptr[nheavy] - h0;
+        for (uint32_t i = tid; i < nheavy << tile_log2; i += kT) hv[i] = make_double2(-0.0, -0.0);
+        for (uint32_t t0 = 0; t0 < nt; t0 += terms.most) {
+            const uint32_t t1 = min(t0 + terms.most, nt);
+            if (t0) __syncthreads();  // the terms before
+            for (uint32_t i = tid; i < t1 - t0; i += kT) terms.put(i, op.terms[h0 + t0 + i]);
+            __syncthreads();
+            for (uint32_t i = tid; i < nheavy << tile_log2; i += kT) {
+                const uint32_t g = i >> tile_log2, r = uint32_t(tile_base) + (i & ((1u << tile_log2) - 1u));
+                const uint32_t a = max(hptr[g] - h0, t0), e = min(hptr[g + 1] - h0, t1);
+                if (a < e) hv[i] = fold_words<kReal>(hv[i], terms, a - t0, e - t0, r);
+            }
         }
         // (the barrier after the lanes' setup, which overlaps the long groups)
     }
 
-    // slot of the lane's group in row rfix, and its change when the batch
-    // index goes from m to m + 1 with t = ctz(m + 1): sigma of bit t minus
-    // those of the bits below, which turn off
-    int32_t sig[kRealMaxLog2] = {0, 0, 0, 0, 0};
-    int32_t slot = int32_t(kSub ? op.gbase + lane : ro * G + lane);
-    auto take = [&](const RankEntry &en, int32_t sign, int32_t &at) {
-        const uint32_t b = uint32_t(en.bit), q = b - rs_log2;  // wraps for b < rs_log2
-        if (q >= m_log2) at += (rfix >> b) & 1u ? sign * en.sigma : 0;
-#pragma unroll
-        for (uint32_t k = 0; k < uint32_t(kRealMaxLog2); ++k)
-            if (q == k && q < m_log2) sig[k] += sign * en.sigma;
-    };
-    int32_t off = 0, osig[kRealMaxLog2] = {0, 0, 0, 0, 0};
+    // place of the lane's group in row rfix, and its change when the batch
+    // index goes from m to m + 1 with t = ctz(m + 1): what bit t adds minus
+    // what the bits below, which turn off, did
+    int32_t slot = int32_t(ro * G + lane);
+    int32_t step[kWordMaxLog2] = {0, 0, 0, 0, 0};
+    // the same of the sub-operator's first entry
+    int32_t off = int32_t(s0), ostep[kWordMaxLog2] = {0, 0, 0, 0, 0};
     if (kSub) {
-        // the sub-operator's first rank (qr_tile.h)
-        off = int32_t(op.gbase);
-        for (uint32_t e = 0; e < op.nanc; ++e) {
-            const RankEntry en = ld_rank(mem.rl + mem.rl_ptr[0] + e);
-            const uint32_t b = uint32_t(en.bit);
-            if (b >= m_log2) off += (rfix >> b) & 1u ? en.sigma : 0;
+        int32_t below = 0;
 #pragma unroll
-            for (uint32_t k = 0; k < uint32_t(kRealMaxLog2); ++k)
-                if (b == k && b < m_log2) osig[k] += en.sigma;
+        for (uint32_t b = 0; b < 32; ++b) {
+            const int32_t v = lf.off[b];
+            if (b >= m_log2) off += (rfix >> b) & 1u ? v : 0;
+            if (b < uint32_t(kWordMaxLog2)) ostep[b] = v - below;
+            below += v;
         }
     }
     const bool valid = lane < G;
     int32_t hs = -1;
     uint32_t xj = 0, n = 0, tf = 0, wi = 0xffffffffu;
-    uint32_t w[kRealHold];
-    double c[kRealHold];
+    uint32_t w[kWordHold];
+    double c[kWordHold];
 #pragma unroll
-    for (int u = 0; u < kRealHold; ++u) {
+    for (int u = 0; u < int(kWordHold); ++u) {
         w[u] = 0xffffffffu;  // -0.0
         c[u] = 0.0;
     }
+    const auto gtz = as_global(op.tz), gttz = as_global(op.ttz);
+    const auto gtc = as_global(reinterpret_cast<const dvec2 *>(op.tc));
+    const auto gttc = as_global(reinterpret_cast<const dvec2 *>(op.ttc));
+    // term u of the lane's group: those past the second from the tail table
+    // (coalesced) as far as it goes
+    auto load = [&](uint32_t u) {
+        const bool tail = u >= 2 && u - 2 < op.ntail;
+        const uint32_t i = tail ? (u - 2) * op.G + s0 + lane : tf + u;
+        const double2 cc = ld2((tail ? gttc : gtc) + i);
+        return WordTerm{cc.x, cc.y, uint32_t(tail ? gttz[i] : gtz[i]), 0};
+    };
     if (valid) {
-        const uint32_t e1 = mem.rl_ptr[lane + 1];
-        for (uint32_t e = mem.rl_ptr[lane]; e < e1; ++e) take(ld_rank(mem.rl + e), 1, slot);
-        uint32_t lo = 0, hi = op.nheavy;  // heavy groups ascend
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (mem.heavy[mid] < lane) lo = mid + 1;
-            else hi = mid;
-        }
-        if (lo < op.nheavy && mem.heavy[lo] == lane) hs = int32_t(lo);
-        xj = uint32_t(mem.gx[lane]);
-        tf = mem.gterm[lane];
-        if (hs < 0) {
-            n = mem.gterm[lane + 1] - tf;
+        const auto rank = as_global(op.rank) + s0 + lane;
+        int32_t below = 0;
 #pragma unroll
-            for (int u = 0; u < kRealHold; ++u) {
-                if (uint32_t(u) >= n) break;
-                // terms past the second from the tail table (coalesced)
-                const bool tail = u >= 2 && uint32_t(u - 2) < op.ntail;
-                const uint32_t at = tail ? uint32_t(u - 2) * op.gstride + lane : tf + uint32_t(u);
-                const uint32_t z = uint32_t(tail ? mem.ttz[at] : mem.tz[at]);
-                const double2 cc = ld2((tail ? mem.ttc : mem.tc) + at);
-                const uint32_t s = sign_word(__popc(rfix & z), (z >> rs_log2) & (M - 1u));
-                w[u] = s ^ (sign_of(cc.x) ? 0xffffffffu : 0u);
-                wi &= s ^ (sign_of(cc.y) ? 0xffffffffu : 0u);
-                c[u] = cc.x;
+        for (uint32_t k = 0; k < uint32_t(kWordMaxLog2); ++k) {
+            const uint32_t b = rs_log2 + k;
+            const int32_t v = k < m_log2 && b < op.nq ? rank[b * op.G] : 0;
+            step[k] = v - below;
+            below += v;
+        }
+        for (uint32_t b = 0; b < rs_log2 && b < op.nq; ++b) slot += (ro >> b) & 1u ? rank[b * op.G] : 0;
+        for (uint32_t b = tile_log2; b < op.nq; ++b)
+            if ((uint32_t(tile_base) >> b) & 1u) slot += rank[b * op.G];
+        const WordGroup gr = op.groups[s0 + lane];
+        xj = gr.x;
+        tf = gr.tf;
+        hs = gr.heavy < int32_t(nheavy) ? gr.heavy : -1;
+        if (hs < 0) {
+            n = gr.n;
+            if constexpr (kReal) {
+#pragma unroll
+                for (int u = 0; u < int(kWordHold); ++u) {
+                    if (uint32_t(u) >= n) break;
+                    const WordTerm t = load(uint32_t(u));
+                    const uint32_t s = sign_word(__popc(rfix & t.z), (t.z >> rs_log2) & (M - 1u));
+                    w[u] = s ^ (sign_of(t.re) ? 0xffffffffu : 0u);
+                    wi &= s ^ (sign_of(t.im) ? 0xffffffffu : 0u);
+                    c[u] = t.re;
+                }
             }
         }
     }
-    slot -= off;
-    int32_t step[kRealMaxLog2];
-    {
-        int32_t below = 0;
-#pragma unroll
-        for (int k = 0; k < kRealMaxLog2; ++k) {
-            const int32_t s = sig[k] - osig[k];
-            step[k] = s - below;
-            below += s;
-        }
-    }
-    if (op.nheavy) __syncthreads();
+    if (nheavy) __syncthreads();
     // the wave's longest group, in registers and past them
-    const bool more2 = __any(n > 2), more4 = __any(n > 4), past = __any(n > uint32_t(kRealHold));
+    const bool more2 = __any(n > 2), more4 = __any(n > 4), past = __any(n > kWordHold);
 
     // the batch's entries, in LDS: written at the lane's slot, copied out by
     // consecutive threads (a batch has at most kT of them)
     const uint32_t stage_entries = G << rs_log2;
     const bool whole = tile_base >= row_begin && tile_base + (uint64_t(M) << rs_log2) <= row_end;
     // output place of the batch's first row (before row_begin: not used)
-    uint64_t dst = (tile_base - row_begin) * (kSub ? op.gstride : G);
+    uint64_t dst = (tile_base - row_begin) * op.G;
     if (kSub) dst += uint64_t(int64_t(off));
-    const uint64_t dst_step = uint64_t(kSub ? op.gstride : G) << rs_log2;
-    int32_t ostep[kRealMaxLog2];
-    {
-        int32_t below = 0;
-#pragma unroll
-        for (int k = 0; k < kRealMaxLog2; ++k) {
-            ostep[k] = osig[k] - below;
-            below += osig[k];
-        }
-    }
-    auto batch = [&](uint32_t m, uint32_t buf) {
+    const uint64_t dst_step = uint64_t(op.G) << rs_log2;
+    const auto indices = as_global(op.indices);
+    const auto data = as_global(reinterpret_cast<dvec2 *>(op.data));
+    auto batch = [&](uint32_t m, uint32_t buf, double2 e) {
         uint64_t *si = reinterpret_cast<uint64_t *>(smem_raw + buf * stage_b);
         double2 *sd = reinterpret_cast<double2 *>(si + batch_pad);
         const uint32_t r = rfix + (m << rs_log2);
         if (valid && (whole || (uint64_t(r) >= row_begin && uint64_t(r) < row_end))) {
-            double v = with_sign(c[0], w[0]);
-            v = v + with_sign(c[1], w[1]);
-            if (more2) {
-                v = v + with_sign(c[2], w[2]);
-                v = v + with_sign(c[3], w[3]);
-            }
-            if (more4) {
-                v = v + with_sign(c[4], w[4]);
-                v = v + with_sign(c[5], w[5]);
-            }
-            uint32_t im = wi;
-            if (past) {
-                for (uint32_t u = kRealHold; u < n; ++u) {
-                    const bool tail = u - 2 < op.ntail;
-                    const uint32_t at = tail ? (u - 2) * op.gstride + lane : tf + u;
-                    const double2 cc = ld2((tail ? mem.ttc : mem.tc) + at);
-                    const uint32_t s = uint32_t(__popc(r & uint32_t(tail ? mem.ttz[at] : mem.tz[at]))) << 31;
-                    v = v + __hiloint2double(__double2hiint(cc.x) ^ int(s), __double2loint(cc.x));
-                    im &= sign_of(cc.y) ^ s;
+            if constexpr (kReal) {
+                // term-order fold: first value, then + (accel.rs:191-208)
+                e.x = with_sign(c[0], w[0]);
+                e.x = e.x + with_sign(c[1], w[1]);
+                if (more2) {
+                    e.x = e.x + with_sign(c[2], w[2]);
+                    e.x = e.x + with_sign(c[3], w[3]);
                 }
+                if (more4) {
+                    e.x = e.x + with_sign(c[4], w[4]);
+                    e.x = e.x + with_sign(c[5], w[5]);
+                }
+                uint32_t im = wi;
+                if (past) {
+                    for (uint32_t u = kWordHold; u < n; ++u) {
+                        const WordTerm t = load(u);
+                        const uint32_t sg = uint32_t(__popc(r & t.z)) << 31;
+                        e.x = e.x + flip(t.re, sg);
+                        im &= sign_of(t.im) ^ sg;
+                    }
+                }
+                e.y = __hiloint2double(int(im & 0x80000000u), 0);
             }
-            double2 e = make_double2(v, __hiloint2double(int(im & 0x80000000u), 0));
             if (hs >= 0) e = hv[(uint32_t(hs) << tile_log2) | (m << rs_log2) | ro];
             si[slot] = r ^ xj;
             sd[slot] = e;
         }
 #pragma unroll
-        for (int u = 0; u < kRealHold; ++u) w[u] <<= 1;
+        for (int u = 0; u < int(kWordHold); ++u) w[u] <<= 1;
         wi <<= 1;
         __syncthreads();
         bool mine = tid < stage_entries;
@@ -330,9 +404,9 @@ __global__ __launch_bounds__(kT, 8) void k_csr_build_real(TileOp op, RealHeavy r
             mine = mine && row >= row_begin && row < row_end;
         }
         if (mine) {
-            mem.indices[dst + tid] = si[tid];
+            indices[dst + tid] = si[tid];
             const double2 dv = sd[tid];
-            mem.data[dst + tid] = dvec2{dv.x, dv.y};
+            data[dst + tid] = dvec2{dv.x, dv.y};
         }
     };
     auto advance = [&](int t) {
@@ -340,15 +414,41 @@ __global__ __launch_bounds__(kT, 8) void k_csr_build_real(TileOp op, RealHeavy r
         dst += dst_step;
         if (kSub) dst += uint64_t(int64_t(ostep[t]));
     };
+    // !kReal: the lane's group in the rows of four batches, each term loaded
+    // once for the four and two in flight (-0.0, the absent term, first: every
+    // sum absorbs it unchanged)
+    double2 e4[4] = {};
+    auto fold4 = [&](uint32_t m) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) e4[k] = make_double2(-0.0, -0.0);
+        const uint32_t r = rfix + (m << rs_log2);
+        auto add = [&](const WordTerm &t) {
+            const uint32_t s0 = uint32_t(__popc(r & t.z)) << 31;
+            const uint32_t za = (t.z >> rs_log2) << 31, zb = (t.z >> (rs_log2 + 1u)) << 31;
+            const uint32_t sg[4] = {s0, s0 ^ za, s0 ^ zb, s0 ^ za ^ zb};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                e4[k].x = e4[k].x + flip(t.re, sg[k]);
+                e4[k].y = e4[k].y + flip(t.im, sg[k]);
+            }
+        };
+        for (uint32_t u = 0; u < n; u += 2) {
+            WordTerm t0 = load(u), t1{-0.0, -0.0, 0, 0};
+            if (u + 1 < n) t1 = load(u + 1);
+            add(t0);
+            add(t1);
+        }
+    };
 #pragma unroll 1
     for (uint32_t m = 0; m < M; m += 4) {  // M is at least 4
-        batch(m, 0);
+        if constexpr (!kReal) fold4(m);
+        batch(m, 0, e4[0]);
         advance(0);
-        batch(m + 1, 1);
+        batch(m + 1, 1, e4[1]);
         advance(1);
-        batch(m + 2, 0);
+        batch(m + 2, 0, e4[2]);
         advance(0);
-        batch(m + 3, 1);
+        batch(m + 3, 1, e4[3]);
         const uint32_t t = uint32_t(__builtin_ctz(m + 4u));  // 2 to 5 (the end)
         if (t == 2) advance(2);
         else if (t == 3) advance(3);
@@ -362,36 +462,39 @@ __global__ __launch_bounds__(256) void k_indptr(uint64_t row_begin, uint64_t nro
     if (i <= nrows) indptr[i] = (row_begin + i) * G;
 }
 
-// Builds of real operators (k_csr_build_real): the whole operator, or one
-// launch per sub-operator of op->real_leaves.
-static int launch_build_real(const qr_op *op, const DeviceTables *t, uint64_t row_begin, uint64_t row_end,
-                             uint64_t *d_indices, double *d_data, hipStream_t s) {
+// Builds by k_csr_build_words: the whole operator, or one launch for all
+// sub-operators of a number of threads.
+static int launch_build_words(const qr_op *op, const DeviceTables *t, uint64_t row_begin, uint64_t row_end,
+                              uint64_t *d_indptr, uint64_t *d_indices, double *d_data, hipStream_t s) {
     const uint32_t G = uint32_t(op->G);
-    auto run = [&](auto sub_t, auto threads_t, TileOp top, uint32_t rs_log2, size_t at) {
+    auto run = [&](auto sub_t, auto threads_t, uint32_t jw, size_t first, size_t last) {
         constexpr bool kSub = decltype(sub_t)::value;
         constexpr int kT = decltype(threads_t)::value;
-        // batches per tile: as many as leave the launch four blocks per CU
-        uint32_t ml = kRealMaxLog2;
-        while (ml > 2 && ((row_end - row_begin) >> (rs_log2 + ml)) < 1024) --ml;
+        const uint32_t nl = uint32_t(last - first), rs_log2 = kSub ? 0u : uint32_t(__builtin_ctz(kT)) - jw;
+        // batches per tile: as many as the sign words of the real form have, and
+        // as many where the tile folds heavy groups; half of that for the rest,
+        // which loads its terms again anyway (20 qubits, 2000 terms 7.5 / 7.4
+        // ms; weights 1 to 4, 2000 terms 2.9 / 3.5); fewer where the launch
+        // would have under four blocks per CU
+        uint32_t ml = op->word_real || t->nheavy ? kWordMaxLog2 : kWordMaxLog2 - 1;
+        while (ml > 2 && nl * ((row_end - row_begin) >> (rs_log2 + ml)) < 1024) --ml;
         const uint32_t tl = rs_log2 + ml;
-        const uint64_t nt = ((row_end - 1) >> tl) - (row_begin >> tl) + 1;
+        const uint64_t nt = nl * (((row_end - 1) >> tl) - (row_begin >> tl) + 1);
         if (nt > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "CSR build grid too large");
-        // heavy groups (their terms first in the stages' place, their values
-        // behind) as LDS allows with two blocks per CU; the rest run term by
-        // term
-        const size_t stage = size_t(((top.G << rs_log2) + 1u) & ~1u) * 24 * 2, each = size_t(16) << tl;
-        const uint32_t *ptr = top.nheavy ? op->real_ptr.data() + at : nullptr;
-        auto front = [&](uint32_t n) {
-            const size_t terms = n ? size_t(ptr[n] - ptr[0]) * sizeof(RealTerm) : 0;
-            return std::max(stage, terms);
-        };
-        while (top.nheavy && front(top.nheavy) + top.nheavy * each > kRealLDS) --top.nheavy;
-        const RealHeavy rh{t->real_ptr + at, t->real_terms, uint32_t(front(top.nheavy))};
-        const size_t shmem = rh.hv_at + top.nheavy * each;
-        auto kern = k_csr_build_real<kSub, kT>;
-        QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
-        hipLaunchKernelGGL(kern, dim3(unsigned(nt)), dim3(kT), shmem, s, top, rh, ml);
+        uint32_t shmem = 0;
+        for (size_t k = first; k < last; ++k) {
+            const WordLeaf &lf = op->word_leaves[k];
+            shmem = std::max(shmem, WordLds(lf.g, rs_log2, tl, lf.hcnt, op->word_ptr.data() + lf.at).total);
+        }
+        const WordOp args{t->word_leaves + first, t->word_groups, t->word_rank, t->tz, t->ttz, t->tc, t->ttc,
+                          t->word_ptr, t->word_terms, d_indptr, d_indices, reinterpret_cast<double2 *>(d_data),
+                          row_begin, row_end, G, uint32_t(op->nq), nl, t->ntail, jw, ml};
+        d_indptr = nullptr;  // by the first launch
+        auto kern = op->word_real ? k_csr_build_words<true, kSub, kT> : k_csr_build_words<false, kSub, kT>;
+        if (shmem > 64 * 1024)
+            QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
+        hipLaunchKernelGGL(kern, dim3(unsigned(nt)), dim3(kT), shmem, s, args);
         QR_HIP_CHECK(hipGetLastError());
         return int(QR_OK);
     };
@@ -400,26 +503,19 @@ static int launch_build_real(const qr_op *op, const DeviceTables *t, uint64_t ro
     using T256 = std::integral_constant<int, 256>;
     using T512 = std::integral_constant<int, 512>;
     using T1024 = std::integral_constant<int, 1024>;
-    auto tile_op = [&](uint32_t g0, uint32_t g, uint32_t depth, const uint32_t *heavy, uint32_t nheavy, uint32_t jw) {
-        return TileOp{t->gx + g0, t->gterm + g0, t->tz, t->tc, t->rl_ptr + g0, t->rl, d_indices,
-                      reinterpret_cast<double2 *>(d_data), nullptr, nullptr, nullptr, row_begin, row_end, g, jw, 1,
-                      1, heavy, nheavy, g0, depth, G, t->ntail ? t->ttz + g0 : nullptr,
-                      t->ntail ? t->ttc + g0 : nullptr, t->ntail, 0};
+    const auto &lv = op->word_leaves;
+    if (lv.size() == 1) return run(F{}, T1024{}, stage_jw_log2(G), 0, 1);
+    auto to = [&](uint32_t most) {
+        size_t k = 0;
+        while (k < lv.size() && lv[k].g <= most) ++k;
+        return k;
     };
-    if (op->real_leaves.empty()) {
-        const uint32_t jw = stage_jw_log2(G);
-        return run(F{}, T1024{}, tile_op(0, G, 0, t->heavy, t->nheavy, jw), 10u - jw, 0);
-    }
-    for (size_t k = 0; k < op->real_leaves.size(); ++k) {
-        const auto &lf = op->real_leaves[k];
-        const uint32_t g = lf.s1 - lf.s0;
-        const TileOp top = tile_op(lf.s0, g, lf.depth, t->real_heavy + lf.hoff, lf.hcnt, 0);
-        const int rc = g <= 256   ? run(T{}, T256{}, top, 0, lf.hoff + k)
-                       : g <= 512 ? run(T{}, T512{}, top, 0, lf.hoff + k)
-                                  : run(T{}, T1024{}, top, 0, lf.hoff + k);
-        if (rc) return rc;
-    }
-    return QR_OK;
+    const size_t a = to(256), b = to(512), c = lv.size();
+    int rc = QR_OK;
+    if (a && (rc = run(T{}, T256{}, 0, 0, a))) return rc;
+    if (b > a && (rc = run(T{}, T512{}, 0, a, b))) return rc;
+    if (c > b) rc = run(T{}, T1024{}, 0, b, c);
+    return rc;
 }
 
 int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin, uint64_t row_end,
@@ -427,6 +523,9 @@ int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin,
     const uint64_t nrows = row_end - row_begin;
     if (op->G > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "too many groups");
     const uint32_t G = uint32_t(op->G);
+    if (op->nq <= 32 && nrows)
+        return launch_build_words(op, t, row_begin, row_end, d_indptr, d_indices, d_data, s);
+    // wider masks: the shared tile builder
     if (d_indptr) {
         uint64_t nb = (nrows + 1 + 255) / 256;
         hipLaunchKernelGGL(k_indptr, dim3(unsigned(nb)), dim3(256), 0, s, row_begin, nrows,
@@ -434,9 +533,6 @@ int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin,
         QR_HIP_CHECK(hipGetLastError());
     }
     if (nrows == 0) return QR_OK;
-    const bool narrow = op->nq <= 32;
-    if (op->real && narrow && (G <= kRealMaxG || 4 * op->T >= 5 * op->G))
-        return launch_build_real(op, t, row_begin, row_end, d_indices, d_data, s);
     if (!op->leaves.empty()) {
         // one sub-operator per subtree of the mask trie, each <= kSubMaxG
         // groups with one row per batch (JW = 1024): the fast 1- and 2-chunk
@@ -459,16 +555,8 @@ int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin,
                        row_begin, row_end, g, jw, nch, dbuf,
                        nh ? t->leaf_heavy + lf.hoff : nullptr, nh, lf.s0, lf.depth, G,
                        t->ntail ? t->ttz + lf.s0 : nullptr, t->ntail ? t->ttc + lf.s0 : nullptr, t->ntail, fl};
-            // (wide masks, and heavy groups, do not fit 64 VGPRs without
-            // spills: one block per CU)
-            auto kst = nh ? (narrow ? (nch <= 1 ? k_csr_build_staged<true, 1, kTileSubHeavy>
-                                                : k_csr_build_staged<true, 2, kTileSubHeavy>)
-                                    : (nch <= 1 ? k_csr_build_staged<false, 1, kTileSubHeavy>
-                                                : k_csr_build_staged<false, 2, kTileSubHeavy>))
-                          : (narrow ? (nch <= 1 ? k_csr_build_sub<true, 1, kTileSub>
-                                                : k_csr_build_sub<true, 2, kTileSub>)
-                                    : (nch <= 1 ? k_csr_build_staged<false, 1, kTileSub>
-                                                : k_csr_build_staged<false, 2, kTileSub>));
+            auto kst = nh ? (nch <= 1 ? k_csr_build_staged<1, kTileSubHeavy> : k_csr_build_staged<2, kTileSubHeavy>)
+                          : (nch <= 1 ? k_csr_build_staged<1, kTileSub> : k_csr_build_staged<2, kTileSub>);
             QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kst),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
             hipLaunchKernelGGL(kst, dim3(unsigned(((nt - 1) >> fl) + 1)), dim3(kStageThreads), shmem, s, top);
@@ -495,14 +583,8 @@ int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin,
     TileOp top{t->gx, t->gterm, t->tz, t->tc, t->rl_ptr, t->rl, d_indices,
                reinterpret_cast<double2 *>(d_data), nullptr, nullptr, nullptr,
                row_begin, row_end, G, jw, nch, dbuf, t->heavy, nh, 0, 0, G, t->ttz, t->ttc, t->ntail, fl};
-    auto pick = [&](auto narrow_t, auto heavy_t) {
-        constexpr bool kN = decltype(narrow_t)::value;
-        constexpr int kH = decltype(heavy_t)::value ? kTileHeavy : kTilePlain;
-        return nch <= 1 ? k_csr_build_staged<kN, 1, kH> : k_csr_build_staged<kN, 2, kH>;
-    };
-    using T = std::true_type;
-    using F = std::false_type;
-    auto kst = narrow ? (nh ? pick(T{}, T{}) : pick(T{}, F{})) : (nh ? pick(F{}, T{}) : pick(F{}, F{}));
+    auto kst = nh ? (nch <= 1 ? k_csr_build_staged<1, kTileHeavy> : k_csr_build_staged<2, kTileHeavy>)
+                  : (nch <= 1 ? k_csr_build_staged<1, kTilePlain> : k_csr_build_staged<2, kTilePlain>);
     QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kst),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
     hipLaunchKernelGGL(kst, dim3(unsigned(((nt - 1) >> fl) + 1)), dim3(kStageThreads), shmem, s, top);

@@ -50,7 +50,8 @@ constexpr uint32_t kMaxHeavy = 128;
 constexpr uint32_t kMaxTail = 16;
 constexpr uint64_t kMaxTailSlots = uint64_t(1) << 22;
 constexpr uint32_t kSubMaxG = 2048;  // groups of one CSR-build sub-operator
-constexpr uint32_t kRealMaxG = 1024;  // the same, operators of real coefficients
+constexpr uint32_t kWordMaxG = 1024;  // the same of the sign-word builder
+constexpr uint32_t kWordHold = 6;     // terms of a group that it holds (real form)
 // CSR matvecs load the CSR stream nontemporally from this many entries per
 // row on (measured crossover; qr_csr.hip)
 constexpr uint64_t kMvNontemporalMinRow = 256;
@@ -136,11 +137,26 @@ constexpr int kMaxWindows = 3;
 
 constexpr int kApplySlots = 6;
 
-// A term of an operator with real coefficients and masks of 32 bits: Re c',
-// z, and the sign of Im c' (a signed zero) in bit 31.
-struct RealTerm {
-    double c;
-    uint32_t z, im;
+// A term of a heavy group (masks of 32 bits): c' and z.
+struct WordTerm {
+    double re, im;
+    uint32_t z, pad;
+};
+
+// A sub-operator of the sign-word builder: the g groups from s0, a subtree of
+// the mask trie; the heavy ones' terms are word_terms[word_ptr[at + k] ..
+// word_ptr[at + k + 1]), k < hcnt.  In row r its groups begin at position
+// s0 + the sum of off[b] over the bits b of r.
+struct WordLeaf {
+    uint32_t s0, g, hcnt, at;
+    int32_t off[32];
+};
+
+// A group: its x mask, its first term, its number of terms, and which of its
+// sub-operator's heavy groups it is (-1: none).
+struct WordGroup {
+    uint32_t x, tf, n;
+    int32_t heavy;
 };
 
 // Device copies of an operator's tables (one set per device that used it).
@@ -159,9 +175,11 @@ struct DeviceTables {
     double2 *ttc = nullptr;
     uint32_t ntail = 0;
     uint32_t *leaf_heavy = nullptr;  // qr_op::leaf_heavy
-    uint32_t *real_heavy = nullptr;  // qr_op::real_heavy, real_ptr, real_terms
-    uint32_t *real_ptr = nullptr;
-    RealTerm *real_terms = nullptr;
+    WordLeaf *word_leaves = nullptr;  // qr_op::word_leaves, word_groups, word_ptr, word_terms
+    WordGroup *word_groups = nullptr;
+    int32_t *word_rank = nullptr;  // [nq][G]: what bit b of r adds to the place of group g in its sub-operator
+    uint32_t *word_ptr = nullptr;
+    WordTerm *word_terms = nullptr;
     // matrix-free apply tables, one set per tile kind and form (slot =
     // 2 * kind + staged; kind 0: FP64, 1: complex64, 2: small complex64 tiles)
     // and pass (slot + kApplySlots * (k + 1): window pass k)
@@ -259,16 +277,16 @@ struct qr_op {
     };
     std::vector<SubLeaf> leaves;
     std::vector<uint32_t> leaf_heavy;  // heavy groups of each leaf, leaf-local
-    // every coefficient c' is real: the builder of k_csr_build_real, on
-    // sub-operators of at most kRealMaxG groups
-    bool real = false;
-    std::vector<SubLeaf> real_leaves;
-    std::vector<uint32_t> real_heavy;
-    // the terms of the heavy groups, one list per real_leaves entry (or one
-    // for the whole operator): group k of list i has the terms
-    // real_terms[real_ptr[hoff + i + k] .. real_ptr[hoff + i + k + 1])
-    std::vector<uint32_t> real_ptr;
-    std::vector<qr::RealTerm> real_terms;
+    // the sign-word builder (k_csr_build_words; at most 32 qubits): its form,
+    // real if every coefficient c' is and few groups have terms past
+    // kWordHold; the whole operator or its sub-operators of at most kWordMaxG
+    // groups, those of at most 256, 512 and 1024 groups one after another;
+    // every group, and the terms of the heavy ones
+    bool word_real = false;
+    std::vector<qr::WordLeaf> word_leaves;
+    std::vector<qr::WordGroup> word_groups;
+    std::vector<uint32_t> word_ptr;
+    std::vector<qr::WordTerm> word_terms;
     // operators with heavy groups: the terms past each group's second,
     // transposed (slot u * G + g holds term gterm[g] + 2 + u, zero where the
     // group is shorter), so that the lanes of a batch -- one group each --

@@ -1,6 +1,6 @@
-"""CSR builds of operators with real coefficients (k_csr_build_real): bit-exact
-against the oracle's rows at the edges of its layout -- groups of 1 to past 6
-terms, zero coefficients of both signs, one and many rows per batch,
+"""CSR builds by sign words (k_csr_build_words), real and complex coefficients:
+bit-exact against the oracle's rows at the edges of its layout -- groups of 1 to
+past the terms held in registers, zero coefficients of both signs, one and many rows per batch,
 sub-operators, more heavy groups than LDS holds, and row windows that begin
 and end inside a tile."""
 import ctypes
@@ -33,20 +33,23 @@ def _label(n, xm, zm):
     return "".join("IXZY"[((xm >> q) & 1) | (((zm >> q) & 1) << 1)] for q in reversed(range(n)))
 
 
-def _real_operator(n, groups, sizes, seed):
+def _operator(n, groups, sizes, seed, real):
     """`groups` masks of sizes[k % len(sizes)] terms each, in shuffled order,
-    every c' real (an even number of Y, or an odd one with an imaginary
-    coefficient), some coefficients 0.0 or -0.0."""
+    some coefficients 0.0 or -0.0.  `real`: every c' real (an even number of Y,
+    or an odd one with an imaginary coefficient)."""
     rng = np.random.default_rng(seed)
     masks = rng.choice(1 << n, size=min(groups, 1 << n), replace=False)
     labels, coeffs = [], []
     for k, xm in enumerate(masks):
         for _ in range(sizes[k % len(sizes)]):
             zm = int(rng.integers(0, 1 << n))
-            c = float(rng.choice([0.0, -0.0, rng.normal()], p=[0.05, 0.05, 0.9]))
-            odd = bin(int(xm) & zm).count("1") % 2
+            c, d = (float(rng.choice([0.0, -0.0, rng.normal()], p=[0.05, 0.05, 0.9])) for _ in range(2))
+            if real:
+                d = float(rng.choice([0.0, -0.0]))
+                if bin(int(xm) & zm).count("1") % 2:
+                    c, d = 0.0, c
             labels.append(_label(n, int(xm), zm))
-            coeffs.append(complex(0.0, c) if odd else complex(c, rng.choice([0.0, -0.0])))
+            coeffs.append(complex(c, d))
     order = rng.permutation(len(labels))
     return [labels[i] for i in order], [coeffs[i] for i in order]
 
@@ -56,12 +59,13 @@ CASES = [(3, 1, [1]), (5, 7, [1, 2]), (9, 25, [2, 2, 2, 48]), (8, 200, [1, 2, 3,
          (12, 90, [40] * 60 + [2] * 30), (10, 130, [12])]
 
 
+@pytest.mark.parametrize("real", [True, False])
 @pytest.mark.parametrize("n,groups,sizes", CASES)
-def test_whole(n, groups, sizes):
-    labels, coeffs = _real_operator(n, groups, sizes, 10 * n + groups)
+def test_whole(n, groups, sizes, real):
+    labels, coeffs = _operator(n, groups, sizes, 10 * n + groups, real)
     p = orc.Params(labels, coeffs)
-    assert np.all(p.cp.view(np.float64)[1::2] == 0.0)
-    print(f"[gpu] real build n={n} groups={groups} T={len(labels)}", flush=True)
+    assert real == bool(np.all(p.cp.view(np.float64)[1::2] == 0.0))
+    print(f"[gpu] build real={real} n={n} groups={groups} T={len(labels)}", flush=True)
     ip, ind, dat = orc.build_csr(p)
     _, data, indices, indptr = _op(labels, coeffs).to_matrix_mode("RowwiseUnsafeChunked/100").export()
     assert indptr.tobytes() == ip.tobytes()
@@ -69,10 +73,11 @@ def test_whole(n, groups, sizes):
     assert data.tobytes() == dat.tobytes()
 
 
+@pytest.mark.parametrize("real", [True, False])
 @pytest.mark.parametrize("n,groups,sizes", [(13, 300, [2, 4, 30]), (13, 1500, [4, 6]), (13, 20, [2, 2, 50])])
-def test_row_windows(n, groups, sizes):
+def test_row_windows(n, groups, sizes, real):
     from qrusty_amd import _lib as L
-    labels, coeffs = _real_operator(n, groups, sizes, n + groups)
+    labels, coeffs = _operator(n, groups, sizes, n + groups, real)
     p, op = orc.Params(labels, coeffs), _op(labels, coeffs)
     h = op._handle(L.QR_PHASE_ROWWISE)
     s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -81,7 +86,7 @@ def test_row_windows(n, groups, sizes):
         # a guard entry on both sides
         ix = torch.full((nnz + 2,), -7, dtype=torch.int64, device="cuda")
         d = torch.full((nnz + 2,), 7.0, dtype=torch.complex128, device="cuda")
-        print(f"[gpu] real build rows {r0}..{r1} of n={n} groups={groups}", flush=True)
+        print(f"[gpu] build real={real} rows {r0}..{r1} of n={n} groups={groups}", flush=True)
         L.check(L.lib.qr_csr_build_rows(h.h, r0, r1, ctypes.c_void_p(ix.data_ptr() + 8),
                                         ctypes.c_void_p(d.data_ptr() + 16), s))
         ih, dh = ix.cpu().numpy(), d.cpu().numpy()
