@@ -39,18 +39,18 @@ static int parse_label(const char *s, uint32_t *nq, uint32_t *base_phase, uint32
     if (*p == 'i' || *p == 'j') { imag = true; ++p; }
     size_t n = std::strlen(p);
     if (n == 0) return fail(QR_ERR_LABEL, "error: malformed label");
+    bool known = true;
     for (size_t k = 0; k < n; ++k)
-        if (p[k] != 'I' && p[k] != 'X' && p[k] != 'Y' && p[k] != 'Z')
-            return fail(QR_ERR_LABEL, "error: malformed label");
+        known &= (p[k] == 'I') | (p[k] == 'X') | (p[k] == 'Y') | (p[k] == 'Z');
+    if (!known) return fail(QR_ERR_LABEL, "error: malformed label");
     if (n > 63) return fail(QR_ERR_SIZE, "Pauli labels of more than 63 qubits are not supported");
     uint64_t xm = 0, zm = 0;
-    uint32_t y = 0;
-    for (size_t q = 0; q < n; ++q) {
-        char c = p[n - 1 - q];
-        if (c == 'X' || c == 'Y') xm |= uint64_t(1) << q;
-        if (c == 'Y' || c == 'Z') zm |= uint64_t(1) << q;
-        if (c == 'Y') ++y;
+    for (size_t k = 0; k < n; ++k) {
+        const char c = p[k];
+        xm = 2 * xm | uint64_t((c == 'X') | (c == 'Y'));
+        zm = 2 * zm | uint64_t((c == 'Y') | (c == 'Z'));
     }
+    const uint32_t y = uint32_t(__builtin_popcountll(xm & zm));
     *nq = uint32_t(n);
     *base_phase = (imag ? 1u : 0u) + (neg ? 2u : 0u);
     *ny = y;
@@ -70,41 +70,39 @@ static int parse_label(const char *s, uint32_t *nq, uint32_t *base_phase, uint32
 // Each (bit, sigma) pair is one RankEntry; a path has at most min(n, G-1) of them.
 static void build_rank_lists(const std::vector<uint64_t> &gx, std::vector<uint32_t> &ptr,
                              std::vector<RankEntry> &out) {
-    const size_t G = gx.size();
-    std::vector<std::vector<RankEntry>> lists(G);
-    struct Range { size_t lo, hi; };
-    std::vector<Range> stack;
-    stack.push_back({0, G});
-    while (!stack.empty()) {
-        Range rg = stack.back();
-        stack.pop_back();
-        if (rg.hi - rg.lo <= 1) continue;
-        uint64_t diff = gx[rg.lo] ^ gx[rg.hi - 1];
-        int b = 63 - __builtin_clzll(diff);
-        uint64_t bit = uint64_t(1) << b;
-        // sorted and sharing all bits above b: first index with bit b set
-        size_t m = size_t(std::partition_point(gx.begin() + rg.lo, gx.begin() + rg.hi,
-                                               [bit](uint64_t v) { return (v & bit) == 0; }) -
-                          gx.begin());
-        int32_t right = int32_t(rg.hi - m), left = int32_t(m - rg.lo);
-        for (size_t j = rg.lo; j < m; ++j) lists[j].push_back({b, right});
-        for (size_t j = m; j < rg.hi; ++j) lists[j].push_back({b, -left});
-        stack.push_back({rg.lo, m});
-        stack.push_back({m, rg.hi});
-    }
-    ptr.assign(G + 1, 0);
-    for (size_t j = 0; j < G; ++j) ptr[j + 1] = ptr[j] + uint32_t(lists[j].size());
+    const uint32_t G = uint32_t(gx.size());
+    ptr.assign(size_t(G) + 1, 0);
     out.clear();
-    out.reserve(ptr[G]);
-    for (size_t j = 0; j < G; ++j) out.insert(out.end(), lists[j].begin(), lists[j].end());
+    RankEntry path[64];
+    auto walk = [&](auto &self, uint32_t lo, uint32_t hi, int depth) -> void {
+        if (hi - lo <= 1) {
+            out.insert(out.end(), path, path + depth);
+            ptr[hi] = uint32_t(out.size());
+            return;
+        }
+        const uint64_t diff = gx[lo] ^ gx[hi - 1];
+        const int b = 63 - __builtin_clzll(diff);
+        const uint64_t bit = uint64_t(1) << b;
+        // sorted and sharing all bits above b: first index with bit b set
+        const uint32_t m = uint32_t(std::partition_point(gx.begin() + lo, gx.begin() + hi,
+                                                         [bit](uint64_t v) { return (v & bit) == 0; }) -
+                                    gx.begin());
+        path[depth] = {b, int32_t(hi - m)};
+        self(self, lo, m, depth + 1);
+        path[depth] = {b, -int32_t(m - lo)};
+        self(self, m, hi, depth + 1);
+    };
+    walk(walk, 0, G, 0);
 }
 
 static void free_patterns(DeviceTables::Patterns &pt);
 
 void free_tables(DeviceTables &t) {
-    void *ptrs[] = {t.gx, t.gterm, t.tz, t.tc, t.rl_ptr, t.rl, t.gkind, t.heavy, t.leaf_heavy, t.word_leaves, t.word_groups, t.word_rank, t.word_ptr, t.word_terms, t.ttz, t.ttc};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
+    if (t.apart)
+        for (void *p : {(void *)t.gx, (void *)t.gterm, (void *)t.tz, (void *)t.tc, (void *)t.rl_ptr, (void *)t.rl,
+                        (void *)t.gkind})
+            if (p) (void)hipFree(p);
+    if (t.mem) (void)hipFree(t.mem);
     for (auto &pt : t.pat) free_patterns(pt);
     t = DeviceTables{};
 }
@@ -117,8 +115,9 @@ struct PartBuild {
     uint64_t basis[kPartRank] = {}, red[kPartRank] = {};
     uint32_t comb[kPartRank] = {};
     int rank = 0;
-    std::vector<size_t> pats;
-    std::vector<uint32_t> code;  // coordinates of each pattern's zl
+    uint32_t n = 0;
+    size_t pats[1 << kPartRank];
+    uint32_t code[1 << kPartRank];  // coordinates of each pattern's zl
     // v minus its component in the span; the component's coordinates in *c
     uint64_t reduce(uint64_t v, uint32_t *c) const {
         *c = 0;
@@ -147,8 +146,8 @@ struct PartBuild {
             c = 1u << rank;  // zl in the basis
             ++rank;
         }
-        pats.push_back(p);
-        code.push_back(c);
+        pats[n] = p;
+        code[n++] = c;
         return true;
     }
     // table index bits of row bit i
@@ -239,24 +238,34 @@ void build_patterns(const qr_op *op, const PatternShape &shape, const std::vecto
         cur_bytes = 0;
         gcls.clear();
     };
+    if (pass.empty()) {
+        out.grp.reserve(op->G);
+        out.tab.reserve(op->G);
+        out.pat.reserve(16 * op->G);
+        out.ptz.reserve(op->T);
+        out.ptc.reserve(2 * op->T);
+    }
+    std::vector<std::pair<uint64_t, uint32_t>> zt;  // a group's (zl, term)
+    std::vector<size_t> heads;                      // first term of each pattern
+    std::vector<PartBuild> parts;
+    std::vector<uint32_t> where;
     for (uint64_t k = 0; k < op->G; ++k) {
         const uint64_t g = staged ? op->G - 1 - k : k;
         if (!pass.empty() && pass[g] != id) continue;
         // window passes keep the mask in the tile's row order
         const uint64_t gm = win.s ? tile_bits(op->gx[g]) : op->gx[g];
-        std::vector<std::pair<uint64_t, uint32_t>> zt;  // (zl, term) by zl, terms in input order
+        zt.clear();
         for (uint32_t i = op->gterm[g]; i < op->gterm[g + 1]; ++i)
             zt.emplace_back(pairs ? pair_row_bits(tile_bits(op->tz[i]), tb) : tile_bits(op->tz[i]), i);
-        std::stable_sort(zt.begin(), zt.end(),
-                         [](const auto &a, const auto &b) { return a.first < b.first; });
-        std::vector<size_t> heads;  // first term of each pattern
+        std::sort(zt.begin(), zt.end());
+        heads.clear();
         for (size_t i = 0; i < zt.size(); ++i)
             if (i == 0 || zt[i].first != zt[i - 1].first) heads.push_back(i);
         heads.push_back(zt.size());
         const size_t npat = heads.size() - 1;
         for (size_t s0 = 0; s0 < npat; s0 += shape.psplit) {
             const size_t s1 = std::min(npat, s0 + shape.psplit);
-            std::vector<PartBuild> parts;
+            parts.clear();
             for (size_t s = s0; s < s1; ++s) {
                 const uint64_t zl = zt[heads[s]].first;
                 bool placed = false;
@@ -281,26 +290,33 @@ void build_patterns(const qr_op *op, const PatternShape &shape, const std::vecto
                 return at;
             };
             if (place(cur_bytes, nullptr) > shape.tcap) close_chunk();
-            std::vector<uint32_t> where;
+            where.clear();
             cur_bytes = place(cur_bytes, &where);
             ApplyGroup a{};
             a.m = gm;
             bool rowvar = false;
             for (size_t k = 0; k < parts.size(); ++k) {
                 const PartBuild &p = parts[k];
-                auto span = [&p](int bit0, int nbits, uint32_t v) {  // index of bits [bit0, bit0 + nbits) = v
-                    uint32_t c = 0;
-                    for (int i = 0; i < nbits; ++i)
-                        if ((v >> i) & 1) c ^= p.col(bit0 + i);
-                    return c;
+                // index of the bits [bit0, bit0 + nbits) = v
+                auto span = [&p](int bit0, int nbits, uint32_t *to) {
+                    to[0] = 0;
+                    for (int i = 0; i < nbits; ++i) {
+                        const uint32_t c = p.col(bit0 + i);
+                        for (uint32_t v = 0; v < 1u << i; ++v) to[v | 1u << i] = to[v] ^ c;
+                    }
                 };
+                uint32_t s0[8], s1[8], s2[4], sr[8];
+                span(0, 3, s0);
+                span(3, 3, s1);
+                span(6, 2, s2);
+                span(tb, 3, sr);
                 ApplyPart ap{};
                 for (uint32_t v = 0; v < 8; ++v) {
-                    ap.w0 |= span(0, 3, v) << (4 * v);
-                    ap.w1 |= span(3, 3, v) << (4 * v);
-                    ap.rc |= uint64_t(span(tb, 3, v) << lg) << (8 * v);
+                    ap.w0 |= s0[v] << (4 * v);
+                    ap.w1 |= s1[v] << (4 * v);
+                    ap.rc |= uint64_t(sr[v] << lg) << (8 * v);
                 }
-                for (uint32_t v = 0; v < 4; ++v) ap.w2 |= (span(6, 2, v) << lg) << (8 * v);
+                for (uint32_t v = 0; v < 4; ++v) ap.w2 |= (s2[v] << lg) << (8 * v);
                 ap.tab = (shape.tab0 + where[k]) / 4;
                 rowvar = rowvar || ap.rc;
                 if (parts.size() == 1) {
@@ -316,8 +332,9 @@ void build_patterns(const qr_op *op, const PatternShape &shape, const std::vecto
                     }
                     out.part.push_back(ap);
                 }
-                std::vector<size_t> by_code(16, npat);
-                for (size_t i = 0; i < p.pats.size(); ++i) by_code[p.code[i]] = p.pats[i];
+                size_t by_code[16];
+                std::fill(by_code, by_code + 16, npat);
+                for (uint32_t i = 0; i < p.n; ++i) by_code[p.code[i]] = p.pats[i];
                 for (uint32_t c = 0; c < 16; ++c) {
                     ApplyRange pr{uint32_t(out.ptz.size()), 0};
                     for (size_t q = by_code[c] < npat ? heads[by_code[c]] : 0;
@@ -340,23 +357,62 @@ void build_patterns(const qr_op *op, const PatternShape &shape, const std::vecto
     close_chunk();
 }
 
-template <typename T>
-static int upload(T **dst, const std::vector<T> &src) {
-    size_t bytes = std::max<size_t>(src.size(), 1) * sizeof(T);
-    QR_HIP_CHECK(hipMalloc((void **)dst, bytes));
-    if (!src.empty()) QR_HIP_CHECK(hipMemcpy(*dst, src.data(), src.size() * sizeof(T),
-                                             hipMemcpyHostToDevice));
-    return QR_OK;
-}
+// Arrays that go to the device in one allocation and, up to kStageBytes, one
+// copy: each allocation and each copy of its own costs 10-20 us, which a small
+// operator's dozen tables made the larger part of its first call.
+class TableSet {
+    static constexpr size_t kStageBytes = size_t(32) << 20;
+    struct Piece {
+        void **dst;
+        const void *src;
+        size_t bytes, at;
+    };
+    std::vector<Piece> pieces_;
+    size_t total_ = 0;
 
-int upload_heavy(const qr_op *op, DeviceTables &t) {
-    int rc;
-    if ((!op->heavy.empty() && (rc = upload(&t.heavy, op->heavy))) ||
-        (!op->leaf_heavy.empty() && (rc = upload(&t.leaf_heavy, op->leaf_heavy))) )
-        return rc;
+  public:
+    template <typename T>
+    void add(T **dst, const void *src, size_t n) {
+        pieces_.push_back({reinterpret_cast<void **>(dst), src, n * sizeof(T), total_});
+        total_ += (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~size_t(255);
+    }
+    template <typename T>
+    void add(T **dst, const std::vector<T> &src) { add(dst, src.data(), src.size()); }
+    int upload(void **mem) const {
+        QR_HIP_CHECK(hipMalloc(mem, total_));
+        unsigned char *base = static_cast<unsigned char *>(*mem);
+        if (total_ <= kStageBytes) {
+            std::vector<unsigned char> host(total_);
+            for (const Piece &p : pieces_)
+                if (p.bytes) std::memcpy(host.data() + p.at, p.src, p.bytes);
+            QR_HIP_CHECK(hipMemcpy(base, host.data(), total_, hipMemcpyHostToDevice));
+        } else {
+            for (const Piece &p : pieces_)
+                if (p.bytes) QR_HIP_CHECK(hipMemcpy(base + p.at, p.src, p.bytes, hipMemcpyHostToDevice));
+        }
+        for (const Piece &p : pieces_) *p.dst = base + p.at;
+        return QR_OK;
+    }
+};
+
+// with_base: also the tables that qr_group.hip builds on the device
+int upload_tables(const qr_op *op, DeviceTables &t, bool with_base) {
+    TableSet set;
+    if (with_base) {
+        set.add(&t.gx, op->gx);
+        set.add(&t.gterm, op->gterm);
+        set.add(&t.tz, op->tz);
+        set.add(&t.tc, op->tc.data(), op->T);
+        set.add(&t.rl_ptr, op->rl_ptr);
+        set.add(&t.rl, op->rl);
+        set.add(&t.gkind, op->gkind);
+    }
+    if (!op->heavy.empty()) set.add(&t.heavy, op->heavy);
+    if (!op->leaf_heavy.empty()) set.add(&t.leaf_heavy, op->leaf_heavy);
+    std::vector<int32_t> rank;
     if (!op->word_leaves.empty()) {
         // rank lists by bit, without the sub-operators' ancestors
-        std::vector<int32_t> rank(uint64_t(op->nq) * op->G, 0);
+        rank.resize(uint64_t(op->nq) * op->G);
         for (const auto &lf : op->word_leaves) {
             uint32_t depth = 0;
             for (int32_t v : lf.off) depth += v != 0;
@@ -364,16 +420,19 @@ int upload_heavy(const qr_op *op, DeviceTables &t) {
                 for (uint32_t e = op->rl_ptr[g] + depth; e < op->rl_ptr[g + 1]; ++e)
                     rank[uint64_t(op->rl[e].bit) * op->G + g] = op->rl[e].sigma;
         }
-        if ((rc = upload(&t.word_leaves, op->word_leaves)) || (rc = upload(&t.word_groups, op->word_groups)) ||
-            (rc = upload(&t.word_rank, rank)) || (rc = upload(&t.word_ptr, op->word_ptr)) ||
-            (!op->word_terms.empty() && (rc = upload(&t.word_terms, op->word_terms))))
-            return rc;
+        set.add(&t.word_leaves, op->word_leaves);
+        set.add(&t.word_groups, op->word_groups);
+        set.add(&t.word_rank, rank);
+        set.add(&t.word_ptr, op->word_ptr);
+        set.add(&t.word_terms, op->word_terms);
     }
+    if (op->ntail) {
+        set.add(&t.ttz, op->ttz);
+        set.add(&t.ttc, op->ttc.data(), op->ttz.size());
+    }
+    t.apart = !with_base;
+    if (int rc = set.upload(&t.mem)) return rc;
     t.nheavy = uint32_t(op->heavy.size());
-    if (!op->ntail) return QR_OK;
-    std::vector<double2> c2(op->ttz.size());
-    for (size_t i = 0; i < c2.size(); ++i) c2[i] = make_double2(op->ttc[2 * i], op->ttc[2 * i + 1]);
-    if ((rc = upload(&t.ttz, op->ttz)) || (rc = upload(&t.ttc, c2))) return rc;
     t.ntail = op->ntail;
     return QR_OK;
 }
@@ -388,14 +447,7 @@ int device_tables(const qr_op *op, DeviceTables **out, bool noalloc) {
         return fail(QR_ERR_ARG, "apply_noalloc: the operator's tables are not on this device "
                                 "(one qr_pauli_apply of it on this device uploads them)");
     if (!t.ready) {
-        int rc;
-        std::vector<double2> tc2(op->T);
-        for (uint64_t i = 0; i < op->T; ++i) tc2[i] = make_double2(op->tc[2 * i], op->tc[2 * i + 1]);
-        if ((rc = upload(&t.gx, op->gx)) || (rc = upload(&t.gterm, op->gterm)) ||
-            (rc = upload(&t.tz, op->tz)) || (rc = upload(&t.tc, tc2)) ||
-            (rc = upload(&t.rl_ptr, op->rl_ptr)) || (rc = upload(&t.rl, op->rl)) ||
-            (rc = upload(&t.gkind, op->gkind)) ||
-            (rc = upload_heavy(op, t))) {
+        if (int rc = upload_tables(op, t, true)) {
             free_tables(t);
             return rc;
         }
@@ -480,15 +532,16 @@ bool choose_windows(const qr_op *op, int L, int elem_log2, std::vector<ApplyWind
 }
 
 static int upload_patterns(DeviceTables::Patterns &pt, const HostPatterns &hp, const PatternShape &shape) {
-    std::vector<double2> c2(hp.ptz.size());
-    for (size_t i = 0; i < c2.size(); ++i) c2[i] = make_double2(hp.ptc[2 * i], hp.ptc[2 * i + 1]);
-    int rc;
-    if ((rc = upload(&pt.grp, hp.grp)) || (rc = upload(&pt.chunk, hp.chunk)) ||
-        (shape.staged && (rc = upload(&pt.run, hp.run))) ||
-        (rc = upload(&pt.part, hp.part)) || (rc = upload(&pt.tab, hp.tab)) ||
-        (rc = upload(&pt.pat, hp.pat)) ||
-        (rc = upload(&pt.ptz, hp.ptz)) || (rc = upload(&pt.ptc, c2)))
-        return rc;
+    TableSet set;
+    set.add(&pt.grp, hp.grp);
+    set.add(&pt.chunk, hp.chunk);
+    if (shape.staged) set.add(&pt.run, hp.run);
+    set.add(&pt.part, hp.part);
+    set.add(&pt.tab, hp.tab);
+    set.add(&pt.pat, hp.pat);
+    set.add(&pt.ptz, hp.ptz);
+    set.add(&pt.ptc, hp.ptc.data(), hp.ptz.size());
+    if (int rc = set.upload(&pt.mem)) return rc;
     pt.ngrp = uint32_t(hp.grp.size());
     pt.nchunk = uint32_t(hp.chunk.size());
     pt.nrun = uint32_t(hp.run.size());
@@ -500,9 +553,7 @@ static int upload_patterns(DeviceTables::Patterns &pt, const HostPatterns &hp, c
 }
 
 static void free_patterns(DeviceTables::Patterns &pt) {
-    for (void *p : {(void *)pt.grp, (void *)pt.chunk, (void *)pt.run, (void *)pt.part, (void *)pt.tab,
-                    (void *)pt.pat, (void *)pt.ptz, (void *)pt.ptc})
-        if (p) (void)hipFree(p);
+    if (pt.mem) (void)hipFree(pt.mem);
     pt = DeviceTables::Patterns{};
 }
 
@@ -738,15 +789,14 @@ int qr_op_create(const char *const *labels, const double *coeffs, uint64_t num_t
         op->cp[2 * t] = M[p][0] * coeffs[2 * t] - M[p][1] * coeffs[2 * t + 1];
         op->cp[2 * t + 1] = M[p][0] * coeffs[2 * t + 1] + M[p][1] * coeffs[2 * t];
     }
-    // group by x: stable sort keeps input order inside a group
-    std::vector<uint32_t> order(T);
-    std::iota(order.begin(), order.end(), 0u);
-    std::stable_sort(order.begin(), order.end(),
-                     [op](uint32_t a, uint32_t b) { return op->x[a] < op->x[b]; });
+    // group by x, input order inside a group
+    std::vector<std::pair<uint64_t, uint32_t>> order(T);
+    for (uint64_t t = 0; t < T; ++t) order[t] = {op->x[t], uint32_t(t)};
+    std::sort(order.begin(), order.end());
     op->tz.resize(T);
     op->tc.resize(2 * T);
     for (uint64_t i = 0; i < T; ++i) {
-        uint32_t t = order[i];
+        const uint32_t t = order[i].second;
         if (i == 0 || op->x[t] != op->gx.back()) {
             op->gx.push_back(op->x[t]);
             op->gterm.push_back(uint32_t(i));

@@ -162,6 +162,10 @@ struct WordGroup {
 // Device copies of an operator's tables (one set per device that used it).
 struct DeviceTables {
     bool ready = false;
+    // what holds the arrays: one allocation, or (tables built on the device,
+    // qr_group.hip) one for those uploaded and gx to gkind each their own
+    void *mem = nullptr;
+    bool apart = false;
     uint64_t *gx = nullptr;      // [G]   distinct x masks, ascending
     uint32_t *gterm = nullptr;   // [G+1] term range of each group
     uint64_t *tz = nullptr;      // [T]   z masks, grouped (term order inside a group)
@@ -185,6 +189,7 @@ struct DeviceTables {
     // and pass (slot + kApplySlots * (k + 1): window pass k)
     struct Patterns {
         int L = -1;
+        void *mem = nullptr;  // holds the arrays
         uint32_t ngrp = 0, nchunk = 0, nrun = 0, max_tab = 0;
         uint32_t nfar = 0;  // groups whose mask reaches outside the tile
         ApplyGroup *grp = nullptr;    // [ngrp]
@@ -314,7 +319,7 @@ int group_terms_device(const char *const *labels, const double *coeffs, uint64_t
 // are set.
 void finish_op(qr_op *op);
 // Uploads the op's heavy groups and tail table (where it has them) into t.
-int upload_heavy(const qr_op *op, DeviceTables &t);
+int upload_tables(const qr_op *op, DeviceTables &t, bool with_base);
 // Frees one device's tables of an op.
 void free_tables(DeviceTables &t);
 
