@@ -342,14 +342,12 @@ int qr_pauli_apply_noalloc(const qr_op *op, int32_t precision, uint32_t nvec, co
 /* ------------------------------------------------------------------------
  * Batches (no counterpart in the reference, which builds and applies one
  * operator at a time: lib.rs:573-585, accel.rs:338-370).  One call builds the
- * CSR of every operator of the batch and one matvec y_k = A_k x_k each, as
- * persistent kernels that take (operator, row tile) items from atomic
- * counters, recorded in a hipGraph (replayed while the buffers and tuning stay
- * the same).  Split form: two build kernels, whose items are every
- * operator's tiles (as sub-operators of at most 2048 groups), then one matvec
- * kernel over the written CSRs.  Fused form: one build-and-apply kernel per
- * register class, plus the single-operator kernels for operators of more
- * than 6144 groups.  CSR entries are bit-identical to qr_csr_build; y_k is
+ * CSR of every operator of the batch and one product y_k = A_k x_k each, as
+ * parallel branches of a hipGraph (replayed while the buffers and tuning stay
+ * the same); operators of at most 2^21 entries share a persistent kernel.
+ * Fused form: y_k by the matrix-free apply (small operators: from the entries
+ * as they are built).  Split form: the builds, then one matvec kernel over
+ * the written CSRs.  CSR entries are bit-identical to qr_csr_build; y_k is
  * computed in FP64 with FMAs.
  *   d_indptr[k], d_indices[k], d_data[k] : CSR outputs sized as for
  *       qr_csr_build, or NULL (all three, or the arrays themselves) to keep
@@ -363,11 +361,13 @@ int qr_pauli_apply_noalloc(const qr_op *op, int32_t precision, uint32_t nvec, co
  * ---------------------------------------------------------------------- */
 typedef struct qr_batch qr_batch;
 typedef struct {
-    uint32_t tiles_per_item;  /* row tiles per work item (1..4096)          */
-    uint32_t blocks_per_cu;   /* persistent blocks per compute unit (1..8)  */
+    uint32_t tiles_per_item;  /* row tiles per work item of the small
+                                 operators' kernel (1..4096)                 */
+    uint32_t blocks_per_cu;   /* blocks per compute unit of that kernel and
+                                 of the matvec kernel (1..8)                 */
     uint32_t order;           /* 0: input order, 1: largest operator first  */
-    uint32_t split;           /* 0: matvec fused into the build (reads no CSR
-                                 back); 1: build pass, then a matvec pass over
+    uint32_t split;           /* 0: y without reading the CSR back; 1: the
+                                 builds, then a matvec pass over
                                  the written CSR (needs every CSR buffer)     */
 } qr_tuning;
 

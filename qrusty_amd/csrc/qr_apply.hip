@@ -958,6 +958,11 @@ static int apply_split(const ApplyPlan &p, bool mixed, uint64_t blocks, int cus)
     return p.small || blocks < uint64_t(4) * cus ? 2 : 1;
 }
 
+int apply_tables(const qr_op *op, DeviceTables *t) {
+    const ApplyPlan plan = make_plan<false, ApplyShape<false>::L>(op, 0);
+    return device_patterns(op, t, plan.slot, plan.shape, plan.win_shape, plan.elem_log2, false);
+}
+
 int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint32_t nvec,
                        const void *d_x, void *d_y, double *d_expect, hipStream_t s,
                        bool noalloc) {

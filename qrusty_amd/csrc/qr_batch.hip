@@ -1,29 +1,29 @@
-// qr_batch.hip -- many operators of uneven size: CSR builds plus one matvec
-// each, as a few persistent kernels captured in one hipGraph, with an
-// autotuner.
+// qr_batch.hip -- many operators of uneven size: CSR builds plus one product
+// each, captured in one hipGraph.
 //
 // The reference builds and applies operators one at a time
-// (qrusty/src/lib.rs:573-585 then accel.rs:338-370).  Here the work of a whole
-// batch is lists of (operator, row tile) items, one per register class.  A
-// persistent grid of 1024-thread blocks takes items from its class's atomic
-// counter; an item builds its
-// rows with the shared LDS-staged tile builder (qr_tile.h) -- CSR entries
-// bit-identical to the single-operator build -- and, fused, the same rows of
-// y = A x from the entries still in registers.  No item depends on another,
-// so every block leaves the loop as soon as the counter passes the end.
-// Two forms (a tuning choice).  Fused: one kernel per register class builds
-// and applies; operators whose G exceeds the largest LDS stage
-// (kStageMaxGLean) are built and applied by the single-operator kernels,
-// recorded in the same graph.  Split (needs every CSR): two build kernels,
-// whose items are the tiles of every operator as sub-operators of at most
-// kSubMaxG groups (an operator of at most kSubMaxG groups is one), then one
-// matvec pass (k_batch_mv) over the written CSRs -- three compute kernels per
-// step whatever the batch holds.
+// (qrusty/src/lib.rs:573-585 then accel.rs:338-370).  Here the operators go to
+// kBranches branches of one graph, each to the branch with the least work so
+// far, so that launches that leave part of the chip idle, and the ends of
+// large ones, run beside others.  An operator's CSR is written by the
+// single-operator build (qr_csr.hip); small operators share the launches of
+// k_batch.  CSR entries are bit-identical either way.  Two forms (a tuning
+// choice):
+//   fused  y = A x by the matrix-free apply of the same operator
+//          (qr_apply.hip), which reads no CSR back and so needs none: 0.5 ps
+//          per entry of a random 20-qubit operator, where reading the entry's
+//          24 bytes takes 4;
+//   split  (needs every CSR) after the builds, one matvec pass (k_batch_mv)
+//          over the written CSRs.
+// Measured, 16 operators of 8 to 18 qubits and 10 to 5000 random terms (443e6
+// entries, 10.6 GB written): one persistent build-and-apply kernel per
+// register class 4850 us, this form 2370.  What bounds it: the CSR stores
+// (1.65 ms at the builds' 6.4 TB/s), then the applies.
 //
-// Tuning knobs (qr_tuning): tiles per item (work granularity), resident
-// blocks per CU (grid size), and the item order (input order or largest
-// operator first).  qr_batch_tune times every candidate on the caller's
-// buffers and keeps the fastest.
+// Tuning knobs (qr_tuning): the order in which operators go to the branches
+// (input order or largest first), the form, and, for k_batch and the matvec
+// pass, tiles per item and resident blocks per CU.  qr_batch_tune times every
+// candidate on the caller's buffers and keeps the fastest.
 #include "qr_internal.h"
 #include "qr_tile.h"
 
@@ -36,27 +36,18 @@ struct BatchOpDesc {
     TileOp op;
     uint64_t item_begin;  // first work item of this operator
     uint64_t tiles;       // row tiles of this operator
-    uint32_t narrow;      // masks fit in 32 bits
-    uint32_t nch;         // group chunks per thread
 };
 
-// One persistent kernel per register class (mask width x chunks per thread):
-// items of that class only, taken from the class's own counter.
-// Minimum waves per SIMD requested from the compiler: 8 means two resident
-// 1024-thread blocks per CU (at most 64 VGPRs), as the single-operator build
-// runs; 1 leaves the register budget alone.  Only the one-chunk build fits
-// 64 VGPRs here: the two-chunk build spilled 25 registers there (its
-// item loop costs a few more than the single-operator kernel), and without
-// the bound the 256-operator batch measured 92.0-93.1 against 93.0-94.1 ms.
-#ifndef QR_BATCH_WAVES
-#define QR_BATCH_WAVES(matvec, chunks, mode) \
-    ((!(matvec) && ((chunks) <= 1 || (mode) == kTileSub)) ? 8 : 1)
-#endif
-template <bool kNarrow, int kChunks, bool kMatvec, int kMode = kTilePlain>
-__global__ __launch_bounds__(kStageThreads, QR_BATCH_WAVES(kMatvec, kChunks, kMode)) void k_batch(const BatchOpDesc *__restrict__ ops,
-                                                         uint32_t nops, uint64_t total_items,
-                                                         uint32_t tiles_per_item,
-                                                         unsigned long long *__restrict__ counter) {
+// Small operators (kBatchSmall): one persistent kernel for those of one group
+// chunk per thread and one for those of two (at most 2048 groups), whose
+// blocks take (operator, tiles) items from an atomic counter and build them
+// with the shared tile builder (qr_tile.h); fused, with the same rows of
+// y = A x from the entries still in registers.  No item depends on another,
+// so every block leaves the loop as soon as the counter passes the end.
+template <int kChunks, bool kMatvec>
+__global__ __launch_bounds__(kStageThreads, !kMatvec && kChunks <= 1 ? 8 : 1) void k_batch(
+    const BatchOpDesc *__restrict__ ops, uint32_t nops, uint64_t total_items, uint32_t tiles_per_item,
+    unsigned long long *__restrict__ counter) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ unsigned long long item_s;
     for (;;) {
@@ -76,11 +67,22 @@ __global__ __launch_bounds__(kStageThreads, QR_BATCH_WAVES(kMatvec, kChunks, kMo
         const uint64_t t0 = (item - d.item_begin) * tiles_per_item;
         const uint64_t t1 = t0 + tiles_per_item < d.tiles ? t0 + tiles_per_item : d.tiles;
         for (uint64_t t = t0; t < t1; ++t) {
-            build_tile_staged<kNarrow, kChunks, kMatvec, kMode>(d.op, t, smem_raw);
+            build_tile_staged<true, kChunks, kMatvec, kTilePlain>(d.op, t, smem_raw);
             __syncthreads();  // the stage is reused by the next tile
         }
     }
 }
+
+// Most groups of an operator whose y the fused form gives without CSR buffers.
+constexpr uint64_t kBatchMostG = 6144;
+
+// Entries up to which an operator is small: it runs in k_batch, which takes
+// all of them in a launch or two, at 11 ps per entry fused, where a build and
+// an apply of its own take two launches and 5.  Measured (us, 2^20 / 2^21 /
+// 2^22 / 2^24): 64 operators of 8 to 14 qubits 442 / 460 / 495 / 560, 16 of
+// 12 to 17 qubits 560 / 560 / 658 / 800, and the first run, which makes the
+// apply's tables, 4 of 8 to 16 qubits 1240 / 710 / 470.
+constexpr uint64_t kBatchSmall = uint64_t(1) << 21;
 
 // Split form, second pass: y_k = A_k x_k from the CSR just written, over
 // (operator, block of kMvRows rows) items taken from one counter.  Operators
@@ -225,10 +227,16 @@ __global__ void k_zero_counter(unsigned long long *counter) { *counter = 0ull; }
 
 using namespace qr;
 
+// (us, 4 / 8 / 16 branches: 16 operators of 8 to 18 qubits 2450 / 2370 / 2670,
+// of 12 to 17 qubits 620 / 565 / 565; one branch 3170 and 930)
+constexpr int kBranches = 8;
+
 struct qr_batch {
     std::vector<const qr_op *> ops;
     int dev = -1;
     hipStream_t cap = nullptr;  // private capture stream (default priority)
+    hipStream_t side[kBranches] = {};  // branches 1 on (0: the recording stream)
+    hipEvent_t fork = nullptr, join[kBranches] = {};
     BatchOpDesc *d_desc = nullptr;
     size_t d_desc_cap = 0;
     BatchMvDesc *d_mv = nullptr;
@@ -246,232 +254,176 @@ struct qr_batch {
 
 namespace {
 
-// register classes: group chunks per thread in {1, 2, kStageMaxChunks,
-// kStageLeanChunks} for whole operators, and {1, 2} for the sub-operators
-// (classes 4 and 5) of the split form's operators of more than kSubMaxG
-// groups.  A batch operator builds all 2^n rows, so n <= 32 and masks are
-// 32-bit.
-constexpr int kClasses = 6;
-constexpr int kSubClass = 4;
-inline int class_of(uint32_t nch) {
-    return nch <= 1 ? 0 : nch <= 2 ? 1 : nch <= uint32_t(kStageMaxChunks) ? 2 : 3;
-}
-
 struct Plan {
-    bool split = false;                       // build pass, then k_batch_mv
-    std::vector<BatchMvDesc> mv;              // split form: one per staged operator
+    // small operators, by group chunks per thread (1 or 2), and their branch
+    int small_branch = 0;
+    std::vector<BatchOpDesc> small[2];
+    uint64_t items[2] = {};
+    size_t shmem[2] = {};
+    std::vector<uint32_t> branch[kBranches];  // the others, in order
+    std::vector<BatchMvDesc> mv;              // split form: one per operator
     uint64_t mv_items = 0;
-    std::vector<BatchOpDesc> desc;            // grouped by class, in item order
-    uint32_t cls_begin[kClasses + 1] = {};    // descriptor range of each class
-    uint64_t cls_items[kClasses] = {};
-    size_t cls_shmem[kClasses] = {};
-    std::vector<uint32_t> big;  // operators built by the single-operator kernels
 };
+
+bool has_csr(uint64_t *const *d_indices, double *const *d_data, size_t k) {
+    return d_indices && d_indices[k] && d_data && d_data[k];
+}
 
 int make_plan(qr_batch *b, uint64_t *const *d_indptr, uint64_t *const *d_indices,
               double *const *d_data, const double *const *d_x, double *const *d_y,
               const qr_tuning &tu, Plan &plan) {
     const uint32_t nops = uint32_t(b->ops.size());
+    // the split form needs every operator's CSR
+    for (uint32_t k = 0; tu.split && k < nops; ++k)
+        if (!has_csr(d_indices, d_data, k))
+            return fail(QR_ERR_ARG, "the split batch form needs CSR output buffers for every operator");
     std::vector<uint32_t> order(nops);
     std::iota(order.begin(), order.end(), 0u);
     if (tu.order == 1)  // largest operator first
         std::stable_sort(order.begin(), order.end(), [b](uint32_t a, uint32_t c) {
             return (b->ops[a]->G << b->ops[a]->nq) > (b->ops[c]->G << b->ops[c]->nq);
         });
-    const uint32_t tpi = tu.tiles_per_item ? tu.tiles_per_item : 1;
-    // the split form needs every staged operator's CSR
-    plan.split = tu.split != 0;
-    for (uint32_t k = 0; plan.split && k < nops; ++k)
-        if (!(d_indices && d_indices[k] && d_data && d_data[k]))
-            return fail(QR_ERR_ARG, "the split batch form needs CSR output buffers for every operator");
-    std::vector<BatchOpDesc> per[kClasses];
-    auto add_item = [&](int c, const TileOp &top, uint64_t tiles, size_t shmem) {
-        BatchOpDesc d{};
-        d.op = top;
-        d.tiles = tiles;
-        d.narrow = 1;
-        d.nch = top.nchunks;
-        d.item_begin = plan.cls_items[c];
-        plan.cls_items[c] += (tiles + tpi - 1) / tpi;
-        plan.cls_shmem[c] = std::max(plan.cls_shmem[c], shmem);
-        per[c].push_back(d);
-    };
+    uint64_t load[kBranches] = {};
     for (uint32_t k : order) {
         const qr_op *op = b->ops[k];
         if (op->nq > 32) return fail(QR_ERR_SIZE, "batch operators are limited to 32 qubits");
         if (!d_x || !d_x[k] || !d_y || !d_y[k]) return fail(QR_ERR_ARG, "null state pointer in batch");
-        const bool has_csr = d_indices && d_indices[k] && d_data && d_data[k];
-        DeviceTables *t;
-        int rc = device_tables(op, &t);
-        if (rc) return rc;
-        const uint32_t G = uint32_t(op->G);
+        const bool csr = has_csr(d_indices, d_data, k);
+        if (!tu.split && op->G > kBatchMostG && !(csr && d_indptr && d_indptr[k]))
+            return fail(QR_ERR_ARG, "batch operators with more than 6144 distinct x masks "
+                                    "need CSR output buffers");
         const uint64_t N = uint64_t(1) << op->nq;
-        uint64_t *ip = d_indptr ? d_indptr[k] : nullptr;
-        auto *dat = has_csr ? reinterpret_cast<double2 *>(d_data[k]) : nullptr;
-        auto *xk = reinterpret_cast<const double2 *>(d_x[k]);
-        auto *yk = reinterpret_cast<double2 *>(d_y[k]);
-        if (plan.split) {
-            // split form: every operator in the two sub-operator classes (1 or
-            // 2 group chunks per thread).  One of at most kSubMaxG groups is a
-            // sub-operator of itself (gbase = nanc = 0, gstride = G); a larger
-            // one is its subtrees of the mask trie, each filling a contiguous
-            // segment of every row, the first of which writes indptr.  Heavy
-            // groups are folded inline.  The matvec pass then reads the CSR.
-            if (op->leaves.empty()) {
-                const uint32_t jw = stage_jw_log2(G), nch = (G + (1u << jw) - 1) >> jw;
-                uint32_t dbuf = 0;
-                const size_t sb = stage_bytes(G, jw, &dbuf);
-                add_item(kSubClass + (nch <= 1 ? 0 : 1),
-                         TileOp{t->gx, t->gterm, t->tz, t->tc, t->rl_ptr, t->rl, d_indices[k], dat, ip, xk,
-                                yk, 0, N, G, jw, nch, dbuf, nullptr, 0, 0, 0, G},
-                         ((N - 1) >> (10 - jw + 4)) + 1, sb);
-            } else {
-                for (const auto &lf : op->leaves) {
-                    const uint32_t g = lf.s1 - lf.s0, nch = (g + 1023) >> 10;
-                    uint32_t dbuf = 0;
-                    const size_t sb = stage_bytes(g, 10, &dbuf);
-                    add_item(kSubClass + (nch <= 1 ? 0 : 1),
-                             TileOp{t->gx + lf.s0, t->gterm + lf.s0, t->tz, t->tc, t->rl_ptr + lf.s0, t->rl,
-                                    d_indices[k], dat, lf.s0 == 0 ? ip : nullptr, xk, yk, 0, N, g, 10, nch,
-                                    dbuf, nullptr, 0, lf.s0, lf.depth, G},
-                             ((N - 1) >> 4) + 1, sb);
-                }
-            }
-            plan.mv.push_back(BatchMvDesc{d_indices[k], dat, xk, yk, N, G, plan.mv_items});
+        if (tu.split) {
+            plan.mv.push_back(BatchMvDesc{d_indices[k], reinterpret_cast<double2 *>(d_data[k]),
+                                          reinterpret_cast<const double2 *>(d_x[k]),
+                                          reinterpret_cast<double2 *>(d_y[k]), N, op->G, plan.mv_items});
             plan.mv_items += (N + kMvRows - 1) / kMvRows;
+        }
+        if (N * op->G <= kBatchSmall && op->G <= kSubMaxG) {
+            DeviceTables *t;
+            if (int rc = device_tables(op, &t)) return rc;
+            const uint32_t G = uint32_t(op->G), jw = stage_jw_log2(G), nch = (G + (1u << jw) - 1) >> jw;
+            const uint32_t c = nch <= 1 ? 0 : 1;
+            uint32_t dbuf = 0;
+            plan.shmem[c] = std::max(plan.shmem[c], stage_bytes(G, jw, &dbuf));
+            BatchOpDesc d{};
+            d.op = TileOp{t->gx, t->gterm, t->tz, t->tc, t->rl_ptr, t->rl, csr ? d_indices[k] : nullptr,
+                          csr ? reinterpret_cast<double2 *>(d_data[k]) : nullptr, d_indptr ? d_indptr[k] : nullptr,
+                          reinterpret_cast<const double2 *>(d_x[k]), reinterpret_cast<double2 *>(d_y[k]), 0, N, G,
+                          jw, nch, dbuf, nullptr, 0, 0, 0, G};
+            d.tiles = ((N - 1) >> (10 - jw + 4)) + 1;
+            d.item_begin = plan.items[c];
+            plan.items[c] += (d.tiles + tu.tiles_per_item - 1) / tu.tiles_per_item;
+            plan.small[c].push_back(d);
             continue;
         }
-        if (op->G > kStageMaxGLean) {
-            // fused form, more than kStageMaxGLean groups: built and applied
-            // by the single-operator kernels
-            if (!has_csr || !ip)
-                return fail(QR_ERR_ARG, "batch operators with more than 6144 distinct x masks "
-                                        "need CSR output buffers");
-            plan.big.push_back(k);
-            continue;
-        }
-        // fused form: the whole operator in the class of its chunk count
-        const uint32_t jw = stage_jw_log2(G), nch = (G + (1u << jw) - 1) >> jw;
-        uint32_t dbuf = 0;
-        const size_t sb = stage_bytes(G, jw, &dbuf);
-        add_item(class_of(nch),
-                 TileOp{t->gx, t->gterm, t->tz, t->tc, t->rl_ptr, t->rl, has_csr ? d_indices[k] : nullptr, dat,
-                        ip, xk, yk, 0, N, G, jw, nch, dbuf, nullptr, 0, 0, 0, G},
-                 ((N - 1) >> (10 - jw + 4)) + 1, sb);
+        // the branch with the least work: entries, and about what a launch of
+        // next to none costs in them
+        const int to = int(std::min_element(load, load + kBranches) - load);
+        load[to] += N * op->G + (uint64_t(1) << 20);
+        plan.branch[to].push_back(k);
     }
-    for (int c = 0; c < kClasses; ++c) {
-        plan.cls_begin[c] = uint32_t(plan.desc.size());
-        plan.desc.insert(plan.desc.end(), per[c].begin(), per[c].end());
-    }
-    plan.cls_begin[kClasses] = uint32_t(plan.desc.size());
+    plan.small_branch = int(std::min_element(load, load + kBranches) - load);
     return QR_OK;
-}
-
-template <bool kNarrow, int kChunks, int kMode = kTilePlain>
-static void launch_class(qr_batch *b, const Plan &plan, int c, uint32_t grid_cap, uint32_t tpi,
-                         hipStream_t s) {
-    const uint64_t items = plan.cls_items[c];
-    if (items == 0) return;
-    const uint64_t grid = std::min<uint64_t>(grid_cap, items);
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(1), 0, s, b->d_counter + c);
-    if (plan.split || kMode != kTilePlain)
-        hipLaunchKernelGGL((k_batch<kNarrow, kChunks, false, kMode>), dim3(unsigned(grid)),
-                           dim3(kStageThreads), plan.cls_shmem[c], s, b->d_desc + plan.cls_begin[c],
-                           plan.cls_begin[c + 1] - plan.cls_begin[c], items, tpi,
-                           b->d_counter + c);
-    else if constexpr (kMode == kTilePlain)
-        hipLaunchKernelGGL((k_batch<kNarrow, kChunks, true>), dim3(unsigned(grid)),
-                           dim3(kStageThreads), plan.cls_shmem[c], s, b->d_desc + plan.cls_begin[c],
-                           plan.cls_begin[c + 1] - plan.cls_begin[c], items, tpi,
-                           b->d_counter + c);
 }
 
 int record(qr_batch *b, const Plan &plan, const qr_tuning &tu, uint64_t *const *d_indptr,
            uint64_t *const *d_indices, double *const *d_data, const double *const *d_x,
            double *const *d_y, hipStream_t s) {
-    const uint32_t bpc = tu.blocks_per_cu ? tu.blocks_per_cu : 1;
-    const uint32_t cap = uint32_t(b->ncu) * bpc;
-    const uint32_t tpi = tu.tiles_per_item ? tu.tiles_per_item : 1u;
-    launch_class<true, 1>(b, plan, 0, cap, tpi, s);
-    launch_class<true, 2>(b, plan, 1, cap, tpi, s);
-    launch_class<true, kStageMaxChunks>(b, plan, 2, cap, tpi, s);
-    launch_class<true, kStageLeanChunks>(b, plan, 3, cap, tpi, s);
-    if (plan.split) {
-        launch_class<true, 1, kTileSub>(b, plan, kSubClass, cap, tpi, s);
-        launch_class<true, 2, kTileSub>(b, plan, kSubClass + 1, cap, tpi, s);
+    int rc;
+    QR_HIP_CHECK(hipEventRecord(b->fork, s));
+    for (int i = 0; i < kBranches; ++i) {
+        if (plan.branch[i].empty() && i != plan.small_branch) continue;
+        const hipStream_t bs = i ? b->side[i] : s;
+        if (i) QR_HIP_CHECK(hipStreamWaitEvent(bs, b->fork, 0));
+        for (uint32_t k : plan.branch[i]) {
+            const qr_op *op = b->ops[k];
+            DeviceTables *t;
+            if ((rc = device_tables(op, &t))) return rc;
+            const uint64_t N = uint64_t(1) << op->nq;
+            uint64_t *ip = d_indptr ? d_indptr[k] : nullptr;
+            if (has_csr(d_indices, d_data, k))
+                rc = launch_csr_build(op, t, 0, N, ip, d_indices[k], d_data[k], bs);
+            else if (ip) rc = launch_csr_indptr(op, 0, N, ip, bs);
+            if (!rc && !tu.split)
+                rc = launch_pauli_apply(op, t, QR_PREC_FP64, 1, d_x[k], d_y[k], nullptr, bs, true);
+            if (rc) return rc;
+        }
+        for (int c = 0; i == plan.small_branch && c < 2; ++c) {
+            if (plan.small[c].empty()) continue;
+            const uint64_t grid = std::min<uint64_t>(uint64_t(b->ncu) * tu.blocks_per_cu, plan.items[c]);
+            auto kern = c == 0 ? (tu.split ? k_batch<1, false> : k_batch<1, true>)
+                               : (tu.split ? k_batch<2, false> : k_batch<2, true>);
+            hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(1), 0, bs, b->d_counter + 1 + c);
+            hipLaunchKernelGGL(kern, dim3(unsigned(grid)), dim3(kStageThreads), plan.shmem[c], bs,
+                               b->d_desc + (c ? plan.small[0].size() : 0), uint32_t(plan.small[c].size()),
+                               plan.items[c], tu.tiles_per_item, b->d_counter + 1 + c);
+            QR_HIP_CHECK(hipGetLastError());
+        }
+        if (i) {
+            QR_HIP_CHECK(hipEventRecord(b->join[i], bs));
+            QR_HIP_CHECK(hipStreamWaitEvent(s, b->join[i], 0));
+        }
     }
-    QR_HIP_CHECK(hipGetLastError());
-    // fused form: operators of more than kStageMaxGLean groups, built and
-    // applied by the single-operator kernels
-    for (uint32_t k : plan.big) {
-        const qr_op *op = b->ops[k];
-        DeviceTables *t;
-        int rc = device_tables(op, &t);
-        if (rc) return rc;
-        const uint64_t N = uint64_t(1) << op->nq;
-        rc = launch_csr_build(op, t, 0, N, d_indptr[k], d_indices[k], d_data[k], s);
-        if (rc) return rc;
-        rc = launch_csr_matvec(N, N, N * op->G, d_indptr[k], d_indices[k], d_data[k], d_x[k], d_y[k], s);
-        if (rc) return rc;
-    }
-    if (plan.split && plan.mv_items) {
+    if (tu.split && plan.mv_items) {
         // 8 resident 256-thread blocks per CU and slot
-        const uint64_t grid = std::min<uint64_t>(uint64_t(b->ncu) * 8 * bpc, plan.mv_items);
-        hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(1), 0, s, b->d_counter + kClasses);
+        const uint64_t grid = std::min<uint64_t>(uint64_t(b->ncu) * 8 * tu.blocks_per_cu, plan.mv_items);
+        hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(1), 0, s, b->d_counter);
         hipLaunchKernelGGL(k_batch_mv, dim3(unsigned(grid)), dim3(256), kBatchMvLds, s, b->d_mv,
-                           uint32_t(plan.mv.size()), plan.mv_items, b->d_counter + kClasses);
+                           uint32_t(plan.mv.size()), plan.mv_items, b->d_counter);
         QR_HIP_CHECK(hipGetLastError());
     }
     return QR_OK;
 }
 
-int prepare(qr_batch *b, const Plan &plan) {
-    int dev = 0;
+// Everything that a recording must not do: streams, the operators' tables,
+// the matvec pass's descriptors.
+int prepare(qr_batch *b, const Plan &plan, const qr_tuning &tu) {
+    int dev = 0, rc;
     QR_HIP_CHECK(hipGetDevice(&dev));
     if (b->dev != dev) {
         if (b->dev >= 0) return fail(QR_ERR_ARG, "a batch is bound to the device it first ran on");
         b->dev = dev;
         QR_HIP_CHECK(hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking));
-        QR_HIP_CHECK(hipMalloc(&b->d_counter, (kClasses + 1) * sizeof(unsigned long long)));
-        hipDeviceProp_t prop;
-        QR_HIP_CHECK(hipGetDeviceProperties(&prop, dev));
-        b->ncu = prop.multiProcessorCount;
-        const int maxsh = int(stage_bytes(kStageMaxGLean, 10, nullptr));
-        // every kernel launch_class may launch (the sub-operator classes run
-        // in the split form only)
-        const void *kerns[] = {
-            reinterpret_cast<const void *>(k_batch<true, 1, true>),
-            reinterpret_cast<const void *>(k_batch<true, 2, true>),
-            reinterpret_cast<const void *>(k_batch<true, kStageMaxChunks, true>),
-            reinterpret_cast<const void *>(k_batch<true, kStageLeanChunks, true>),
-            reinterpret_cast<const void *>(k_batch<true, 1, false>),
-            reinterpret_cast<const void *>(k_batch<true, 2, false>),
-            reinterpret_cast<const void *>(k_batch<true, kStageMaxChunks, false>),
-            reinterpret_cast<const void *>(k_batch<true, kStageLeanChunks, false>),
-            reinterpret_cast<const void *>(k_batch<true, 1, false, kTileSub>),
-            reinterpret_cast<const void *>(k_batch<true, 2, false, kTileSub>)};
-        for (const void *kf : kerns)
-            QR_HIP_CHECK(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, maxsh));
+        QR_HIP_CHECK(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
+        QR_HIP_CHECK(hipMalloc(&b->d_counter, 3 * sizeof(unsigned long long)));
+        for (const void *kf : {reinterpret_cast<const void *>(k_batch<1, true>), reinterpret_cast<const void *>(k_batch<2, true>),
+                               reinterpret_cast<const void *>(k_batch<1, false>), reinterpret_cast<const void *>(k_batch<2, false>)})
+            QR_HIP_CHECK(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             int(stage_bytes(kSubMaxG, 10, nullptr))));
+        QR_HIP_CHECK(hipDeviceGetAttribute(&b->ncu, hipDeviceAttributeMultiprocessorCount, dev));
     }
-    // a previous graph or tuning pass may still read the descriptors
-    QR_HIP_CHECK(hipDeviceSynchronize());
-    if (b->d_desc_cap < plan.desc.size()) {
-        if (b->d_desc) (void)hipFree(b->d_desc);
-        b->d_desc = nullptr;
-        b->d_desc_cap = 0;
-        QR_HIP_CHECK(hipMalloc(&b->d_desc, std::max<size_t>(plan.desc.size(), 1) * sizeof(BatchOpDesc)));
-        b->d_desc_cap = plan.desc.size();
+    for (int i = 0; i < kBranches; ++i) {
+        const auto &branch = plan.branch[i];
+        if (i && !b->join[i] && (!branch.empty() || i == plan.small_branch)) {
+            QR_HIP_CHECK(hipStreamCreateWithFlags(&b->side[i], hipStreamNonBlocking));
+            QR_HIP_CHECK(hipEventCreateWithFlags(&b->join[i], hipEventDisableTiming));
+        }
+        for (uint32_t k : branch) {
+            DeviceTables *t;
+            if ((rc = device_tables(b->ops[k], &t))) return rc;
+            if (!tu.split && (rc = apply_tables(b->ops[k], t))) return rc;
+        }
     }
-    if (!plan.desc.empty())
-        QR_HIP_CHECK(hipMemcpy(b->d_desc, plan.desc.data(), plan.desc.size() * sizeof(BatchOpDesc),
-                               hipMemcpyHostToDevice));
-    if (b->d_mv_cap < plan.mv.size()) {
-        if (b->d_mv) (void)hipFree(b->d_mv);
-        b->d_mv = nullptr;
-        b->d_mv_cap = 0;
-        QR_HIP_CHECK(hipMalloc(&b->d_mv, plan.mv.size() * sizeof(BatchMvDesc)));
-        b->d_mv_cap = plan.mv.size();
-    }
+    const size_t nsmall = plan.small[0].size() + plan.small[1].size();
+    if (nsmall || !plan.mv.empty())
+        // a previous graph or tuning pass may still read the descriptors
+        QR_HIP_CHECK(hipDeviceSynchronize());
+    auto room = [](auto **d, size_t *cap, size_t n) {
+        if (*cap >= n) return int(QR_OK);
+        if (*d) (void)hipFree(*d);
+        *d = nullptr;
+        *cap = 0;
+        QR_HIP_CHECK(hipMalloc(d, n * sizeof(**d)));
+        *cap = n;
+        return int(QR_OK);
+    };
+    if ((rc = room(&b->d_desc, &b->d_desc_cap, nsmall)) || (rc = room(&b->d_mv, &b->d_mv_cap, plan.mv.size())))
+        return rc;
+    for (size_t c = 0, at = 0; c < 2; at += plan.small[c++].size())
+        if (!plan.small[c].empty())
+            QR_HIP_CHECK(hipMemcpy(b->d_desc + at, plan.small[c].data(), plan.small[c].size() * sizeof(BatchOpDesc),
+                                   hipMemcpyHostToDevice));
     if (!plan.mv.empty())
         QR_HIP_CHECK(hipMemcpy(b->d_mv, plan.mv.data(), plan.mv.size() * sizeof(BatchMvDesc),
                                hipMemcpyHostToDevice));
@@ -531,6 +483,11 @@ int qr_batch_destroy(qr_batch *b) {
     if (b->d_desc) (void)hipFree(b->d_desc);
     if (b->d_mv) (void)hipFree(b->d_mv);
     if (b->d_counter) (void)hipFree(b->d_counter);
+    for (int i = 1; i < kBranches; ++i) {
+        if (b->side[i]) (void)hipStreamDestroy(b->side[i]);
+        if (b->join[i]) (void)hipEventDestroy(b->join[i]);
+    }
+    if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->cap) (void)hipStreamDestroy(b->cap);
     delete b;
     return QR_OK;
@@ -550,7 +507,7 @@ int qr_batch_run(qr_batch *b, uint64_t *const *d_indptr, uint64_t *const *d_indi
         Plan plan;
         int rc = make_plan(b, d_indptr, d_indices, d_data, d_x, d_y, tu, plan);
         if (rc) return rc;
-        rc = prepare(b, plan);
+        rc = prepare(b, plan, tu);
         if (rc) return rc;
         drop_graph(b);
         QR_HIP_CHECK(hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal));
@@ -596,7 +553,7 @@ int qr_batch_tune(qr_batch *b, uint64_t *const *d_indptr, uint64_t *const *d_ind
                 const qr_tuning tu{tpi, bpc, order, split};
                 Plan plan;
                 if ((rc = make_plan(b, d_indptr, d_indices, d_data, d_x, d_y, tu, plan)) ||
-                    (rc = prepare(b, plan)))
+                    (rc = prepare(b, plan, tu)))
                     goto done;
                 // one untimed pass (first touch), then one timed pass
                 for (int rep = 0; rep < 2; ++rep) {

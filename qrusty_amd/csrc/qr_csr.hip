@@ -518,6 +518,13 @@ static int launch_build_words(const qr_op *op, const DeviceTables *t, uint64_t r
     return rc;
 }
 
+int launch_csr_indptr(const qr_op *op, uint64_t row_begin, uint64_t nrows, uint64_t *d_indptr, hipStream_t s) {
+    const uint64_t nb = (nrows + 1 + 255) / 256;
+    hipLaunchKernelGGL(k_indptr, dim3(unsigned(nb)), dim3(256), 0, s, row_begin, nrows, op->G, d_indptr);
+    QR_HIP_CHECK(hipGetLastError());
+    return QR_OK;
+}
+
 int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin, uint64_t row_end,
                      uint64_t *d_indptr, uint64_t *d_indices, double *d_data, hipStream_t s) {
     const uint64_t nrows = row_end - row_begin;
@@ -526,12 +533,8 @@ int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin,
     if (op->nq <= 32 && nrows)
         return launch_build_words(op, t, row_begin, row_end, d_indptr, d_indices, d_data, s);
     // wider masks: the shared tile builder
-    if (d_indptr) {
-        uint64_t nb = (nrows + 1 + 255) / 256;
-        hipLaunchKernelGGL(k_indptr, dim3(unsigned(nb)), dim3(256), 0, s, row_begin, nrows,
-                           uint64_t(G), d_indptr);
-        QR_HIP_CHECK(hipGetLastError());
-    }
+    int rc;
+    if (d_indptr && (rc = launch_csr_indptr(op, row_begin, nrows, d_indptr, s))) return rc;
     if (nrows == 0) return QR_OK;
     if (!op->leaves.empty()) {
         // one sub-operator per subtree of the mask trie, each <= kSubMaxG

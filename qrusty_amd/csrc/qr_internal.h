@@ -327,6 +327,7 @@ void free_tables(DeviceTables &t);
 int device_tables(const qr_op *op, DeviceTables **out, bool noalloc = false);
 
 // Kernel launchers (qr_csr.hip, qr_apply.hip).
+int launch_csr_indptr(const qr_op *op, uint64_t row_begin, uint64_t nrows, uint64_t *d_indptr, hipStream_t s);
 int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin,
                      uint64_t row_end, uint64_t *d_indptr, uint64_t *d_indices,
                      double *d_data, hipStream_t s);
@@ -360,6 +361,9 @@ int io_read_raw(const char *path, uint64_t rows, uint64_t nnz, uint64_t *ip, uin
 int io_write_mm(const char *path, uint64_t rows, uint64_t cols, uint64_t nnz, const uint64_t *ip,
                 const uint64_t *ix, const double *d, int sym, hipStream_t s);
 int io_read_mm(const char *path, qr_mm_reader **out, hipStream_t s);
+// the tables of an FP64 apply of the operator, so that a launch_pauli_apply
+// without allocation finds them
+int apply_tables(const qr_op *op, DeviceTables *t);
 // noalloc: no device allocation -- the tables must be on the device already
 // and the <x|y> block partials go to the file-scope scratch array (qr_apply.hip)
 int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint32_t nvec,

@@ -1,5 +1,6 @@
-// qr_tile.h -- the LDS-staged row-tile builder shared by the single-operator
-// CSR build (qr_csr.hip) and the batched build+matvec (qr_batch.hip).
+// qr_tile.h -- the LDS-staged row-tile builder shared by the CSR build of
+// operators past 32 qubits (qr_csr.hip) and the batch's small operators
+// (qr_batch.hip).
 //
 // Replaces accel::rowwise::make_row (qrusty/src/accel.rs:171-210) for one tile
 // of rows.  Thread layout: 1024 threads = RS rows x JW groups (JW a power of
@@ -29,13 +30,6 @@ namespace qr {
 
 constexpr int kBuildM = 16;            // batches per tile (4 varying row bits)
 constexpr int kStageThreads = 1024;
-constexpr uint32_t kStageMaxG = 4096;  // 24 B per entry: 96 KB of LDS for one row
-constexpr int kStageMaxChunks = 4;
-// "lean" class: up to 6 chunks (G <= 6144, a 144 KB row stage); only the rank
-// data and term offsets stay in registers, the first term of each group is
-// re-read (from L2) for every batch
-constexpr int kStageLeanChunks = 6;
-constexpr uint32_t kStageMaxGLean = 6144;
 
 template <bool kNarrow>
 __device__ __forceinline__ uint32_t parity_and(uint64_t a, uint64_t b) {
@@ -303,22 +297,9 @@ __device__ __forceinline__ void build_tile_staged(const TileOp &op, uint64_t til
                                                   unsigned char *smem_raw, uint32_t sub = 0) {
     constexpr bool kHeavy = kMode == kTileHeavy || kMode == kTileSubHeavy;
     constexpr bool kSub = kMode == kTileSub || kMode == kTileSubHeavy;
-    // the second term of each group stays in registers when few chunks leave
-    // room; with more than kStageMaxChunks not even the first one does.  Not
-    // in the sub-operator mode without heavy groups (random operators of more
-    // than 2048 groups, and every operator of the batch's split form), whose
-    // groups rarely have a second term: there the held term cost the batch's
-    // two-chunk kernel 10 of its 14 spilled registers (256-operator batch
-    // 79.6-79.9 -> 78.0-78.3 ms)
-    constexpr bool kHold2 = kChunks <= 2 && kMode != kTileSub;
-    // instances of operators with heavy groups (whose other groups run to 4-6
-    // terms) that run one block per CU also hold terms 2 and 3, loaded after
-    // the heavy fold so that they do not add to its registers (narrow masks:
-    // the 64-bit ones would spill)
-    constexpr bool kHold4 = kHold2 && kNarrow && fold_tiles<kChunks, kMode>();
-    // the one-chunk sub-operators have room for terms 4 and 5 as well
-    constexpr bool kHold6 = kHold4 && kChunks == 1;
-    constexpr bool kLean = kChunks > kStageMaxChunks;
+    // the second term of each group stays in registers, but in sub-operators
+    // without heavy groups, whose groups rarely have one
+    constexpr bool kHold2 = kMode != kTileSub;
     const TileMem mem = tile_mem(op);
     const uint32_t G = op.G, jw_log2 = op.jw_log2, nchunks = op.nchunks;
     const uint64_t row_begin = op.row_begin, row_end = op.row_end;
@@ -381,7 +362,7 @@ __device__ __forceinline__ void build_tile_staged(const TileOp &op, uint64_t til
     // masks of <= 32-qubit operators are held in 32 bits
     using mask_t = typename std::conditional<kNarrow, uint32_t, uint64_t>::type;
     // rank offsets of the four batch bits, two 16-bit values per register
-    // (|sigma| < G <= kStageMaxGLean)
+    // (|sigma| < G <= kSubMaxG)
     int32_t rfx[kChunks], s01[kChunks], s23[kChunks];
     mask_t xj[kChunks], z0[kChunks], z1[kChunks];
     double2 c0[kChunks], c1[kChunks];
@@ -424,10 +405,8 @@ __device__ __forceinline__ void build_tile_staged(const TileOp &op, uint64_t til
         xj[c] = mask_t(mem.gx[j]);
         t0[c] = mem.gterm[j];
         t1[c] = mem.gterm[j + 1];
-        if (!kLean) {
-            z0[c] = mask_t(mem.tz[t0[c]]);
-            c0[c] = ld2(mem.tc + t0[c]);
-        }
+        z0[c] = mask_t(mem.tz[t0[c]]);
+        c0[c] = ld2(mem.tc + t0[c]);
         if (kHold2 && t1[c] > t0[c] + 1) {
             z1[c] = mask_t(mem.tz[t0[c] + 1]);
             c1[c] = ld2(mem.tc + t0[c] + 1);
@@ -465,33 +444,6 @@ __device__ __forceinline__ void build_tile_staged(const TileOp &op, uint64_t til
         }
         __syncthreads();
     }
-    mask_t z2[kChunks], z3[kChunks], z4[kChunks], z5[kChunks];
-    double2 c2[kChunks], c3[kChunks], c4[kChunks], c5[kChunks];
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-        z2[c] = z3[c] = z4[c] = z5[c] = 0;
-        c2[c] = c3[c] = c4[c] = c5[c] = make_double2(0.0, 0.0);
-        const uint32_t j = (uint32_t(c) << jw_log2) + lane;
-        if (!kHold4 || uint32_t(c) >= nchunks || j >= G) continue;
-        // term 2 + u from the tail table (u < ntail) or the group's own range
-        auto hold = [&](uint32_t u, mask_t &z, double2 &cc) {
-            if (t1[c] <= t0[c] + 2 + u) return;
-            if (u < op.ntail) {
-                z = mask_t(mem.ttz[u * op.gstride + j]);
-                cc = ld2(mem.ttc + u * op.gstride + j);
-            } else {
-                z = mask_t(mem.tz[t0[c] + 2 + u]);
-                cc = ld2(mem.tc + t0[c] + 2 + u);
-            }
-        };
-        hold(0, z2[c], c2[c]);
-        hold(1, z3[c], c3[c]);
-        if (kHold6) {
-            hold(2, z4[c], c4[c]);
-            hold(3, z5[c], c5[c]);
-        }
-    }
-
 #pragma unroll 1
     for (int m = 0; m < kBuildM; ++m) {
         const int buf = op.dbuf ? (m & 1) : 0;
@@ -520,8 +472,7 @@ __device__ __forceinline__ void build_tile_staged(const TileOp &op, uint64_t til
             uint32_t tf = t0[c];
             asm volatile("" : "+v"(tf));
             // term-order fold: first value, then + (accel.rs:191-208)
-            double2 v = kLean ? signed_coeff(ld2(mem.tc + tf), parity_and<kNarrow>(r, mem.tz[tf]))
-                              : signed_coeff(c0[c], parity_and<kNarrow>(r, z0[c]));
+            double2 v = signed_coeff(c0[c], parity_and<kNarrow>(r, z0[c]));
             if (kHeavy && hs[c] >= 0) {
                 v = hv[(uint32_t(hs[c]) << (tile_log2 + fold_log2)) | (sub << tile_log2) |
                        (uint32_t(m) << rs_log2) | ro];
@@ -531,41 +482,13 @@ __device__ __forceinline__ void build_tile_staged(const TileOp &op, uint64_t til
                                                         parity_and<kNarrow>(r, mem.tz[tf + 1]));
                 v.x = v.x + e.x;
                 v.y = v.y + e.y;
-                uint32_t u0 = 0;
-                if (kHold4) {
-                    // terms 2 and 3 from registers
-                    if (t1[c] > tf + 2) {
-                        const double2 e2 = signed_coeff(c2[c], parity_and<kNarrow>(r, z2[c]));
-                        v.x = v.x + e2.x;
-                        v.y = v.y + e2.y;
-                    }
-                    if (t1[c] > tf + 3) {
-                        const double2 e3 = signed_coeff(c3[c], parity_and<kNarrow>(r, z3[c]));
-                        v.x = v.x + e3.x;
-                        v.y = v.y + e3.y;
-                    }
-                    u0 = 2;
-                    if (kHold6) {
-                        if (t1[c] > tf + 4) {
-                            const double2 e4 = signed_coeff(c4[c], parity_and<kNarrow>(r, z4[c]));
-                            v.x = v.x + e4.x;
-                            v.y = v.y + e4.y;
-                        }
-                        if (t1[c] > tf + 5) {
-                            const double2 e5 = signed_coeff(c5[c], parity_and<kNarrow>(r, z5[c]));
-                            v.x = v.x + e5.x;
-                            v.y = v.y + e5.y;
-                        }
-                        u0 = 4;
-                    }
-                }
                 // the remaining terms, in term order: from the transposed tail
                 // table while it has them -- the lanes, one group each, then
                 // read one contiguous run per position (u counts iterations,
                 // so the choice is the same for every active lane) -- else
                 // from the group's own term range.  Four loads in flight were
                 // slower than this serial loop, from either table.
-                for (uint32_t t = tf + 2 + u0, u = u0; t < t1[c]; ++t, ++u) {
+                for (uint32_t t = tf + 2, u = 0; t < t1[c]; ++t, ++u) {
                     double2 ct;
                     if (u < op.ntail) {
                         const uint32_t slot = u * op.gstride + j;
