@@ -8,15 +8,17 @@
 // are dropped.  Two passes over the rows -- count, then (after a scan of the
 // counts into indptr) fill.
 //
-// A block takes a tile of consecutive rows.  Their entries are contiguous in
-// both inputs, so the block loads them coalesced into LDS (column and the
-// already scaled value a*v1 or b*v2), a group of lanes per row merges in LDS
-// (each lane from its own merge-path split of the row), and
-// the fill pass writes the tile's merged entries to LDS and from there
-// coalesced to the output, whose tile range is contiguous too.  A tile whose
-// entries exceed the LDS capacity (long or uneven rows) is merged from global
-// memory, one thread per row.
+// Two kernels.  k_spadd_few, where one matrix has up to kSpFew entries per row
+// in the mean.  Otherwise k_spadd_tile: a block takes a tile of consecutive
+// rows.  Their entries are contiguous in both inputs, so the block loads them
+// coalesced into LDS (column and the already scaled value a*v1 or b*v2), a
+// group of lanes per row merges in LDS (each lane from its own merge-path split
+// of the row), and the fill pass writes the tile's merged entries to LDS and
+// from there coalesced to the output, whose tile range is contiguous too.  A
+// tile whose entries exceed the LDS capacity (long or uneven rows) is merged
+// from global memory, one thread per row.
 #include "qr_internal.h"
+#include "qr_mv.h"
 
 #include <hipcub/device/device_scan.hpp>
 
@@ -270,6 +272,220 @@ __global__ __launch_bounds__(kT) void k_spadd_tile(uint64_t nrows, uint32_t rows
     }
 }
 
+// One matrix with few entries per row (H - e*I): 2^lpr_log2 lanes hold a row's
+// entries of the longer matrix (in), that many at a time, and pass over the
+// shorter one's; ballots give every entry its place among the kept ones.
+// Nothing is staged: inputs are read and outputs written by consecutive lanes.
+// Results as merge_row's, whichever matrix is the longer (the sums commute).
+// A wave takes 2^rpw_log2 consecutive rows, one per lane for their bounds and
+// their entry of the shorter matrix, which the lanes of a row then fetch by
+// shuffles; where all rows have one such entry at most and fit their lanes,
+// kSpDepth of them are in flight per lane group and a row takes few vector
+// instructions.  Otherwise one row at a time in pieces.
+// What bounds it: the fill pass memory (10 GB at 5.3 TB/s for the 23-qubit
+// ring), the count pass (5.2 GB at 5) that and its instructions.  Measured
+// (H - e*I, count + fill us, staged tiles / this): 23-qubit ring 1540 + 3040 /
+// 1130 + 1895; 16-qubit molecule (981 entries per row, which overflow the
+// staged tile) 12350 + 21090 / 330 + 500; 992 random terms, 16 qubits 12430 +
+// 22960 / 320 + 720.  Without the shared loads of the bounds (one row of two
+// per lane group at a time) the ring took 1640 + 2065; 4 rows in flight 1190 +
+// 1970.
+constexpr int kSpDepth = 8;
+
+__device__ __forceinline__ double2 nt_value(const double2 *p) {
+    const dvec2 v = __builtin_nontemporal_load(reinterpret_cast<const dvec2 *>(p));
+    return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ void nt_store(uint64_t c, double2 v, uint64_t *ix, double2 *d) {
+    __builtin_nontemporal_store(c, ix);
+    __builtin_nontemporal_store(dvec2{v.x, v.y}, reinterpret_cast<dvec2 *>(d));
+}
+__device__ __forceinline__ uint64_t first_lane(uint64_t v) {
+    return uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(v >> 32)))) << 32 |
+           uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
+}
+
+template <bool kFill>
+__global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_log2, uint32_t rpw_log2, SpAddIn in,
+                                                   uint64_t *__restrict__ counts,
+                                                   const uint64_t *__restrict__ ipo,
+                                                   uint64_t *__restrict__ ixo, double2 *__restrict__ dout) {
+    const uint32_t wl = threadIdx.x & 63u, lpr = 1u << lpr_log2, lane = wl & (lpr - 1u), group = wl >> lpr_log2;
+    const uint32_t gw = 64u >> lpr_log2, shift = wl & ~(lpr - 1u);
+    const uint64_t gmask = lpr == 64 ? ~uint64_t(0) : ((uint64_t(1) << lpr) - 1);
+    const uint32_t mine0 = uint32_t(gmask << shift), mine1 = uint32_t((gmask << shift) >> 32);
+    const uint64_t rw = (uint64_t(blockIdx.x) * 4 + threadIdx.x / 64u) << rpw_log2;  // the wave's first row
+    if (rw >= nrows) return;
+    const uint32_t rows = uint32_t(nrows - rw < (uint64_t(1) << rpw_log2) ? nrows - rw : uint64_t(1) << rpw_log2);
+    // row rw + wl of each lane (of the last lanes: the last row)
+    uint64_t i0, i1, j0, j1, po = 0, pe = 0;
+    {
+        const uint64_t r = rw + (wl < rows ? wl : rows - 1);
+        i0 = in.ip1[r];
+        i1 = in.ip1[r + 1];
+        j0 = in.ip2[r];
+        j1 = in.ip2[r + 1];
+        if (kFill) {
+            po = ipo[r];
+            pe = ipo[r + 1];
+        }
+        i1 = i1 < in.nnz1 ? i1 : in.nnz1;
+        i0 = i0 < i1 ? i0 : i1;
+        j1 = j1 < in.nnz2 ? j1 : in.nnz2;
+        j0 = j0 < j1 ? j0 : j1;
+    }
+    const uint64_t iw = first_lane(i0), pw = first_lane(po);
+    const bool fits = i1 - i0 <= lpr && j1 - j0 <= 1 && i0 - iw < (1u << 27) &&
+                      (!kFill || (po - pw < (1u << 27) && pe - po < (1u << 27)));
+    if (__all(fits)) {
+        // (iw < nnz1 unless the wave's rows are empty or the last)
+        const uint64_t ia = iw < in.nnz1 ? iw : in.nnz1 - 1, left = in.nnz1 - 1 - ia;
+        const uint32_t most = left < (1u << 28) ? uint32_t(left) : 1u << 28;
+        const uint64_t jc = j0 < in.nnz2 ? j0 : in.nnz2 - 1;
+        const uint64_t cb = in.ix2[jc];
+        const double2 q = cmul2(in.b, in.d2[jc]);
+        const bool hb = j1 > j0;
+        // the row's entries, whether it has one of the shorter matrix and
+        // whether that alone is kept, and the room in the output
+        const uint32_t meta = uint32_t(i1 - i0) | (hb ? 0x100u : 0u) |
+                              (hb && (0.0 + q.x != 0.0 || 0.0 + q.y != 0.0) ? 0x200u : 0u) |
+                              (kFill ? uint32_t(pe - po < 0xffff ? pe - po : 0xffff) << 16 : 0u);
+        const uint32_t rel = uint32_t(i0 - iw), orel = uint32_t(po - pw);
+        const uint64_t *ix1 = in.ix1 + ia;
+        const double2 *d1 = in.d1 + ia;
+        uint32_t count = 0;
+        for (uint32_t s = 0; s * gw < rows; s += kSpDepth) {
+            uint64_t c[kSpDepth];
+            double2 v[kSpDepth];
+            uint32_t mt[kSpDepth];
+#pragma unroll
+            for (int u = 0; u < kSpDepth; ++u) {
+                const uint32_t row = (s + uint32_t(u)) * gw + group;
+                mt[u] = uint32_t(__shfl(int(meta), int(row & 63u)));
+                uint32_t at = uint32_t(__shfl(int(rel), int(row & 63u))) + lane;
+                at = at < most ? at : most;
+                c[u] = __builtin_nontemporal_load(ix1 + at);
+                v[u] = nt_value(d1 + at);
+            }
+            // (all their loads before the first is used)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < kSpDepth; ++u) {
+                const uint32_t row = (s + uint32_t(u)) * gw + group;
+                const bool have = row < rows && lane < (mt[u] & 0xffu);
+                const uint64_t cr = __shfl(cb, int(row & 63u));
+                const double qx = __shfl(q.x, int(row & 63u)), qy = __shfl(q.y, int(row & 63u));
+                const bool both = have && (mt[u] & 0x100u) && c[u] == cr;
+                const double2 p = cmul2(in.a, v[u]);
+                // one side only: + 0 as the reference's binop does
+                const double2 x = make_double2(p.x + (both ? qx : 0.0), p.y + (both ? qy : 0.0));
+                const bool keep = have && (x.x != 0.0 || x.y != 0.0);
+                const uint64_t kept = __ballot(keep), met = __ballot(both);
+                const uint32_t k0 = uint32_t(kept) & mine0, k1 = uint32_t(kept >> 32) & mine1;
+                uint32_t n = __popc(k0) + __popc(k1);
+                uint32_t before = kFill ? __builtin_amdgcn_mbcnt_hi(k1, __builtin_amdgcn_mbcnt_lo(k0, 0)) : 0;
+                const bool alone = row < rows && (mt[u] & 0x200u) &&
+                                   ((uint32_t(met) & mine0) | (uint32_t(met >> 32) & mine1)) == 0;
+                const uint32_t to = kFill ? uint32_t(__shfl(int(orel), int(row & 63u))) : 0;
+                if (__any(alone)) {
+                    const uint64_t lower = __ballot(keep && c[u] < cr);
+                    const uint32_t at = __popc(uint32_t(lower) & mine0) + __popc(uint32_t(lower >> 32) & mine1);
+                    if (kFill && alone && lane == 0 && at < mt[u] >> 16)
+                        nt_store(cr, make_double2(0.0 + qx, 0.0 + qy), ixo + pw + to + at, dout + pw + to + at);
+                    before += alone && c[u] > cr ? 1u : 0u;
+                    n += alone ? 1u : 0u;
+                }
+                if (kFill) {
+                    if (keep && before < mt[u] >> 16) nt_store(c[u], x, ixo + pw + to + before, dout + pw + to + before);
+                } else {
+                    // to the lane of the row
+                    const uint32_t mine = uint32_t(__shfl(int(n), int((wl & (gw - 1u)) << lpr_log2)));
+                    if (wl >> (6u - lpr_log2) == s + uint32_t(u)) count = mine;
+                }
+            }
+        }
+        if (!kFill && wl < rows) counts[rw + wl] = count;
+        return;
+    }
+    auto vote = [&](bool p) { return (__ballot(p) >> shift) & gmask; };
+    for (uint32_t s = 0; s * gw < rows; ++s) {
+        const uint32_t row = s * gw + group;
+        const int src = int(row & 63u);
+        uint64_t i = __shfl(i0, src), j = __shfl(j0, src), pos = __shfl(po, src);
+        const uint64_t iend = __shfl(i1, src), jend = __shfl(j1, src), kend = __shfl(pe, src);
+        if (row >= rows) break;
+        uint64_t next = 0;
+        double2 vnext = make_double2(0.0, 0.0);
+        auto load = [&](uint64_t at) {
+            if (at + lane < iend) {
+                next = __builtin_nontemporal_load(in.ix1 + at + lane);
+                vnext = nt_value(in.d1 + at + lane);
+            }
+        };
+        load(i);
+        for (;;) {
+            const bool have = i + lane < iend, last = i + lpr >= iend;
+            const uint64_t col = next;
+            const double2 va = vnext;
+            load(i + lpr);  // the piece after this one
+            const uint64_t top = __shfl(col, int(lpr - 1u), int(lpr));
+            const double2 p = cmul2(in.a, va);
+            double2 q = make_double2(0.0, 0.0);
+            uint64_t je = j;
+            for (; je < jend; ++je) {
+                const uint64_t cc = in.ix2[je];
+                if (!last && cc > top) break;
+                if (have && col == cc) q = cmul2(in.b, in.d2[je]);
+            }
+            const double2 x = make_double2(p.x + q.x, p.y + q.y);
+            const bool keep = have && (x.x != 0.0 || x.y != 0.0);
+            const uint64_t kept = vote(keep);
+            uint32_t before = uint32_t(__popcll(kept & ((uint64_t(1) << lane) - 1))), nb = 0;
+            for (uint64_t t = j; t < je; ++t) {
+                const uint64_t cc = in.ix2[t];
+                if (vote(have && col == cc)) continue;
+                const double2 y = cmul2(in.b, in.d2[t]), z = make_double2(0.0 + y.x, 0.0 + y.y);
+                if (z.x == 0.0 && z.y == 0.0) continue;
+                if (kFill) {
+                    const uint64_t at = pos + uint32_t(__popcll(vote(keep && col < cc))) + nb;
+                    if (lane == 0 && at < kend) nt_store(cc, z, ixo + at, dout + at);
+                    if (have && col > cc) ++before;
+                }
+                ++nb;
+            }
+            if (kFill && keep && pos + before < kend) nt_store(col, x, ixo + pos + before, dout + pos + before);
+            pos += uint32_t(__popcll(kept)) + nb;
+            if (last) break;
+            i += lpr;
+            j = je;
+        }
+        if (!kFill && lane == 0) counts[rw + row] = pos;
+    }
+}
+
+// Whether k_spadd_few takes a sum (the shorter matrix has up to kSpFew entries
+// per row in the mean): its lanes per row, the longer matrix's mean length
+// rounded up to a power of two from 4 to 64; its rows per wave, 64 or what
+// leaves the launch 16 waves per CU, or 256 if rows are long (16-qubit
+// molecule, fill pass, 16 / 64 / 256 waves per CU 612 / 563 / 498 us; 18-qubit
+// ring 58 / 49 / 87); and `in` with the longer first.
+constexpr double kSpFew = 2.0;
+struct SpFew {
+    uint32_t lpr_log2, rpw_log2;
+    uint64_t blocks;
+};
+static bool spadd_few(uint64_t nrows, SpAddIn &in, SpFew &f) {
+    if (in.nnz1 < in.nnz2) in = SpAddIn{in.b, in.a, in.nnz2, in.nnz1, in.ip2, in.ix2, in.ip1, in.ix1, in.d2, in.d1};
+    if (in.nnz2 == 0 || double(in.nnz2) > kSpFew * double(nrows)) return false;
+    f.lpr_log2 = 2;
+    while (f.lpr_log2 < 6 && (nrows << f.lpr_log2) < in.nnz1) ++f.lpr_log2;
+    f.rpw_log2 = 6;
+    const uint64_t waves = f.lpr_log2 == 6 ? 65536 : 4096;
+    while (f.rpw_log2 > 6 - f.lpr_log2 && (nrows >> f.rpw_log2) < waves) --f.rpw_log2;
+    f.blocks = (nrows + (uint64_t(4) << f.rpw_log2) - 1) / (uint64_t(4) << f.rpw_log2);
+    return true;
+}
+
 // Rows per tile: the staged capacity over the mean merged row length, with
 // room for rows up to 1/0.85 times the mean.  Lanes per row: enough that the
 // tile's rows keep the block's threads busy (a power of two, at most 64).
@@ -298,7 +514,7 @@ int launch_spadd_count(uint64_t nrows, const double *a, uint64_t nnz1, const uin
                        const uint64_t *ix1, const double *d1, const double *b, uint64_t nnz2,
                        const uint64_t *ip2, const uint64_t *ix2, const double *d2, uint64_t *ipo,
                        uint64_t *nnz_out, hipStream_t s) {
-    const SpAddIn in = spadd_in(a, nnz1, ip1, ix1, d1, b, nnz2, ip2, ix2, d2);
+    SpAddIn in = spadd_in(a, nnz1, ip1, ix1, d1, b, nnz2, ip2, ix2, d2);
     size_t tmp_bytes = 0;
     QR_HIP_CHECK(hipcub::DeviceScan::InclusiveSum(nullptr, tmp_bytes, ipo, ipo + 1, nrows, s));
     // per-row counts, then their inclusive scan into indptr[1..nrows]
@@ -307,13 +523,19 @@ int launch_spadd_count(uint64_t nrows, const double *a, uint64_t nnz1, const uin
     QR_HIP_CHECK(hipMallocAsync(&tmp, cbytes + tmp_bytes, s));
     uint64_t *counts = static_cast<uint64_t *>(tmp);
     const SpTiling tl = spadd_tiling(nrows, nnz1, nnz2, kSpCountThreads, kSpCountCap);
-    const uint64_t ntiles = (nrows + tl.rows - 1) / tl.rows;
+    SpFew f;
+    const bool few = spadd_few(nrows, in, f);
+    const uint64_t ntiles = few ? f.blocks : (nrows + tl.rows - 1) / tl.rows;
     if (ntiles > 0x7FFFFFFFull) {
         (void)hipFreeAsync(tmp, s);
         return fail(QR_ERR_SIZE, "sparse add: too many row tiles");
     }
     hipLaunchKernelGGL(k_set_zero_u64, dim3(1), dim3(1), 0, s, ipo);
-    hipLaunchKernelGGL((k_spadd_tile<false, kSpCountThreads, kSpCountCap>), dim3(unsigned(ntiles)), dim3(kSpCountThreads), 0, s, nrows,
+    if (few)
+        hipLaunchKernelGGL(k_spadd_few<false>, dim3(unsigned(ntiles)), dim3(256), 0, s, nrows, f.lpr_log2, f.rpw_log2, in, counts,
+                           nullptr, nullptr, nullptr);
+    else
+        hipLaunchKernelGGL((k_spadd_tile<false, kSpCountThreads, kSpCountCap>), dim3(unsigned(ntiles)), dim3(kSpCountThreads), 0, s, nrows,
                        tl.rows, tl.lpr, in, counts, nullptr, nullptr, nullptr);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
@@ -330,10 +552,16 @@ int launch_spadd_fill(uint64_t nrows, const double *a, uint64_t nnz1, const uint
                       const uint64_t *ix1, const double *d1, const double *b, uint64_t nnz2,
                       const uint64_t *ip2, const uint64_t *ix2, const double *d2,
                       const uint64_t *ipo, uint64_t *ixo, double *dout, hipStream_t s) {
-    const SpAddIn in = spadd_in(a, nnz1, ip1, ix1, d1, b, nnz2, ip2, ix2, d2);
+    SpAddIn in = spadd_in(a, nnz1, ip1, ix1, d1, b, nnz2, ip2, ix2, d2);
     const SpTiling tl = spadd_tiling(nrows, nnz1, nnz2, kSpFillThreads, kSpCap);
-    const uint64_t ntiles = (nrows + tl.rows - 1) / tl.rows;
+    SpFew f;
+    const bool few = spadd_few(nrows, in, f);
+    const uint64_t ntiles = few ? f.blocks : (nrows + tl.rows - 1) / tl.rows;
     if (ntiles > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "sparse add: too many row tiles");
+    if (few)
+        hipLaunchKernelGGL(k_spadd_few<true>, dim3(unsigned(ntiles)), dim3(256), 0, s, nrows, f.lpr_log2, f.rpw_log2, in, nullptr,
+                           ipo, ixo, reinterpret_cast<double2 *>(dout));
+    else
     hipLaunchKernelGGL((k_spadd_tile<true, kSpFillThreads, kSpCap>), dim3(unsigned(ntiles)), dim3(kSpFillThreads), 0, s, nrows,
                        tl.rows, tl.lpr, in, nullptr, ipo, ixo, reinterpret_cast<double2 *>(dout));
     QR_HIP_CHECK(hipGetLastError());
