@@ -8,7 +8,7 @@
 // products (a.re x.re - a.im x.im, a.re x.im + a.im x.re) and sums with no
 // fused multiply-add (the library is built with -ffp-contract=off), division
 // ((a c + b d) / (c c + d d), (b c - a d) / (c c + d d)), norm = hypot.
-// Every kernel is a grid-stride loop over its elements.
+// Every kernel but k_diag_scan is a grid-stride loop over its elements.
 #include "qr_internal.h"
 
 namespace qr {
@@ -52,6 +52,64 @@ __global__ __launch_bounds__(256) void k_csr_diagonal(uint64_t n, uint64_t nnz,
         out[r] = diag_entry(r, nnz, indptr, indices, data);
 }
 
+// out = dx / reg(d - e, tol), reg(v) = tol + 0i when |v| < tol, else v
+__device__ __forceinline__ double2 precond_entry(double2 d, double2 dx, double2 e, double tol) {
+    double2 v = make_double2(d.x - e.x, d.y - e.y);
+    if (hypot(v.x, v.y) < tol) v = make_double2(tol, 0.0);
+    return cdiv(dx, v);
+}
+
+// Rows of 8 to kDiagScan entries in the mean: 2^lpr_log2 lanes read a row's
+// columns, four each at a time, and the lane that meets the diagonal writes
+// the row's result (the first lane, if none does).
+// What bounds it: memory.  A binary search per row, the other way, leaves its
+// lines in the caches between dependent probes, where they thrash, but reads
+// few lines of a long row.  Measured (precond, us, search / scan): rings of 20,
+// 23, 24 qubits (21 to 25 entries) 109 / 66, 815 / 582, 1671 / 1190; random
+// operators of 4 entries, 24 qubits 214 / 400, 60, 22 qubits 442 / 474, 120, 21
+// qubits 269 / 470.
+constexpr double kDiagScan = 48.0;
+template <bool kPrecond>
+__global__ __launch_bounds__(256) void k_diag_scan(uint64_t n, uint32_t lpr_log2, uint64_t nnz,
+                                                   const uint64_t *__restrict__ indptr,
+                                                   const uint64_t *__restrict__ indices,
+                                                   const double2 *__restrict__ data,
+                                                   const double2 *__restrict__ dx, double2 e, double tol,
+                                                   double2 *__restrict__ out) {
+    const uint32_t lpr = 1u << lpr_log2, lane = threadIdx.x & (lpr - 1u);
+    const uint64_t r = uint64_t(blockIdx.x) * (256u >> lpr_log2) + (threadIdx.x >> lpr_log2);
+    if (r >= n) return;
+    const uint64_t hi = indptr[r + 1] < nnz ? indptr[r + 1] : nnz;
+    uint64_t at = ~uint64_t(0);
+    for (uint64_t k = indptr[r] + lane; k < hi; k += 4 * lpr) {
+        uint64_t c[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint64_t i = k + uint32_t(u) * lpr;
+            c[u] = indices[i < nnz ? i : nnz - 1];
+        }
+#pragma unroll
+        for (int u = 3; u >= 0; --u) {
+            const uint64_t i = k + uint32_t(u) * lpr;
+            if (c[u] == r && i < hi && i < at) at = i;
+        }
+    }
+    const uint64_t met = __ballot(at != ~uint64_t(0)) >> ((threadIdx.x & 63u) & ~(lpr - 1u));
+    const uint64_t mine = met & (lpr == 64 ? ~uint64_t(0) : (uint64_t(1) << lpr) - 1);
+    // (a column that comes twice in a row: the lower lane's)
+    if (mine ? lane != uint32_t(__ffsll((unsigned long long)mine)) - 1u : lane != 0) return;
+    const double2 d = mine ? data[at] : make_double2(0.0, 0.0);
+    out[r] = kPrecond ? precond_entry(d, dx[r], e, tol) : d;
+}
+
+// Lanes per row of k_diag_scan (0: not by it): a quarter of the mean length
+static uint32_t diag_lanes_log2(uint64_t nrows, uint64_t nnz) {
+    if (double(nnz) < 8.0 * double(nrows) || double(nnz) > kDiagScan * double(nrows)) return 0;
+    uint32_t l = 2;
+    while (l < 6 && (nrows << (l + 2)) < nnz) ++l;
+    return l;
+}
+
 // z = a x + b y  (mode 0), a x + y (mode 1), a x (mode 2)
 __global__ __launch_bounds__(256) void k_axpby(uint64_t n, int mode, double2 a,
                                                const double2 *__restrict__ x, double2 b,
@@ -69,8 +127,8 @@ __global__ __launch_bounds__(256) void k_axpby(uint64_t n, int mode, double2 a,
     }
 }
 
-// out = dx / reg(d - e, tol), reg(v) = tol + 0i when |v| < tol, else v; the
-// diagonal d either given (precond2) or read from the CSR (precond)
+// precond_entry of every row, the diagonal d either given (precond2) or
+// searched in the CSR (precond)
 __global__ __launch_bounds__(256) void k_precond(uint64_t n, const double2 *__restrict__ diag,
                                                  uint64_t nnz, const uint64_t *__restrict__ indptr,
                                                  const uint64_t *__restrict__ indices,
@@ -80,9 +138,7 @@ __global__ __launch_bounds__(256) void k_precond(uint64_t n, const double2 *__re
     for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < n;
          i += uint64_t(gridDim.x) * 256) {
         const double2 d = diag ? diag[i] : diag_entry(i, nnz, indptr, indices, data);
-        double2 v = make_double2(d.x - e.x, d.y - e.y);
-        if (hypot(v.x, v.y) < tol) v = make_double2(tol, 0.0);
-        out[i] = cdiv(dx[i], v);
+        out[i] = precond_entry(d, dx[i], e, tol);
     }
 }
 
@@ -95,6 +151,16 @@ int launch_csr_diagonal(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint
                         const uint64_t *indices, const double *data, double *out, hipStream_t s) {
     const uint64_t n = nrows < ncols ? nrows : ncols;
     if (n == 0) return QR_OK;
+    if (const uint32_t l = diag_lanes_log2(nrows, nnz)) {
+        const uint64_t blocks = (n + (256u >> l) - 1) / (256u >> l);
+        if (blocks <= 0x7FFFFFFFull) {
+            hipLaunchKernelGGL(k_diag_scan<false>, dim3(unsigned(blocks)), dim3(256), 0, s, n, l, nnz, indptr,
+                               indices, reinterpret_cast<const double2 *>(data), nullptr, double2{}, 0.0,
+                               reinterpret_cast<double2 *>(out));
+            QR_HIP_CHECK(hipGetLastError());
+            return QR_OK;
+        }
+    }
     hipLaunchKernelGGL(k_csr_diagonal, dim3(grid_for(n)), dim3(256), 0, s, n, nnz, indptr,
                        indices, reinterpret_cast<const double2 *>(data),
                        reinterpret_cast<double2 *>(out));
@@ -118,6 +184,15 @@ int launch_precond(uint64_t n, const double *diag, uint64_t nnz, const uint64_t 
                    const uint64_t *indices, const double *data, const double *dx, const double *e,
                    double tol, double *out, hipStream_t s) {
     if (n == 0) return QR_OK;
+    const uint32_t l = diag ? 0 : diag_lanes_log2(n, nnz);
+    const uint64_t blocks = l ? (n + (256u >> l) - 1) / (256u >> l) : 0;
+    if (l && blocks <= 0x7FFFFFFFull) {
+        hipLaunchKernelGGL(k_diag_scan<true>, dim3(unsigned(blocks)), dim3(256), 0, s, n, l, nnz, indptr, indices,
+                           reinterpret_cast<const double2 *>(data), reinterpret_cast<const double2 *>(dx),
+                           make_double2(e[0], e[1]), tol, reinterpret_cast<double2 *>(out));
+        QR_HIP_CHECK(hipGetLastError());
+        return QR_OK;
+    }
     hipLaunchKernelGGL(k_precond, dim3(grid_for(n)), dim3(256), 0, s, n,
                        reinterpret_cast<const double2 *>(diag), nnz, indptr, indices,
                        reinterpret_cast<const double2 *>(data),
