@@ -692,14 +692,24 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
     if (row < nrows && lane == 0) y[row] = acc;
 }
 
-// Rows of 16..32 entries on average (8 lanes per row): each 8-lane slot of a
-// wave takes two rows, base + s and base + s + 8, and issues the loads of
-// both rows' first 32 entries before the first gather -- twice the rows per
-// wave of k_csr_matvec<8>, in half the waves.  Entries beyond the 32nd (a
-// general CSR may have such rows) are added in the same per-lane order.
-// The sums are bit-identical to k_csr_matvec<8, false>.  Measured on the
-// 24-qubit Heisenberg CSR (25 entries per row): 2.61 -> 2.47 ms; four rows
-// per slot: 2.65 ms.
+// Rows of 16..32 entries on average: a wave takes 8 consecutive rows, whose
+// entries are contiguous, streams them in whole lines (four loads of 64
+// consecutive entries, nontemporal: the x lines keep the caches), and reads them
+// back from LDS in the gather layout of qr_mv.h: lane (s, t) takes the entries
+// s, s + 8, ... of row t, so that the 8 rows that read one x line do so in one
+// instruction.  Waves whose rows do not fit that (a general CSR) read them from
+// memory in the same per-lane order; the sums are bit-identical to
+// k_csr_matvec<8, false>.
+// What bounds it: memory, 6.2 TB/s with the x lines read again past L2 (the
+// 24-qubit ring: 10.1 GB of CSR, 12.8 GB fetched).  Two rows per 8-lane slot,
+// loaded straight to the gather layout / this, us: rings of 20, 23, 24 qubits
+// 118 / 96, 1122 / 948, 2460 / 2056; terms of weight 1 to 4, 23 qubits (29
+// entries) 1385 / 1140; random operators of 20 entries, 23 qubits 1044 / 938, 31,
+// 22 qubits 731 / 676; 24, 22 qubits 547 / 564, where x comes past L2 for every
+// entry.  Plain loads: ring of 24 qubits 2190; four times eight rows per wave,
+// the next ones' loads behind the gathers, 2125.
+// U: loads per lane; rows of up to 8 U entries.
+template <uint32_t U>
 __global__ __launch_bounds__(256) void k_csr_matvec_short(uint64_t nrows, uint64_t ncols, uint64_t nnz,
                                                           uint32_t nblocks_xcd,
                                                           const uint64_t *__restrict__ indptr,
@@ -707,70 +717,77 @@ __global__ __launch_bounds__(256) void k_csr_matvec_short(uint64_t nrows, uint64
                                                           const double2 *__restrict__ data,
                                                           const double2 *__restrict__ x,
                                                           double2 *__restrict__ y) {
-    constexpr int LPR = 8, U = 4, H = 2;
+    constexpr uint32_t kFit = 64 * U;  // entries of a wave's rows
+    __shared__ uint64_t s_idx[4][kFit];
+    __shared__ dvec2 s_dat[4][kFit];
     uint32_t b = blockIdx.x;
     if (nblocks_xcd) b = (b % 8) * nblocks_xcd + b / 8;
-    const uint32_t wave = threadIdx.x / 64, slot = (threadIdx.x % 64) / LPR;
-    const uint32_t lane = threadIdx.x % LPR;
-    const uint64_t base = (uint64_t(b) * 4 + wave) * (LPR * H);
-    uint64_t c[H][U], k0[H], k1[H];
-    double2 a[H][U], acc[H];
+    const uint32_t wave = threadIdx.x / 64, l = threadIdx.x % 64, ls = l / 8, lt = l % 8;
+    const uint64_t r0 = (uint64_t(b) * 4 + wave) * 8;
+    if (r0 >= nrows) return;
+    const uint64_t rl = r0 + (l < 8 ? l : 8);
+    const uint64_t pl = min(indptr[rl < nrows ? rl : nrows], nnz);  // lane j <= 8: where row r0 + j begins
+    const uint64_t first = readlane_u64(pl, 0), end = readlane_u64(pl, 8);
+    const uint64_t row = r0 + lt, k0 = __shfl(pl, int(lt)), k1 = __shfl(pl, int(lt) + 1);
+    double2 acc = make_double2(0.0, 0.0);
+    auto add = [&](dvec2 a, double2 bx) {
+        acc.x = fma(a.x, bx.x, acc.x);
+        acc.x = fma(-a.y, bx.y, acc.x);
+        acc.y = fma(a.x, bx.y, acc.y);
+        acc.y = fma(a.y, bx.x, acc.y);
+    };
+    if (__all(k0 <= k1 && first <= k0 && k1 <= end && end - first <= kFit)) {
+        const uint32_t at = uint32_t(k0 - first), len = uint32_t(k1 - k0);
+        // U loads and U gathers per lane, none behind a branch
+        const uint64_t top = end > first ? end - 1 : first ? first - 1 : 0;
+        uint64_t c[U];
+        dvec2 a[U];
 #pragma unroll
-    for (int h = 0; h < H; ++h) {
-        acc[h] = make_double2(0.0, 0.0);
-        const uint64_t row = base + slot + LPR * h;
-        k0[h] = k1[h] = 0;
-        if (row < nrows) {
-            k0[h] = min(indptr[row], nnz);
-            k1[h] = min(indptr[row + 1], nnz);
+        for (uint32_t u = 0; u < U; ++u) {
+            // (lanes past the rows repeat their last entry: the entries there
+            // would be fetched twice)
+            const uint64_t k = min(first + l + 64 * u, top);
+            c[u] = __builtin_nontemporal_load(indices + k);
+            a[u] = __builtin_nontemporal_load(reinterpret_cast<const dvec2 *>(data + k));
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint64_t k = k0[h] + lane + u * LPR;
-            c[h][u] = ~uint64_t(0);
-            a[h][u] = make_double2(0.0, 0.0);
-            if (k < k1[h]) {
-                c[h][u] = indices[k];
-                const dvec2 av = *reinterpret_cast<const dvec2 *>(data + k);
-                a[h][u] = make_double2(av.x, av.y);
-            }
+        for (uint32_t u = 0; u < U; ++u) {
+            s_idx[wave][l + 64 * u] = c[u];
+            s_dat[wave][l + 64 * u] = a[u];
+        }
+        // LDS writes of other lanes visible to this wave's reads below
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        double2 bx[U];
+        bool ok[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t p = ls + 8 * u;
+            c[u] = s_idx[wave][(at + p) % kFit];
+            a[u] = s_dat[wave][(at + p) % kFit];
+            ok[u] = p < len && c[u] < ncols;
+            bx[u] = x[ok[u] ? c[u] : 0];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (ok[u]) add(a[u], bx[u]);
+        for (uint32_t p = ls + 8 * U; p < len; p += 8) {
+            const uint64_t cc = s_idx[wave][at + p];
+            if (cc < ncols) add(s_dat[wave][at + p], x[cc]);
+        }
+    } else {
+        for (uint64_t k = k0 + ls; k < k1; k += 8) {
+            const uint64_t cc = indices[k];
+            if (cc < ncols) add(*reinterpret_cast<const dvec2 *>(data + k), x[cc]);
         }
     }
 #pragma unroll
-    for (int h = 0; h < H; ++h)
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (c[h][u] < ncols) {
-                const double2 bx = x[c[h][u]];
-                acc[h].x = fma(a[h][u].x, bx.x, acc[h].x);
-                acc[h].x = fma(-a[h][u].y, bx.y, acc[h].x);
-                acc[h].y = fma(a[h][u].x, bx.y, acc[h].y);
-                acc[h].y = fma(a[h][u].y, bx.x, acc[h].y);
-            }
-        }
-#pragma unroll
-    for (int h = 0; h < H; ++h) {
-        const uint64_t row = base + slot + LPR * h;
-        if (k1[h] > k0[h] + U * LPR) {
-            // a row longer than U * LPR entries: the rest, in the same order
-            for (uint64_t k = k0[h] + lane + U * LPR; k < k1[h]; k += LPR) {
-                const uint64_t cc = indices[k];
-                if (cc < ncols) {
-                    const double2 av = data[k], bx = x[cc];
-                    acc[h].x = fma(av.x, bx.x, acc[h].x);
-                    acc[h].x = fma(-av.y, bx.y, acc[h].x);
-                    acc[h].y = fma(av.x, bx.y, acc[h].y);
-                    acc[h].y = fma(av.y, bx.x, acc[h].y);
-                }
-            }
-        }
-#pragma unroll
-        for (int off = LPR / 2; off > 0; off /= 2) {
-            acc[h].x += __shfl_xor(acc[h].x, off, LPR);
-            acc[h].y += __shfl_xor(acc[h].y, off, LPR);
-        }
-        if (row < nrows && lane == 0) y[row] = acc[h];
+    for (int off = 32; off >= 8; off /= 2) {
+        acc.x += __shfl_xor(acc.x, off);
+        acc.y += __shfl_xor(acc.y, off);
     }
+    if (ls == 0 && row < nrows) y[row] = acc;
 }
 
 // k_csr_matvec_staged (the walker of qr_mv.h over a general CSR): which band
@@ -871,15 +888,16 @@ int launch_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint64
     auto y = reinterpret_cast<double2 *>(d_y);
     const dim3 grid(static_cast<unsigned>(nblocks)), block(256);
     const bool nt = avg >= kMvNontemporalMinRow;
-    if (lpr == 8 && avg <= 32) {
-        // 16..32 entries per row on average: two rows per 8-lane slot
-        const uint64_t nb = (nrows + 63) / 64;
+    if (lpr == 8 && avg <= 32 && ncols) {
+        // 16..32 entries per row on average; a wave's eight rows are to fit,
+        // with a quarter to spare where they cannot be equal
+        const uint64_t nb = (nrows + 31) / 32;
         if (nb > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "CSR matvec grid too large");
         const uint32_t nbx_short = (nb % 8 == 0) ? uint32_t(nb / 8) : 0;
-        hipLaunchKernelGGL(k_csr_matvec_short, dim3(unsigned(nb)), dim3(256), 0, s, nrows, ncols,
-                           nnz, nbx_short, d_indptr, d_indices,
-                           reinterpret_cast<const double2 *>(d_data),
-                           reinterpret_cast<const double2 *>(d_x), reinterpret_cast<double2 *>(d_y));
+        const uint64_t need = nnz % nrows == 0 ? avg : avg + avg / 4 + 1;
+        auto kern = need <= 16 ? k_csr_matvec_short<2> : need <= 24 ? k_csr_matvec_short<3> : k_csr_matvec_short<4>;
+        hipLaunchKernelGGL(kern, dim3(unsigned(nb)), dim3(256), 0, s, nrows, ncols, nnz, nbx_short, d_indptr,
+                           d_indices, data, x, y);
         QR_HIP_CHECK(hipGetLastError());
         return QR_OK;
     }

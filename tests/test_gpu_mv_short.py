@@ -1,0 +1,46 @@
+"""CSR matvec of rows of 16 to 32 entries in the mean (k_csr_matvec_short): each
+load count per lane, rows that do not fit beside rows that do, row counts around
+a wave's eight, columns past the state (skipped), an indptr that descends.
+Against numpy within (2 len + 8) eps sum |a||x| per row."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import qrusty_amd  # noqa: F401
+    yield
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows,lens", [(1, [16]), (7, [16]), (9, [17]), (64, [24]), (257, [25]), (1000, [32]), (33, [31]),
+                                       (513, [0, 40]), (100, [1, 1, 1, 1, 1, 1, 1, 200]), (4000, [5, 20, 33, 16])])
+@pytest.mark.parametrize("kind", ["valid", "past", "descends"])
+def test_short(rows, lens, kind):
+    import qrusty_amd as qa
+    rng = np.random.default_rng(rows + len(lens))
+    cols = 300
+    lens = np.resize(lens, rows)
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    ind = np.concatenate([np.sort(rng.choice(cols, size=int(n), replace=False)) for n in lens]).astype(np.uint64)
+    data = rng.standard_normal(len(ind)) + 1j * rng.standard_normal(len(ind))
+    if kind == "past":
+        ind[::7] += np.uint64(10**6)
+    if kind == "descends" and rows > 3:
+        indptr[rows // 2] = indptr[rows // 2 - 1] // np.uint64(2)
+    x = rng.standard_normal(cols) + 1j * rng.standard_normal(cols)
+    m = qa.SpMat.new_unchecked((rows, cols), data, ind, indptr)
+    print(f"[gpu] short rows={rows} {kind}", flush=True)
+    y = qa.spmat_dot_densevec(m, torch.from_numpy(x).cuda()).cpu().numpy()
+    for r in range(rows):
+        k0, k1 = int(indptr[r]), max(int(indptr[r]), int(indptr[r + 1]))
+        c, a = ind[k0:k1], data[k0:k1]
+        c, a = c[c < cols].astype(np.int64), a[c < cols]
+        bound = (2 * len(c) + 8) * 2.3e-16 * np.sum(np.abs(a) * np.abs(x[c]))
+        assert abs(y[r] - np.sum(a * x[c])) <= bound + 1e-300
