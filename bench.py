@@ -132,9 +132,9 @@ def bench_csr(args, torch, qa):
     }
     res["build_pct_hbm"] = 100 * res["build_GBps"] / HBM_PEAK_GBPS
     res["matvec_pct_hbm"] = 100 * res["matvec_GBps"] / HBM_PEAK_GBPS
-    # the kernels that run here: k_csr_build_staged (G <= 2048) and
-    # k_csr_matvec_staged (rows of 256+ entries)
-    dom = ("k_csr_build_staged", bm, b_build) if bm >= mm else ("k_csr_matvec_staged", mm, b_mv)
+    # the kernels that run here: k_csr_build_words and k_csr_matvec_staged (rows
+    # of 256+ entries)
+    dom = ("k_csr_build_words", bm, b_build) if bm >= mm else ("k_csr_matvec_staged", mm, b_mv)
     res["roofline"] = {
         "kernel": dom[0], "bound": "hbm", "achieved": dom[2] / dom[1] / 1e6, "peak": HBM_PEAK_GBPS,
         "unit": "GB/s", "frac": dom[2] / dom[1] / 1e6 / HBM_PEAK_GBPS,
@@ -369,14 +369,13 @@ def bench_batch(args, torch, qa):
     ms = [ev[k].elapsed_time(ev[k + 1]) for k in range(args.steps)]
     m = statistics.mean(ms)
     # algorithmic bytes: CSR written (24 B/nnz + indptr), then y = A x (x read,
-    # y written).  The split form's matvec pass reads every CSR back (its two
-    # build kernels take every operator as sub-operators); the fused form
-    # reads back only the operators of more than 6144 groups, which run the
-    # single-operator kernels.
+    # y written).  The split form's matvec pass reads every CSR back, the fused
+    # form none.  Operators of more than 2^21 entries run the single-operator
+    # kernels.
     split = bool(best.get("split", 0))
-    big = [] if split else [k for k, h in enumerate(b._h) if h.G > 6144]
+    big = [k for k, h in enumerate(b._h) if h.nnz > 1 << 21]
     nnz_big = sum(b._h[k].nnz for k in big)
-    nnz_reread = nnz if split else sum(h.nnz for h in b._h if h.G > 6144)
+    nnz_reread = nnz if split else 0
     byts = 24 * nnz + 8 * (rows + len(ops)) + 24 * nnz_reread + 32 * rows
     res = {"workload": "batch of 256 uneven random operators (8..18 qubits, 10..5000 terms): "
                        "CSR build + one matvec each, one graph launch",
