@@ -503,6 +503,37 @@ static SpTiling spadd_tiling(uint64_t nrows, uint64_t nnz1, uint64_t nnz2, int t
 
 __global__ void k_set_zero_u64(uint64_t *p) { *p = 0; }
 
+// indptr of few rows: the counts at ipo[1 ..] become their inclusive sums, by
+// one block, in place (the device scan takes three launches and a workspace of
+// its own).  What bounds it: latency.  H - e*I, both calls, rings of 8, 12, 14
+// qubits 70, 74, 73 -> 46, 46, 62 us.
+constexpr uint32_t kScanSmallPer = 16;
+__global__ __launch_bounds__(1024) void k_scan_small(uint32_t n, uint64_t *__restrict__ ipo) {
+    __shared__ uint64_t waves[16];
+    const uint32_t t = threadIdx.x, per = (n + 1023u) / 1024u, at = t * per, lane = t & 63u;
+    uint64_t v[kScanSmallPer], sum = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kScanSmallPer; ++i) {
+        v[i] = i < per && at + i < n ? ipo[1 + at + i] : 0;
+        sum += v[i];
+    }
+    uint64_t incl = sum;
+    for (uint32_t o = 1; o < 64; o <<= 1) {
+        const uint64_t u = __shfl_up(incl, o);
+        if (lane >= o) incl += u;
+    }
+    if (lane == 63) waves[t / 64] = incl;
+    __syncthreads();
+    uint64_t run = incl - sum;
+    for (uint32_t w = 0; w < t / 64; ++w) run += waves[w];
+    if (t == 0) ipo[0] = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kScanSmallPer; ++i) {
+        run += v[i];
+        if (i < per && at + i < n) ipo[1 + at + i] = run;
+    }
+}
+
 static SpAddIn spadd_in(const double *a, uint64_t nnz1, const uint64_t *ip1, const uint64_t *ix1,
                         const double *d1, const double *b, uint64_t nnz2, const uint64_t *ip2,
                         const uint64_t *ix2, const double *d2) {
@@ -515,33 +546,39 @@ int launch_spadd_count(uint64_t nrows, const double *a, uint64_t nnz1, const uin
                        const uint64_t *ip2, const uint64_t *ix2, const double *d2, uint64_t *ipo,
                        uint64_t *nnz_out, hipStream_t s) {
     SpAddIn in = spadd_in(a, nnz1, ip1, ix1, d1, b, nnz2, ip2, ix2, d2);
-    size_t tmp_bytes = 0;
-    QR_HIP_CHECK(hipcub::DeviceScan::InclusiveSum(nullptr, tmp_bytes, ipo, ipo + 1, nrows, s));
-    // per-row counts, then their inclusive scan into indptr[1..nrows]
-    void *tmp = nullptr;
-    const size_t cbytes = (size_t(nrows) * sizeof(uint64_t) + 255) & ~size_t(255);
-    QR_HIP_CHECK(hipMallocAsync(&tmp, cbytes + tmp_bytes, s));
-    uint64_t *counts = static_cast<uint64_t *>(tmp);
     const SpTiling tl = spadd_tiling(nrows, nnz1, nnz2, kSpCountThreads, kSpCountCap);
     SpFew f;
     const bool few = spadd_few(nrows, in, f);
     const uint64_t ntiles = few ? f.blocks : (nrows + tl.rows - 1) / tl.rows;
-    if (ntiles > 0x7FFFFFFFull) {
-        (void)hipFreeAsync(tmp, s);
-        return fail(QR_ERR_SIZE, "sparse add: too many row tiles");
+    if (ntiles > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "sparse add: too many row tiles");
+    // per-row counts, then their inclusive scan into indptr[1..nrows]
+    const bool small = nrows <= 1024 * kScanSmallPer;
+    size_t tmp_bytes = 0;
+    void *tmp = nullptr;
+    const size_t cbytes = (size_t(nrows) * sizeof(uint64_t) + 255) & ~size_t(255);
+    uint64_t *counts = ipo + 1;
+    if (!small) {
+        QR_HIP_CHECK(hipcub::DeviceScan::InclusiveSum(nullptr, tmp_bytes, ipo, ipo + 1, nrows, s));
+        QR_HIP_CHECK(hipMallocAsync(&tmp, cbytes + tmp_bytes, s));
+        counts = static_cast<uint64_t *>(tmp);
+        hipLaunchKernelGGL(k_set_zero_u64, dim3(1), dim3(1), 0, s, ipo);
     }
-    hipLaunchKernelGGL(k_set_zero_u64, dim3(1), dim3(1), 0, s, ipo);
     if (few)
-        hipLaunchKernelGGL(k_spadd_few<false>, dim3(unsigned(ntiles)), dim3(256), 0, s, nrows, f.lpr_log2, f.rpw_log2, in, counts,
-                           nullptr, nullptr, nullptr);
+        hipLaunchKernelGGL(k_spadd_few<false>, dim3(unsigned(ntiles)), dim3(256), 0, s, nrows, f.lpr_log2, f.rpw_log2,
+                           in, counts, nullptr, nullptr, nullptr);
     else
-        hipLaunchKernelGGL((k_spadd_tile<false, kSpCountThreads, kSpCountCap>), dim3(unsigned(ntiles)), dim3(kSpCountThreads), 0, s, nrows,
-                       tl.rows, tl.lpr, in, counts, nullptr, nullptr, nullptr);
+        hipLaunchKernelGGL((k_spadd_tile<false, kSpCountThreads, kSpCountCap>), dim3(unsigned(ntiles)),
+                           dim3(kSpCountThreads), 0, s, nrows, tl.rows, tl.lpr, in, counts, nullptr, nullptr, nullptr);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess)
-        e = hipcub::DeviceScan::InclusiveSum(static_cast<unsigned char *>(tmp) + cbytes, tmp_bytes,
-                                             counts, ipo + 1, nrows, s);
-    (void)hipFreeAsync(tmp, s);
+    if (small) {
+        hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, s, uint32_t(nrows), ipo);
+        if (e == hipSuccess) e = hipGetLastError();
+    } else {
+        if (e == hipSuccess)
+            e = hipcub::DeviceScan::InclusiveSum(static_cast<unsigned char *>(tmp) + cbytes, tmp_bytes,
+                                                 counts, ipo + 1, nrows, s);
+        (void)hipFreeAsync(tmp, s);
+    }
     if (e != hipSuccess) return hip_fail(e, "sparse add count / scan");
     QR_HIP_CHECK(hipMemcpyAsync(nnz_out, ipo + nrows, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     QR_HIP_CHECK(hipStreamSynchronize(s));

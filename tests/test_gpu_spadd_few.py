@@ -2,7 +2,7 @@
 oracle's merge at the edges of the layout -- rows that fill and overflow their
 lanes, none, one or several entries of the short matrix before, between, on
 and after the long one's, exact cancellations, -0.0, both argument orders, row
-counts around a wave's 64."""
+counts around a wave's 64 and the one-block scan's 1024 and 2^14."""
 import numpy as np
 import pytest
 
@@ -36,7 +36,8 @@ def _csr(rows, cols, lens, rng):
 CASES = [(1, 1, [1], [1]), (63, 40, [4], [1]), (64, 40, [5, 8], [1]), (65, 40, [24], [1, 0]),
          (4097, 64, [24], [1]), (1000, 64, [32], [1]), (1000, 64, [33, 20], [0, 1, 2]), (200, 200, [64], [1]),
          (200, 300, [65, 130, 1], [1]), (300, 2000, [981, 3, 0], [5, 0, 1, 0]), (70000, 30, [3], [1]),
-         (130, 900, [0, 0, 0, 900], [2, 1, 0])]
+         (130, 900, [0, 0, 0, 900], [2, 1, 0]), (1023, 20, [2], [1]), (1025, 20, [0, 5], [1]),
+         (16384, 20, [2], [1]), (16385, 20, [2], [1])]
 
 
 @pytest.mark.parametrize("rows,cols,long,short", CASES)
