@@ -692,7 +692,7 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
     if (row < nrows && lane == 0) y[row] = acc;
 }
 
-// Rows of 16..64 entries on average: a wave takes 8 consecutive rows, whose
+// Rows of 8..64 entries on average: a wave takes 8 consecutive rows, whose
 // entries are contiguous, streams them in whole lines (U loads of 64
 // consecutive entries, nontemporal: the x lines keep the caches), and reads them
 // back from LDS in the gather layout of qr_mv.h: lane (s, t) takes the entries
@@ -708,7 +708,9 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
 // 22 qubits 731 / 676; 24, 22 qubits 547 / 564, where x comes past L2 for every
 // entry; and for k_csr_matvec<8> / this, 35, 48, 64 entries, 22 qubits 836 /
 // 754, 1077 / 1073, 1439 / 1373; terms of weight 1 to 4 (45 and 57 entries) 1060
-// / 835, 1318 / 1076.  (More than 64 would leave one block per CU the LDS.)  Plain loads: ring of 24 qubits 2190; four times eight rows per wave,
+// / 835, 1318 / 1076; for 2 and 4 lanes per row / this, 8, 10, 24 qubits 949 /
+// 867, 1190 / 1020, 12, 15, 23 qubits 668 / 544, 839 / 703, but 6, 24 qubits 710
+// / 789.  (More than 64 would leave one block per CU the LDS.)  Plain loads: ring of 24 qubits 2190; four times eight rows per wave,
 // the next ones' loads behind the gathers, 2125.
 // U: loads per lane; rows of up to 8 U entries.
 template <uint32_t U>
@@ -890,14 +892,15 @@ int launch_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint64
     auto y = reinterpret_cast<double2 *>(d_y);
     const dim3 grid(static_cast<unsigned>(nblocks)), block(256);
     const bool nt = avg >= kMvNontemporalMinRow;
-    if (lpr == 8 && avg <= 64 && ncols) {
-        // 16..64 entries per row on average; a wave's eight rows are to fit,
+    if (avg >= 8 && avg <= 64 && ncols) {
+        // 8..64 entries per row on average; a wave's eight rows are to fit,
         // with a quarter to spare where they cannot be equal
         const uint64_t nb = (nrows + 31) / 32;
         if (nb > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "CSR matvec grid too large");
         const uint32_t nbx_short = (nb % 8 == 0) ? uint32_t(nb / 8) : 0;
         const uint64_t need = nnz % nrows == 0 ? avg : avg + avg / 4 + 1;
-        auto kern = need <= 16   ? k_csr_matvec_short<2>
+        auto kern = need <= 8    ? k_csr_matvec_short<1>
+                    : need <= 16 ? k_csr_matvec_short<2>
                     : need <= 24 ? k_csr_matvec_short<3>
                     : need <= 32 ? k_csr_matvec_short<4>
                     : need <= 48 ? k_csr_matvec_short<6>

@@ -1,4 +1,4 @@
-"""CSR matvec of rows of 16 to 64 entries in the mean (k_csr_matvec_short): each
+"""CSR matvec of rows of 8 to 64 entries in the mean (k_csr_matvec_short): each
 load count per lane, rows that do not fit beside rows that do, row counts around
 a wave's eight, columns past the state (skipped), an indptr that descends.
 Against numpy within (2 len + 8) eps sum |a||x| per row."""
@@ -20,7 +20,7 @@ def _gpu():
 
 
 @pytest.mark.parametrize("rows,lens", [(1, [16]), (7, [16]), (9, [17]), (64, [24]), (257, [25]), (1000, [32]), (33, [31]),
-                                       (513, [0, 40]), (100, [1, 1, 1, 1, 1, 1, 1, 200]), (4000, [5, 20, 33, 16]), (65, [33]), (130, [48]), (70, [49]), (300, [64]), (77, [63, 30, 90])])
+                                       (513, [0, 40]), (100, [1, 1, 1, 1, 1, 1, 1, 200]), (4000, [5, 20, 33, 16]), (65, [33]), (130, [48]), (70, [49]), (300, [64]), (77, [63, 30, 90]), (41, [8]), (90, [9]), (200, [12, 0, 30])])
 @pytest.mark.parametrize("kind", ["valid", "past", "descends"])
 def test_short(rows, lens, kind):
     import qrusty_amd as qa
