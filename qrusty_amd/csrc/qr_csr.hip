@@ -692,7 +692,7 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
     if (row < nrows && lane == 0) y[row] = acc;
 }
 
-// Rows of 8..64 entries on average: a wave takes 8 consecutive rows, whose
+// Rows of 8..64 entries on average (128 past the MALL): a wave takes 8 consecutive rows, whose
 // entries are contiguous, streams them in whole lines (U loads of 64
 // consecutive entries, nontemporal: the x lines keep the caches), and reads them
 // back from LDS in the gather layout of qr_mv.h: lane (s, t) takes the entries
@@ -710,11 +710,15 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
 // 754, 1077 / 1073, 1439 / 1373; terms of weight 1 to 4 (45 and 57 entries) 1060
 // / 835, 1318 / 1076; for 2 and 4 lanes per row / this, 8, 10, 24 qubits 949 /
 // 867, 1190 / 1020, 12, 15, 23 qubits 668 / 544, 839 / 703, but 6, 24 qubits 710
-// / 789.  (More than 64 would leave one block per CU the LDS.)  Plain loads: ring of 24 qubits 2190; four times eight rows per wave,
-// the next ones' loads behind the gathers, 2125.
+// / 789.  Rows of 65 to 128 run blocks of two waves (three blocks' LDS per CU),
+// only in matrices of equal rows and 2^25 entries on: 70, 96, 22 qubits 1666 /
+// 1489, 2123 / 2150, 110, 128, 21 qubits 1309 / 1170, 1442 / 1346, weights 1 to
+// 4, 82 and 110 entries 1681 / 1525, 2205 / 2115; where the MALL holds the
+// matrix 28 / 33 (100 entries, 16 qubits).
 // U: loads per lane; rows of up to 8 U entries.
-template <uint32_t U>
-__global__ __launch_bounds__(256) void k_csr_matvec_short(uint64_t nrows, uint64_t ncols, uint64_t nnz,
+constexpr uint64_t kShortLongNnz = uint64_t(1) << 25;
+template <uint32_t U, uint32_t kWaves = 4>
+__global__ __launch_bounds__(64 * kWaves) void k_csr_matvec_short(uint64_t nrows, uint64_t ncols, uint64_t nnz,
                                                           uint32_t nblocks_xcd,
                                                           const uint64_t *__restrict__ indptr,
                                                           const uint64_t *__restrict__ indices,
@@ -722,12 +726,12 @@ __global__ __launch_bounds__(256) void k_csr_matvec_short(uint64_t nrows, uint64
                                                           const double2 *__restrict__ x,
                                                           double2 *__restrict__ y) {
     constexpr uint32_t kFit = 64 * U;  // entries of a wave's rows
-    __shared__ uint64_t s_idx[4][kFit];
-    __shared__ dvec2 s_dat[4][kFit];
+    __shared__ uint64_t s_idx[kWaves][kFit];
+    __shared__ dvec2 s_dat[kWaves][kFit];
     uint32_t b = blockIdx.x;
     if (nblocks_xcd) b = (b % 8) * nblocks_xcd + b / 8;
     const uint32_t wave = threadIdx.x / 64, l = threadIdx.x % 64, ls = l / 8, lt = l % 8;
-    const uint64_t r0 = (uint64_t(b) * 4 + wave) * 8;
+    const uint64_t r0 = (uint64_t(b) * kWaves + wave) * 8;
     if (r0 >= nrows) return;
     const uint64_t rl = r0 + (l < 8 ? l : 8);
     const uint64_t pl = min(indptr[rl < nrows ? rl : nrows], nnz);  // lane j <= 8: where row r0 + j begins
@@ -892,20 +896,23 @@ int launch_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint64
     auto y = reinterpret_cast<double2 *>(d_y);
     const dim3 grid(static_cast<unsigned>(nblocks)), block(256);
     const bool nt = avg >= kMvNontemporalMinRow;
-    if (avg >= 8 && avg <= 64 && ncols) {
-        // 8..64 entries per row on average; a wave's eight rows are to fit,
-        // with a quarter to spare where they cannot be equal
-        const uint64_t nb = (nrows + 31) / 32;
+    if (ncols && avg >= 8 && (avg <= 64 || (avg <= 128 && nnz >= kShortLongNnz && nnz % nrows == 0))) {
+        // a wave's eight rows are to fit, with a quarter to spare where they
+        // cannot be equal
+        const uint64_t need = nnz % nrows == 0 ? avg : avg + avg / 4 + 1;
+        const uint32_t waves = need > 64 ? 2 : 4;  // (the LDS of three blocks per CU)
+        const uint64_t nb = (nrows + 8 * waves - 1) / (8 * waves);
         if (nb > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "CSR matvec grid too large");
         const uint32_t nbx_short = (nb % 8 == 0) ? uint32_t(nb / 8) : 0;
-        const uint64_t need = nnz % nrows == 0 ? avg : avg + avg / 4 + 1;
         auto kern = need <= 8    ? k_csr_matvec_short<1>
                     : need <= 16 ? k_csr_matvec_short<2>
                     : need <= 24 ? k_csr_matvec_short<3>
                     : need <= 32 ? k_csr_matvec_short<4>
                     : need <= 48 ? k_csr_matvec_short<6>
-                                 : k_csr_matvec_short<8>;
-        hipLaunchKernelGGL(kern, dim3(unsigned(nb)), dim3(256), 0, s, nrows, ncols, nnz, nbx_short, d_indptr,
+                    : need <= 64 ? k_csr_matvec_short<8>
+                    : need <= 96 ? k_csr_matvec_short<12, 2>
+                                 : k_csr_matvec_short<16, 2>;
+        hipLaunchKernelGGL(kern, dim3(unsigned(nb)), dim3(64 * waves), 0, s, nrows, ncols, nnz, nbx_short, d_indptr,
                            d_indices, data, x, y);
         QR_HIP_CHECK(hipGetLastError());
         return QR_OK;

@@ -44,3 +44,24 @@ def test_short(rows, lens, kind):
         c, a = c[c < cols].astype(np.int64), a[c < cols]
         bound = (2 * len(c) + 8) * 2.3e-16 * np.sum(np.abs(a) * np.abs(x[c]))
         assert abs(y[r] - np.sum(a * x[c])) <= bound + 1e-300
+
+
+@pytest.mark.parametrize("n,terms", [(19, 70), (19, 110), (18, 129)])
+def test_long_rows_of_large_matrices(n, terms):
+    """65 to 128 entries per row from 2^25 entries on (and past both limits):
+    the product against the oracle on sampled rows, within 1e-12 of
+    sum |c'||x|."""
+    import qrusty_amd as qa
+    from oracle import oracle as orc
+    from qrusty_amd import workloads
+    labels, coeffs = workloads.random_op(n, terms, seed=0x6100 + terms)
+    p = orc.Params(labels, coeffs)
+    op = qa.SparsePauliOp([qa.Pauli(l) for l in labels], coeffs)
+    m = op.to_matrix_mode("RowwiseUnsafeChunked/100")
+    x = workloads.random_states(p.N, 1, 17)[0]
+    print(f"[gpu] matvec n={n} terms={terms}", flush=True)
+    y = qa.spmat_dot_densevec(m, torch.from_numpy(x).cuda()).cpu().numpy()
+    rows = np.unique(np.concatenate([[0, p.N - 1], np.random.default_rng(3).integers(0, p.N, 200)])).astype(np.uint64)
+    ref = orc.apply_rows(p, x, rows)[0]
+    bound = sum(abs(c) * np.abs(x[(rows ^ xm).astype(np.int64)]) for c, xm in zip(p.cp.view(np.complex128), p.x))
+    assert np.all(np.abs(y[rows.astype(np.int64)] - ref) <= 1e-12 * bound)
