@@ -406,9 +406,9 @@ int prepare(qr_batch *b, const Plan &plan, const qr_tuning &tu) {
         }
     }
     const size_t nsmall = plan.small[0].size() + plan.small[1].size();
-    if (nsmall || !plan.mv.empty())
-        // a previous graph or tuning pass may still read the descriptors
-        QR_HIP_CHECK(hipDeviceSynchronize());
+    // a previous graph, which the caller destroys next, or tuning pass may
+    // still run and read the descriptors
+    QR_HIP_CHECK(hipDeviceSynchronize());
     auto room = [](auto **d, size_t *cap, size_t n) {
         if (*cap >= n) return int(QR_OK);
         if (*d) (void)hipFree(*d);

@@ -321,13 +321,13 @@ __global__ __launch_bounds__(kT, 8) void k_csr_build_words(WordOp op) {
 #pragma unroll
         for (uint32_t k = 0; k < uint32_t(kWordMaxLog2); ++k) {
             const uint32_t b = rs_log2 + k;
-            const int32_t v = k < m_log2 && b < op.nq ? rank[b * op.G] : 0;
+            const int32_t v = k < m_log2 && b < op.nq ? rank[uint64_t(b) * op.G] : 0;
             step[k] = v - below;
             below += v;
         }
-        for (uint32_t b = 0; b < rs_log2 && b < op.nq; ++b) slot += (ro >> b) & 1u ? rank[b * op.G] : 0;
+        for (uint32_t b = 0; b < rs_log2 && b < op.nq; ++b) slot += (ro >> b) & 1u ? rank[uint64_t(b) * op.G] : 0;
         for (uint32_t b = tile_log2; b < op.nq; ++b)
-            if ((uint32_t(tile_base) >> b) & 1u) slot += rank[b * op.G];
+            if ((uint32_t(tile_base) >> b) & 1u) slot += rank[uint64_t(b) * op.G];
         const WordGroup gr = op.groups[s0 + lane];
         xj = gr.x;
         tf = gr.tf;
