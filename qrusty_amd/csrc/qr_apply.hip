@@ -332,15 +332,15 @@ __device__ __forceinline__ void merge_splits(dvec2 *area, uint32_t tid, uint32_t
     }
 }
 
-// The end of a tile: y of the thread's rows, and the block's <x|y> partial.  y is written once and not read again by the
-// kernel: nontemporal stores, so that it does not displace x, which the
-// partner tiles still gather, from the caches.
-// row(l) is the state's row of the tile's row l, x(l) its element.  kAdd: y
-// and the partial are added to (a window pass).
-template <bool kFull, bool kPairs, bool kAdd, int kSplit, int R, typename cT, typename Row, typename X>
-__device__ __forceinline__ void finish_tile(uint32_t tid, uint32_t sub, uint64_t tile_rows, Row row, X x,
-                                            cT *__restrict__ yv, double *__restrict__ partials, double *red, const double (&ar)[R],
-                                            const double (&ai)[R]) {
+// The end of a tile: y of the thread's rows, and the block's <x|y> partial.  y
+// is written once and not read again by the kernel: nontemporal stores, so that
+// it does not displace x, which the partner tiles still gather, from the caches.
+// row(l) is the state's row of the tile's row l, x(l) its element.  add: y
+// and the partial are added to (a window pass after another pass).
+template <bool kFull, bool kPairs, int kSplit, int R, typename cT, typename Row, typename X>
+__device__ __forceinline__ void finish_tile(uint32_t tid, uint32_t sub, uint64_t tile_rows, bool add, Row row, X x,
+                                            cT *__restrict__ yv, double *__restrict__ partials, double *red,
+                                            const double (&ar)[R], const double (&ai)[R]) {
     double er = 0.0, ei = 0.0;
     if (kSplit == 1 || sub == 0) {
 #pragma unroll
@@ -356,7 +356,7 @@ __device__ __forceinline__ void finish_tile(uint32_t tid, uint32_t sub, uint64_t
                     if (k & 1) {
                         fvec4 *at = reinterpret_cast<fvec4 *>(yv + row(l - 1));
                         fvec4 was = {0.0f, 0.0f, 0.0f, 0.0f};
-                        if (kAdd) was = __builtin_nontemporal_load(at);
+                        if (add) was = __builtin_nontemporal_load(at);
                         __builtin_nontemporal_store(
                             fvec4{float(ar[k - 1] + was.x), float(ai[k - 1] + was.y), float(ar[k] + was.z),
                                   float(ai[k] + was.w)}, at);
@@ -364,7 +364,7 @@ __device__ __forceinline__ void finish_tile(uint32_t tid, uint32_t sub, uint64_t
                 } else {
                     cT *at = yv + row(l);
                     cT was = {0, 0};
-                    if (kAdd) was = __builtin_nontemporal_load(at);
+                    if (add) was = __builtin_nontemporal_load(at);
                     __builtin_nontemporal_store(cT{eT(ar[k] + was.x), eT(ai[k] + was.y)}, at);
                 }
             }
@@ -388,8 +388,8 @@ __device__ __forceinline__ void finish_tile(uint32_t tid, uint32_t sub, uint64_t
             double s0 = 0.0, s1 = 0.0;
             for (int w = 0; w < kApplyThreads / 64; ++w) { s0 += red[2 * w]; s1 += red[2 * w + 1]; }
             double *at = partials + 2 * uint64_t(blockIdx.x);
-            at[0] = kAdd ? at[0] + s0 : s0;
-            at[1] = kAdd ? at[1] + s1 : s1;
+            at[0] = add ? at[0] + s0 : s0;
+            at[1] = add ? at[1] + s1 : s1;
         }
     }
 }
@@ -518,10 +518,12 @@ __device__ __forceinline__ void chunk_tables(const ApplyChunk &ch, uint32_t t, u
     __syncthreads();
 }
 
-// kWin: a window pass (ApplyWindow), whose groups all gather inside the tile.
+// kWin: a window pass (ApplyWindow), whose groups all gather inside the tile;
+// win_add: it adds to y and the partials.  nchunk is at least 1: the wait for
+// the tile's loads is chunk_tables'.
 template <bool kMixed, bool kNarrow, bool kCplx, bool kFull, int kL, int kSplit, bool kWin>
 __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
-    uint64_t N, ApplyWindow win, uint32_t ntiles, uint32_t tiles_per_xcd, uint32_t nchunk,
+    uint64_t N, ApplyWindow win, uint32_t ntiles, uint32_t tiles_per_xcd, uint32_t nchunk, uint32_t win_add,
     const ApplyGroup *__restrict__ grp, const ApplyChunk *__restrict__ chunks,
     const ApplyPart *__restrict__ part, const uint32_t *__restrict__ tab,
     const ApplyRange *__restrict__ pat, const uint64_t *__restrict__ ptz,
@@ -613,7 +615,7 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
     if (kSplit > 1) merge_splits<kSplit, R>(reinterpret_cast<dvec2 *>(smem_raw), tid, sub, ar, ai);
     // x from the tile in LDS, or from global memory where the merge used it
     const auto x = [&](uint64_t l) { return kSplit == 1 ? xt[l] : xv[row(l)]; };
-    finish_tile<kFull, kPairs, kWin, kSplit, R, cT>(tid, sub, tile_rows, row, x,
+    finish_tile<kFull, kPairs, kSplit, R, cT>(tid, sub, tile_rows, kWin && win_add, row, x,
                                               yout ? reinterpret_cast<cT *>(yout) + uint64_t(v) * N : nullptr,
                                               partials, reinterpret_cast<double *>(smem_raw), ar, ai);
 }
@@ -706,7 +708,7 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_staged(
     const auto row = [base](uint64_t l) { return base + l; };
     // (the buffers hold partner tiles)
     const auto x = [&](uint64_t l) { return xv[base + l]; };
-    finish_tile<true, false, false, kSplit, R, cT>(tid, sub, tile_rows, row, x,
+    finish_tile<true, false, kSplit, R, cT>(tid, sub, tile_rows, false, row, x,
                                             yout ? reinterpret_cast<cT *>(yout) + uint64_t(v) * N : nullptr,
                                             partials, reinterpret_cast<double *>(smem_raw), ar, ai);
 }
@@ -737,7 +739,7 @@ __global__ __launch_bounds__(256) void k_reduce_partials(uint32_t ntiles,
 
 template <bool kMixed, bool kNarrow, int kL, int kSplit, bool kWin = false>
 static int launch_tiled(const qr_op *op, DeviceTables *t, int slot, uint32_t nvec, const void *d_x,
-                        void *d_y, double *partials, uint32_t ntiles, hipStream_t s) {
+                        void *d_y, double *partials, uint32_t ntiles, hipStream_t s, bool add = false) {
     using Shape = ApplyShape<kMixed, kL>;
     const uint64_t N = uint64_t(1) << op->nq;
     const uint64_t tile_rows = N < (uint64_t(1) << Shape::L) ? N : (uint64_t(1) << Shape::L);
@@ -759,7 +761,7 @@ static int launch_tiled(const qr_op *op, DeviceTables *t, int slot, uint32_t nve
     const uint64_t nblocks = uint64_t(ntiles) * nvec;
     if (nblocks > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "apply grid too large");
     hipLaunchKernelGGL(kern, dim3(unsigned(nblocks)), dim3(kApplyThreads * kSplit), shmem, s, N, pt.win, ntiles,
-                       tpx, pt.nchunk, pt.grp, pt.chunk, pt.part, pt.tab, pt.pat,
+                       tpx, pt.nchunk, uint32_t(add), pt.grp, pt.chunk, pt.part, pt.tab, pt.pat,
                        pt.ptz, pt.ptc, d_x, d_y, partials);
     QR_HIP_CHECK(hipGetLastError());
     return QR_OK;
@@ -1041,17 +1043,21 @@ int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint
             const void *x = static_cast<const unsigned char *>(d_x) + off;
             void *y = d_y ? static_cast<unsigned char *>(d_y) + off : nullptr;
             double *e = partials ? partials + 2 * uint64_t(ntiles) * v : nullptr;
-            int r;
-            if (plan.form != kFormGather)
+            // (window passes may have taken every group: then the first of
+            // them writes y)
+            const bool rows_pass = t->pat[plan.slot].nchunk > 0;
+            int r = QR_OK;
+            if (rows_pass && plan.form != kFormGather)
                 r = narrow ? launch_staged<kMixed, true, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s)
                            : launch_staged<kMixed, false, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s);
-            else
+            else if (rows_pass)
                 r = narrow ? launch_tiled<kMixed, true, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s)
                            : launch_tiled<kMixed, false, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s);
             for (uint32_t k = 0; !r && k < nwin; ++k) {
                 const int sl = plan.slot + kApplySlots * int(k + 1);
-                r = narrow ? launch_tiled<kMixed, true, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s)
-                           : launch_tiled<kMixed, false, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s);
+                const bool add = rows_pass || k > 0;
+                r = narrow ? launch_tiled<kMixed, true, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, add)
+                           : launch_tiled<kMixed, false, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, add);
             }
             if (r) return r;
         }

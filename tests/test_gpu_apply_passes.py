@@ -138,3 +138,26 @@ def test_window_passes(kind, n, nvec):
     rows = np.unique(np.r_[0, p.N - 1, rng.choice(p.N, size=4096)]).astype(np.uint64)
     print(f"[gpu] apply window passes {kind} n={n} nvec={nvec}", flush=True)
     _check(p, op, x, rows, "fp64")
+
+
+@pytest.mark.parametrize("n,kind,nvec", [(21, "x", 3), (22, "x", 1), (23, "bonds", 2), (24, "x", 1)])
+def test_windows_take_every_group(n, kind, nvec):
+    """Operators of high masks alone, without a diagonal: X on the top qubits,
+    XX + YY bonds of qubits 17 and up.  Window passes hold all their groups, and
+    the first of them writes y."""
+    from qrusty_amd import workloads
+
+    def term(ops):
+        return "".join(ops.get(n - 1 - k, "I") for k in range(n))
+
+    if kind == "bonds":
+        labels = [term({q: p, q + 1: p}) for q in range(17, n - 1) for p in "XY"]
+    else:
+        labels = [term({q: "X"}) for q in range(17, n)]
+    rng = np.random.default_rng(n)
+    coeffs = list(rng.uniform(-1, 1, len(labels)).astype(complex))
+    p, op = orc.Params(labels, coeffs), _op(labels, coeffs)
+    x = workloads.random_states(p.N, nvec, 800 + n)
+    rows = np.unique(np.r_[0, p.N - 1, rng.choice(p.N, size=4096)]).astype(np.uint64)
+    print(f"[gpu] apply windows only {kind} n={n} nvec={nvec}", flush=True)
+    _check(p, op, x, rows, "fp64")

@@ -1,0 +1,77 @@
+"""CPU tests of which kernels the library launches and what it allocates: each
+runs in a process of its own over hip_stub.c, a HIP runtime that runs nothing,
+with addresses that nothing reads."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes, sys
+stub = ctypes.CDLL({stub!r}, mode=ctypes.RTLD_GLOBAL)
+stub.stub_name.restype = ctypes.c_char_p
+stub.stub_arg.restype = stub.stub_blocks.restype = ctypes.c_uint32
+stub.stub_malloc_bytes.restype = ctypes.c_uint64
+sys.path.insert(0, {repo!r})
+from qrusty_amd import _lib as L
+GB = 1 << 30
+
+def op_of(labels, coeffs=None):
+    n = len(labels)
+    coeffs = coeffs or [1.0 + 0.5 * k for k in range(n)]
+    c = (ctypes.c_double * (2 * n))(*[v for z in coeffs for v in (complex(z).real, complex(z).imag)])
+    h = ctypes.c_void_p()
+    L.check(L.lib.qr_op_create((ctypes.c_char_p * n)(*[s.encode() for s in labels]), c, n, 0, ctypes.byref(h)))
+    return h
+
+def term(n, ops):
+    chars = ["I"] * n
+    for q, ch in ops.items():
+        chars[n - 1 - q] = ch
+    return "".join(chars)
+
+def launched(part):
+    return [(stub.stub_name(i).decode(), stub.stub_arg(i), stub.stub_blocks(i))
+            for i in range(stub.stub_launches()) if part in stub.stub_name(i).decode()]
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    stub = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", stub, os.path.join(HERE, "hip_stub.c")], check=True)
+
+    def go(body):
+        res = subprocess.run([sys.executable, "-c", PRELUDE.format(stub=stub, repo=REPO) + body],
+                             capture_output=True, text=True, timeout=120)
+        assert res.returncode == 0, res.stdout + res.stderr
+
+    return go
+
+
+@pytest.mark.parametrize("split", ["", "1"])
+@pytest.mark.parametrize("n,prec,kind", [(22, 0, "x17"), (23, 0, "bonds17"), (24, 0, "x17"), (28, 0, "x21"),
+                                         (28, 1, "x21")])
+def test_every_apply_pass_has_groups(run, n, prec, kind, split):
+    """The wait for a tile's loads into LDS lies in the loop over the pass's
+    chunks, so no pass may run without one: operators that window passes take
+    whole."""
+    run(f"""
+import os
+if {split!r}:
+    os.environ["QR_APPLY_SPLIT"] = {split!r}
+n = {n}
+if {kind!r} == "bonds17":
+    labels = [term(n, {{q: p, q + 1: p}}) for q in range(17, n - 1) for p in "XY"]
+else:
+    labels = [term(n, {{q: "X"}}) for q in range(int({kind!r}[1:]), n)]
+stub.stub_watch(b"k_apply_tiled", 4)
+op = op_of(labels)
+L.check(L.lib.qr_pauli_apply(op, {prec}, 1, 64 * GB, 128 * GB, 192 * GB, None))
+passes = launched("k_apply_tiled")
+assert passes and all(nchunk > 0 for _, nchunk, _ in passes), passes
+""")
