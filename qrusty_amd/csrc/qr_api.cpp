@@ -463,34 +463,35 @@ bool tables_ready(const qr_op *op, const DeviceTables *t, int slot, int L) {
 }
 
 // Which groups run in window passes.  In the pass over tiles of consecutive
-// rows, every distinct value of the mask bits above the tile is a partner tile
-// that each tile reads; those whose mask stays within about 2^17 complex128
-// (2^18 complex64) rows find it in the XCD's 4 MB L2, the others read it past
-// L2, at the 6.2-7 TB/s that HBM and the MALL deliver (L2: 31 TB/s).  A window
+// rows, every distinct value of the mask bits above the tile is a partner
+// tile that each tile reads; those whose mask stays within about 2^17
+// complex128 rows find it in the XCD's 4 MB L2, the others read it past L2,
+// at the 6.2-7 TB/s that HBM and the MALL deliver (L2: 31 TB/s).  A window
 // pass reads x once, and y once and writes it once more, whatever the number
 // of masks it holds: three streams of the state.  So the windows [s, s + w)
 // that save the most partner streams are taken in turn while they save at
 // least kWindowMinSaved (a partner stream is saved when all groups that share
-// it move).  Up to the MALL's 256 MB that is done for FP64 if together they
-// save half of the partners past L2 (the return value): nearest-neighbour
-// rings and chains, whose masks are a few adjacent bits.  Measured, one state
-// / 8 states, without and with: 24-qubit ring 432 -> 301 us / 3.49 -> 2.91 ms,
-// 22 qubits 107 -> 78 / 697 -> 633 us; k-local and molecular operators, where
-// windows save a sixth of the partners, lost 1-5% with them, and so did
-// complex64 rings, whose arithmetic takes as long as the streams.  For states
-// past the MALL every partner is read from HBM: 28-qubit k-local, complex64,
-// 242 -> 235 ms.
+// it move).  Up to the MALL's 256 MB that is done if together they save half
+// of the partners past L2 (the return value): nearest-neighbour rings and
+// chains, whose masks are a few adjacent bits.  Measured, one state 8 states,
+// without and with: 24-qubit ring 432 -> 301 us / 3.49 -> 2.91 ms, 22 qubits
+// 107 -> 78 / 697 -> 633 us; k-local and molecular operators, where windows
+// save a sixth of the partners, lost 1-5% with them.  For states past the
+// MALL every partner is read from HBM: k-local, 28 qubits and 1000 terms 94
+// -> 80 ms, 26 qubits and 3000 terms 35.2 -> 33.9.
+// FP64 only: y goes through memory from pass to pass, which keeps a sum of
+// doubles and would round the running sum of a complex64 state once per pass.
 constexpr uint32_t kWindowMinSaved = 5;
 constexpr int kWindowMinStateLog2 = 25, kMallLog2 = 28;  // bytes of one state
-bool choose_windows(const qr_op *op, int L, int elem_log2, std::vector<ApplyWindow> &wins,
+bool choose_windows(const qr_op *op, int L, std::vector<ApplyWindow> &wins,
                     std::vector<uint8_t> &pass) {
     wins.clear();
     pass.assign(op->G, 0);
-    const int n = int(op->nq);
-    const bool past_mall = n + elem_log2 > kMallLog2;
-    if (!past_mall && (elem_log2 != 4 || n + elem_log2 < kWindowMinStateLog2)) return false;
-    const int f = 7 - elem_log2;  // 128-byte segments
-    const int w = L - f, near = 21 - elem_log2;
+    const int n = int(op->nq), state_log2 = n + 4;
+    const bool past_mall = state_log2 > kMallLog2;
+    if (state_log2 < kWindowMinStateLog2) return false;
+    const int f = 3;  // 128-byte segments
+    const int w = L - f, near = 17;
     // gx ascends: the groups of one partner are adjacent
     struct Partner { uint64_t g0, g1, bits; };
     std::vector<Partner> far;
@@ -558,7 +559,7 @@ static void free_patterns(DeviceTables::Patterns &pt) {
 }
 
 int device_patterns(const qr_op *op, DeviceTables *t, int slot, const PatternShape &shape,
-                    const PatternShape &win_shape, int elem_log2, bool noalloc) {
+                    const PatternShape &win_shape, bool noalloc) {
     std::lock_guard<std::mutex> lock(op->mu);
     DeviceTables::Patterns &pt = t->pat[slot];
     if (pt.L == shape.L) return QR_OK;
@@ -569,7 +570,7 @@ int device_patterns(const qr_op *op, DeviceTables *t, int slot, const PatternSha
     for (int k = 0; k <= kMaxWindows; ++k) free_patterns(t->pat[slot + kApplySlots * k]);
     std::vector<ApplyWindow> wins;
     std::vector<uint8_t> pass;
-    if (win_shape.L) choose_windows(op, win_shape.L, elem_log2, wins, pass);
+    if (win_shape.L) choose_windows(op, win_shape.L, wins, pass);
     HostPatterns hp;
     int rc;
     for (size_t k = 0; k < wins.size(); ++k) {

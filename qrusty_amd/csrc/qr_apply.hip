@@ -43,7 +43,7 @@
 //    partner tile (their masks agree above the tile), the groups are ordered
 //    by partner and each partner tile is loaded into LDS once, double-
 //    buffered, instead of being gathered once per group.
-//  * Window passes (ApplyWindow): groups whose partner tiles would be
+//  * Window passes (ApplyWindow; FP64): groups whose partner tiles would be
 //    read past L2 are applied in a second pass over tiles made of the low bits
 //    and a window of high ones, where their masks stay inside the tile.
 //
@@ -354,12 +354,9 @@ __device__ __forceinline__ void finish_tile(uint32_t tid, uint32_t sub, uint64_t
                 if constexpr (kPairs) {
                     // the pair's two rows in one 16-byte store, at the odd row
                     if (k & 1) {
-                        fvec4 *at = reinterpret_cast<fvec4 *>(yv + row(l - 1));
-                        fvec4 was = {0.0f, 0.0f, 0.0f, 0.0f};
-                        if (add) was = __builtin_nontemporal_load(at);
                         __builtin_nontemporal_store(
-                            fvec4{float(ar[k - 1] + was.x), float(ai[k - 1] + was.y), float(ar[k] + was.z),
-                                  float(ai[k] + was.w)}, at);
+                            fvec4{float(ar[k - 1]), float(ai[k - 1]), float(ar[k]), float(ai[k])},
+                            reinterpret_cast<fvec4 *>(yv + row(l - 1)));
                     }
                 } else {
                     cT *at = yv + row(l);
@@ -815,7 +812,6 @@ static int apply_form(const qr_op *op, int kind, int L, const PatternShape &win_
     if (e && atoi(e) == 1) return kFormGather;
     int form = op->form[kind].load(std::memory_order_relaxed) - 1;
     if (form < 0) {
-        const int elem_log2 = kind == 0 ? 4 : 3;
         // gx ascends, so groups with equal bits above the tile are adjacent
         uint64_t far = 0, distinct = 0, prev = 0;
         for (uint64_t g = 0; g < op->G; ++g) {
@@ -828,9 +824,9 @@ static int apply_form(const qr_op *op, int kind, int L, const PatternShape &win_
         std::vector<ApplyWindow> wins;
         std::vector<uint8_t> pass;
         // (then the partners left are mostly in L2)
-        const bool windows = win_shape.L && choose_windows(op, win_shape.L, elem_log2, wins, pass);
+        const bool windows = win_shape.L && choose_windows(op, win_shape.L, wins, pass);
         const bool dense = far >= 8 * distinct;
-        const int state_log2 = int(op->nq) + elem_log2;
+        const int state_log2 = int(op->nq) + (kind == 0 ? 4 : 3);
         bool staged = far > 0 && kind != 2 && !windows;
         if (kind == 0)
             staged = staged && (dense || state_log2 >= 26 || (state_log2 >= 24 && 2 * far >= 3 * distinct));
@@ -928,9 +924,9 @@ static ApplyPlan make_plan(const qr_op *op, int kind) {
     ApplyPlan p;
     p.L = int(op->nq) < kL ? int(op->nq) : kL;
     p.elem_log2 = kMixed ? 3 : 4;
-    if (p.L == kL)
+    if (!kMixed && p.L == kL)
         p.win_shape = {p.L, kApplyThreadBits, Shape::kPatSplit, Shape::kTabChunk,
-                       uint32_t(Shape::kTile), false, kMixed, {}};
+                       uint32_t(Shape::kTile), false, false, {}};
     p.form = p.L == kL ? apply_form(op, kind, p.L, p.win_shape) : kFormGather;
     const bool staged = p.form != kFormGather;
     // the gather form on full complex64 tiles runs the paired-row layout
@@ -962,7 +958,7 @@ static int apply_split(const ApplyPlan &p, bool mixed, uint64_t blocks, int cus)
 
 int apply_tables(const qr_op *op, DeviceTables *t) {
     const ApplyPlan plan = make_plan<false, ApplyShape<false>::L>(op, 0);
-    return device_patterns(op, t, plan.slot, plan.shape, plan.win_shape, plan.elem_log2, false);
+    return device_patterns(op, t, plan.slot, plan.shape, plan.win_shape, false);
 }
 
 int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint32_t nvec,
@@ -999,7 +995,7 @@ int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint
                 plan = other;
         }
     }
-    rc = device_patterns(op, t, plan.slot, plan.shape, plan.win_shape, plan.elem_log2, noalloc);
+    rc = device_patterns(op, t, plan.slot, plan.shape, plan.win_shape, noalloc);
     if (rc) return rc;
     const int L = plan.L;
     if ((N >> L) * uint64_t(nvec) > 0x7FFFFFFFull)
@@ -1053,12 +1049,13 @@ int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint
             else if (rows_pass)
                 r = narrow ? launch_tiled<kMixed, true, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s)
                            : launch_tiled<kMixed, false, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s);
-            for (uint32_t k = 0; !r && k < nwin; ++k) {
-                const int sl = plan.slot + kApplySlots * int(k + 1);
-                const bool add = rows_pass || k > 0;
-                r = narrow ? launch_tiled<kMixed, true, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, add)
-                           : launch_tiled<kMixed, false, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, add);
-            }
+            if constexpr (!kMixed)
+                for (uint32_t k = 0; !r && k < nwin; ++k) {
+                    const int sl = plan.slot + kApplySlots * int(k + 1);
+                    const bool add = rows_pass || k > 0;
+                    r = narrow ? launch_tiled<false, true, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, add)
+                               : launch_tiled<false, false, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, add);
+                }
             if (r) return r;
         }
         return int(QR_OK);

@@ -126,7 +126,7 @@ struct ApplyRun {
     uint32_t g1, pad;
 };
 
-// Window pass of the apply: tiles of 2^L rows whose index bits are the
+// Window pass of an FP64 apply: tiles of 2^L rows whose index bits are the
 // state's bits [0, f) and [s, s + L - f).  The groups whose masks lie in those
 // bits gather inside the tile there, where tiles of consecutive rows would
 // read a partner tile each; y is added to.  s = 0: no window.
@@ -244,7 +244,7 @@ void build_patterns(const qr_op *op, const PatternShape &shape, const std::vecto
 // The window passes of an operator: pass[g] = 0 for the groups of the pass
 // over tiles of consecutive rows, k + 1 for those of wins[k] (see qr_api.cpp).
 // Returns whether they hold most of the masks that reach past L2.
-bool choose_windows(const qr_op *op, int L, int elem_log2, std::vector<ApplyWindow> &wins,
+bool choose_windows(const qr_op *op, int L, std::vector<ApplyWindow> &wins,
                     std::vector<uint8_t> &pass);
 // Whether slot `slot` holds the apply tables for tile size L.
 bool tables_ready(const qr_op *op, const DeviceTables *t, int slot, int L);
@@ -252,7 +252,7 @@ bool tables_ready(const qr_op *op, const DeviceTables *t, int slot, int L);
 // wanted).  With `noalloc` they must already be on the device (QR_ERR_ARG if
 // not): nothing is allocated or uploaded.
 int device_patterns(const qr_op *op, DeviceTables *t, int slot, const PatternShape &shape,
-                    const PatternShape &win_shape, int elem_log2, bool noalloc = false);
+                    const PatternShape &win_shape, bool noalloc = false);
 
 }  // namespace qr
 

@@ -161,3 +161,22 @@ def test_windows_take_every_group(n, kind, nvec):
     rows = np.unique(np.r_[0, p.N - 1, rng.choice(p.N, size=4096)]).astype(np.uint64)
     print(f"[gpu] apply windows only {kind} n={n} nvec={nvec}", flush=True)
     _check(p, op, x, rows, "fp64")
+
+
+def test_complex64_sum_is_rounded_once():
+    """26 qubits, complex64: groups inside a tile and groups of high masks whose
+    sums cancel to 1e-6 of either.  On a constant state y is the sum of the
+    coefficients times it; one rounding of each part (2^-24) and FP64 before."""
+    import qrusty_amd as qa
+    from qrusty_amd import workloads
+    n = 26
+    qubits = [0, 1, 2, 3] + list(range(19, n))
+    coeffs = [1 / 12] * 4 + [-1 / 21 + 1e-6 / 7] * 7
+    op = qa.SparsePauliOp([qa.Pauli(workloads._label(n, {q: "X"})) for q in qubits], [complex(c) for c in coeffs])
+    v = complex(np.float32(0.1), np.float32(0.3))
+    print("[gpu] complex64 cancelling sum", flush=True)
+    x = torch.full((1, 1 << n), v, dtype=torch.complex64, device="cuda")
+    y = op.apply(x, "mixed")
+    ref = sum(coeffs) * v
+    err = (torch.view_as_real(y).double() - torch.tensor([ref.real, ref.imag], device="cuda")).abs().amax().item()
+    assert err <= 1.01 * 2.0**-24 * abs(ref)

@@ -75,3 +75,16 @@ L.check(L.lib.qr_pauli_apply(op, {prec}, 1, 64 * GB, 128 * GB, 192 * GB, None))
 passes = launched("k_apply_tiled")
 assert passes and all(nchunk > 0 for _, nchunk, _ in passes), passes
 """)
+
+
+@pytest.mark.parametrize("n", [24, 26, 28])
+def test_complex64_apply_is_one_pass(run, n):
+    """y of a complex64 state is rounded once, when it is written: its sum does
+    not go through memory between passes."""
+    run(f"""
+n = {n}
+labels = [term(n, {{q: "X", (q + 1) % n: "X"}}) for q in range(n)]
+op = op_of(labels)
+L.check(L.lib.qr_pauli_apply(op, L.QR_PREC_MIXED, 1, 64 * GB, 128 * GB, None, None))
+assert len(launched("k_apply")) == 1, launched("k_apply")
+""")
