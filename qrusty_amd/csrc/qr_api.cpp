@@ -473,7 +473,7 @@ bool tables_ready(const qr_op *op, const DeviceTables *t, int slot, int L) {
 // least kWindowMinSaved (a partner stream is saved when all groups that share
 // it move).  Up to the MALL's 256 MB that is done if together they save half
 // of the partners past L2 (the return value): nearest-neighbour rings and
-// chains, whose masks are a few adjacent bits.  Measured, one state 8 states,
+// chains, whose masks are a few adjacent bits.  Measured, one state / 8 states,
 // without and with: 24-qubit ring 432 -> 301 us / 3.49 -> 2.91 ms, 22 qubits
 // 107 -> 78 / 697 -> 633 us; k-local and molecular operators, where windows
 // save a sixth of the partners, lost 1-5% with them.  For states past the

@@ -276,7 +276,9 @@ __global__ __launch_bounds__(kT) void k_spadd_tile(uint64_t nrows, uint32_t rows
 // entries of the longer matrix (in), that many at a time, and pass over the
 // shorter one's; ballots give every entry its place among the kept ones.
 // Nothing is staged: inputs are read and outputs written by consecutive lanes.
-// Results as merge_row's, whichever matrix is the longer (the sums commute).
+// Results as merge_row's, whichever matrix is the longer (the sums commute), and
+// for rows in any order: a short entry meets the first of the long ones left
+// whose column is not below its own, and joins it or comes before it.
 // A wave takes 2^rpw_log2 consecutive rows, one per lane for their bounds and
 // their entry of the shorter matrix, which the lanes of a row then fetch by
 // shuffles; where all rows have one such entry at most and fit their lanes,
@@ -354,6 +356,10 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
         const uint64_t *ix1 = in.ix1 + ia;
         const double2 *d1 = in.d1 + ia;
         uint32_t count = 0;
+        // the lowest and the highest lane of every row
+        uint64_t lows = 1;
+        for (uint32_t k = lpr; k < 64; k <<= 1) lows |= lows << k;
+        const uint64_t highs = lows << (lpr - 1u);
         for (uint32_t s = 0; s * gw < rows; s += kSpDepth) {
             uint64_t c[kSpDepth];
             double2 v[kSpDepth];
@@ -375,12 +381,16 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
                 const bool have = row < rows && lane < (mt[u] & 0xffu);
                 const uint64_t cr = __shfl(cb, int(row & 63u));
                 const double qx = __shfl(q.x, int(row & 63u)), qy = __shfl(q.y, int(row & 63u));
-                const bool both = have && (mt[u] & 0x100u) && c[u] == cr;
+                // of each row, the first entry whose column is not below the
+                // short one's (no borrow leaves a row: its highest bit is set)
+                const uint64_t from = __ballot(have && (mt[u] & 0x100u) && c[u] >= cr), any = from | highs;
+                const uint64_t met = from & any & ~(any - lows) & __ballot(c[u] == cr);
+                const bool both = __builtin_amdgcn_inverse_ballot_w64(met);
                 const double2 p = cmul2(in.a, v[u]);
                 // one side only: + 0 as the reference's binop does
                 const double2 x = make_double2(p.x + (both ? qx : 0.0), p.y + (both ? qy : 0.0));
                 const bool keep = have && (x.x != 0.0 || x.y != 0.0);
-                const uint64_t kept = __ballot(keep), met = __ballot(both);
+                const uint64_t kept = __ballot(keep);
                 const uint32_t k0 = uint32_t(kept) & mine0, k1 = uint32_t(kept >> 32) & mine1;
                 uint32_t n = __popc(k0) + __popc(k1);
                 uint32_t before = kFill ? __builtin_amdgcn_mbcnt_hi(k1, __builtin_amdgcn_mbcnt_lo(k0, 0)) : 0;
@@ -388,11 +398,12 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
                                    ((uint32_t(met) & mine0) | (uint32_t(met >> 32) & mine1)) == 0;
                 const uint32_t to = kFill ? uint32_t(__shfl(int(orel), int(row & 63u))) : 0;
                 if (__any(alone)) {
-                    const uint64_t lower = __ballot(keep && c[u] < cr);
-                    const uint32_t at = __popc(uint32_t(lower) & mine0) + __popc(uint32_t(lower >> 32) & mine1);
+                    const uint64_t mine = uint64_t(mine1) << 32 | mine0, above = from & mine;
+                    const uint64_t below = (above & (0 - above)) - 1;  // the lanes before it, or all
+                    const uint32_t at = uint32_t(__popcll(kept & mine & below));
                     if (kFill && alone && lane == 0 && at < mt[u] >> 16)
                         nt_store(cr, make_double2(0.0 + qx, 0.0 + qy), ixo + pw + to + at, dout + pw + to + at);
-                    before += alone && c[u] > cr ? 1u : 0u;
+                    before += alone && !((below >> wl) & 1u) ? 1u : 0u;
                     n += alone ? 1u : 0u;
                 }
                 if (kFill) {
@@ -428,28 +439,40 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
             const uint64_t col = next;
             const double2 va = vnext;
             load(i + lpr);  // the piece after this one
-            const uint64_t top = __shfl(col, int(lpr - 1u), int(lpr));
             const double2 p = cmul2(in.a, va);
             double2 q = make_double2(0.0, 0.0);
+            // the lane that a short entry of column cc meets, of those from
+            // `left` on (lpr: none, it comes after them); whether it joins it
+            uint32_t left = 0;
+            auto meet = [&](uint64_t cc, uint32_t &f) {
+                const uint64_t ge = vote(have && lane >= left && col >= cc);
+                f = ge ? uint32_t(__builtin_ctzll(ge)) : lpr;
+                const bool joins = ge && __shfl(col, int(f & (lpr - 1u)), int(lpr)) == cc;
+                left = f + (joins ? 1u : 0u);
+                return joins;
+            };
             uint64_t je = j;
             for (; je < jend; ++je) {
-                const uint64_t cc = in.ix2[je];
-                if (!last && cc > top) break;
-                if (have && col == cc) q = cmul2(in.b, in.d2[je]);
+                uint32_t f;
+                const bool joins = meet(in.ix2[je], f);
+                if (f == lpr && !last) break;  // the next piece's
+                if (joins && lane == f) q = cmul2(in.b, in.d2[je]);
             }
+            left = 0;
             const double2 x = make_double2(p.x + q.x, p.y + q.y);
             const bool keep = have && (x.x != 0.0 || x.y != 0.0);
             const uint64_t kept = vote(keep);
             uint32_t before = uint32_t(__popcll(kept & ((uint64_t(1) << lane) - 1))), nb = 0;
             for (uint64_t t = j; t < je; ++t) {
                 const uint64_t cc = in.ix2[t];
-                if (vote(have && col == cc)) continue;
+                uint32_t f;
+                if (meet(cc, f)) continue;
                 const double2 y = cmul2(in.b, in.d2[t]), z = make_double2(0.0 + y.x, 0.0 + y.y);
                 if (z.x == 0.0 && z.y == 0.0) continue;
                 if (kFill) {
-                    const uint64_t at = pos + uint32_t(__popcll(vote(keep && col < cc))) + nb;
+                    const uint64_t at = pos + uint32_t(__popcll(f < 64 ? kept & ((uint64_t(1) << f) - 1) : kept)) + nb;
                     if (lane == 0 && at < kend) nt_store(cc, z, ixo + at, dout + at);
-                    if (have && col > cc) ++before;
+                    if (lane >= f) ++before;
                 }
                 ++nb;
             }

@@ -66,3 +66,30 @@ def test_few(rows, cols, long, short):
             ref = orc.csr_add(rows, s, first, t, second)
             assert np.array_equal(indptr, ref[0]) and np.array_equal(indices, ref[1])
             assert np.array_equal(np.asarray(data).view(np.uint64), np.asarray(ref[2]).view(np.uint64))
+
+
+@pytest.mark.parametrize("rows,cols,long,short", [(300, 9, [8, 3, 5], [1]), (300, 9, [8, 3, 5], [1, 2, 0, 3]),
+                                                  (130, 6, [24, 1, 0], [1, 0]), (130, 40, [64], [1]),
+                                                  (130, 12, [70, 200, 2], [1, 3]), (1, 6, [2], [1])])
+def test_few_of_any_order(rows, cols, long, short):
+    """Rows whose columns do not ascend or come twice: every entry keeps a place
+    of its own, those of the merge."""
+    import qrusty_amd as qa
+    rng = np.random.default_rng(rows + cols + len(short))
+
+    def matrix(lens):
+        lens = np.resize(lens, rows)
+        indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+        n = int(indptr[-1])
+        return indptr, rng.integers(0, cols, n).astype(np.uint64), rng.integers(-1, 2, n) + 1j * rng.integers(-1, 2, n)
+
+    a, b = matrix(long), matrix(short)
+    if rows == 1:
+        a[1][:], b[1][:], a[2][:], b[2][:] = [5, 2], [3], [1, 2], [4]
+    ma, mb = (qa.SpMat.new_unchecked((rows, cols), m[2], m[1], m[0]) for m in (a, b))
+    print(f"[gpu] spadd few, any order rows={rows} cols={cols} long={long} short={short}", flush=True)
+    for first, second, m1, m2 in [(a, b, ma, mb), (b, a, mb, ma)]:
+        _, data, indices, indptr = qa.a_spmat_p_b_spmat(1.0, m1, -1.0, m2).export()
+        ref = orc.csr_add(rows, 1.0, first, -1.0, second)
+        assert np.array_equal(indptr, ref[0]) and np.array_equal(indices, ref[1])
+        assert np.array_equal(np.asarray(data).view(np.uint64), np.asarray(ref[2]).view(np.uint64))
