@@ -8,10 +8,10 @@
 // are dropped.  Two passes over the rows -- count, then (after a scan of the
 // counts into indptr) fill.
 //
-// Two kernels.  k_spadd_few, where one matrix has up to kSpFew entries per row
-// in the mean.  Otherwise k_spadd_tile: a block takes a tile of consecutive
-// rows.  Their entries are contiguous in both inputs, so the block loads them
-// coalesced into LDS (column and the already scaled value a*v1 or b*v2), a
+// Two kernels.  k_spadd_few, where one matrix has one or two entries per row in
+// the mean (spadd_few).  Otherwise k_spadd_tile: a block takes a tile of
+// consecutive rows.  Their entries are contiguous in both inputs, so the block
+// loads them coalesced into LDS (column and the already scaled value a*v1 or b*v2), a
 // group of lanes per row merges in LDS (each lane from its own merge-path split
 // of the row), and the fill pass writes the tile's merged entries to LDS and
 // from there coalesced to the output, whose tile range is contiguous too.  A
@@ -281,9 +281,9 @@ __global__ __launch_bounds__(kT) void k_spadd_tile(uint64_t nrows, uint32_t rows
 // whose column is not below its own, and joins it or comes before it.
 // A wave takes 2^rpw_log2 consecutive rows, one per lane for their bounds and
 // their entry of the shorter matrix, which the lanes of a row then fetch by
-// shuffles; where all rows have one such entry at most and fit their lanes,
-// kSpDepth of them are in flight per lane group and a row takes few vector
-// instructions.  Otherwise one row at a time in pieces.
+// shuffles.  Rows that have one such entry at most and fit their lanes run
+// kSpDepth at a time per lane group and take few vector instructions; the others
+// follow, one at a time, in pieces (kPieces: all do).
 // What bounds it: the fill pass memory (10 GB at 5.3 TB/s for the 23-qubit
 // ring), the count pass (5.2 GB at 5) that and its instructions.  Measured
 // (H - e*I, count + fill us, staged tiles / this): 23-qubit ring 1540 + 3040 /
@@ -307,7 +307,7 @@ __device__ __forceinline__ uint64_t first_lane(uint64_t v) {
            uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
 }
 
-template <bool kFill>
+template <bool kFill, bool kPieces>
 __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_log2, uint32_t rpw_log2, SpAddIn in,
                                                    uint64_t *__restrict__ counts,
                                                    const uint64_t *__restrict__ ipo,
@@ -337,22 +337,22 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
         j0 = j0 < j1 ? j0 : j1;
     }
     const uint64_t iw = first_lane(i0), pw = first_lane(po);
-    const bool fits = i1 - i0 <= lpr && j1 - j0 <= 1 && i0 - iw < (1u << 27) &&
+    const bool fits = !kPieces && i1 - i0 <= lpr && j1 - j0 <= 1 && i0 - iw < (1u << 27) &&
                       (!kFill || (po - pw < (1u << 27) && pe - po < (1u << 27)));
-    if (__all(fits)) {
+    if (!kPieces && __any(fits)) {
         // (iw < nnz1 unless the wave's rows are empty or the last)
         const uint64_t ia = iw < in.nnz1 ? iw : in.nnz1 - 1, left = in.nnz1 - 1 - ia;
         const uint32_t most = left < (1u << 28) ? uint32_t(left) : 1u << 28;
         const uint64_t jc = j0 < in.nnz2 ? j0 : in.nnz2 - 1;
         const uint64_t cb = in.ix2[jc];
         const double2 q = cmul2(in.b, in.d2[jc]);
-        const bool hb = j1 > j0;
-        // the row's entries, whether it has one of the shorter matrix and
+        const bool hb = fits && j1 > j0;
+        // (of a row that does not fit: none) the row's entries, whether it has one of the shorter matrix and
         // whether that alone is kept, and the room in the output
-        const uint32_t meta = uint32_t(i1 - i0) | (hb ? 0x100u : 0u) |
+        const uint32_t meta = (fits ? uint32_t(i1 - i0) : 0u) | (hb ? 0x100u : 0u) |
                               (hb && (0.0 + q.x != 0.0 || 0.0 + q.y != 0.0) ? 0x200u : 0u) |
                               (kFill ? uint32_t(pe - po < 0xffff ? pe - po : 0xffff) << 16 : 0u);
-        const uint32_t rel = uint32_t(i0 - iw), orel = uint32_t(po - pw);
+        const uint32_t rel = fits ? uint32_t(i0 - iw) : 0u, orel = fits ? uint32_t(po - pw) : 0u;
         const uint64_t *ix1 = in.ix1 + ia;
         const double2 *d1 = in.d1 + ia;
         uint32_t count = 0;
@@ -415,16 +415,18 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
                 }
             }
         }
-        if (!kFill && wl < rows) counts[rw + wl] = count;
-        return;
+        if (!kFill && wl < rows && fits) counts[rw + wl] = count;
     }
     auto vote = [&](bool p) { return (__ballot(p) >> shift) & gmask; };
-    for (uint32_t s = 0; s * gw < rows; ++s) {
-        const uint32_t row = s * gw + group;
+    // the rows left, the lowest gw of them at a time
+    for (uint64_t rest = __ballot(wl < rows && !fits); rest;) {
+        uint32_t row = 64;
+        for (uint32_t g = 0; g < gw && rest; ++g, rest &= rest - 1)
+            if (group == g) row = uint32_t(__builtin_ctzll(rest));
         const int src = int(row & 63u);
         uint64_t i = __shfl(i0, src), j = __shfl(j0, src), pos = __shfl(po, src);
         const uint64_t iend = __shfl(i1, src), jend = __shfl(j1, src), kend = __shfl(pe, src);
-        if (row >= rows) break;
+        if (row == 64) continue;
         uint64_t next = 0;
         double2 vnext = make_double2(0.0, 0.0);
         auto load = [&](uint64_t at) {
@@ -486,22 +488,38 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
     }
 }
 
-// Whether k_spadd_few takes a sum (the shorter matrix has up to kSpFew entries
-// per row in the mean): its lanes per row, the longer matrix's mean length
-// rounded up to a power of two from 4 to 64; its rows per wave, 64 or what
-// leaves the launch 16 waves per CU, or 256 if rows are long (16-qubit
+// Whether k_spadd_few takes a sum, its lanes per row (the longer matrix's mean
+// length rounded up to a power of two from 4 to 64), its rows per wave (64 or
+// what leaves the launch 16 waves per CU, or 256 if rows are long: 16-qubit
 // molecule, fill pass, 16 / 64 / 256 waves per CU 612 / 563 / 498 us; 18-qubit
-// ring 58 / 49 / 87); and `in` with the longer first.
-constexpr double kSpFew = 2.0;
+// ring 58 / 49 / 87), and `in` with the longer matrix first.
+// Rows of up to 64 entries in the mean: sums with as many short entries as rows
+// (a diagonal, one Pauli string), where one each is what to expect.  Staged
+// tiles / this, count + fill, us: 20 qubits, 4 to 64 random terms 570-900 /
+// 500-600; rows of 10.6 to 12.7 entries in the mean (isotropic rings without
+// their zeros, 20, 23, 24 qubits) 405 / 340, 3500 / 2860, 6340 / 6110; Poisson
+// lengths of 8, 20, 40 330 / 320, 595 / 525, 1050 / 837; one row in 100 of 600
+// entries 4360 / 656; but half of the rows 3 and half 40 long 930 / 1020.  Other
+// sums stay with the tiles: rows with two short entries (Z + X) run one at a
+// time here, 20-qubit ring 657 / 1290, 0 to 2 each 600 / 900 (and as many as
+// rows, alternately 0 and 2, 23 qubits 4780 / 6800).
+// Longer rows, which leave the tiles few rows or overflow them: from 128 entries
+// per row with one short one, 192 with two.  One / two short entries: 90
+// entries 1012 / 1055, 972 / 1280; 128: 784 / 666, 772 / 763; 220: 811 / 535,
+// 828 / 578; 400: 1084 / 868, 1097 / 952; 600: 21200 / 685, 21300 / 676.
 struct SpFew {
     uint32_t lpr_log2, rpw_log2;
     uint64_t blocks;
+    bool pieces;
 };
 static bool spadd_few(uint64_t nrows, SpAddIn &in, SpFew &f) {
     if (in.nnz1 < in.nnz2) in = SpAddIn{in.b, in.a, in.nnz2, in.nnz1, in.ip2, in.ix2, in.ip1, in.ix1, in.d2, in.d1};
-    if (in.nnz2 == 0 || double(in.nnz2) > kSpFew * double(nrows)) return false;
     f.lpr_log2 = 2;
     while (f.lpr_log2 < 6 && (nrows << f.lpr_log2) < in.nnz1) ++f.lpr_log2;
+    f.pieces = (nrows << f.lpr_log2) < in.nnz1;
+    if (f.pieces ? in.nnz2 == 0 || in.nnz2 > 2 * nrows || in.nnz1 / 64 < nrows + in.nnz2
+                 : in.nnz2 != nrows)
+        return false;
     f.rpw_log2 = 6;
     const uint64_t waves = f.lpr_log2 == 6 ? 65536 : 4096;
     while (f.rpw_log2 > 6 - f.lpr_log2 && (nrows >> f.rpw_log2) < waves) --f.rpw_log2;
@@ -587,8 +605,8 @@ int launch_spadd_count(uint64_t nrows, const double *a, uint64_t nnz1, const uin
         hipLaunchKernelGGL(k_set_zero_u64, dim3(1), dim3(1), 0, s, ipo);
     }
     if (few)
-        hipLaunchKernelGGL(k_spadd_few<false>, dim3(unsigned(ntiles)), dim3(256), 0, s, nrows, f.lpr_log2, f.rpw_log2,
-                           in, counts, nullptr, nullptr, nullptr);
+        hipLaunchKernelGGL((f.pieces ? k_spadd_few<false, true> : k_spadd_few<false, false>), dim3(unsigned(ntiles)),
+                           dim3(256), 0, s, nrows, f.lpr_log2, f.rpw_log2, in, counts, nullptr, nullptr, nullptr);
     else
         hipLaunchKernelGGL((k_spadd_tile<false, kSpCountThreads, kSpCountCap>), dim3(unsigned(ntiles)),
                            dim3(kSpCountThreads), 0, s, nrows, tl.rows, tl.lpr, in, counts, nullptr, nullptr, nullptr);
@@ -619,11 +637,12 @@ int launch_spadd_fill(uint64_t nrows, const double *a, uint64_t nnz1, const uint
     const uint64_t ntiles = few ? f.blocks : (nrows + tl.rows - 1) / tl.rows;
     if (ntiles > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "sparse add: too many row tiles");
     if (few)
-        hipLaunchKernelGGL(k_spadd_few<true>, dim3(unsigned(ntiles)), dim3(256), 0, s, nrows, f.lpr_log2, f.rpw_log2, in, nullptr,
-                           ipo, ixo, reinterpret_cast<double2 *>(dout));
+        hipLaunchKernelGGL((f.pieces ? k_spadd_few<true, true> : k_spadd_few<true, false>), dim3(unsigned(ntiles)),
+                           dim3(256), 0, s, nrows, f.lpr_log2, f.rpw_log2, in, nullptr, ipo, ixo,
+                           reinterpret_cast<double2 *>(dout));
     else
-    hipLaunchKernelGGL((k_spadd_tile<true, kSpFillThreads, kSpCap>), dim3(unsigned(ntiles)), dim3(kSpFillThreads), 0, s, nrows,
-                       tl.rows, tl.lpr, in, nullptr, ipo, ixo, reinterpret_cast<double2 *>(dout));
+        hipLaunchKernelGGL((k_spadd_tile<true, kSpFillThreads, kSpCap>), dim3(unsigned(ntiles)), dim3(kSpFillThreads),
+                           0, s, nrows, tl.rows, tl.lpr, in, nullptr, ipo, ixo, reinterpret_cast<double2 *>(dout));
     QR_HIP_CHECK(hipGetLastError());
     return QR_OK;
 }

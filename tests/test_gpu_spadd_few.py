@@ -68,12 +68,14 @@ def test_few(rows, cols, long, short):
             assert np.array_equal(np.asarray(data).view(np.uint64), np.asarray(ref[2]).view(np.uint64))
 
 
-@pytest.mark.parametrize("rows,cols,long,short", [(300, 9, [8, 3, 5], [1]), (300, 9, [8, 3, 5], [1, 2, 0, 3]),
-                                                  (130, 6, [24, 1, 0], [1, 0]), (130, 40, [64], [1]),
-                                                  (130, 12, [70, 200, 2], [1, 3]), (1, 6, [2], [1])])
+@pytest.mark.parametrize("rows,cols,long,short", [(300, 9, [8, 2, 5], [1]), (300, 9, [8, 2, 5], [0, 2, 1, 1]),
+                                                  (130, 6, [24, 2], [1]), (130, 6, [24, 2], [2, 0]), (130, 40, [64], [1]),
+                                                  (130, 12, [300, 900, 2], [1, 3]), (1, 6, [2], [1])])
 def test_few_of_any_order(rows, cols, long, short):
     """Rows whose columns do not ascend or come twice: every entry keeps a place
-    of its own, those of the merge."""
+    of its own, those of the merge.  (As many short entries as rows and a whole
+    number of long ones per row, or rows too long for the staged tile: the sums
+    that lane groups take.)"""
     import qrusty_amd as qa
     rng = np.random.default_rng(rows + cols + len(short))
 
@@ -93,3 +95,15 @@ def test_few_of_any_order(rows, cols, long, short):
         ref = orc.csr_add(rows, 1.0, first, -1.0, second)
         assert np.array_equal(indptr, ref[0]) and np.array_equal(indices, ref[1])
         assert np.array_equal(np.asarray(data).view(np.uint64), np.asarray(ref[2]).view(np.uint64))
+
+
+# rows that do and do not fit their lanes side by side (as many short entries as
+# rows), and long rows on both sides of the rule
+UNEVEN = [(64, 40, [5, 30], [0, 2]), (1000, 90, [3, 70, 20, 40], [0, 2, 1, 1]), (131, 90, [2, 90, 1], [1]),
+          (4, 30, [3, 9], [4, 0, 0, 0]), (77, 300, [127], [1]), (77, 300, [128], [1]), (50, 400, [190, 194], [2]),
+          (50, 400, [190, 193], [2]), (40, 900, [1, 800, 0, 300], [1])]
+
+
+@pytest.mark.parametrize("rows,cols,long,short", UNEVEN)
+def test_few_uneven(rows, cols, long, short):
+    test_few(rows, cols, long, short)
