@@ -692,33 +692,46 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
     if (row < nrows && lane == 0) y[row] = acc;
 }
 
-// Rows of 8..64 entries on average (128 past the MALL): a wave takes 8 consecutive rows, whose
-// entries are contiguous, streams them in whole lines (U loads of 64
-// consecutive entries, nontemporal: the x lines keep the caches), and reads them
-// back from LDS in the gather layout of qr_mv.h: lane (s, t) takes the entries
-// s, s + 8, ... of row t, so that the 8 rows that read one x line do so in one
-// instruction.  Waves whose rows do not fit that (a general CSR) read them from
-// memory in the same per-lane order; the sums are bit-identical to
-// k_csr_matvec<8, false>.
+// Rows of 8 to 64 entries on average (128 past the MALL): a wave takes 8
+// consecutive rows, whose entries are contiguous, streams them in whole lines (U
+// loads of 64 consecutive entries, nontemporal: the x lines keep the caches), and
+// reads them back from LDS in the gather layout of qr_mv.h: lane (s, t) takes the
+// entries s, s + 8, ... of row t, so that the 8 rows that read one x line do so
+// in one instruction.  Waves whose rows do not fit that (a general CSR) read them
+// from memory in the same per-lane order, kD entries per lane in flight; the sums
+// are bit-identical to k_csr_matvec<8, false>.
 // What bounds it: memory, 6.2 TB/s with the x lines read again past L2 (the
-// 24-qubit ring: 10.1 GB of CSR, 12.8 GB fetched).  Two rows per 8-lane slot,
-// loaded straight to the gather layout / this, us: rings of 20, 23, 24 qubits
-// 118 / 96, 1122 / 948, 2460 / 2056; terms of weight 1 to 4, 23 qubits (29
-// entries) 1385 / 1140; random operators of 20 entries, 23 qubits 1044 / 938, 31,
-// 22 qubits 731 / 676; 24, 22 qubits 547 / 564, where x comes past L2 for every
-// entry; and for k_csr_matvec<8> / this, 35, 48, 64 entries, 22 qubits 836 /
-// 754, 1077 / 1073, 1439 / 1373; terms of weight 1 to 4 (45 and 57 entries) 1060
-// / 835, 1318 / 1076; for 2 and 4 lanes per row / this, 8, 10, 24 qubits 949 /
-// 867, 1190 / 1020, 12, 15, 23 qubits 668 / 544, 839 / 703, but 6, 24 qubits 710
-// / 789.  Rows of 65 to 128 run blocks of two waves (three blocks' LDS per CU),
-// only in matrices of equal rows and 2^25 entries on: 70, 96, 22 qubits 1666 /
-// 1489, 2123 / 2150, 110, 128, 21 qubits 1309 / 1170, 1442 / 1346, weights 1 to
-// 4, 82 and 110 entries 1681 / 1525, 2205 / 2115; where the MALL holds the
-// matrix 28 / 33 (100 entries, 16 qubits).
+// 24-qubit ring: 10.1 GB of CSR, 12.8 GB fetched).
+// Matrices past the MALL's 256 MB.  Two rows per 8-lane slot, loaded straight to
+// the gather layout / this, us: rings of 20, 23, 24 qubits 118 / 96, 1122 / 948,
+// 2460 / 2056; terms of weight 1 to 4, 23 qubits (29 entries) 1385 / 1140; random
+// operators of 20 entries, 23 qubits 1044 / 938, 31, 22 qubits 731 / 676; 24, 22
+// qubits 547 / 564, where x comes past L2 for every entry; and for
+// k_csr_matvec<8> / this, 35, 48, 64 entries, 22 qubits 836 / 754, 1077 / 1073,
+// 1439 / 1373; terms of weight 1 to 4 (45 and 57 entries) 1060 / 835, 1318 /
+// 1076; for 2 and 4 lanes per row / this, 8, 10, 24 qubits 949 / 867, 1190 /
+// 1020, 12, 15, 23 qubits 668 / 544, 839 / 703, but 6, 24 qubits 710 / 789.
+// Rows of uneven length (as many lanes per row / this): isotropic rings without
+// their zeros, 23, 24, 26 qubits (12.5 to 14 entries in the mean) 727 / 611, 1494
+// / 1284, 6690 / 5490; Poisson lengths of 20, 28, 40, 50, 20 to 21 qubits 164 /
+// 133, 431 / 329, 267 / 226, 331 / 283; half of the rows 3 and half 40 long 150 /
+// 125; one row in 100 of 600 entries, the others 15, 328 / 194 (with one entry per
+// lane in flight for the waves that do not fit 422); half 30 and half 90 long,
+// the one kind measured slower, 171 / 180.
+// Rows of 65 to 128 run blocks of two waves (three blocks' LDS per CU), only in
+// matrices of equal rows and 2^25 entries on: 70, 96, 22 qubits 1666 / 1489, 2123
+// / 2150, 110, 128, 21 qubits 1309 / 1170, 1442 / 1346, weights 1 to 4, 82 and 110
+// entries 1681 / 1525, 2205 / 2115; where the MALL holds the matrix 28 / 33 (100
+// entries, 16 qubits).
+// Where the MALL holds the matrix the streams gain nothing, and only equal rows
+// from 11 entries on run here: 19 qubits, 12, 20 entries 46 / 46, 58 / 58, 16
+// qubits, 17 entries 18 / 16.5; but 8 and 10 entries, 20 and 19 qubits 58 / 65,
+// 41 / 44, Poisson lengths of 12, 50, 19 and 17 qubits 42 / 49, 40 / 44.
 // U: loads per lane; rows of up to 8 U entries.
+constexpr uint64_t kMallBytes = uint64_t(1) << 28;
 constexpr uint64_t kShortLongNnz = uint64_t(1) << 25;
 template <uint32_t U, uint32_t kWaves = 4>
-__global__ __launch_bounds__(64 * kWaves) void k_csr_matvec_short(uint64_t nrows, uint64_t ncols, uint64_t nnz,
+__global__ __launch_bounds__(64 * kWaves, U <= 3 ? 8 : 1) void k_csr_matvec_short(uint64_t nrows, uint64_t ncols, uint64_t nnz,
                                                           uint32_t nblocks_xcd,
                                                           const uint64_t *__restrict__ indptr,
                                                           const uint64_t *__restrict__ indices,
@@ -726,6 +739,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_csr_matvec_short(uint64_t nrows
                                                           const double2 *__restrict__ x,
                                                           double2 *__restrict__ y) {
     constexpr uint32_t kFit = 64 * U;  // entries of a wave's rows
+    constexpr uint32_t kD = U <= 3 ? 4 : 8;
     __shared__ uint64_t s_idx[kWaves][kFit];
     __shared__ dvec2 s_dat[kWaves][kFit];
     uint32_t b = blockIdx.x;
@@ -785,9 +799,28 @@ __global__ __launch_bounds__(64 * kWaves) void k_csr_matvec_short(uint64_t nrows
             if (cc < ncols) add(s_dat[wave][at + p], x[cc]);
         }
     } else {
-        for (uint64_t k = k0 + ls; k < k1; k += 8) {
-            const uint64_t cc = indices[k];
-            if (cc < ncols) add(*reinterpret_cast<const dvec2 *>(data + k), x[cc]);
+        // kD entries per lane in flight
+        for (uint64_t k = k0 + ls; k < k1; k += 8 * kD) {
+            uint64_t c[kD];
+            dvec2 a[kD];
+            double2 bx[kD];
+#pragma unroll
+            for (uint32_t u = 0; u < kD; ++u) {
+                c[u] = ~uint64_t(0);
+                a[u] = dvec2{0.0, 0.0};
+                if (k + 8 * u < k1) {
+                    c[u] = indices[k + 8 * u];
+                    a[u] = *reinterpret_cast<const dvec2 *>(data + k + 8 * u);
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kD; ++u) {
+                bx[u] = make_double2(0.0, 0.0);
+                if (c[u] < ncols) bx[u] = x[c[u]];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kD; ++u)
+                if (c[u] < ncols) add(a[u], bx[u]);
         }
     }
 #pragma unroll
@@ -896,10 +929,12 @@ int launch_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint64
     auto y = reinterpret_cast<double2 *>(d_y);
     const dim3 grid(static_cast<unsigned>(nblocks)), block(256);
     const bool nt = avg >= kMvNontemporalMinRow;
-    if (ncols && avg >= 8 && (avg <= 64 || (avg <= 128 && nnz >= kShortLongNnz && nnz % nrows == 0))) {
-        // a wave's eight rows are to fit, with a quarter to spare where they
+    const bool equal = nnz % nrows == 0, in_mall = nnz * 24 <= kMallBytes;
+    if (ncols && avg >= 8 && (in_mall ? equal && avg >= 11 && avg <= 64
+                                      : avg <= 64 || (avg <= 128 && equal && nnz >= kShortLongNnz))) {
+        // a wave's eight rows are to fit, with an eighth to spare where they
         // cannot be equal
-        const uint64_t need = nnz % nrows == 0 ? avg : avg + avg / 4 + 1;
+        const uint64_t need = equal ? avg : avg + avg / 8 + 1;
         const uint32_t waves = need > 64 ? 2 : 4;  // (the LDS of three blocks per CU)
         const uint64_t nb = (nrows + 8 * waves - 1) / (8 * waves);
         if (nb > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "CSR matvec grid too large");

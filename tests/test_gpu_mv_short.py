@@ -65,3 +65,32 @@ def test_long_rows_of_large_matrices(n, terms):
     ref = orc.apply_rows(p, x, rows)[0]
     bound = sum(abs(c) * np.abs(x[(rows ^ xm).astype(np.int64)]) for c, xm in zip(p.cp.view(np.complex128), p.x))
     assert np.all(np.abs(y[rows.astype(np.int64)] - ref) <= 1e-12 * bound)
+
+
+@pytest.mark.parametrize("n,mean,dense", [(21, 8.0, 40), (20, 12.0, 600), (19, 25.0, 200), (18, 60.0, 90)])
+def test_uneven_rows_of_large_matrices(n, mean, dense):
+    """Matrices past 256 MB whose rows vary about their mean, one in 100 with
+    `dense` entries: waves that fit beside waves that do not.  Against numpy
+    within (2 len + 8) eps sum |a||x| per row."""
+    import qrusty_amd as qa
+    rng = np.random.default_rng(n)
+    rows = 1 << n
+    lens = np.where(rng.random(rows) < 0.01, dense, rng.poisson(mean, rows)).astype(np.int64)
+    lens[-3:] = [dense, 0, dense]
+    indptr = np.concatenate([[0], np.cumsum(lens)])
+    nnz = int(indptr[-1])
+    which = np.repeat(np.arange(rows), lens)
+    k = np.arange(nnz) - indptr[which]
+    ind = (which // 1024 * 1024 + k).clip(0, rows + 5)  # (the last past the state)
+    data = rng.standard_normal(nnz) + 1j * rng.standard_normal(nnz)
+    x = rng.standard_normal(rows) + 1j * rng.standard_normal(rows)
+    m = qa.SpMat.new_unchecked((rows, rows), data, ind.astype(np.uint64), indptr.astype(np.uint64))
+    print(f"[gpu] uneven rows n={n} mean={mean} dense={dense} nnz={nnz}", flush=True)
+    assert 24 * nnz > 1 << 28
+    y = qa.spmat_dot_densevec(m, torch.from_numpy(x).cuda()).cpu().numpy()
+    prod = np.where(ind < rows, data * x[np.minimum(ind, rows - 1)], 0)
+    size = np.where(ind < rows, np.abs(data) * np.abs(x[np.minimum(ind, rows - 1)]), 0)
+    starts = np.minimum(indptr[:-1], nnz - 1)
+    ref = np.where(lens > 0, np.add.reduceat(prod, starts), 0)
+    bound = np.where(lens > 0, np.add.reduceat(size, starts), 0) * (2 * lens + 8) * 2.3e-16
+    assert np.all(np.abs(y - ref) <= bound + 1e-300)
