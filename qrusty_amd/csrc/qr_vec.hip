@@ -96,8 +96,14 @@ __global__ __launch_bounds__(256) void k_diag_scan(uint64_t n, uint32_t lpr_log2
     }
     const uint64_t met = __ballot(at != ~uint64_t(0)) >> ((threadIdx.x & 63u) & ~(lpr - 1u));
     const uint64_t mine = met & (lpr == 64 ? ~uint64_t(0) : (uint64_t(1) << lpr) - 1);
-    // (a column that comes twice in a row: the lower lane's)
-    if (mine ? lane != uint32_t(__ffsll((unsigned long long)mine)) - 1u : lane != 0) return;
+    // (a column that comes more than once in the row: its first entry)
+    uint64_t first = at;
+    if (mine & (mine - 1))
+        for (uint32_t o = 1; o < lpr; o <<= 1) {
+            const uint64_t other = __shfl_xor(first, int(o));
+            first = other < first ? other : first;
+        }
+    if (mine ? at == ~uint64_t(0) || at != first : lane != 0) return;
     const double2 d = mine ? data[at] : make_double2(0.0, 0.0);
     out[r] = kPrecond ? precond_entry(d, dx[r], e, tol) : d;
 }

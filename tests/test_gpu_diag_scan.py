@@ -47,3 +47,27 @@ def test_scan(rows, cols, lens):
     for e, tol in [(0.3 - 0.1j, 1e-3), (0.0, 0.5)]:
         assert np.array_equal(np.asarray(qa.precond(m, dx, e, tol)).view(np.uint64),
                               np.asarray(qa.precond2(want, dx, e, tol)).view(np.uint64))
+
+
+@pytest.mark.parametrize("rows,mean", [(200, 8), (200, 13), (300, 31), (129, 47)])
+def test_scan_of_repeated_columns(rows, mean):
+    """Rows in any order that hold their diagonal column more than once: the
+    first entry of the row that has it, whichever lanes read them."""
+    import qrusty_amd as qa
+    from oracle import oracle as orc
+    rng = np.random.default_rng(rows + mean)
+    indptr = np.arange(rows + 1, dtype=np.uint64) * np.uint64(mean)
+    indices = rng.integers(0, rows, (rows, mean))
+    for r in range(rows):
+        if r % 2:
+            indices[r].sort()
+        at = (r // 2) % mean  # the pair on every place of the row, on two lanes or one
+        indices[r, at] = indices[r, min(at + 1 + r % 5, mean - 1)] = r
+        if r % 2:
+            indices[r].sort()
+    data = rng.standard_normal(rows * mean) + 1j * rng.standard_normal(rows * mean)
+    indices = indices.reshape(-1).astype(np.uint64)
+    want = orc.csr_diagonal((rows, rows), indptr, indices, data)
+    m = qa.SpMat.new_unchecked((rows, rows), data, indices, indptr)
+    print(f"[gpu] diagonal scan, repeated columns rows={rows} mean={mean}", flush=True)
+    assert np.array_equal(np.asarray(m.diagonal()), want)
