@@ -478,6 +478,23 @@ static int launch_build_words(const qr_op *op, const DeviceTables *t, uint64_t r
         // would have under four blocks per CU
         uint32_t ml = op->word_real || t->nheavy ? kWordMaxLog2 : kWordMaxLog2 - 1;
         while (ml > 2 && nl * ((row_end - row_begin) >> (rs_log2 + ml)) < 1024) --ml;
+        // and as few as the LDS holds all heavy groups' values for (by 8 batches
+        // it does: a heavy group has 4 times the mean of terms, so they are at
+        // most a quarter of the operator's, and kMaxHeavy).  The lanes of a group
+        // that does not fit load its terms for every row: 32 batches whether they
+        // fit or not / this, us: 24 qubits, 8 groups, one of 64, 300 terms 4230 /
+        // 644, 20900 / 1270, with complex coefficients 8270 / 1270; 23 qubits, 12
+        // groups, two of 200 13800 / 935; 21 qubits, 64 groups, 15 of 100 11060 /
+        // 1045; 20 qubits, 200 groups, 40 of 100 7640 / 1490.
+        auto all_fit = [&]() {
+            for (size_t k = first; k < last; ++k) {
+                const WordLeaf &lf = op->word_leaves[k];
+                if (WordLds(lf.g, rs_log2, rs_log2 + ml, lf.hcnt, op->word_ptr.data() + lf.at).nheavy < lf.hcnt)
+                    return false;
+            }
+            return true;
+        };
+        while (ml > 2 && !all_fit()) --ml;
         const uint32_t tl = rs_log2 + ml;
         const uint64_t nt = nl * (((row_end - 1) >> tl) - (row_begin >> tl) + 1);
         if (nt > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "CSR build grid too large");

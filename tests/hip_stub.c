@@ -10,7 +10,7 @@
 enum { kMaxLaunch = 4096, kMaxKernel = 4096 };
 static struct { const void *host; const char *name; } kernels[kMaxKernel];
 static int nkernels;
-static struct { const char *name; uint32_t arg, blocks; } launches[kMaxLaunch];
+static struct { const char *name; uint32_t arg, blocks; size_t shmem; } launches[kMaxLaunch];
 static int nlaunches;
 static const char *watch_name = "";
 static int watch_arg;
@@ -22,6 +22,7 @@ int stub_launches(void) { return nlaunches; }
 const char *stub_name(int i) { return launches[i].name; }
 uint32_t stub_arg(int i) { return launches[i].arg; }
 uint32_t stub_blocks(int i) { return launches[i].blocks; }
+uint32_t stub_shmem(int i) { return (uint32_t)launches[i].shmem; }
 void stub_reset(void) { nlaunches = 0; malloc_bytes = 0; }
 void stub_watch(const char *name, int arg) { watch_name = strdup(name); watch_arg = arg; }
 void stub_fail_malloc_after(long n) { malloc_left = n; }
@@ -57,13 +58,14 @@ int __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *s, void **st) {
     return 0;
 }
 int hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t shmem, void *stream) {
-    (void)block; (void)shmem; (void)stream;
+    (void)block; (void)stream;
     if (nlaunches == kMaxLaunch) return 1;
     const char *name = "";
     for (int i = 0; i < nkernels; ++i)
         if (kernels[i].host == f) name = kernels[i].name;
     launches[nlaunches].name = name;
     launches[nlaunches].blocks = grid.x;
+    launches[nlaunches].shmem = shmem;
     launches[nlaunches].arg = 0;
     if (*watch_name && strstr(name, watch_name)) memcpy(&launches[nlaunches].arg, args[watch_arg], 4);
     ++nlaunches;

@@ -88,3 +88,24 @@ op = op_of(labels)
 L.check(L.lib.qr_pauli_apply(op, L.QR_PREC_MIXED, 1, 64 * GB, 128 * GB, None, None))
 assert len(launched("k_apply")) == 1, launched("k_apply")
 """)
+
+
+@pytest.mark.parametrize("groups,heavy", [(5, 1), (8, 1), (12, 2), (32, 6), (64, 15), (128, 30)])
+def test_build_folds_every_heavy_group(run, groups, heavy):
+    """A tile of the CSR build has room for the values of all heavy groups (16
+    bytes a row each, after two stages of 24 bytes per entry of a batch): those
+    that it does not fold it loads term by term for every row."""
+    run(f"""
+n, groups, heavy = 24, {groups}, {heavy}
+labels = []
+for g in range(groups):
+    for t in range(64 if g < heavy else 1):
+        xz = (g << 12, t)
+        labels.append("".join("IZXY"[2 * (xz[0] >> q & 1) + (xz[1] >> q & 1)] for q in reversed(range(n))))
+op = op_of(labels)
+L.check(L.lib.qr_csr_build(op, 64 * GB, 128 * GB, 192 * GB, None))
+(k,) = [i for i in range(stub.stub_launches()) if "k_csr_build" in stub.stub_name(i).decode()]
+rows = (1 << n) // stub.stub_blocks(k)
+per_batch = 1024 >> (groups - 1).bit_length()
+assert stub.stub_shmem(k) >= 48 * groups * per_batch + 16 * heavy * rows, (stub.stub_shmem(k), rows)
+""")
