@@ -756,7 +756,10 @@ __global__ __launch_bounds__(64 * kWaves, U <= 3 ? 8 : 1) void k_csr_matvec_shor
                                                           const double2 *__restrict__ x,
                                                           double2 *__restrict__ y) {
     constexpr uint32_t kFit = 64 * U;  // entries of a wave's rows
-    constexpr uint32_t kD = U <= 3 ? 4 : 8;
+    // entries per lane in flight where the rows do not fit: 8 take 92 VGPRs, which
+    // cost U = 4 a wave per SIMD (25 and 29 equal entries, 22 qubits, 4 / 8: 515 /
+    // 526, 572 / 581 us; one row in 100 of 600 entries, the others 18, 236 / 213)
+    constexpr uint32_t kD = U <= 4 ? 4 : 8;
     __shared__ uint64_t s_idx[kWaves][kFit];
     __shared__ dvec2 s_dat[kWaves][kFit];
     uint32_t b = blockIdx.x;
