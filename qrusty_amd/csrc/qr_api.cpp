@@ -103,6 +103,7 @@ void free_tables(DeviceTables &t) {
                         (void *)t.gkind})
             if (p) (void)hipFree(p);
     if (t.mem) (void)hipFree(t.mem);
+    if (t.word_mem) (void)hipFree(t.word_mem);
     for (auto &pt : t.pat) free_patterns(pt);
     t = DeviceTables{};
 }
@@ -379,6 +380,7 @@ class TableSet {
     template <typename T>
     void add(T **dst, const std::vector<T> &src) { add(dst, src.data(), src.size()); }
     int upload(void **mem) const {
+        if (!total_) return QR_OK;
         QR_HIP_CHECK(hipMalloc(mem, total_));
         unsigned char *base = static_cast<unsigned char *>(*mem);
         if (total_ <= kStageBytes) {
@@ -395,8 +397,27 @@ class TableSet {
     }
 };
 
-// with_base: also the tables that qr_group.hip builds on the device
-int upload_tables(const qr_op *op, DeviceTables &t, bool with_base) {
+// The sign-word builder's tables; `rank` holds one of them until the upload.
+static void add_words(const qr_op *op, DeviceTables &t, TableSet &set, std::vector<int32_t> &rank) {
+    // rank lists by bit, without the sub-operators' ancestors
+    rank.resize(uint64_t(op->nq) * op->G);
+    for (const auto &lf : op->word_leaves) {
+        uint32_t depth = 0;
+        for (int32_t v : lf.off) depth += v != 0;
+        for (uint32_t g = lf.s0; g < lf.s0 + lf.g; ++g)
+            for (uint32_t e = op->rl_ptr[g] + depth; e < op->rl_ptr[g + 1]; ++e)
+                rank[uint64_t(op->rl[e].bit) * op->G + g] = op->rl[e].sigma;
+    }
+    set.add(&t.word_leaves, op->word_leaves);
+    set.add(&t.word_groups, op->word_groups);
+    set.add(&t.word_rank, rank);
+    set.add(&t.word_ptr, op->word_ptr);
+    set.add(&t.word_terms, op->word_terms);
+}
+
+// with_base: also the tables that qr_group.hip builds on the device;
+// with_words: also the sign-word builder's, in the same copy
+int upload_tables(const qr_op *op, DeviceTables &t, bool with_base, bool with_words) {
     TableSet set;
     if (with_base) {
         set.add(&t.gx, op->gx);
@@ -410,22 +431,8 @@ int upload_tables(const qr_op *op, DeviceTables &t, bool with_base) {
     if (!op->heavy.empty()) set.add(&t.heavy, op->heavy);
     if (!op->leaf_heavy.empty()) set.add(&t.leaf_heavy, op->leaf_heavy);
     std::vector<int32_t> rank;
-    if (!op->word_leaves.empty()) {
-        // rank lists by bit, without the sub-operators' ancestors
-        rank.resize(uint64_t(op->nq) * op->G);
-        for (const auto &lf : op->word_leaves) {
-            uint32_t depth = 0;
-            for (int32_t v : lf.off) depth += v != 0;
-            for (uint32_t g = lf.s0; g < lf.s0 + lf.g; ++g)
-                for (uint32_t e = op->rl_ptr[g] + depth; e < op->rl_ptr[g + 1]; ++e)
-                    rank[uint64_t(op->rl[e].bit) * op->G + g] = op->rl[e].sigma;
-        }
-        set.add(&t.word_leaves, op->word_leaves);
-        set.add(&t.word_groups, op->word_groups);
-        set.add(&t.word_rank, rank);
-        set.add(&t.word_ptr, op->word_ptr);
-        set.add(&t.word_terms, op->word_terms);
-    }
+    with_words = with_words && !op->word_leaves.empty();
+    if (with_words) add_words(op, t, set, rank);
     if (op->ntail) {
         set.add(&t.ttz, op->ttz);
         set.add(&t.ttc, op->ttc.data(), op->ttz.size());
@@ -434,10 +441,29 @@ int upload_tables(const qr_op *op, DeviceTables &t, bool with_base) {
     if (int rc = set.upload(&t.mem)) return rc;
     t.nheavy = uint32_t(op->heavy.size());
     t.ntail = op->ntail;
+    t.words = with_words;
     return QR_OK;
 }
 
-int device_tables(const qr_op *op, DeviceTables **out, bool noalloc) {
+int word_tables(const qr_op *op, DeviceTables *t, hipStream_t s, bool *have) {
+    std::lock_guard<std::mutex> lock(op->mu);
+    *have = t->words;
+    if (t->words || op->word_leaves.empty()) return QR_OK;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return QR_OK;
+    }
+    if (st != hipStreamCaptureStatusNone) return QR_OK;
+    TableSet set;
+    std::vector<int32_t> rank;
+    add_words(op, *t, set, rank);
+    if (int rc = set.upload(&t->word_mem)) return rc;
+    *have = t->words = true;
+    return QR_OK;
+}
+
+int device_tables(const qr_op *op, DeviceTables **out, bool noalloc, bool with_words) {
     int dev = 0;
     QR_HIP_CHECK(hipGetDevice(&dev));
     if (dev < 0 || dev >= kMaxDevices) return fail(QR_ERR_ARG, "device index out of range");
@@ -447,7 +473,7 @@ int device_tables(const qr_op *op, DeviceTables **out, bool noalloc) {
         return fail(QR_ERR_ARG, "apply_noalloc: the operator's tables are not on this device "
                                 "(one qr_pauli_apply of it on this device uploads them)");
     if (!t.ready) {
-        if (int rc = upload_tables(op, t, true)) {
+        if (int rc = upload_tables(op, t, true, with_words)) {
             free_tables(t);
             return rc;
         }
@@ -954,7 +980,7 @@ int qr_csr_build(const qr_op *op, uint64_t *d_indptr, uint64_t *d_indices, doubl
     if (!op || !d_indptr || !d_indices || !d_data) return fail(QR_ERR_ARG, "null argument");
     if (op->nq > 40) return fail(QR_ERR_SIZE, "CSR of more than 40 qubits is not supported");
     DeviceTables *t;
-    int rc = device_tables(op, &t);
+    int rc = device_tables(op, &t, false, /*with_words=*/true);
     if (rc) return rc;
     return launch_csr_build(op, t, 0, uint64_t(1) << op->nq, d_indptr, d_indices, d_data,
                             (hipStream_t)stream);
@@ -968,7 +994,7 @@ int qr_csr_build_rows(const qr_op *op, uint64_t row_begin, uint64_t row_end, uin
         return fail(QR_ERR_ARG, "row range out of bounds");
     if (row_end == row_begin) return QR_OK;
     DeviceTables *t;
-    int rc = device_tables(op, &t);
+    int rc = device_tables(op, &t, false, /*with_words=*/true);
     if (rc) return rc;
     return launch_csr_build(op, t, row_begin, row_end, nullptr, d_indices, d_data,
                             (hipStream_t)stream);

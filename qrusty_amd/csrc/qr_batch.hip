@@ -261,6 +261,7 @@ struct Plan {
     uint64_t items[2] = {};
     size_t shmem[2] = {};
     std::vector<uint32_t> branch[kBranches];  // the others, in order
+    std::vector<bool> csr;                    // whether operator k's CSR is built
     std::vector<BatchMvDesc> mv;              // split form: one per operator
     uint64_t mv_items = 0;
 };
@@ -284,11 +285,12 @@ int make_plan(qr_batch *b, uint64_t *const *d_indptr, uint64_t *const *d_indices
             return (b->ops[a]->G << b->ops[a]->nq) > (b->ops[c]->G << b->ops[c]->nq);
         });
     uint64_t load[kBranches] = {};
+    plan.csr.resize(nops);
     for (uint32_t k : order) {
         const qr_op *op = b->ops[k];
         if (op->nq > 32) return fail(QR_ERR_SIZE, "batch operators are limited to 32 qubits");
         if (!d_x || !d_x[k] || !d_y || !d_y[k]) return fail(QR_ERR_ARG, "null state pointer in batch");
-        const bool csr = has_csr(d_indices, d_data, k);
+        const bool csr = plan.csr[k] = has_csr(d_indices, d_data, k);
         if (!tu.split && op->G > kBatchMostG && !(csr && d_indptr && d_indptr[k]))
             return fail(QR_ERR_ARG, "batch operators with more than 6144 distinct x masks "
                                     "need CSR output buffers");
@@ -401,7 +403,9 @@ int prepare(qr_batch *b, const Plan &plan, const qr_tuning &tu) {
         }
         for (uint32_t k : branch) {
             DeviceTables *t;
-            if ((rc = device_tables(b->ops[k], &t))) return rc;
+            bool have;
+            if ((rc = device_tables(b->ops[k], &t, false, plan.csr[k]))) return rc;
+            if (plan.csr[k] && (rc = word_tables(b->ops[k], t, b->cap, &have))) return rc;
             if (!tu.split && (rc = apply_tables(b->ops[k], t))) return rc;
         }
     }

@@ -542,15 +542,17 @@ int launch_csr_indptr(const qr_op *op, uint64_t row_begin, uint64_t nrows, uint6
     return QR_OK;
 }
 
-int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin, uint64_t row_end,
+int launch_csr_build(const qr_op *op, DeviceTables *t, uint64_t row_begin, uint64_t row_end,
                      uint64_t *d_indptr, uint64_t *d_indices, double *d_data, hipStream_t s) {
     const uint64_t nrows = row_end - row_begin;
     if (op->G > 0x7FFFFFFFull) return fail(QR_ERR_SIZE, "too many groups");
     const uint32_t G = uint32_t(op->G);
-    if (op->nq <= 32 && nrows)
-        return launch_build_words(op, t, row_begin, row_end, d_indptr, d_indices, d_data, s);
-    // wider masks: the shared tile builder
     int rc;
+    bool words = false;
+    if (nrows && (rc = word_tables(op, t, s, &words))) return rc;
+    if (words) return launch_build_words(op, t, row_begin, row_end, d_indptr, d_indices, d_data, s);
+    // wider masks, and captures that come before any build of the operator: the
+    // shared tile builder
     if (d_indptr && (rc = launch_csr_indptr(op, row_begin, nrows, d_indptr, s))) return rc;
     if (nrows == 0) return QR_OK;
     if (!op->leaves.empty()) {

@@ -480,7 +480,7 @@ int group_terms_device(const char *const *labels, const double *coeffs, uint64_t
     for (void *p : {(void *)d_gx, (void *)d_gterm, (void *)d_tz, (void *)d_tc, (void *)d_rlptr,
                     (void *)d_rl, (void *)d_gkind})
         B.release(p);
-    if ((rc = upload_tables(op, t, false))) {
+    if ((rc = upload_tables(op, t, false, false))) {
         free_tables(t);
         delete op;
         return rc;

@@ -179,6 +179,10 @@ struct DeviceTables {
     double2 *ttc = nullptr;
     uint32_t ntail = 0;
     uint32_t *leaf_heavy = nullptr;  // qr_op::leaf_heavy
+    // the sign-word builder's, from the first CSR build on (word_tables): in
+    // `mem`, or in word_mem where another call made that one
+    bool words = false;
+    void *word_mem = nullptr;
     WordLeaf *word_leaves = nullptr;  // qr_op::word_leaves, word_groups, word_ptr, word_terms
     WordGroup *word_groups = nullptr;
     int32_t *word_rank = nullptr;  // [nq][G]: what bit b of r adds to the place of group g in its sub-operator
@@ -318,17 +322,23 @@ int group_terms_device(const char *const *labels, const double *coeffs, uint64_t
 // Sub-operators, heavy groups and tail table of an op whose grouped tables
 // are set.
 void finish_op(qr_op *op);
-// Uploads the op's heavy groups and tail table (where it has them) into t.
-int upload_tables(const qr_op *op, DeviceTables &t, bool with_base);
+// Uploads the op's heavy groups and tail table (where it has them) into t;
+// with_base, with_words: the grouped tables, the sign-word builder's as well.
+int upload_tables(const qr_op *op, DeviceTables &t, bool with_base, bool with_words);
 // Frees one device's tables of an op.
 void free_tables(DeviceTables &t);
 
 // Uploads the op's tables to the current device if needed; returns the tables.
-int device_tables(const qr_op *op, DeviceTables **out, bool noalloc = false);
+// with_words: for a CSR build, whose own tables then come in the same copy.
+int device_tables(const qr_op *op, DeviceTables **out, bool noalloc = false, bool with_words = false);
+// The sign-word builder's tables (4 n bytes per group and more, which only it
+// reads).  *have = false: they are not on the device and `s` is being captured,
+// which allows no upload; the shared tile builder needs none of them.
+int word_tables(const qr_op *op, DeviceTables *t, hipStream_t s, bool *have);
 
 // Kernel launchers (qr_csr.hip, qr_apply.hip).
 int launch_csr_indptr(const qr_op *op, uint64_t row_begin, uint64_t nrows, uint64_t *d_indptr, hipStream_t s);
-int launch_csr_build(const qr_op *op, const DeviceTables *t, uint64_t row_begin,
+int launch_csr_build(const qr_op *op, DeviceTables *t, uint64_t row_begin,
                      uint64_t row_end, uint64_t *d_indptr, uint64_t *d_indices,
                      double *d_data, hipStream_t s);
 int launch_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint64_t *d_indptr,

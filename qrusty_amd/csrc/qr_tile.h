@@ -1,6 +1,6 @@
 // qr_tile.h -- the LDS-staged row-tile builder shared by the CSR build of
-// operators past 32 qubits (qr_csr.hip) and the batch's small operators
-// (qr_batch.hip).
+// operators past 32 qubits, or captured before any build of the operator
+// (qr_csr.hip), and the batch's small operators (qr_batch.hip).
 //
 // Replaces accel::rowwise::make_row (qrusty/src/accel.rs:171-210) for one tile
 // of rows.  Thread layout: 1024 threads = RS rows x JW groups (JW a power of

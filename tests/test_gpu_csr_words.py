@@ -96,3 +96,31 @@ def test_row_windows(n, groups, sizes, real):
             a = 1 + (r - r0) * h.G
             assert np.array_equal(ih[a:a + h.G].view(np.uint64), cols)
             assert dh[a:a + h.G].tobytes() == vals.tobytes()
+
+
+@pytest.mark.parametrize("n,groups,sizes", [(9, 25, [2, 2, 2, 48]), (10, 300, [1, 3]), (12, 2600, [4, 4, 4, 6, 9])])
+def test_captured_before_any_build(n, groups, sizes):
+    """An operator whose first build is recorded into a graph, after an apply put
+    its other tables on the device: the tile builder's entries, on every replay."""
+    from qrusty_amd import _lib as L
+    labels, coeffs = _operator(n, groups, sizes, 3 * n + groups, False)
+    p, op = orc.Params(labels, coeffs), _op(labels, coeffs)
+    h = op._handle(L.QR_PHASE_ROWWISE)
+    ip, ind, dat = orc.build_csr(p)
+    x = torch.ones(p.N, dtype=torch.complex128, device="cuda")
+    op.apply(x)
+    out = [torch.empty(p.N + 1, dtype=torch.int64, device="cuda"), torch.empty(len(ind), dtype=torch.int64, device="cuda"),
+           torch.empty(len(ind), dtype=torch.complex128, device="cuda")]
+    print(f"[gpu] captured first build n={n} groups={groups}", flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        L.check(L.lib.qr_csr_build(h.h, *(ctypes.c_void_p(t.data_ptr()) for t in out),
+                                   ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    for _ in range(3):
+        for t in out:
+            t.fill_(7)
+        op.apply(x)
+        torch.cuda.synchronize()
+        graph.replay()
+        for t, want in zip(out, (ip, ind, dat)):
+            assert t.cpu().numpy().tobytes() == want.tobytes()

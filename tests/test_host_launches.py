@@ -109,3 +109,36 @@ rows = (1 << n) // stub.stub_blocks(k)
 per_batch = 1024 >> (groups - 1).bit_length()
 assert stub.stub_shmem(k) >= 48 * groups * per_batch + 16 * heavy * rows, (stub.stub_shmem(k), rows)
 """)
+
+
+def test_apply_uploads_no_build_tables(run):
+    """The sign-word builder's tables, 4 n bytes per group and more, come to the
+    device with the first CSR build; one that is captured before takes the tile
+    builder, which needs none, and neither allocates nor copies."""
+    run("""
+n = 24
+labels = [term(n, {q: c for q, c in zip(range(a, a + 6), cs)}) for a in range(18)
+          for cs in __import__("itertools").product("XY", "XYZ", "XI", "XZ", "IX", "XI")]
+labels = list(dict.fromkeys(labels))
+op, same = op_of(labels), op_of(labels)
+groups = ctypes.c_uint64()
+L.check(L.lib.qr_op_info(op, None, None, ctypes.byref(groups), None))
+rank = 4 * n * groups.value
+L.check(L.lib.qr_pauli_apply(op, 0, 1, 64 * GB, 128 * GB, None, None))
+applied = stub.stub_malloc_bytes()
+stub.stub_capture(1)
+L.check(L.lib.qr_csr_build(op, 64 * GB, 128 * GB, 192 * GB, None))
+stub.stub_capture(0)
+assert stub.stub_syncs_in_capture() == 0 and stub.stub_malloc_bytes() == applied
+assert launched("k_csr_build_staged") and not launched("k_csr_build_words")
+L.check(L.lib.qr_csr_build(op, 64 * GB, 128 * GB, 192 * GB, None))
+assert launched("k_csr_build_words") and stub.stub_malloc_bytes() >= applied + rank
+built = stub.stub_malloc_bytes()
+stub.stub_capture(1)
+L.check(L.lib.qr_csr_build(op, 64 * GB, 128 * GB, 192 * GB, None))
+stub.stub_capture(0)
+assert stub.stub_syncs_in_capture() == 0 and stub.stub_malloc_bytes() == built
+stub.stub_reset()
+L.check(L.lib.qr_csr_build(same, 64 * GB, 128 * GB, 192 * GB, None))
+assert rank <= stub.stub_malloc_bytes() and launched("k_csr_build_words")
+""")
