@@ -378,6 +378,14 @@ int record(qr_batch *b, const Plan &plan, const qr_tuning &tu, uint64_t *const *
     return QR_OK;
 }
 
+void drop_graph(qr_batch *b) {
+    if (b->exec) (void)hipGraphExecDestroy(b->exec);
+    if (b->graph) (void)hipGraphDestroy(b->graph);
+    b->exec = nullptr;
+    b->graph = nullptr;
+    b->have_graph = false;
+}
+
 // Everything that a recording must not do: streams, the operators' tables,
 // the matvec pass's descriptors.
 int prepare(qr_batch *b, const Plan &plan, const qr_tuning &tu) {
@@ -410,9 +418,10 @@ int prepare(qr_batch *b, const Plan &plan, const qr_tuning &tu) {
         }
     }
     const size_t nsmall = plan.small[0].size() + plan.small[1].size();
-    // a previous graph, which the caller destroys next, or tuning pass may
-    // still run and read the descriptors
+    // a previous graph or tuning pass may still run and read the descriptors; no
+    // graph outlives them
     QR_HIP_CHECK(hipDeviceSynchronize());
+    drop_graph(b);
     auto room = [](auto **d, size_t *cap, size_t n) {
         if (*cap >= n) return int(QR_OK);
         if (*d) (void)hipFree(*d);
@@ -432,14 +441,6 @@ int prepare(qr_batch *b, const Plan &plan, const qr_tuning &tu) {
         QR_HIP_CHECK(hipMemcpy(b->d_mv, plan.mv.data(), plan.mv.size() * sizeof(BatchMvDesc),
                                hipMemcpyHostToDevice));
     return QR_OK;
-}
-
-void drop_graph(qr_batch *b) {
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
-    b->have_graph = false;
 }
 
 std::vector<uintptr_t> key_of(const qr_batch *b, uint64_t *const *d_indptr,
@@ -513,7 +514,6 @@ int qr_batch_run(qr_batch *b, uint64_t *const *d_indptr, uint64_t *const *d_indi
         if (rc) return rc;
         rc = prepare(b, plan, tu);
         if (rc) return rc;
-        drop_graph(b);
         QR_HIP_CHECK(hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal));
         rc = record(b, plan, tu, d_indptr, d_indices, d_data, d_x, d_y, b->cap);
         hipGraph_t g = nullptr;
@@ -576,7 +576,6 @@ done:
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    drop_graph(b);  // the descriptors now hold the last candidate's plan
     b->tuned = bt;
     b->have_tuned = true;
     if (best) *best = bt;

@@ -142,3 +142,27 @@ stub.stub_reset()
 L.check(L.lib.qr_csr_build(same, 64 * GB, 128 * GB, 192 * GB, None))
 assert rank <= stub.stub_malloc_bytes() and launched("k_csr_build_words")
 """)
+
+
+def test_batch_graph_ends_with_its_descriptors(run):
+    """A tuning pass that fails part of the way has replaced the descriptors that
+    the recorded graph reads: the next run records again."""
+    run("""
+ops = [op_of([term(8, {q: "X"}) for q in range(k)]) for k in (2, 5)]
+batch = ctypes.c_void_p()
+L.check(L.lib.qr_batch_create((ctypes.c_void_p * 2)(*ops), 2, ctypes.byref(batch)))
+
+def args(at):
+    return [ctypes.cast((ctypes.c_void_p * 2)((at + 2 * k) * GB, (at + 2 * k + 1) * GB), ctypes.c_void_p) for k in range(5)]
+
+first, second = args(64), args(128)
+L.check(L.lib.qr_batch_run(batch, *first, None, None))
+L.check(L.lib.qr_batch_run(batch, *first, None, None))
+assert stub.stub_graphs_made() == 1
+stub.stub_fail_malloc_after.argtypes = [ctypes.c_long]
+stub.stub_fail_malloc_after(0)  # the matvec pass's descriptors, in the split candidates
+assert L.lib.qr_batch_tune(batch, *second, None, None) == -6
+stub.stub_fail_malloc_after(-1)
+L.check(L.lib.qr_batch_run(batch, *first, None, None))
+assert stub.stub_graphs_made() == 2
+""")
