@@ -146,7 +146,9 @@ typedef double dvec2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) unsigned char lds_byte;
 
 // LDS by absolute byte address.  The tile buffers and tables are aligned to
-// their sizes, so places in them are formed with XOR.
+// their sizes, so places in them are formed with XOR.  Both hold because the
+// apply kernels' dynamic LDS begins at address 0: they have no static LDS
+// (tests/test_apply_lds.py reads that from the built library).
 template <typename T>
 __device__ __forceinline__ T lds_load(uint32_t at) {
     return *(const __attribute__((address_space(3))) T *)(at);
