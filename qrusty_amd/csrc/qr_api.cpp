@@ -228,8 +228,6 @@ void build_patterns(const qr_op *op, const PatternShape &shape, const std::vecto
                 for (uint32_t c = 0; c <= uint32_t(kApplyClasses); ++c) cur.cg[c] = g0;
                 cur.cg[kApplyClasses] = g1;
             }
-            for (uint32_t i = 0; i < n; ++i)
-                if (was[i].m & far_mask) ++out.nfar;
             out.chunk.push_back(cur);
             out.max_tab = std::max(out.max_tab, cur_bytes);
         }
@@ -569,10 +567,8 @@ static int upload_patterns(DeviceTables::Patterns &pt, const HostPatterns &hp, c
     set.add(&pt.ptz, hp.ptz);
     set.add(&pt.ptc, hp.ptc.data(), hp.ptz.size());
     if (int rc = set.upload(&pt.mem)) return rc;
-    pt.ngrp = uint32_t(hp.grp.size());
     pt.nchunk = uint32_t(hp.chunk.size());
     pt.nrun = uint32_t(hp.run.size());
-    pt.nfar = hp.nfar;
     pt.max_tab = hp.max_tab;
     pt.cplx = hp.cplx;
     pt.win = shape.win;

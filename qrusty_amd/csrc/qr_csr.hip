@@ -626,17 +626,9 @@ int launch_csr_build(const qr_op *op, DeviceTables *t, uint64_t row_begin, uint6
 // gathers coalesce.  Blocks are handed to the 8 XCDs round-robin; the block
 // index is remapped so that each XCD works on one contiguous range of rows
 // and its L2 sees the neighbouring rows' x lines.
-// CSR stream loads: nontemporal (kNT) for long rows, plain for short ones.
-// Measured (MI355X, complex128): nontemporal wins from about 256 entries per
-// row (400: 5%, 1000: 7%, 2000: 2.4%) and loses below (150: 3%, 60: 8%,
-// 25 -- the 24-qubit Heisenberg CSR: 13%).
-template <bool kNT, typename T>
-__device__ __forceinline__ T mv_load(const T *p) {
-    if constexpr (kNT) return __builtin_nontemporal_load(p);
-    else return *p;
-}
-
-template <int LPR, bool kNT>
+// Plain stream loads: nontemporal ones lose in the rows that come here (150
+// entries: 3%, 60: 8%, 25 -- the 24-qubit Heisenberg CSR: 13%).
+template <int LPR>
 __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz,
                                                     uint32_t nblocks_xcd,
                                                     const uint64_t *__restrict__ indptr,
@@ -662,8 +654,8 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
             double2 a[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                c[u] = mv_load<kNT>(indices + k + u * LPR);
-                const dvec2 av = mv_load<kNT>(reinterpret_cast<const dvec2 *>(data + k + u * LPR));
+                c[u] = indices[k + u * LPR];
+                const dvec2 av = *reinterpret_cast<const dvec2 *>(data + k + u * LPR);
                 a[u] = make_double2(av.x, av.y);
             }
 #pragma unroll
@@ -686,8 +678,8 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
                 c[u] = ~uint64_t(0);
                 a[u] = make_double2(0.0, 0.0);
                 if (k + u * LPR < k1) {
-                    c[u] = mv_load<kNT>(indices + k + u * LPR);
-                    const dvec2 av = mv_load<kNT>(reinterpret_cast<const dvec2 *>(data + k + u * LPR));
+                    c[u] = indices[k + u * LPR];
+                    const dvec2 av = *reinterpret_cast<const dvec2 *>(data + k + u * LPR);
                     a[u] = make_double2(av.x, av.y);
                 }
             }
@@ -718,7 +710,7 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
 // entries s, s + 8, ... of row t, so that the 8 rows that read one x line do so
 // in one instruction.  Waves whose rows do not fit that (a general CSR) read them
 // from memory in the same per-lane order, kD entries per lane in flight; the sums
-// are bit-identical to k_csr_matvec<8, false>.
+// are bit-identical to k_csr_matvec<8>.
 // What bounds it: memory, 6.2 TB/s with the x lines read again past L2 (the
 // 24-qubit ring: 10.1 GB of CSR, 12.8 GB fetched).
 // Matrices past the MALL's 256 MB.  Two rows per 8-lane slot, loaded straight to
@@ -950,7 +942,6 @@ int launch_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint64
     auto data = reinterpret_cast<const double2 *>(d_data);
     auto y = reinterpret_cast<double2 *>(d_y);
     const dim3 grid(static_cast<unsigned>(nblocks)), block(256);
-    const bool nt = avg >= kMvNontemporalMinRow;
     const bool equal = nnz % nrows == 0, in_mall = nnz * 24 <= kMallBytes;
     if (ncols && avg >= 8 && (in_mall ? equal && avg >= 11 && avg <= 64
                                       : avg <= 64 || (avg <= 128 && equal && nnz >= kShortLongNnz))) {
@@ -974,22 +965,8 @@ int launch_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint64
         QR_HIP_CHECK(hipGetLastError());
         return QR_OK;
     }
-#define QR_MV_CASE(L)                                                                        \
-    case L:                                                                                  \
-        if (nt)                                                                              \
-            hipLaunchKernelGGL((k_csr_matvec<L, true>), grid, block, 0, s, nrows, ncols, nnz, \
-                               nbx, d_indptr, d_indices, data, x, y);                        \
-        else                                                                                 \
-            hipLaunchKernelGGL((k_csr_matvec<L, false>), grid, block, 0, s, nrows, ncols, nnz, \
-                               nbx, d_indptr, d_indices, data, x, y);                        \
-        break;
-    switch (lpr) {
-        QR_MV_CASE(1)
-        QR_MV_CASE(2)
-        QR_MV_CASE(4)
-        default: QR_MV_CASE(8)
-    }
-#undef QR_MV_CASE
+    auto kern = lpr == 1 ? k_csr_matvec<1> : lpr == 2 ? k_csr_matvec<2> : lpr == 4 ? k_csr_matvec<4> : k_csr_matvec<8>;
+    hipLaunchKernelGGL(kern, grid, block, 0, s, nrows, ncols, nnz, nbx, d_indptr, d_indices, data, x, y);
     QR_HIP_CHECK(hipGetLastError());
     return QR_OK;
 }

@@ -52,9 +52,6 @@ constexpr uint64_t kMaxTailSlots = uint64_t(1) << 22;
 constexpr uint32_t kSubMaxG = 2048;  // groups of one CSR-build sub-operator
 constexpr uint32_t kWordMaxG = 1024;  // the same of the sign-word builder
 constexpr uint32_t kWordHold = 6;     // terms of a group that it holds (real form)
-// CSR matvecs load the CSR stream nontemporally from this many entries per
-// row on (measured crossover; qr_csr.hip)
-constexpr uint64_t kMvNontemporalMinRow = 256;
 
 // Row-ordering entry: while building row r, a group whose sorted-x position is j
 // moves by `sigma` positions when bit `bit` of r is set (see build_rank_lists).
@@ -194,9 +191,8 @@ struct DeviceTables {
     struct Patterns {
         int L = -1;
         void *mem = nullptr;  // holds the arrays
-        uint32_t ngrp = 0, nchunk = 0, nrun = 0, max_tab = 0;
-        uint32_t nfar = 0;  // groups whose mask reaches outside the tile
-        ApplyGroup *grp = nullptr;    // [ngrp]
+        uint32_t nchunk = 0, nrun = 0, max_tab = 0;
+        ApplyGroup *grp = nullptr;    // by chunk
         ApplyChunk *chunk = nullptr;  // [nchunk]
         ApplyRun *run = nullptr;      // [nrun] (staged form only)
         ApplyPart *part = nullptr;  // parts of the groups that have more than one
@@ -232,7 +228,7 @@ struct HostPatterns {
     std::vector<uint64_t> ptz;
     std::vector<double> ptc;  // 2 per term
     std::vector<ApplyRun> run;  // staged form only
-    uint32_t max_tab = 0, nfar = 0;
+    uint32_t max_tab = 0;
     bool cplx = false;
 };
 // Paired-row layout of the mixed gather form: thread t owns the row pairs
