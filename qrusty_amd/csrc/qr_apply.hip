@@ -84,6 +84,7 @@ namespace qr {
 constexpr int kApplyThreads = 256;
 constexpr int kApplyThreadBits = 8;
 constexpr size_t kApplyMaxLDS = 40 * 1024;  // LDS of one block
+constexpr size_t kApplyFewLDS = 80 * 1024;  // of kFormGatherFew: two blocks per CU
 // of an operator with a group that needs more than a chunk's share of it
 constexpr size_t kApplyLDSLimit = 160 * 1024;
 // dynamic LDS that a launch may ask for without raising the kernel's limit
@@ -738,12 +739,14 @@ __global__ __launch_bounds__(256) void k_reduce_partials(uint32_t ntiles,
 
 template <bool kMixed, bool kNarrow, int kL, int kSplit, bool kWin = false>
 static int launch_tiled(const qr_op *op, DeviceTables *t, int slot, uint32_t nvec, const void *d_x,
-                        void *d_y, double *partials, uint32_t ntiles, hipStream_t s, bool add = false) {
+                        void *d_y, double *partials, uint32_t ntiles, hipStream_t s, bool few = false,
+                        bool add = false) {
     using Shape = ApplyShape<kMixed, kL>;
     const uint64_t N = uint64_t(1) << op->nq;
     const uint64_t tile_rows = N < (uint64_t(1) << Shape::L) ? N : (uint64_t(1) << Shape::L);
     const DeviceTables::Patterns &pt = t->pat[slot];
-    const size_t shmem = apply_lds_bytes(Shape::kTile, pt.max_tab, Shape::merge_bytes(kSplit));
+    size_t shmem = apply_lds_bytes(Shape::kTile, pt.max_tab, Shape::merge_bytes(kSplit));
+    if (few && shmem < kApplyFewLDS) shmem = kApplyFewLDS;
     if (shmem > kApplyLDSLimit) return fail(QR_ERR_SIZE, "apply: LDS stage too large");
     const uint32_t tpx = (ntiles % 8 == 0) ? ntiles / 8 : 0;
     const bool full = tile_rows == (uint64_t(1) << Shape::L);
@@ -790,23 +793,47 @@ static int launch_staged(const qr_op *op, DeviceTables *t, int slot, uint32_t nv
 
 // Which form applies the operator (of the state's size, not of the number of
 // states, so that every call finds the same tables).  F groups reach outside
-// the tile, on D partner tiles.
+// the tile, on D partner tiles, P of them past an L2 (as in choose_windows).
 constexpr int kFormGather = 0;       // F gathers from memory
 constexpr int kFormStaged = 1;       // D partner tiles through LDS
 constexpr int kFormStagedDense = 2;  // the same with F >= 8 D
+constexpr int kFormGatherFew = 3;    // gathers, two blocks per CU
+constexpr int kFormStagedFew = 4;    // staged, two thread groups per block
 // Measured (us, one state, gather / partner-staged):
 //   FP64: reference's molecules (F/D 9..), 16 / 20 / 22 qubits 134 / 113,
 //     1360 / 928, 7750 / 5050; k-local 24 qubits, 3000 terms (F/D 3.6) 7784 /
 //     7436, 300 terms, two states (1.4) 4140 / 3340, 20 qubits 459 / 400;
-//     random 20 qubits, 2000 terms (2.3) 1123 / 1104, 300 terms (1.1) 185 /
-//     203; below 2^20 rows, where x stays in L2,
-//     gathers win up to F/D 8: 18 qubits, 100 terms 50 / 60, k-local 16
-//     qubits 28 / 33.  Operators with window passes keep only partners that
-//     the L2 holds: 24-qubit ring 300 / 321.
+//     random 20 qubits, 2000 terms (2.3) 1123 / 1104; below 2^20 rows, where x
+//     stays in L2, gathers win up to F/D 8: 18 qubits, 100 terms 50 / 60,
+//     k-local 16 qubits 28 / 33.  Operators with window passes keep only
+//     partners that the L2 holds: 24-qubit ring 300 / 321.
 //   complex64 (2^11-row tiles): molecule 20 qubits 804 / 883, random 20 qubits
 //     762 / 840, k-local 24 qubits, 3000 terms 4940 / 5160, ring 24 qubits 183
 //     / 199; a state past the 256 MB MALL: k-local 28 qubits 236 / 229 ms.
 //   small complex64 tiles: gathers in all cases, within 5% at the worst.
+// Where most partners lie past L2 (random operators), and hardly any group
+// shares its partner, each group is a pass over x, and what counts is that the
+// blocks find each other's partners in L2: masks ascend, so those of one step
+// lie in a region as large as the tiles that the XCD works on, and neighbouring
+// masks go to the same region.  Four blocks of 256 threads per CU make that 2 MB
+// of the 4 MB L2, and once the blocks have drifted apart by a region every
+// partner comes from the MALL or HBM; two make it 1 MB, which held in all cases.
+// FP64, four states or one, gathers from four blocks per CU / staged / this, us:
+// 24 qubits, 1000, 1500, 3000 terms 34400 / 34200 / 17100, 49300 / 48800 / 23200,
+// 102800 / 96200 / 41300; 23 qubits, 300, 1000 4640 / 4650 / 3350, 14600 / 14900 /
+// 6950, four states 68200 / 68900 / 27800; 22 qubits, 300 1790 / 1840 / 1170, four
+// states 8890 / 9310 / 4710; 21 qubits (two blocks of 512 threads, as 20), 300
+// 447 / 442 / 406, four states 3320 / 3260 / 1790; 25 qubits, 1000 59300 / 70500 /
+// 46700.  With few partners the tile itself, which gathers load for groups
+// inside it, counts: staged wins, 20 qubits, 8, 30 terms 24 / 17, 52 / 35; 21
+// qubits, 100 terms 222 / 212 (but 20 qubits and 100 terms, two blocks, 71 / 82); one
+// term, 19 qubits, four states 16 / 12.  Complex64 gains from the staged form,
+// from 2^23 rows on with two thread groups per block (gathers / staged, one
+// thread group / two): 22 qubits, 300 and 1000 terms 630 / 588 / 730, 2200 / 1800
+// / 2250, four states 3750 / 2260 / 2780, 12100 / 6840 / 8750; 23 qubits, 300 terms
+// 1970 / 1890 / 1475; 24 qubits, 300, 1000, 3000 terms 4680 / 4710 / 3220, 15300 /
+// 8570 / 10200, 44100 / 23500 / 27300; 25 qubits, 1000 34500 / 34500 / 23100; but
+// 21 qubits, 300 terms 236 / 287 (x in L2).
 // The environment variable QR_APPLY_FORM (1 gather, 2 staged) overrides the
 // choice, for tests and measurement.
 static int apply_form(const qr_op *op, int kind, int L, const PatternShape &win_shape) {
@@ -815,12 +842,16 @@ static int apply_form(const qr_op *op, int kind, int L, const PatternShape &win_
     int form = op->form[kind].load(std::memory_order_relaxed) - 1;
     if (form < 0) {
         // gx ascends, so groups with equal bits above the tile are adjacent
-        uint64_t far = 0, distinct = 0, prev = 0;
+        uint64_t far = 0, distinct = 0, past = 0, prev = 0;
+        const int near = kind == 0 ? 17 : 18;
         for (uint64_t g = 0; g < op->G; ++g) {
             const uint64_t hi = op->gx[g] >> L;
             if (!hi) continue;
             ++far;
-            if (distinct == 0 || hi != prev) ++distinct;
+            if (distinct == 0 || hi != prev) {
+                ++distinct;
+                past += (op->gx[g] >> near) != 0;
+            }
             prev = hi;
         }
         std::vector<ApplyWindow> wins;
@@ -828,15 +859,24 @@ static int apply_form(const qr_op *op, int kind, int L, const PatternShape &win_
         // (then the partners left are mostly in L2)
         const bool windows = win_shape.L && choose_windows(op, win_shape.L, wins, pass);
         const bool dense = far >= 8 * distinct;
+        const bool scattered = 4 * past >= 3 * distinct, lone = scattered && 4 * far < 5 * distinct;
         const int state_log2 = int(op->nq) + (kind == 0 ? 4 : 3);
-        bool staged = far > 0 && kind != 2 && !windows;
-        if (kind == 0)
-            staged = staged && (dense || state_log2 >= 26 || (state_log2 >= 24 && 2 * far >= 3 * distinct));
-        else staged = staged && state_log2 >= 28 && 2 * far >= 3 * distinct;
-        form = !staged ? kFormGather : dense ? kFormStagedDense : kFormStaged;
+        bool staged = far > 0 && kind != 2 && !windows, few = false;
+        if (kind == 0) {
+            few = staged && lone && distinct >= 64 && state_log2 >= 24;
+            staged = staged && !few &&
+                     (dense || state_log2 >= 26 || (state_log2 >= 24 && (scattered || 2 * far >= 3 * distinct)) ||
+                      (far == op->G && 4 * far < 5 * distinct && distinct <= 16));
+        } else {
+            staged = staged && ((state_log2 >= 28 && 2 * far >= 3 * distinct) ||
+                                (state_log2 >= 25 && scattered && distinct >= 64));
+            few = staged && lone && distinct >= 64 && state_log2 >= 26;
+        }
+        form = few ? (kind == 0 ? kFormGatherFew : kFormStagedFew)
+                   : !staged ? kFormGather : dense ? kFormStagedDense : kFormStaged;
         op->form[kind].store(form + 1, std::memory_order_relaxed);
     }
-    if (e && atoi(e) == 2) return form == kFormStagedDense ? form : kFormStaged;
+    if (e && atoi(e) == 2) return form == kFormStagedDense || form == kFormStagedFew ? form : kFormStaged;
     return form;
 }
 
@@ -914,8 +954,8 @@ static int apply_cus(int *out) {
 // slot that holds its tables (2 * kind + staged; kind 0: FP64, 1: complex64,
 // 2: small complex64 tiles).
 struct ApplyPlan {
-    int L = 0, slot = 0, form = kFormGather;
-    bool small = false;
+    int L = 0, tiles_log2 = 0, slot = 0, form = kFormGather;
+    bool small = false, staged = false, single = false;  // single: one group
     PatternShape shape = {}, win_shape = {};
     int elem_log2 = 4;
 };
@@ -925,12 +965,14 @@ static ApplyPlan make_plan(const qr_op *op, int kind) {
     using Shape = ApplyShape<kMixed, kL>;
     ApplyPlan p;
     p.L = int(op->nq) < kL ? int(op->nq) : kL;
+    p.tiles_log2 = int(op->nq) - p.L;
+    p.single = op->G == 1;
     p.elem_log2 = kMixed ? 3 : 4;
     if (!kMixed && p.L == kL)
         p.win_shape = {p.L, kApplyThreadBits, Shape::kPatSplit, Shape::kTabChunk,
                        uint32_t(Shape::kTile), false, false, {}};
     p.form = p.L == kL ? apply_form(op, kind, p.L, p.win_shape) : kFormGather;
-    const bool staged = p.form != kFormGather;
+    const bool staged = p.staged = p.form != kFormGather && p.form != kFormGatherFew;
     // the gather form on full complex64 tiles runs the paired-row layout
     const bool pairs = kMixed && !staged && p.L == kL;
     p.shape = {p.L, kApplyThreadBits, staged ? Shape::kPatSplitS : Shape::kPatSplit,
@@ -948,13 +990,17 @@ static ApplyPlan make_plan(const qr_op *op, int kind) {
 // FP64 molecules, 12 qubits 86 / 50 / 35, 16: 272 / 161 / 113, 18 (256 tiles):
 // 613 / 371 / 235, 20 (1024 tiles, staged, F/D 9): 1007 / 928 / 989, 22: 6020
 // / 5050 / 5570; k-local 20 qubits, 3000 terms (staged, F/D 5): 400 / 486 /
-// 716; ring 24 qubits (gather) 320 / 300 / 358.  Complex64, 2^11-row tiles:
-// molecule 20 qubits (512 tiles) 1085 / 804, k-local 24 qubits (8192 tiles)
-// 4940 / 5250; 2^10-row tiles: molecule 18 qubits (256 tiles) 439 / 256 / 183,
-// random 18 qubits, 3 states (768 tiles) 47 / 36 / 41.
+// 716 (one term, 19 qubits, four states 12 / 13 / 23); ring 24 qubits (gather)
+// 320 / 300 / 358, a diagonal, 26 qubits 722 / 854; gathers with two blocks per
+// CU, random, 300 terms, 21 qubits 491 / 406, 22 qubits 1170 / 1670.  Complex64,
+// 2^11-row tiles: molecule 20 qubits (512 tiles) 1085 / 804, k-local 24 qubits
+// (8192 tiles) 4940 / 5250; 2^10-row tiles: molecule 18 qubits (256 tiles) 439 /
+// 256 / 183, random 18 qubits, 3 states (768 tiles) 47 / 36 / 41.
 static int apply_split(const ApplyPlan &p, bool mixed, uint64_t blocks, int cus) {
+    if (!mixed && p.form == kFormStaged) return 1;
+    if (p.form == kFormGatherFew) return p.tiles_log2 <= 11 ? 2 : 1;
     if ((!mixed || p.small) && blocks <= uint64_t(2) * cus) return 4;
-    if (!mixed) return p.form == kFormStaged ? 1 : 2;
+    if (!mixed || p.form == kFormStagedFew) return p.single ? 1 : 2;
     return p.small || blocks < uint64_t(4) * cus ? 2 : 1;
 }
 
@@ -1043,20 +1089,20 @@ int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint
             double *e = partials ? partials + 2 * uint64_t(ntiles) * v : nullptr;
             // (window passes may have taken every group: then the first of
             // them writes y)
-            const bool rows_pass = t->pat[plan.slot].nchunk > 0;
+            const bool rows_pass = t->pat[plan.slot].nchunk > 0, few = plan.form == kFormGatherFew;
             int r = QR_OK;
-            if (rows_pass && plan.form != kFormGather)
+            if (rows_pass && plan.staged)
                 r = narrow ? launch_staged<kMixed, true, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s)
                            : launch_staged<kMixed, false, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s);
             else if (rows_pass)
-                r = narrow ? launch_tiled<kMixed, true, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s)
-                           : launch_tiled<kMixed, false, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s);
+                r = narrow ? launch_tiled<kMixed, true, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s, few)
+                           : launch_tiled<kMixed, false, kL, kSplit>(op, t, plan.slot, nv, x, y, e, ntiles, s, few);
             if constexpr (!kMixed)
                 for (uint32_t k = 0; !r && k < nwin; ++k) {
                     const int sl = plan.slot + kApplySlots * int(k + 1);
                     const bool add = rows_pass || k > 0;
-                    r = narrow ? launch_tiled<false, true, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, add)
-                               : launch_tiled<false, false, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, add);
+                    r = narrow ? launch_tiled<false, true, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, false, add)
+                               : launch_tiled<false, false, kL, 1, true>(op, t, sl, nv, x, y, e, ntiles, s, false, add);
                 }
             if (r) return r;
         }

@@ -180,3 +180,20 @@ def test_complex64_sum_is_rounded_once():
     ref = sum(coeffs) * v
     err = (torch.view_as_real(y).double() - torch.tensor([ref.real, ref.imag], device="cuda")).abs().amax().item()
     assert err <= 1.01 * 2.0**-24 * abs(ref)
+
+
+@pytest.mark.parametrize("n,terms,nvec,prec", [(20, 70, 2, "fp64"), (22, 70, 1, "fp64"), (20, 40, 1, "fp64"),
+                                               (16, 3, 4, "fp64"), (14, 15, 1, "fp64"), (22, 70, 2, "mixed"),
+                                               (23, 70, 1, "mixed")])
+def test_scattered_partners(n, terms, nvec, prec):
+    """Random operators, whose groups have partners of their own far from the
+    tile: on both sides of the rule's numbers of partners and rows."""
+    from qrusty_amd import workloads
+    rng = np.random.default_rng(n + terms)
+    labels = ["X" + "".join(rng.choice(list("IXYZ"), size=n - 1)) for _ in range(terms)]
+    coeffs = list(rng.standard_normal(terms) + 1j * rng.standard_normal(terms))
+    p, op = orc.Params(labels, coeffs), _op(labels, coeffs)
+    x = workloads.random_states(p.N, nvec, 900 + n)
+    rows = np.unique(np.r_[0, p.N - 1, rng.choice(p.N, size=4096)]).astype(np.uint64)
+    print(f"[gpu] apply scattered n={n} terms={terms} nvec={nvec} {prec}", flush=True)
+    _check(p, op, x, rows, prec)

@@ -166,3 +166,30 @@ stub.stub_fail_malloc_after(-1)
 L.check(L.lib.qr_batch_run(batch, *first, None, None))
 assert stub.stub_graphs_made() == 2
 """)
+
+
+@pytest.mark.parametrize("n,prec,groups,form,few", [(24, 0, 100, "tiled", True), (20, 0, 90, "tiled", True),
+                                                    (20, 0, 40, "staged", False), (19, 0, 100, "tiled", False),
+                                                    (16, 0, 1, "staged", False), (22, 1, 100, "staged", False),
+                                                    (24, 1, 100, "staged", False), (21, 1, 100, "tiled", False),
+                                                    (24, 0, "ring", "tiled", False), (24, 0, "shared", "staged", False)])
+def test_apply_form(run, n, prec, groups, form, few):
+    """Groups on partners of their own past L2: gathers by two blocks per CU, or
+    staged where they are few or the state is complex64 (past its caches); others
+    as before."""
+    run(f"""
+import random
+rng, n, groups = random.Random(5), {n}, {groups!r}
+if groups == "ring":
+    labels = [term(n, {{q: p, (q + 1) % n: p}}) for q in range(n) for p in "XYZ"]
+elif groups == "shared":
+    labels = [term(n, {{q: "X", p: "X"}}) for q in range(10, n) for p in range(10)]
+else:
+    labels = ["X" + "".join(rng.choice("IXYZ") for _ in range(n - 1)) for _ in range(groups)]
+op = op_of(labels)
+L.check(L.lib.qr_pauli_apply(op, {prec}, 1, 64 * GB, 128 * GB, None, None))
+names = launched("k_apply_")
+assert all("k_apply_{form}" in k[0] for k in names), names
+lds = max(stub.stub_shmem(i) for i in range(stub.stub_launches()))
+assert (lds >= 80 << 10) == {few}, lds
+""")
