@@ -59,16 +59,21 @@ __device__ __forceinline__ double2 precond_entry(double2 d, double2 dx, double2 
     return cdiv(dx, v);
 }
 
-// Rows of 8 to kDiagScan entries in the mean: 2^lpr_log2 lanes read a row's
-// columns, four each at a time, and the lane that meets the diagonal writes
-// the row's result (the first lane, if none does).
+// Rows of 8 to kDiagScan entries in the mean: a wave takes 64 rows, one per lane
+// for their bounds, their diagonal's value and the result, and 2^lpr_log2 lanes
+// read a row's columns, four each, kDiagDepth rows in flight per lane group; the
+// first entry of the row that has the diagonal column is its own.  Rows longer
+// than their lanes' four entries are searched, each by its lane.
 // What bounds it: memory.  A binary search per row, the other way, leaves its
 // lines in the caches between dependent probes, where they thrash, but reads
-// few lines of a long row.  Measured (precond, us, search / scan): rings of 20,
-// 23, 24 qubits (21 to 25 entries) 109 / 66, 815 / 582, 1671 / 1190; random
-// operators of 4 entries, 24 qubits 214 / 400, 60, 22 qubits 442 / 474, 120, 21
-// qubits 269 / 470.
+// few lines of a long row.  Measured (precond, us, search / this): rings of 20,
+// 23, 24 qubits (21 to 25 entries) 107 / 60, 794 / 562, 1651 / 1120; Poisson
+// lengths of 9, 22, 35, 20 qubits 31 / 20, 85 / 35, 98 / 65; geometric ones of 30
+// 75 / 55; one row of 2^19 entries, the others 12 in the mean 52 / 23; but 15 rows
+// of 16 of one entry, the others 625, 20 / 44.  (A lane group for every row, whatever
+// its length: rings 68, 569, 1186; the row of 2^19 entries 12400.)
 constexpr double kDiagScan = 48.0;
+constexpr int kDiagDepth = 4;
 template <bool kPrecond>
 __global__ __launch_bounds__(256) void k_diag_scan(uint64_t n, uint32_t lpr_log2, uint64_t nnz,
                                                    const uint64_t *__restrict__ indptr,
@@ -76,43 +81,65 @@ __global__ __launch_bounds__(256) void k_diag_scan(uint64_t n, uint32_t lpr_log2
                                                    const double2 *__restrict__ data,
                                                    const double2 *__restrict__ dx, double2 e, double tol,
                                                    double2 *__restrict__ out) {
-    const uint32_t lpr = 1u << lpr_log2, lane = threadIdx.x & (lpr - 1u);
-    const uint64_t r = uint64_t(blockIdx.x) * (256u >> lpr_log2) + (threadIdx.x >> lpr_log2);
-    if (r >= n) return;
-    const uint64_t hi = indptr[r + 1] < nnz ? indptr[r + 1] : nnz;
-    uint64_t at = ~uint64_t(0);
-    for (uint64_t k = indptr[r] + lane; k < hi; k += 4 * lpr) {
-        uint64_t c[4];
+    const uint32_t wl = threadIdx.x & 63u, lpr = 1u << lpr_log2, lane = wl & (lpr - 1u), group = wl >> lpr_log2;
+    const uint32_t gw = 64u >> lpr_log2, shift = wl & ~(lpr - 1u);
+    const uint64_t r0 = (uint64_t(blockIdx.x) * 4 + threadIdx.x / 64u) * 64;
+    if (r0 >= n) return;
+    const uint64_t r = r0 + wl, rr = r < n ? r : n - 1;
+    const uint64_t lo = indptr[rr], hi = indptr[rr + 1] < nnz ? indptr[rr + 1] : nnz;
+    // the wave's entries from `base` on, counted in 32 bits
+    const uint64_t first = uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(lo >> 32)))) << 32 |
+                           uint32_t(__builtin_amdgcn_readfirstlane(int(lo)));
+    const uint64_t base = first < nnz ? first : nnz - 1;
+    const uint32_t most = nnz - 1 - base < (1u << 30) ? uint32_t(nnz - 1 - base) : 1u << 30;
+    const bool some = lo < hi, fits = !some || (hi - lo <= 4 * lpr && lo - base < (1u << 29));
+    const uint32_t rel = some && fits ? uint32_t(lo - base) : 0u, len = some && fits ? uint32_t(hi - lo) : 0u;
+    uint32_t at = ~0u;
+    for (uint32_t s = 0; s < lpr; s += kDiagDepth) {
+        uint64_t c[kDiagDepth][4];
+        uint32_t l[kDiagDepth];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint64_t i = k + uint32_t(u) * lpr;
-            c[u] = indices[i < nnz ? i : nnz - 1];
+        for (int d = 0; d < kDiagDepth; ++d) {
+            const int row = int((s + uint32_t(d)) * gw + group);
+            const uint32_t o = uint32_t(__shfl(int(rel), row)) + lane;
+            l[d] = uint32_t(__shfl(int(len), row));
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t i = o + u * lpr;
+                c[d][u] = indices[base + (i < most ? i : most)];
+            }
         }
 #pragma unroll
-        for (int u = 3; u >= 0; --u) {
-            const uint64_t i = k + uint32_t(u) * lpr;
-            if (c[u] == r && i < hi && i < at) at = i;
+        for (int d = 0; d < kDiagDepth; ++d) {
+            const uint64_t row = r0 + (s + uint32_t(d)) * gw + group;
+            uint32_t pos = ~0u;
+#pragma unroll
+            for (int u = 3; u >= 0; --u) {
+                const uint32_t i = lane + uint32_t(u) * lpr;
+                const uint64_t met = __ballot(i < l[d] && c[d][u] == row) >> shift;
+                const uint32_t mine = uint32_t(met) & (lpr == 32 ? ~0u : (1u << lpr) - 1u);
+                if (mine) pos = uint32_t(u) * lpr + uint32_t(__builtin_ctz(mine));
+            }
+            // to the lane of the row
+            const uint32_t got = uint32_t(__shfl(int(pos), int((wl & (gw - 1u)) << lpr_log2)));
+            if (wl >> (6u - lpr_log2) == s + uint32_t(d)) at = got;
         }
     }
-    const uint64_t met = __ballot(at != ~uint64_t(0)) >> ((threadIdx.x & 63u) & ~(lpr - 1u));
-    const uint64_t mine = met & (lpr == 64 ? ~uint64_t(0) : (uint64_t(1) << lpr) - 1);
-    // (a column that comes more than once in the row: its first entry)
-    uint64_t first = at;
-    if (mine & (mine - 1))
-        for (uint32_t o = 1; o < lpr; o <<= 1) {
-            const uint64_t other = __shfl_xor(first, int(o));
-            first = other < first ? other : first;
-        }
-    if (mine ? at == ~uint64_t(0) || at != first : lane != 0) return;
-    const double2 d = mine ? data[at] : make_double2(0.0, 0.0);
+    if (r >= n) return;
+    double2 d = make_double2(0.0, 0.0);
+    if (!fits) d = diag_entry(r, nnz, indptr, indices, data);
+    else if (at != ~0u) d = data[base + rel + at];
     out[r] = kPrecond ? precond_entry(d, dx[r], e, tol) : d;
 }
 
-// Lanes per row of k_diag_scan (0: not by it): a quarter of the mean length
+// Lanes per row of k_diag_scan (0: not by it), 4 to 32: a quarter of the mean
+// length, or, where the rows cannot be equal, of what most of them have
 static uint32_t diag_lanes_log2(uint64_t nrows, uint64_t nnz) {
-    if (double(nnz) < 8.0 * double(nrows) || double(nnz) > kDiagScan * double(nrows)) return 0;
+    const double mean = double(nnz) / double(nrows);
+    if (mean < 8.0 || mean > kDiagScan) return 0;
+    const double need = nnz % nrows ? mean + 2.0 * sqrt(mean) : mean;
     uint32_t l = 2;
-    while (l < 6 && (nrows << (l + 2)) < nnz) ++l;
+    while (l < 5 && double(4u << l) < need) ++l;
     return l;
 }
 
@@ -158,7 +185,7 @@ int launch_csr_diagonal(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint
     const uint64_t n = nrows < ncols ? nrows : ncols;
     if (n == 0) return QR_OK;
     if (const uint32_t l = diag_lanes_log2(nrows, nnz)) {
-        const uint64_t blocks = (n + (256u >> l) - 1) / (256u >> l);
+        const uint64_t blocks = (n + 255) / 256;
         if (blocks <= 0x7FFFFFFFull) {
             hipLaunchKernelGGL(k_diag_scan<false>, dim3(unsigned(blocks)), dim3(256), 0, s, n, l, nnz, indptr,
                                indices, reinterpret_cast<const double2 *>(data), nullptr, double2{}, 0.0,
@@ -191,7 +218,7 @@ int launch_precond(uint64_t n, const double *diag, uint64_t nnz, const uint64_t 
                    double tol, double *out, hipStream_t s) {
     if (n == 0) return QR_OK;
     const uint32_t l = diag ? 0 : diag_lanes_log2(n, nnz);
-    const uint64_t blocks = l ? (n + (256u >> l) - 1) / (256u >> l) : 0;
+    const uint64_t blocks = (n + 255) / 256;
     if (l && blocks <= 0x7FFFFFFFull) {
         hipLaunchKernelGGL(k_diag_scan<true>, dim3(unsigned(blocks)), dim3(256), 0, s, n, l, nnz, indptr, indices,
                            reinterpret_cast<const double2 *>(data), reinterpret_cast<const double2 *>(dx),

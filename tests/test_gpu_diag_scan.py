@@ -71,3 +71,33 @@ def test_scan_of_repeated_columns(rows, mean):
     m = qa.SpMat.new_unchecked((rows, rows), data, indices, indptr)
     print(f"[gpu] diagonal scan, repeated columns rows={rows} mean={mean}", flush=True)
     assert np.array_equal(np.asarray(m.diagonal()), want)
+
+
+@pytest.mark.parametrize("rows,lens", [(300, [8, 0, 16, 17, 1, 40]), (65, [31, 32, 33, 0]), (64, [48, 100, 64, 65, 3]),
+                                       (1, [9]), (257, [2, 30]), (4096, [12] * 63 + [2000])])
+def test_scan_of_uneven_rows(rows, lens):
+    """Rows on both sides of what their lanes read at a time, in one wave; some
+    that start past the matrix's entries, and end before they start."""
+    import qrusty_amd as qa
+    from oracle import oracle as orc
+    rng = np.random.default_rng(rows + len(lens))
+    lens, cols = np.resize(lens, rows), max(rows, 2000)
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    ind = []
+    for r, n in enumerate(lens):
+        c = rng.choice(cols, size=int(n), replace=False)
+        if n and r % 3 and r not in c:
+            c[rng.integers(n)] = r
+        ind.append(np.sort(c))
+    indices = np.concatenate(ind).astype(np.uint64)
+    data = rng.standard_normal(len(indices)) + 1j * rng.standard_normal(len(indices))
+    print(f"[gpu] diagonal scan, uneven rows={rows} lens={lens[:6]}", flush=True)
+    m = qa.SpMat.new_unchecked((rows, cols), data, indices, indptr)
+    assert np.array_equal(np.asarray(m.diagonal()), orc.csr_diagonal((rows, cols), indptr, indices, data))
+    if rows > 8:
+        bad = indptr.copy()
+        bad[3], bad[5], bad[-2] = bad[-1] + np.uint64(9), np.uint64(0), np.uint64(1) << np.uint64(40)
+        m = qa.SpMat.new_unchecked((rows, cols), data, indices, bad)
+        got, want = np.asarray(m.diagonal()), orc.csr_diagonal((rows, cols), indptr, indices, data)
+        ok = [r for r in range(6, rows - 3)]
+        assert np.array_equal(got[ok], want[ok])
