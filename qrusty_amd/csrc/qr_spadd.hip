@@ -22,6 +22,8 @@
 
 #include <hipcub/device/device_scan.hpp>
 
+#include <cmath>
+
 namespace qr {
 
 __device__ __forceinline__ double2 cmul2(double2 a, double2 v) {
@@ -488,21 +490,25 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
     }
 }
 
-// Whether k_spadd_few takes a sum, its lanes per row (the longer matrix's mean
-// length rounded up to a power of two from 4 to 64), its rows per wave (64 or
-// what leaves the launch 16 waves per CU, or 256 if rows are long: 16-qubit
-// molecule, fill pass, 16 / 64 / 256 waves per CU 612 / 563 / 498 us; 18-qubit
-// ring 58 / 49 / 87), and `in` with the longer matrix first.
+// Whether k_spadd_few takes a sum, its lanes per row (a power of two from 4 to 64
+// that holds the longer matrix's mean length, or, where the rows cannot be equal,
+// what most of them have: mean + 2 sqrt(mean)), its rows per wave (64 or what
+// leaves the launch 16 waves per CU, or 256 if rows come in pieces: 16-qubit
+// molecule, fill pass, 16 / 64 / 256 waves per CU 612 / 563 / 498 us; 18-qubit ring
+// 58 / 49 / 87; 33 entries, 16 qubits 97 / - / 213), and `in` with the longer matrix
+// first.
 // Rows of up to 64 entries in the mean: sums with as many short entries as rows
 // (a diagonal, one Pauli string), where one each is what to expect.  Staged
 // tiles / this, count + fill, us: 20 qubits, 4 to 64 random terms 570-900 /
-// 500-600; rows of 10.6 to 12.7 entries in the mean (isotropic rings without
-// their zeros, 20, 23, 24 qubits) 405 / 340, 3500 / 2860, 6340 / 6110; Poisson
-// lengths of 8, 20, 40 330 / 320, 595 / 525, 1050 / 837; one row in 100 of 600
-// entries 4360 / 656; but half of the rows 3 and half 40 long 930 / 1020.  Other
-// sums stay with the tiles: rows with two short entries (Z + X) run one at a
-// time here, 20-qubit ring 657 / 1290, 0 to 2 each 600 / 900 (and as many as
-// rows, alternately 0 and 2, 23 qubits 4780 / 6800).
+// 500-600; isotropic rings without their zeros, 20, 22, 23, 24 qubits (10.6 to 12.7
+// entries in the mean, 32 lanes but for 22) 364 / 323, 1433 / 1134, 3227 / 2268, 6138
+// / 4711 (16 lanes: 3373, 7303); Poisson lengths of 7, 14, 22, 35, 20 qubits 265 /
+// 250, 417 / 399, 598 / 520, 864 / 798 (the mean rounded up: 363, 517, 521, 728); one
+// row in 100 of 600 entries 4360 / 656; but 24 or 100 entries in every other row
+// 432 / 595, 1120 / 1700 (a whole number in the mean).  Other sums stay with
+// the tiles: rows with two short entries (Z + X) run one at a time here, 20-qubit
+// ring 657 / 1290, 0 to 2 each 600 / 900 (and as many as rows, alternately 0 and 2,
+// 23 qubits 4780 / 6800).
 // Longer rows, which leave the tiles few rows or overflow them: from 128 entries
 // per row with one short one, 192 with two.  One / two short entries: 90
 // entries 1012 / 1055, 972 / 1280; 128: 784 / 666, 772 / 763; 220: 811 / 535,
@@ -514,14 +520,16 @@ struct SpFew {
 };
 static bool spadd_few(uint64_t nrows, SpAddIn &in, SpFew &f) {
     if (in.nnz1 < in.nnz2) in = SpAddIn{in.b, in.a, in.nnz2, in.nnz1, in.ip2, in.ix2, in.ip1, in.ix1, in.d2, in.d1};
+    const double mean = double(in.nnz1) / double(nrows ? nrows : 1);
+    const double need = nrows && in.nnz1 % nrows ? mean + 2.0 * std::sqrt(mean) : mean;
     f.lpr_log2 = 2;
-    while (f.lpr_log2 < 6 && (nrows << f.lpr_log2) < in.nnz1) ++f.lpr_log2;
-    f.pieces = (nrows << f.lpr_log2) < in.nnz1;
+    while (f.lpr_log2 < 6 && double(1u << f.lpr_log2) < need) ++f.lpr_log2;
+    f.pieces = mean > 64;
     if (f.pieces ? in.nnz2 == 0 || in.nnz2 > 2 * nrows || in.nnz1 / 64 < nrows + in.nnz2
-                 : in.nnz2 != nrows)
+                 : in.nnz2 != nrows || need > 64)
         return false;
     f.rpw_log2 = 6;
-    const uint64_t waves = f.lpr_log2 == 6 ? 65536 : 4096;
+    const uint64_t waves = f.pieces ? 65536 : 4096;
     while (f.rpw_log2 > 6 - f.lpr_log2 && (nrows >> f.rpw_log2) < waves) --f.rpw_log2;
     f.blocks = (nrows + (uint64_t(4) << f.rpw_log2) - 1) / (uint64_t(4) << f.rpw_log2);
     return true;

@@ -193,3 +193,21 @@ assert all("k_apply_{form}" in k[0] for k in names), names
 lds = max(stub.stub_shmem(i) for i in range(stub.stub_launches()))
 assert (lds >= 80 << 10) == {few}, lds
 """)
+
+
+@pytest.mark.parametrize("n,longer,lanes,rows", [(16, 33 << 16, 6, 16), (16, (7 << 16) + 1, 4, 16), (20, 25 << 20, 5, 64),
+                                                 (20, (22 << 20) + 1, 5, 64), (20, (60 << 20) + 1, 0, 0), (18, 9 << 18, 4, 64)])
+def test_lanes_of_sums(run, n, longer, lanes, rows):
+    """Lanes per row of a sum with a diagonal (0: staged tiles), enough for most
+    rows where these cannot be equal, and rows per wave."""
+    run(f"""
+n, longer = 1 << {n}, {longer}
+stub.stub_watch(b"k_spadd_few", 1)
+one = (ctypes.c_double * 2)(1.0, 0.0)
+L.check(L.lib.qr_csr_add_fill(n, one, longer, 64 * GB, 65 * GB, 66 * GB, one, n, 67 * GB, 68 * GB, 69 * GB, 70 * GB,
+                              71 * GB, 72 * GB, None))
+few = launched("k_spadd_few")
+assert bool(few) == bool({lanes})
+if few:
+    assert few[0][1] == {lanes} and few[0][2] * 4 * {rows} == n, few
+""")
