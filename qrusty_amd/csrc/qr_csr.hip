@@ -734,10 +734,12 @@ __global__ __launch_bounds__(256) void k_csr_matvec(uint64_t nrows, uint64_t nco
 // / 2150, 110, 128, 21 qubits 1309 / 1170, 1442 / 1346, weights 1 to 4, 82 and 110
 // entries 1681 / 1525, 2205 / 2115; where the MALL holds the matrix 28 / 33 (100
 // entries, 16 qubits).
-// Where the MALL holds the matrix the streams gain nothing, and only equal rows
-// from 11 entries on run here: 19 qubits, 12, 20 entries 46 / 46, 58 / 58, 16
-// qubits, 17 entries 18 / 16.5; but 8 and 10 entries, 20 and 19 qubits 58 / 65,
-// 41 / 44, Poisson lengths of 12, 50, 19 and 17 qubits 42 / 49, 40 / 44.
+// Where the MALL holds the matrix the streams gain little, and only equal rows
+// of 11 to 63 entries run here: 19 qubits, 12, 20 entries 46 / 46, 58 / 58; random
+// operators, 17 qubits, 16, 30, 44, 56 entries 13.7 / 11.3, 21.3 / 18.7, 28.8 / 27.1,
+// 34.7 / 36, 16 qubits, 44, 56 entries 15.8 / 13.2, 18.7 / 17.6; but 64, 16 and 17
+// qubits 17.5 / 20, 36.4 / 40.8, 8 and 10 entries, 20 and 19 qubits 58 / 65, 41 /
+// 44, Poisson lengths of 12, 50, 19 and 17 qubits 42 / 49, 40 / 44.
 // U: loads per lane; rows of up to 8 U entries.
 constexpr uint64_t kMallBytes = uint64_t(1) << 28;
 constexpr uint64_t kShortLongNnz = uint64_t(1) << 25;
@@ -943,7 +945,7 @@ int launch_csr_matvec(uint64_t nrows, uint64_t ncols, uint64_t nnz, const uint64
     auto y = reinterpret_cast<double2 *>(d_y);
     const dim3 grid(static_cast<unsigned>(nblocks)), block(256);
     const bool equal = nnz % nrows == 0, in_mall = nnz * 24 <= kMallBytes;
-    if (ncols && avg >= 8 && (in_mall ? equal && avg >= 11 && avg <= 64
+    if (ncols && avg >= 8 && (in_mall ? equal && avg >= 11 && avg < 64
                                       : avg <= 64 || (avg <= 128 && equal && nnz >= kShortLongNnz))) {
         // a wave's eight rows are to fit, with an eighth to spare where they
         // cannot be equal
