@@ -28,12 +28,15 @@
 //    l, so a thread finds it with a few shifts and XORs of two words of the
 //    group's descriptor (ApplyPart) whatever the number of terms.  Summing the
 //    signed coefficients per thread instead took 5-6 vector instructions per
-//    pattern: 103 per group and 8 rows on the 28-qubit k-local operator (now
-//    70), 90 per group and 4 rows on a 20-qubit molecule (now 30); molecules
-//    of 12 / 16 / 20 / 22 qubits, FP64, one state: 290 / 556 / 1633 / 10100 ->
-//    35 / 114 / 912 / 5120 us, 20 qubits and 2000 random terms 1590 -> 1100.
-//    What bounds them now is the chain of descriptor loads, lookups and
-//    gathers of each group (vector ALU about half busy).
+//    pattern; molecules of 12 / 16 / 20 / 22 qubits, FP64, one state: 290 / 556
+//    / 1633 / 10100 -> 35 / 114 / 890 / 5120 us, 20 qubits and 2000 random terms
+//    1590 -> 1100.  What bounds them now (counters): the 20-qubit molecule the
+//    LDS, four fifths of its 128 B per cycle (6.7 reads per group and wave), and
+//    the vector ALU, 64% busy (34 instructions per group and 4 rows); the
+//    28-qubit k-local operator, complex64, the vector ALU, 78% (90 per group
+//    and 8 rows, with the tables); the 24-qubit complex64 ring the partners past
+//    L2, 7.8 TB/s; small states the chain of descriptor loads, lookups and
+//    gathers of each group.
 //  * Thread `tid` owns rows l = tid + 256*k.  The gather form on full
 //    complex64 tiles owns row pairs instead, l = 2*tid + (k & 1) + 512*(k >>
 //    1), so that one 16-byte load gathers both partners of a pair and one

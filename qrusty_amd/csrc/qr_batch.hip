@@ -73,7 +73,8 @@ __global__ __launch_bounds__(kStageThreads, !kMatvec && kChunks <= 1 ? 8 : 1) vo
     }
 }
 
-// Most groups of an operator whose y the fused form gives without CSR buffers.
+// Most groups of an operator whose y the fused form gives without CSR buffers (a
+// limit of the interface: the apply has none).
 constexpr uint64_t kBatchMostG = 6144;
 
 // Entries up to which an operator is small: it runs in k_batch, which takes

@@ -212,8 +212,8 @@ struct WordOp {
 };
 
 // LDS of a block: two stages, whose place the heavy groups' terms take first
-// (in turns of that size), and those groups' values: as many of them as leave
-// two blocks to a CU; the rest run term by term.
+// (in turns of that size), and those groups' values, as many as leave two blocks
+// to a CU (all of them: the launch takes fewer batches per tile until they fit).
 struct WordLds {
     uint32_t nheavy, hv_at, total;
     __host__ __device__ WordLds(uint32_t g, uint32_t rs_log2, uint32_t tile_log2, uint32_t hcnt, const uint32_t *ptr) {
@@ -567,8 +567,9 @@ int launch_csr_build(const qr_op *op, DeviceTables *t, uint64_t row_begin, uint6
             const uint32_t g = lf.s1 - lf.s0, nch = (g + 1023) >> 10;
             uint32_t dbuf = 0;
             const uint32_t nh = heavy_fit(lf.hcnt, jw);
-            // (sub-operators keep one stage: the second would cost them
-            // tiles per heavy fold, H10 14.12 -> 14.38 ms)
+            // (sub-operators keep one stage: the second would cost them tiles
+            // per heavy fold; 20-qubit molecule, when it was built here, 14.12
+            // -> 14.38 ms)
             const size_t sb = stage_bytes(g, jw, &dbuf);
             const uint32_t fl = fold_tiles_log2(true, sb, heavy_bytes(nh, jw), nt);
             const size_t shmem = sb + (heavy_bytes(nh, jw) << fl);

@@ -40,8 +40,8 @@ int hip_fail(hipError_t e, const char *what);
 constexpr int kMaxDevices = 16;
 // heavy groups the CSR build folds per row in a pass of their own: molecular
 // Hamiltonians (the reference's H8..H12) have 17-111 groups of 22-301 terms
-// next to groups of at most 6 (as many as the tile's LDS holds are folded
-// that way, heavy_fit in qr_tile.h)
+// next to groups of at most 6 (the sign-word builder's tiles hold all of them;
+// of the shared tile builder, as many as the LDS holds, heavy_fit in qr_tile.h)
 constexpr uint32_t kMaxHeavy = 128;
 // Tail table of an operator with heavy groups: terms 2, 3, ... of every group
 // transposed, slot u * G + g = term 2 + u of group g, for u < ntail <=

@@ -164,8 +164,10 @@ __host__ __device__ inline uint32_t heavy_fit(uint32_t nheavy, uint32_t jw_log2)
 // values within kFoldBudget bytes of LDS (those instances run one block per
 // CU for their registers) and leave at least kFoldMinBlocks blocks of the
 // launch's ntiles tiles, so that small operators still fill the chip.
-// up to 8 tiles: H12 (2^19 rows) 4.66 -> 4.42 ms against up to 4, H10 and
-// H11 unchanged; 16 do not fit the LDS budget there
+// Up to 8 tiles: a 24-qubit molecule (2^19 rows) 4.66 -> 4.42 ms against up to
+// 4, 20 and 22 qubits unchanged; 16 do not fit the LDS budget there.  (The
+// molecules' figures here are from before operators of at most 32 qubits had a
+// builder of their own; wider ones have the same tiles.)
 #ifndef QR_FOLD_MAX_LOG2
 #define QR_FOLD_MAX_LOG2 3
 #endif
@@ -174,7 +176,7 @@ constexpr size_t kFoldBudget = 150 * 1024;
 // block overlaps a batch's copy-out with the next batch's build)
 // double-buffer the stage when it and one tile's heavy values fit the
 // budget; the tiles per block are then chosen with the double stage.
-// Measured on H12 (2^19 rows): 3.93 -> 3.72-3.76 ms.
+// Measured on a 24-qubit molecule (2^19 rows): 3.93 -> 3.72-3.76 ms.
 #ifndef QR_HEAVY_DBUF
 #define QR_HEAVY_DBUF 1
 #endif
@@ -281,8 +283,8 @@ constexpr int kTilePlain = 0, kTileHeavy = 1, kTileSub = 2, kTileSubHeavy = 3;
 // Heavy-group instances that build several tiles per block, folding the heavy
 // groups once for all of them: the two-chunk ones (one block per CU anyway)
 // and the one-chunk sub-operators, which the tile loop takes from 60 to 78
-// VGPRs and one block per CU.  Measured (ms): H10 16.75 -> 16.45 and H11
-// 13.92 -> 13.48 with the one-chunk sub-operators in; the whole one-chunk
+// VGPRs and one block per CU.  Measured (ms, molecules): 20 qubits 16.75 -> 16.45
+// and 22 qubits 13.92 -> 13.48 with the one-chunk sub-operators in; the whole one-chunk
 // operators (the 24-qubit Heisenberg build) stay at one tile per block
 // (2.25 ms against 3.03 with it).
 template <int kChunks, int kMode>
