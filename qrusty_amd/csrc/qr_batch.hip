@@ -557,9 +557,13 @@ int qr_batch_tune(qr_batch *b, uint64_t *const *d_indptr, uint64_t *const *d_ind
             for (uint32_t tpi : tpis) {
                 const qr_tuning tu{tpi, bpc, order, split};
                 Plan plan;
-                if ((rc = make_plan(b, d_indptr, d_indices, d_data, d_x, d_y, tu, plan)) ||
-                    (rc = prepare(b, plan, tu)))
-                    goto done;
+                if ((rc = make_plan(b, d_indptr, d_indices, d_data, d_x, d_y, tu, plan))) goto done;
+                // without small operators the tiles per item reach no kernel, and
+                // the blocks per CU the matvec pass alone
+                if (plan.small[0].empty() && plan.small[1].empty() &&
+                    (tpi != tpis[0] || (!split && bpc != bpcs[0])))
+                    continue;
+                if ((rc = prepare(b, plan, tu))) goto done;
                 // one untimed pass (first touch), then one timed pass
                 for (int rep = 0; rep < 2; ++rep) {
                     if (rep == 1 && hipEventRecord(e0, s) != hipSuccess) { rc = fail(QR_ERR_HIP, "event"); goto done; }

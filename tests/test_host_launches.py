@@ -211,3 +211,18 @@ assert bool(few) == bool({lanes})
 if few:
     assert few[0][1] == {lanes} and few[0][2] * 4 * {rows} == n, few
 """)
+
+
+@pytest.mark.parametrize("qubits,candidates", [((22, 23), 6), ((22, 8), 32)])
+def test_tuning_times_no_candidate_twice(run, qubits, candidates):
+    """Batches without small operators: orders, forms, and the matvec pass's blocks
+    per CU, without the knobs that reach no kernel of the plan."""
+    run(f"""
+ops = [op_of([term(q, {{0: "X"}})]) for q in {qubits}]
+batch = ctypes.c_void_p()
+L.check(L.lib.qr_batch_create((ctypes.c_void_p * 2)(*ops), 2, ctypes.byref(batch)))
+args = [ctypes.cast((ctypes.c_void_p * 2)((64 + 4 * k) * GB, (66 + 4 * k) * GB), ctypes.c_void_p) for k in range(5)]
+L.check(L.lib.qr_batch_tune(batch, *args, None, None))
+large = sum(q > 20 for q in {qubits})
+assert len(launched("k_csr_build")) == {candidates} * 2 * large, len(launched("k_csr_build"))
+""")
