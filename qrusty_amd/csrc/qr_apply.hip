@@ -522,9 +522,10 @@ __device__ __forceinline__ void chunk_tables(const ApplyChunk &ch, uint32_t t, u
 }
 
 // kWin: a window pass (ApplyWindow), whose groups all gather inside the tile;
-// win_add: it adds to y and the partials.  nchunk is at least 1: the wait for
-// the tile's loads is chunk_tables'.
-template <bool kMixed, bool kNarrow, bool kCplx, bool kFull, int kL, int kSplit, bool kWin>
+// win_add: it adds to y and the partials.  kParts: vector v of y is the sum over
+// the v-th share of the groups of one state (launch_apply_parts).  nchunk is at
+// least 1: the wait for the tile's loads is chunk_tables'.
+template <bool kMixed, bool kNarrow, bool kCplx, bool kFull, int kL, int kSplit, bool kWin, bool kParts>
 __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
     uint64_t N, ApplyWindow win, uint32_t ntiles, uint32_t tiles_per_xcd, uint32_t nchunk, uint32_t win_add,
     const ApplyGroup *__restrict__ grp, const ApplyChunk *__restrict__ chunks,
@@ -556,7 +557,10 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
     auto row = [&](uint64_t l) {
         return kWin ? base + ((l & ((1u << win.f) - 1u)) | ((l >> win.f) << win.s)) : base + l;
     };
-    const cT *__restrict__ xv = reinterpret_cast<const cT *>(xin) + uint64_t(v) * N;
+    const cT *__restrict__ xv = reinterpret_cast<const cT *>(xin) + uint64_t(kParts ? 0u : v) * N;
+    // the thread group's share of the groups: every `stride`-th from `share` on
+    const uint32_t share = kParts ? v * kSplit + sub : sub;
+    const uint32_t stride = kParts ? gridDim.x / ntiles * kSplit : uint32_t(kSplit);
 
     cT *xt = reinterpret_cast<cT *>(smem_raw);
     const uint32_t lds0 = uint32_t(uintptr_t((lds_byte *)smem_raw));
@@ -589,8 +593,10 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
         auto run_class = [&](auto far_t, auto swap_t, int cls) {
             constexpr bool kFar = decltype(far_t)::value, kSwap = decltype(swap_t)::value;
             const uint32_t g1 = ch.cg[cls + 1];
-            // thread group `sub` takes every kSplit-th group of the chunk
-            uint32_t g = ch.cg[cls] + (kSplit == 1 ? 0u : (sub - (ch.cg[cls] - ch.cg[0])) % kSplit);
+            // (in the order of the chunk)
+            uint32_t g = ch.cg[cls];
+            if constexpr (kParts) g += (share - (ch.cg[cls] - ch.cg[0])) & (stride - 1);
+            else if constexpr (kSplit > 1) g += (share - (ch.cg[cls] - ch.cg[0])) % kSplit;
             if (g >= g1) return;
             ApplyGroup nx = grp[g];
             do {
@@ -598,7 +604,7 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
                 // all descriptor fields in SGPRs before the gathers are issued,
                 // so that no later scalar-load wait also waits for them
                 asm volatile("" ::"s"(gd.m), "s"(gd.w0), "s"(gd.w1), "s"(gd.w2), "s"(gd.tab_n), "s"(gd.rc));
-                g += kSplit;
+                g += stride;
                 const auto fetch = [&]() {
                     gather<kFar, kFull, kPairs, R>(gd.m, tid, tile_rows, base, lds0, xv, xg);
                 };
@@ -630,7 +636,7 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
 // groups use it.  The load of run r + 1 (LDS-DMA: global memory straight into
 // LDS, no registers) is in flight while run r is computed.
 
-template <bool kMixed, bool kNarrow, bool kCplx, int kL, int kSplit>
+template <bool kMixed, bool kNarrow, bool kCplx, int kL, int kSplit, bool kParts>
 __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_staged(
     uint64_t N, uint32_t ntiles, uint32_t tiles_per_xcd, uint32_t nchunk, uint32_t nrun,
     const ApplyGroup *__restrict__ grp,
@@ -657,7 +663,10 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_staged(
     uint32_t tile = blockIdx.x % ntiles;
     if (tiles_per_xcd) tile = (tile % 8) * tiles_per_xcd + tile / 8;
     const uint64_t base = uint64_t(tile) * tile_rows;
-    const cT *__restrict__ xv = reinterpret_cast<const cT *>(xin) + uint64_t(v) * N;
+    const cT *__restrict__ xv = reinterpret_cast<const cT *>(xin) + uint64_t(kParts ? 0u : v) * N;
+    // the thread group's share of the groups: every `stride`-th from `share` on
+    const uint32_t share = kParts ? v * kSplit + sub : sub;
+    const uint32_t stride = kParts ? gridDim.x / ntiles * kSplit : uint32_t(kSplit);
 
     const uint32_t lds0 = uint32_t(uintptr_t((lds_byte *)smem_raw));
     const TabView tv = tab_view(tid);
@@ -679,7 +688,7 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_staged(
     for (int k = 0; k < R; ++k) ar[k] = ai[k] = 0.0;
     cT xg[R];
     if (nrun) stage(runs[0].hi, 0);
-    uint32_t r = 0, g = sub;
+    uint32_t r = 0, g = share;
     const uint32_t glast = nrun ? runs[nrun - 1].g1 - 1 : 0;
     ApplyGroup nx = grp[g < glast ? g : glast];
     for (uint32_t c = 0; c < nchunk; ++c) {
@@ -693,12 +702,12 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_staged(
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
             __syncthreads();
             if (r + 1 < nrun) stage(runs[r + 1].hi, (r + 1) & 1u);
-            // the run's groups (every kSplit-th), gathering from that tile
+            // the thread group's share of the run's groups, gathering from that tile
             const uint32_t g1 = runs[r].g1, xt = lds0 + (r & 1u) * kStageTileBytes;
             while (g < g1) {
                 const ApplyGroup gd = nx;
                 asm volatile("" ::"s"(gd.m), "s"(gd.w0), "s"(gd.w1), "s"(gd.w2), "s"(gd.tab_n), "s"(gd.rc));
-                g += kSplit;
+                g += stride;
                 const auto fetch = [&]() {
                     gather<false, true, false, R>(gd.m, tid, tile_rows, base, xt, xv, xg);
                 };
@@ -740,7 +749,17 @@ __global__ __launch_bounds__(256) void k_reduce_partials(uint32_t ntiles,
     if (threadIdx.x == 0) { out[2 * v] = ra[0]; out[2 * v + 1] = rb[0]; }
 }
 
-template <bool kMixed, bool kNarrow, int kL, int kSplit, bool kWin = false>
+// y = the sum of its parts y_p (launch_apply_parts), in order
+__global__ __launch_bounds__(256) void k_sum_parts(uint32_t n, uint32_t parts, const dvec2 *__restrict__ from,
+                                                   dvec2 *__restrict__ y) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    dvec2 v = from[i];
+    for (uint32_t p = 1; p < parts; ++p) v += from[uint64_t(p) * n + i];
+    y[i] = v;
+}
+
+template <bool kMixed, bool kNarrow, int kL, int kSplit, bool kWin = false, bool kParts = false>
 static int launch_tiled(const qr_op *op, DeviceTables *t, int slot, uint32_t nvec, const void *d_x,
                         void *d_y, double *partials, uint32_t ntiles, hipStream_t s, bool few = false,
                         bool add = false) {
@@ -755,11 +774,11 @@ static int launch_tiled(const qr_op *op, DeviceTables *t, int slot, uint32_t nve
     const bool full = tile_rows == (uint64_t(1) << Shape::L);
     auto pick = [&](auto cplx_t) {
         constexpr bool kC = decltype(cplx_t)::value;
-        return full ? k_apply_tiled<kMixed, kNarrow, kC, true, kL, kSplit, kWin>
-                    : k_apply_tiled<kMixed, kNarrow, kC, false, kL, kSplit, false>;
+        return full ? k_apply_tiled<kMixed, kNarrow, kC, true, kL, kSplit, kWin, kParts>
+                    : k_apply_tiled<kMixed, kNarrow, kC, false, kL, kSplit, false, false>;
     };
     auto kern = pt.cplx ? pick(std::true_type{}) : pick(std::false_type{});
-    if (kWin && !full) return fail(QR_ERR_ARG, "apply: a window pass of partial tiles");
+    if ((kWin || kParts) && !full) return fail(QR_ERR_ARG, "apply: partial tiles");
     if (shmem > kDefaultLDS)
         QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
@@ -772,7 +791,7 @@ static int launch_tiled(const qr_op *op, DeviceTables *t, int slot, uint32_t nve
     return QR_OK;
 }
 
-template <bool kMixed, bool kNarrow, int kL, int kSplit>
+template <bool kMixed, bool kNarrow, int kL, int kSplit, bool kParts = false>
 static int launch_staged(const qr_op *op, DeviceTables *t, int slot, uint32_t nvec, const void *d_x,
                          void *d_y, double *partials, uint32_t ntiles, hipStream_t s) {
     using Shape = ApplyShape<kMixed, kL>;
@@ -781,8 +800,8 @@ static int launch_staged(const qr_op *op, DeviceTables *t, int slot, uint32_t nv
     const size_t shmem = apply_lds_bytes(2 * Shape::kTile, pt.max_tab, Shape::merge_bytes(kSplit));
     if (shmem > kApplyLDSLimit) return fail(QR_ERR_SIZE, "apply: LDS stage too large");
     const uint32_t tpx = (ntiles % 8 == 0) ? ntiles / 8 : 0;
-    auto kern = pt.cplx ? k_apply_staged<kMixed, kNarrow, true, kL, kSplit>
-                        : k_apply_staged<kMixed, kNarrow, false, kL, kSplit>;
+    auto kern = pt.cplx ? k_apply_staged<kMixed, kNarrow, true, kL, kSplit, kParts>
+                        : k_apply_staged<kMixed, kNarrow, false, kL, kSplit, kParts>;
     if (shmem > kDefaultLDS)
         QR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)));
@@ -1010,6 +1029,46 @@ static int apply_split(const ApplyPlan &p, bool mixed, uint64_t blocks, int cus)
 int apply_tables(const qr_op *op, DeviceTables *t) {
     const ApplyPlan plan = make_plan<false, ApplyShape<false>::L>(op, 0);
     return device_patterns(op, t, plan.slot, plan.shape, plan.win_shape, false);
+}
+
+// FP64 applies of one state of few tiles and many groups, for a caller with
+// memory for the sums: a tile's blocks take a share of the groups each and write
+// what they add to y, which k_sum_parts sums.  In few blocks such an apply is a
+// chain over the groups, 0.08-0.1 us each, which a batch of few operators ends up
+// waiting for.  Measured, batches of one random operator (build and y, us), y from
+// the entries in the tile builder's registers / whole applies / shares of 64 blocks
+// in all: 12 qubits, 1000, 2000, 3500 terms 67, 85, 115 / 128, 222, 324 / 58, 89,
+// 119; 13 qubits, 5000 323 / 686 / 308; 14 qubits, 500, 2000 114, 323 / 102, 418 /
+// 69, 262; 15 qubits, 300, 2000 173, 676 / 94, 571 / 80, 463.  32, 64, 128 and 256
+// blocks: 64 operators of 8 to 14 qubits 760, 746, 774, 789, 32 of 11 to 14 2650,
+// 2605, 2680, 2930, but one of 15 qubits and 1000 terms 301, 245, 221, 207.
+constexpr uint32_t kPartsBlocks = 64, kPartsGroups = 32;
+
+uint32_t apply_parts(const qr_op *op) {
+    constexpr int L = ApplyShape<false>::L;
+    if (int(op->nq) < L || op->nq > 32) return 1;
+    const uint64_t tiles = uint64_t(1) << (op->nq - L);
+    uint32_t parts = 1;
+    while (2 * parts * tiles <= kPartsBlocks && 2 * parts * kPartsGroups <= op->G) parts *= 2;
+    return parts;
+}
+
+int launch_apply_parts(const qr_op *op, DeviceTables *t, uint32_t parts, const void *d_x, void *d_y, void *d_sums,
+                       hipStream_t s) {
+    constexpr int L = ApplyShape<false>::L;
+    const ApplyPlan plan = make_plan<false, L>(op, 0);
+    int rc = device_patterns(op, t, plan.slot, plan.shape, plan.win_shape, true);
+    if (rc) return rc;
+    const uint32_t n = 1u << op->nq, ntiles = n >> L;
+    // (no window passes: the states are far below their least size)
+    rc = plan.staged
+             ? launch_staged<false, true, L, 4, true>(op, t, plan.slot, parts, d_x, d_sums, nullptr, ntiles, s)
+             : launch_tiled<false, true, L, 4, false, true>(op, t, plan.slot, parts, d_x, d_sums, nullptr, ntiles, s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_sum_parts, dim3((n + 255) / 256), dim3(256), 0, s, n, parts,
+                       static_cast<const dvec2 *>(d_sums), static_cast<dvec2 *>(d_y));
+    QR_HIP_CHECK(hipGetLastError());
+    return QR_OK;
 }
 
 int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint32_t nvec,

@@ -12,7 +12,8 @@
 //   fused  y = A x by the matrix-free apply of the same operator
 //          (qr_apply.hip), which reads no CSR back and so needs none: 0.5 ps
 //          per entry of a random 20-qubit operator, where reading the entry's
-//          24 bytes takes 4;
+//          24 bytes takes 4; states of few tiles with the operator's groups
+//          in shares (launch_apply_parts);
 //   split  (needs every CSR) after the builds, one matvec pass (k_batch_mv)
 //          over the written CSRs.
 // Measured, 16 operators of 8 to 18 qubits and 10 to 5000 random terms (443e6
@@ -242,6 +243,8 @@ struct qr_batch {
     size_t d_desc_cap = 0;
     BatchMvDesc *d_mv = nullptr;
     size_t d_mv_cap = 0;
+    double *d_sums = nullptr;  // of the applies in shares (apply_parts), one after another
+    size_t d_sums_cap = 0;
     unsigned long long *d_counter = nullptr;
     int ncu = 0;
     // graph of the last (buffers, tuning)
@@ -263,6 +266,8 @@ struct Plan {
     size_t shmem[2] = {};
     std::vector<uint32_t> branch[kBranches];  // the others, in order
     std::vector<bool> csr;                    // whether operator k's CSR is built
+    std::vector<size_t> sums_at;              // operator k's place in d_sums
+    size_t sums = 0;                          // doubles there
     std::vector<BatchMvDesc> mv;              // split form: one per operator
     uint64_t mv_items = 0;
 };
@@ -287,6 +292,7 @@ int make_plan(qr_batch *b, uint64_t *const *d_indptr, uint64_t *const *d_indices
         });
     uint64_t load[kBranches] = {};
     plan.csr.resize(nops);
+    plan.sums_at.resize(nops);
     for (uint32_t k : order) {
         const qr_op *op = b->ops[k];
         if (op->nq > 32) return fail(QR_ERR_SIZE, "batch operators are limited to 32 qubits");
@@ -325,6 +331,9 @@ int make_plan(qr_batch *b, uint64_t *const *d_indptr, uint64_t *const *d_indices
         const int to = int(std::min_element(load, load + kBranches) - load);
         load[to] += N * op->G + (uint64_t(1) << 20);
         plan.branch[to].push_back(k);
+        const uint32_t parts = tu.split ? 1 : apply_parts(op);
+        plan.sums_at[k] = plan.sums;
+        if (parts > 1) plan.sums += 2 * N * parts;
     }
     plan.small_branch = int(std::min_element(load, load + kBranches) - load);
     return QR_OK;
@@ -348,7 +357,10 @@ int record(qr_batch *b, const Plan &plan, const qr_tuning &tu, uint64_t *const *
             if (has_csr(d_indices, d_data, k))
                 rc = launch_csr_build(op, t, 0, N, ip, d_indices[k], d_data[k], bs);
             else if (ip) rc = launch_csr_indptr(op, 0, N, ip, bs);
-            if (!rc && !tu.split)
+            const uint32_t parts = tu.split ? 1 : apply_parts(op);
+            if (!rc && parts > 1)
+                rc = launch_apply_parts(op, t, parts, d_x[k], d_y[k], b->d_sums + plan.sums_at[k], bs);
+            else if (!rc && !tu.split)
                 rc = launch_pauli_apply(op, t, QR_PREC_FP64, 1, d_x[k], d_y[k], nullptr, bs, true);
             if (rc) return rc;
         }
@@ -432,7 +444,8 @@ int prepare(qr_batch *b, const Plan &plan, const qr_tuning &tu) {
         *cap = n;
         return int(QR_OK);
     };
-    if ((rc = room(&b->d_desc, &b->d_desc_cap, nsmall)) || (rc = room(&b->d_mv, &b->d_mv_cap, plan.mv.size())))
+    if ((rc = room(&b->d_desc, &b->d_desc_cap, nsmall)) || (rc = room(&b->d_mv, &b->d_mv_cap, plan.mv.size())) ||
+        (rc = room(&b->d_sums, &b->d_sums_cap, plan.sums)))
         return rc;
     for (size_t c = 0, at = 0; c < 2; at += plan.small[c++].size())
         if (!plan.small[c].empty())
@@ -488,6 +501,7 @@ int qr_batch_destroy(qr_batch *b) {
     drop_graph(b);
     if (b->d_desc) (void)hipFree(b->d_desc);
     if (b->d_mv) (void)hipFree(b->d_mv);
+    if (b->d_sums) (void)hipFree(b->d_sums);
     if (b->d_counter) (void)hipFree(b->d_counter);
     for (int i = 1; i < kBranches; ++i) {
         if (b->side[i]) (void)hipStreamDestroy(b->side[i]);

@@ -370,6 +370,11 @@ int io_read_mm(const char *path, qr_mm_reader **out, hipStream_t s);
 // the tables of an FP64 apply of the operator, so that a launch_pauli_apply
 // without allocation finds them
 int apply_tables(const qr_op *op, DeviceTables *t);
+// The same apply of one state without <x|y>, its groups in apply_parts(op)
+// shares (1: not in shares), given memory for as many states in d_sums.
+uint32_t apply_parts(const qr_op *op);
+int launch_apply_parts(const qr_op *op, DeviceTables *t, uint32_t parts, const void *d_x, void *d_y, void *d_sums,
+                       hipStream_t s);
 // noalloc: no device allocation -- the tables must be on the device already
 // and the <x|y> block partials go to the file-scope scratch array (qr_apply.hip)
 int launch_pauli_apply(const qr_op *op, DeviceTables *t, int32_t precision, uint32_t nvec,

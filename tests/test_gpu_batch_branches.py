@@ -82,3 +82,37 @@ def test_indptr_alone(n, t):
     G = len(np.unique(params[0].x))
     assert np.array_equal(ip.cpu().numpy(), np.arange((1 << n) + 1) * G)
     _check_y(params[0], x, b.y[0].cpu().numpy())
+
+
+# states of 2 to 32 tiles: every mask of the tile and a few past it (gathers), or
+# masks all over (partner tiles staged); from 64 groups, shares of few, on
+@pytest.mark.parametrize("form", ["1", "2"])
+@pytest.mark.parametrize("n,groups,real", [(11, 1025, True), (11, 1500, False), (12, 1100, True), (13, 2049, False),
+                                           (14, 150, True), (15, 70, False)])
+def test_groups_in_shares(monkeypatch, n, groups, real, form):
+    import qrusty_amd as qa
+    from qrusty_amd import workloads
+    monkeypatch.setenv("QR_APPLY_FORM", form)
+    rng = np.random.default_rng(n * groups)
+    low = rng.permutation(min(1 << 10, groups - 3))[:groups - 3]
+    masks = list(low) + list(rng.choice(np.arange(1 << 10, 1 << n), groups - len(low), replace=False))
+    labels, coeffs = [], []
+    for m in masks:
+        for _ in range(rng.integers(1, 4)):
+            z = int(rng.integers(1 << n))
+            labels.append("".join("IZXY"[2 * (int(m) >> q & 1) + (z >> q & 1)] for q in reversed(range(n))))
+            ny = bin(int(m) & z).count("1")
+            c = complex(rng.standard_normal(), 0 if real else rng.standard_normal())
+            coeffs.append(c * 1j ** ny if real else c)
+    op = qa.SparsePauliOp([qa.Pauli(s) for s in labels], coeffs)
+    p = orc.Params(labels, coeffs)
+    assert len(np.unique(p.x)) == groups and groups << n > 1 << 21
+    for keep in (True, False):
+        b = qa.Batch([op], keep_csr=keep)
+        for rep in range(3):
+            x = workloads.random_states(p.N, 1, 11 * rep + n)[0]
+            b.set_states([x])
+            print(f"[gpu] batch, groups in shares n={n} groups={groups} real={real} form={form} run {rep}", flush=True)
+            b.run()
+            torch.cuda.synchronize()
+            _check_y(p, x, b.y[0].cpu().numpy())

@@ -226,3 +226,22 @@ L.check(L.lib.qr_batch_tune(batch, *args, None, None))
 large = sum(q > 20 for q in {qubits})
 assert len(launched("k_csr_build")) == {candidates} * 2 * large, len(launched("k_csr_build"))
 """)
+
+
+@pytest.mark.parametrize("n,groups", [(11, 1500), (12, 2000), (12, 3500), (14, 300)])
+def test_batch_applies_of_few_tiles_fill_more_blocks(run, n, groups):
+    """y of a batch's operator whose state has few tiles: its many groups are
+    shared among blocks, not walked by one per tile."""
+    run(f"""
+import random
+rng = random.Random(7)
+masks = rng.sample(range(1 << {n}), {groups})
+op = op_of(["".join("IX"[m >> q & 1] for q in reversed(range({n}))) for m in masks])
+batch = ctypes.c_void_p()
+L.check(L.lib.qr_batch_create((ctypes.c_void_p * 1)(op), 1, ctypes.byref(batch)))
+args = [ctypes.cast((ctypes.c_void_p * 1)((64 + 4 * k) * GB), ctypes.c_void_p) for k in range(5)]
+L.check(L.lib.qr_batch_run(batch, *args, None, None))
+applies = launched("k_apply_")
+assert len(applies) == 1 and applies[0][2] >= min(64, {groups} // 64 << ({n} - 10)), applies
+assert len(launched("k_sum_parts")) == 1
+""")
