@@ -98,6 +98,32 @@ def test_row_windows(n, groups, sizes, real):
             assert dh[a:a + h.G].tobytes() == vals.tobytes()
 
 
+@pytest.mark.parametrize("n,groups,sizes", [(13, 1500, [1, 2]), (13, 40, [3]), (40, 60, [2]), (34, 2100, [1])])
+def test_every_row_of_a_window(n, groups, sizes):
+    """Windows of any number of tiles (the XCDs' ranges are not equal): every row
+    as in the window that holds them all."""
+    from qrusty_amd import _lib as L
+    low = min(n, 13)
+    labels, coeffs = _operator(low, groups, sizes, groups, False)
+    op = _op(["Z" * (n - low) + s for s in labels], coeffs)
+    h = op._handle(L.QR_PHASE_ROWWISE)
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def rows(r0, r1):
+        ix = torch.full(((r1 - r0) * h.G,), -7, dtype=torch.int64, device="cuda")
+        d = torch.full(((r1 - r0) * h.G,), 7.0, dtype=torch.complex128, device="cuda")
+        L.check(L.lib.qr_csr_build_rows(h.h, r0, r1, ctypes.c_void_p(ix.data_ptr()), ctypes.c_void_p(d.data_ptr()), s))
+        return ix, d
+
+    print(f"[gpu] build windows n={n} groups={groups}", flush=True)
+    ix, d = rows(0, 4096)
+    assert int((ix == -7).sum()) == 0
+    for tiles in range(1, 16):
+        r0, r1 = 16 * (tiles % 5), min(4096, 16 * (tiles % 5) + (16 if groups > 500 else 256) * tiles + tiles % 3)
+        for got, want in zip(rows(r0, r1), (ix, d)):
+            assert torch.equal(got.view(torch.uint8), want[r0 * h.G:r1 * h.G].view(torch.uint8)), (r0, r1)
+
+
 @pytest.mark.parametrize("n,groups,sizes", [(9, 25, [2, 2, 2, 48]), (10, 300, [1, 3]), (12, 2600, [4, 4, 4, 6, 9])])
 def test_captured_before_any_build(n, groups, sizes):
     """An operator whose first build is recorded into a graph, after an apply put
