@@ -660,14 +660,31 @@ void finish_op(qr_op *op) {
         };
         split(op->leaves, op->leaf_heavy);
     }
+    // the form of the sign-word builder: terms past those it holds are loaded
+    // again for every row, so they have to be few
+    bool real = true;
+    for (uint64_t i = 0; i < op->T; ++i) real = real && op->tc[2 * i + 1] == 0.0;
+    uint64_t past = 0;
+    for (uint64_t g = 0; g < op->G; ++g) {
+        const uint64_t n = op->gterm[g + 1] - op->gterm[g];
+        if (n > kWordHold && !std::binary_search(op->heavy.begin(), op->heavy.end(), uint32_t(g)))
+            past += n - kWordHold;
+    }
+    op->word_real = real && 16 * past <= op->G;
     if (op->nq <= 32) {
         std::vector<qr_op::SubLeaf> leaves;
         cut(kWordMaxG, leaves);
         if (leaves.empty()) leaves.push_back({0, uint32_t(op->G), 0, 0, 0});
-        std::stable_sort(leaves.begin(), leaves.end(), [](const auto &a, const auto &b) {
-            auto threads = [](const auto &l) { return l.s1 - l.s0 <= 256 ? 0 : l.s1 - l.s0 <= 512 ? 1 : 2; };
-            return threads(a) < threads(b);
-        });
+        auto threads = [](const auto &l) { return l.s1 - l.s0 <= 256 ? 256u : l.s1 - l.s0 <= 512 ? 512u : 1024u; };
+        uint64_t most = 0, sum = 0;
+        for (const auto &l : leaves) {
+            most = std::max<uint64_t>(most, threads(l));
+            sum += threads(l);
+        }
+        op->word_joint = most * leaves.size() <= 2 * sum && (op->word_real || op->T <= 4 * op->G);
+        if (!op->word_joint)
+            std::stable_sort(leaves.begin(), leaves.end(),
+                             [&](const auto &a, const auto &b) { return threads(a) < threads(b); });
         op->word_groups.resize(op->G);
         for (const auto &l : leaves) {
             WordLeaf lf{l.s0, l.s1 - l.s0, 0, uint32_t(op->word_ptr.size()), {}};
@@ -685,17 +702,6 @@ void finish_op(qr_op *op) {
             op->word_leaves.push_back(lf);
         }
     }
-    // the form of the sign-word builder: terms past those it holds are loaded
-    // again for every row, so they have to be few
-    bool real = true;
-    for (uint64_t i = 0; i < op->T; ++i) real = real && op->tc[2 * i + 1] == 0.0;
-    uint64_t past = 0;
-    for (uint64_t g = 0; g < op->G; ++g) {
-        const uint64_t n = op->gterm[g + 1] - op->gterm[g];
-        if (n > kWordHold && !std::binary_search(op->heavy.begin(), op->heavy.end(), uint32_t(g)))
-            past += n - kWordHold;
-    }
-    op->word_real = real && 16 * past <= op->G;
     // tail table: operators with heavy groups, whose other groups also run
     // past two terms (the molecular Hamiltonians: 4 and 6), and those of many
     // terms per group

@@ -100,8 +100,8 @@ __global__ __launch_bounds__(kStageThreads) void k_csr_build_staged(TileOp op) {
 // tile, one thread per (group, row), their terms in LDS.  The additions are
 // the same, in the same order, as build_tile_staged's, so the values are
 // bit-identical.  Operators of more than kWordMaxG groups are built as
-// sub-operators of at most that many (kSub), each with the power of two of
-// threads that holds it, consecutive blocks building the same rows.
+// sub-operators of at most that many (kSub), consecutive blocks building the same
+// rows (launch_build_words).
 // What bounds it: the stores (5.2 or 6.5 TB/s of 24 B per entry, by the place
 // of the output in memory; fills reach 6.65), and from about five terms per
 // group on the additions and the loads of the terms.  The two-group-chunk
@@ -463,8 +463,19 @@ __global__ __launch_bounds__(256) void k_indptr(uint64_t row_begin, uint64_t nro
     if (i <= nrows) indptr[i] = (row_begin + i) * G;
 }
 
-// Builds by k_csr_build_words: the whole operator, or one launch for all
-// sub-operators of a number of threads.
+// Builds by k_csr_build_words: the whole operator, or its sub-operators, in one
+// launch with the threads that the largest needs, or in one for each number of
+// threads.  One launch writes every row from end to end, while its lines are in L2;
+// several write it in pieces, whose ends leave the caches in between.  But it idles
+// the threads that small sub-operators don't need, which counts where the lanes load
+// their terms again; so one (word_joint) for the real form and up to 4 terms per
+// group, where it takes at most twice the threads.  Several / one, us: molecules of
+// 18, 20, 22 qubits (4 to 6 GB) 1249 / 1085, 928 / 822, 1330 / 1197; random, 17
+// qubits, 1025 groups (488 + 537) 837 / 592 (638 by the builder before this one), 18
+// qubits, 2086 736 / 589; 880 + 220 groups of 1, 3 (complex), 6 terms 798 / 662, 795
+// / 730, 812 / 693; 200 + 150, 900, 210 of 4 complex terms 1173 / 954; but 900 + 300
+// of 8 1063 / 1260, 1000 + 60 of 6 853 / 1055; 1000, 60, 120, 240 of 1 (2.3 times the
+// threads) 985 / 1079.
 static int launch_build_words(const qr_op *op, const DeviceTables *t, uint64_t row_begin, uint64_t row_end,
                               uint64_t *d_indptr, uint64_t *d_indices, double *d_data, hipStream_t s) {
     const uint32_t G = uint32_t(op->G);
@@ -528,7 +539,14 @@ static int launch_build_words(const qr_op *op, const DeviceTables *t, uint64_t r
         while (k < lv.size() && lv[k].g <= most) ++k;
         return k;
     };
-    const size_t a = to(256), b = to(512), c = lv.size();
+    size_t a = to(256), b = to(512);
+    const size_t c = lv.size();
+    if (op->word_joint) {
+        uint32_t most = 0;
+        for (const auto &l : lv) most = std::max(most, l.g);
+        a = most <= 256 ? c : 0;
+        b = most <= 512 ? c : 0;
+    }
     int rc = QR_OK;
     if (a && (rc = run(T{}, T256{}, 0, 0, a))) return rc;
     if (b > a && (rc = run(T{}, T512{}, 0, a, b))) return rc;

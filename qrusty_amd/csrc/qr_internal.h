@@ -285,9 +285,10 @@ struct qr_op {
     // the sign-word builder (k_csr_build_words; at most 32 qubits): its form,
     // real if every coefficient c' is and few groups have terms past
     // kWordHold; the whole operator or its sub-operators of at most kWordMaxG
-    // groups, those of at most 256, 512 and 1024 groups one after another;
-    // every group, and the terms of the heavy ones
-    bool word_real = false;
+    // groups, in the order of their place (word_joint: one launch builds them
+    // all, launch_build_words) or those of at most 256, 512 and 1024 groups one
+    // after another; every group, and the terms of the heavy ones
+    bool word_real = false, word_joint = false;
     std::vector<qr::WordLeaf> word_leaves;
     std::vector<qr::WordGroup> word_groups;
     std::vector<uint32_t> word_ptr;

@@ -98,6 +98,28 @@ def test_row_windows(n, groups, sizes, real):
             assert dh[a:a + h.G].tobytes() == vals.tobytes()
 
 
+@pytest.mark.parametrize("real,terms", [(True, [1]), (True, [4, 6]), (False, [1, 2]), (False, [6])])
+@pytest.mark.parametrize("parts", [(488, 537), (700, 330, 20, 1), (300, 480, 10, 400), (1000, 30, 3, 200)])
+def test_uneven_sub_operators(parts, real, terms):
+    """Sub-operators of unlike sizes, in one launch or several."""
+    rng, n = np.random.default_rng(sum(parts)), 12
+    labels, coeffs = [], []
+    for k, size in enumerate(parts):
+        for j, m in enumerate(rng.choice(1 << 10, size, replace=False)):
+            for _ in range(terms[j % len(terms)]):
+                x, z = int(m) | k << 10, int(rng.integers(1 << n))
+                c = complex(rng.normal(), 0.0 if real else rng.normal())
+                labels.append(_label(n, x, z))
+                coeffs.append(c * 1j ** bin(x & z).count("1") if real else c)
+    p = orc.Params(labels, coeffs)
+    print(f"[gpu] build by uneven sub-operators {parts} real={real} terms={terms}", flush=True)
+    ip, ind, dat = orc.build_csr(p)
+    _, data, indices, indptr = _op(labels, coeffs).to_matrix_mode("RowwiseUnsafeChunked/100").export()
+    assert indptr.tobytes() == ip.tobytes()
+    assert indices.tobytes() == ind.tobytes()
+    assert data.tobytes() == dat.tobytes()
+
+
 @pytest.mark.parametrize("n,groups,sizes", [(13, 1500, [1, 2]), (13, 40, [3]), (40, 60, [2]), (34, 2100, [1])])
 def test_every_row_of_a_window(n, groups, sizes):
     """Windows of any number of tiles (the XCDs' ranges are not equal): every row

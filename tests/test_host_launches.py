@@ -245,3 +245,30 @@ applies = launched("k_apply_")
 assert len(applies) == 1 and applies[0][2] >= min(64, {groups} // 64 << ({n} - 10)), applies
 assert len(launched("k_sum_parts")) == 1
 """)
+
+
+@pytest.mark.parametrize("sizes,terms,real,launches", [((488, 537), 1, True, 1), ((1000, 520, 505), 1, False, 1),
+                                                       ((880, 220), 4, False, 1), ((880, 220), 6, False, 2),
+                                                       ((40, 50, 60, 1000), 1, True, 2), ((900, 700, 600), 6, False, 1)])
+def test_sub_operators_of_one_launch(run, sizes, terms, real, launches):
+    """A build by sub-operators writes its rows from end to end, in one launch, but
+    where that idles too many threads."""
+    run(f"""
+import random
+rng, n = random.Random(3), 22
+sizes, terms, real = {sizes}, {terms}, {real}
+labels = []
+for k, size in enumerate(sizes):
+    # prefixes 0, 10, 110, ...: each leaves the subtree of those after it
+    top = ((1 << k) - 1) << (12 - k)
+    for m in rng.sample(range(1 << 9), min(size, 1 << 9)) + [512 + i for i in range(size - 512)]:
+        for z in rng.sample(range(1 << 10), terms):
+            x = (top << 10) | m
+            labels.append("".join("IZXY"[2 * (x >> q & 1) + (z >> q & 1)] for q in reversed(range(n))))
+op = op_of(labels, [1.0 + 0.5 * k if real else complex(1, 1 + k) for k in range(len(labels))])
+groups = ctypes.c_uint64()
+L.check(L.lib.qr_op_info(op, None, None, ctypes.byref(groups), None))
+assert groups.value == sum(sizes)
+L.check(L.lib.qr_csr_build(op, 64 * GB, 128 * GB, 192 * GB, None))
+assert len(launched("k_csr_build_words")) == {launches}, launched("k_csr_build_words")
+""")
