@@ -428,8 +428,9 @@ __device__ __forceinline__ double2 pattern_coeff(uint64_t base, uint32_t t0, uin
     return make_double2(a_r, a_i);
 }
 
-// LDS: x tile (gather form) or two tile buffers (partner-staged form) |
-// tables; at the end the split's sums and the <x|y> partials take it over.
+// LDS: x tile (gather form) or two tile buffers (partner-staged form) | tables;
+// at the end the split's sums take over the tables (gather form) or all of it
+// (partner-staged), and the <x|y> partials the first bytes.
 __host__ __device__ inline size_t apply_lds_bytes(size_t tiles, uint32_t max_tab, size_t merge) {
     const size_t all = tiles + ((size_t(max_tab) + 15) & ~size_t(15));
     return all > merge + 64 ? all : merge + 64;
@@ -621,9 +622,12 @@ __global__ __launch_bounds__(kApplyThreads * kSplit) void k_apply_tiled(
             if constexpr (kPairs) run_class(T{}, T{}, 3);
         }
     }
-    if (kSplit > 1) merge_splits<kSplit, R>(reinterpret_cast<dvec2 *>(smem_raw), tid, sub, ar, ai);
-    // x from the tile in LDS, or from global memory where the merge used it
-    const auto x = [&](uint64_t l) { return kSplit == 1 ? xt[l] : xv[row(l)]; };
+    // the sums are added up where the tables were, so that <x|y> takes x from the
+    // tile (y and energy, read again / this, us: 26 qubits, 1, 8 groups 569 / 512, 689
+    // / 571, rings of 23, 24 qubits 205 / 192, 376 / 359; 574 for the 8 groups before
+    // there were two thread groups)
+    if (kSplit > 1) merge_splits<kSplit, R>(reinterpret_cast<dvec2 *>(smem_raw + Shape::kTile), tid, sub, ar, ai);
+    const auto x = [&](uint64_t l) { return xt[l]; };
     finish_tile<kFull, kPairs, kSplit, R, cT>(tid, sub, tile_rows, kWin && win_add, row, x,
                                               yout ? reinterpret_cast<cT *>(yout) + uint64_t(v) * N : nullptr,
                                               partials, reinterpret_cast<double *>(smem_raw), ar, ai);
@@ -767,7 +771,7 @@ static int launch_tiled(const qr_op *op, DeviceTables *t, int slot, uint32_t nve
     const uint64_t N = uint64_t(1) << op->nq;
     const uint64_t tile_rows = N < (uint64_t(1) << Shape::L) ? N : (uint64_t(1) << Shape::L);
     const DeviceTables::Patterns &pt = t->pat[slot];
-    size_t shmem = apply_lds_bytes(Shape::kTile, pt.max_tab, Shape::merge_bytes(kSplit));
+    size_t shmem = Shape::kTile + apply_lds_bytes(0, pt.max_tab, Shape::merge_bytes(kSplit));
     if (few && shmem < kApplyFewLDS) shmem = kApplyFewLDS;
     if (shmem > kApplyLDSLimit) return fail(QR_ERR_SIZE, "apply: LDS stage too large");
     const uint32_t tpx = (ntiles % 8 == 0) ? ntiles / 8 : 0;

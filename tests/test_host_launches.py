@@ -272,3 +272,19 @@ assert groups.value == sum(sizes)
 L.check(L.lib.qr_csr_build(op, 64 * GB, 128 * GB, 192 * GB, None))
 assert len(launched("k_csr_build_words")) == {launches}, launched("k_csr_build_words")
 """)
+
+
+@pytest.mark.parametrize("n,groups", [(14, 3), (22, 8), (23, 30)])
+def test_sums_leave_the_tile_in_place(run, n, groups):
+    """The LDS of an apply by gathers holds the tile of x (2^10 complex128) beside
+    the sums of its thread groups (16 bytes a row for every second of them): <x|y>
+    does not read x again."""
+    run(f"""
+import re
+op = op_of([term({n}, {{q % 4: "X", q // 4: "Y" if q // 4 != q % 4 else "X"}}) for q in range({groups})])
+L.check(L.lib.qr_pauli_apply(op, 0, 1, 64 * GB, 128 * GB, 192 * GB, None))
+applies = [(re.search("k_apply_tiled.*Li10ELi([24])E", stub.stub_name(i).decode()), stub.stub_shmem(i))
+           for i in range(stub.stub_launches())]
+applies = [(int(m[1]), lds) for m, lds in applies if m]
+assert applies and all(lds >= (16 << 10) * (1 + split // 2) for split, lds in applies), applies
+""")
