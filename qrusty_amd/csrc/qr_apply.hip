@@ -825,6 +825,7 @@ constexpr int kFormStaged = 1;       // D partner tiles through LDS
 constexpr int kFormStagedDense = 2;  // the same with F >= 8 D
 constexpr int kFormGatherFew = 3;    // gathers, two blocks per CU
 constexpr int kFormStagedFew = 4;    // staged, two thread groups per block
+constexpr int kFormGatherNear = 5;   // FP64, more than 8 groups, F = 0
 // Measured (us, one state, gather / partner-staged):
 //   FP64: reference's molecules (F/D 9..), 16 / 20 / 22 qubits 134 / 113,
 //     1360 / 928, 7750 / 5050; k-local 24 qubits, 3000 terms (F/D 3.6) 7784 /
@@ -898,8 +899,9 @@ static int apply_form(const qr_op *op, int kind, int L, const PatternShape &win_
                                 (state_log2 >= 25 && scattered && distinct >= 64));
             few = staged && lone && distinct >= 64 && state_log2 >= 26;
         }
-        form = few ? (kind == 0 ? kFormGatherFew : kFormStagedFew)
-                   : !staged ? kFormGather : dense ? kFormStagedDense : kFormStaged;
+        form = few       ? (kind == 0 ? kFormGatherFew : kFormStagedFew)
+               : staged  ? (dense ? kFormStagedDense : kFormStaged)
+               : kind == 0 && far == 0 && op->G > 8 ? kFormGatherNear : kFormGather;
         op->form[kind].store(form + 1, std::memory_order_relaxed);
     }
     if (e && atoi(e) == 2) return form == kFormStagedDense || form == kFormStagedFew ? form : kFormStaged;
@@ -998,7 +1000,8 @@ static ApplyPlan make_plan(const qr_op *op, int kind) {
         p.win_shape = {p.L, kApplyThreadBits, Shape::kPatSplit, Shape::kTabChunk,
                        uint32_t(Shape::kTile), false, false, {}};
     p.form = p.L == kL ? apply_form(op, kind, p.L, p.win_shape) : kFormGather;
-    const bool staged = p.staged = p.form != kFormGather && p.form != kFormGatherFew;
+    const bool staged = p.staged =
+        p.form == kFormStaged || p.form == kFormStagedDense || p.form == kFormStagedFew;
     // the gather form on full complex64 tiles runs the paired-row layout
     const bool pairs = kMixed && !staged && p.L == kL;
     p.shape = {p.L, kApplyThreadBits, staged ? Shape::kPatSplitS : Shape::kPatSplit,
@@ -1017,7 +1020,10 @@ static ApplyPlan make_plan(const qr_op *op, int kind) {
 // 613 / 371 / 235, 20 (1024 tiles, staged, F/D 9): 1007 / 928 / 989, 22: 6020
 // / 5050 / 5570; k-local 20 qubits, 3000 terms (staged, F/D 5): 400 / 486 /
 // 716 (one term, 19 qubits, four states 12 / 13 / 23); ring 24 qubits (gather)
-// 320 / 300 / 358, a diagonal, 26 qubits 722 / 854; gathers with two blocks per
+// 320 / 300 / 358, a diagonal, 26 qubits 722 / 854; all groups inside the tile, y /
+// y and energy, split 1 against 2: 24 qubits, 12, 24 groups 84 / 141 against 96 / 176,
+// 130 / 187 against 144 / 229, 26 qubits, 16 414 / 522 against 470 / 665, but 24 qubits,
+// 6 90 / 147 against 81 / 157, and below 2^22 rows equal; gathers with two blocks per
 // CU, random, 300 terms, 21 qubits 491 / 406, 22 qubits 1170 / 1670.  Complex64,
 // 2^11-row tiles: molecule 20 qubits (512 tiles) 1085 / 804, k-local 24 qubits
 // (8192 tiles) 4940 / 5250; 2^10-row tiles: molecule 18 qubits (256 tiles) 439 /
@@ -1025,6 +1031,7 @@ static ApplyPlan make_plan(const qr_op *op, int kind) {
 static int apply_split(const ApplyPlan &p, bool mixed, uint64_t blocks, int cus) {
     if (!mixed && p.form == kFormStaged) return 1;
     if (p.form == kFormGatherFew) return p.tiles_log2 <= 11 ? 2 : 1;
+    if (p.form == kFormGatherNear && p.tiles_log2 >= 12) return 1;
     if ((!mixed || p.small) && blocks <= uint64_t(2) * cus) return 4;
     if (!mixed || p.form == kFormStagedFew) return p.single ? 1 : 2;
     return p.small || blocks < uint64_t(4) * cus ? 2 : 1;

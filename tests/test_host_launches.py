@@ -274,7 +274,7 @@ assert len(launched("k_csr_build_words")) == {launches}, launched("k_csr_build_w
 """)
 
 
-@pytest.mark.parametrize("n,groups", [(14, 3), (22, 8), (23, 30)])
+@pytest.mark.parametrize("n,groups", [(14, 3), (22, 8), (20, 30)])
 def test_sums_leave_the_tile_in_place(run, n, groups):
     """The LDS of an apply by gathers holds the tile of x (2^10 complex128) beside
     the sums of its thread groups (16 bytes a row for every second of them): <x|y>
@@ -287,4 +287,23 @@ applies = [(re.search("k_apply_tiled.*Li10ELi([24])E", stub.stub_name(i).decode(
            for i in range(stub.stub_launches())]
 applies = [(int(m[1]), lds) for m, lds in applies if m]
 assert applies and all(lds >= (16 << 10) * (1 + split // 2) for split, lds in applies), applies
+""")
+
+
+@pytest.mark.parametrize("n,groups,far,split", [(22, 9, 0, 1), (26, 16, 0, 1), (24, 8, 0, 2), (21, 16, 0, 2), (23, 12, 1, 2),
+                                                (14, 12, 0, 4)])
+def test_thread_groups_inside_the_tile(run, n, groups, far, split):
+    """Operators of more than 8 groups, all inside the tile, have one thread group
+    per block where the tiles fill the chip many times."""
+    run(f"""
+import itertools
+pairs = list(itertools.combinations(range(8), 2))
+labels = [term({n}, {{a: "X", b: "X", 13: "Z"}}) for a, b in pairs[:{groups} - {far}]]
+labels += [term({n}, {{12: "X", a: "X"}}) for a in range({far})]
+op = op_of(labels)
+if {far}:
+    __import__("os").environ["QR_APPLY_FORM"] = "1"
+L.check(L.lib.qr_pauli_apply(op, 0, 1, 64 * GB, 128 * GB, None, None))
+names = [k[0] for k in launched("k_apply_")]
+assert names and all("tiled" in k and "Li10ELi{split}E" in k for k in names), names
 """)
