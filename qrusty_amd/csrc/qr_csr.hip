@@ -486,9 +486,10 @@ static int launch_build_words(const qr_op *op, const DeviceTables *t, uint64_t r
         // batches per tile: as many as the sign words of the real form have, and
         // as many where the tile folds heavy groups; half of that for the rest,
         // which loads its terms again anyway (20 qubits, 2000 terms 7.5 / 7.4
-        // ms; weights 1 to 4, 2000 terms 2.9 / 3.5); fewer where the launch
-        // would have under four blocks per CU
-        uint32_t ml = op->word_real || t->nheavy ? kWordMaxLog2 : kWordMaxLog2 - 1;
+        // ms; weights 1 to 4, 2000 terms 2.9 / 3.5), and for one or two groups, whose
+        // tiles are the longest (24 and 25 qubits 187 / 166, 211 / 186 us); fewer where
+        // the launch would have under four blocks per CU
+        uint32_t ml = (op->word_real && G > 2) || t->nheavy ? kWordMaxLog2 : kWordMaxLog2 - 1;
         while (ml > 2 && nl * ((row_end - row_begin) >> (rs_log2 + ml)) < 1024) --ml;
         // and as few as the LDS holds all heavy groups' values for (by 8 batches
         // it does: a heavy group has 4 times the mean of terms, so they are at

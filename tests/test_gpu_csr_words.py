@@ -74,6 +74,13 @@ def test_whole(n, groups, sizes, real):
 
 
 @pytest.mark.parametrize("real", [True, False])
+@pytest.mark.parametrize("n,groups,sizes", [(1, 2, [1]), (14, 1, [1]), (16, 2, [1, 3]), (17, 1, [9]), (16, 3, [2])])
+def test_few_groups(n, groups, sizes, real):
+    """One to three groups: the tiles of the most rows, several of them."""
+    test_whole(n, groups, sizes, real)
+
+
+@pytest.mark.parametrize("real", [True, False])
 @pytest.mark.parametrize("n,groups,sizes", [(13, 300, [2, 4, 30]), (13, 1500, [4, 6]), (13, 20, [2, 2, 50])])
 def test_row_windows(n, groups, sizes, real):
     from qrusty_amd import _lib as L
