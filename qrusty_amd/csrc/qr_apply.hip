@@ -835,7 +835,13 @@ constexpr int kFormGatherNear = 5;   // FP64, more than 8 groups, F = 0
 //     random 20 qubits, 2000 terms (2.3) 1123 / 1104; below 2^20 rows, where x
 //     stays in L2, gathers win up to F/D 8: 18 qubits, 100 terms 50 / 60,
 //     k-local 16 qubits 28 / 33.  Operators with window passes keep only
-//     partners that the L2 holds: 24-qubit ring 300 / 321.
+//     partners that the L2 holds: 24-qubit ring 300 / 321.  So do those with 5 to 12
+//     partners, many of them in L2, for half of the groups or more: random
+//     bonds, y / y and energy, 24 qubits, 14, 12 groups 210 / 270 against 275 / 285,
+//     200 / 259 against 256 / 277, 25 qubits, 12 415 / 496 against 482 / 502, k-local,
+//     23 qubits, 12 114 / 162 against 134 / 179; but k-local, 24 qubits, 21 groups, 10
+//     of them far, 337 / 397 against 332 / 379, 36 groups, 23 partners 611 / 660
+//     against 594 / 659, 4 groups, 3 partners, two states 221 / 303 against 204 / 300.
 //   complex64 (2^11-row tiles): molecule 20 qubits 804 / 883, random 20 qubits
 //     762 / 840, k-local 24 qubits, 3000 terms 4940 / 5160, ring 24 qubits 183
 //     / 199; a state past the 256 MB MALL: k-local 28 qubits 236 / 229 ms.
@@ -893,8 +899,9 @@ static int apply_form(const qr_op *op, int kind, int L, const PatternShape &win_
         bool staged = far > 0 && kind != 2 && !windows, few = false;
         if (kind == 0) {
             few = staged && lone && distinct >= 64 && state_log2 >= 24;
+            const bool some = distinct >= 5 && distinct <= 12 && 2 * far >= op->G;
             staged = staged && !few &&
-                     (dense || state_log2 >= 26 || (state_log2 >= 24 && (scattered || 2 * far >= 3 * distinct)) ||
+                     (dense || (state_log2 >= 26 && !some) || (state_log2 >= 24 && (scattered || 2 * far >= 3 * distinct)) ||
                       (far == op->G && 4 * far < 5 * distinct && distinct <= 16));
         } else {
             staged = staged && ((state_log2 >= 28 && 2 * far >= 3 * distinct) ||

@@ -307,3 +307,19 @@ L.check(L.lib.qr_pauli_apply(op, 0, 1, 64 * GB, 128 * GB, None, None))
 names = [k[0] for k in launched("k_apply_")]
 assert names and all("tiled" in k and "Li10ELi{split}E" in k for k in names), names
 """)
+
+
+@pytest.mark.parametrize("n,bonds,near,form", [(24, range(10, 22, 2), 3, "tiled"), (22, range(9, 20), 2, "tiled"),
+                                               (24, range(10, 18, 2), 0, "staged"), (24, range(10, 22, 2), 6, "staged"),
+                                               (21, range(10, 20, 2), 3, "tiled")])
+def test_form_of_some_partners(run, n, bonds, near, form):
+    """FP64, partners of their own for 5 to 12 groups, half of them or more, half
+    of the partners in L2: gathers; with fewer, or more groups inside the
+    tile, staged from 2^22 rows on."""
+    run(f"""
+labels = [term({n}, {{q: "X", q + 1: "Y"}}) for q in {list(bonds)}] + [term({n}, {{q: "X"}}) for q in range({near})]
+op = op_of(labels)
+L.check(L.lib.qr_pauli_apply(op, 0, 1, 64 * GB, 128 * GB, None, None))
+names = [k[0] for k in launched("k_apply_")]
+assert names and all("k_apply_{form}" in k for k in names), names
+""")
