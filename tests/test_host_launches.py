@@ -310,7 +310,7 @@ assert names and all("tiled" in k and "Li10ELi{split}E" in k for k in names), na
 
 
 @pytest.mark.parametrize("n,bonds,near,form", [(24, range(10, 22, 2), 3, "tiled"), (22, range(9, 20), 2, "tiled"),
-                                               (24, range(10, 18, 2), 0, "staged"), (24, range(10, 22, 2), 6, "staged"),
+                                               (24, range(10, 18, 2), 0, "staged"), (24, range(10, 22, 2), 7, "staged"),
                                                (21, range(10, 20, 2), 3, "tiled")])
 def test_form_of_some_partners(run, n, bonds, near, form):
     """FP64, partners of their own for 5 to 12 groups, half of them or more, half
