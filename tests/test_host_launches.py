@@ -323,3 +323,15 @@ L.check(L.lib.qr_pauli_apply(op, 0, 1, 64 * GB, 128 * GB, None, None))
 names = [k[0] for k in launched("k_apply_")]
 assert names and all("k_apply_{form}" in k for k in names), names
 """)
+
+
+@pytest.mark.parametrize("longer,few", [(1, False), (2, False), (3, True)])
+def test_sums_of_few_strings(run, longer, few):
+    """One entry per row in one matrix and one or two in the other: the staged tiles."""
+    run(f"""
+n = 1 << 20
+one = (ctypes.c_double * 2)(1.0, 0.0)
+L.check(L.lib.qr_csr_add_fill(n, one, {longer} * n, 64 * GB, 65 * GB, 66 * GB, one, n, 67 * GB, 68 * GB, 69 * GB, 70 * GB,
+                              71 * GB, 72 * GB, None))
+assert bool(launched("k_spadd_few")) == {few} and bool(launched("k_spadd_tile")) != {few}
+""")
