@@ -506,7 +506,7 @@ __global__ __launch_bounds__(256) void k_spadd_few(uint64_t nrows, uint32_t lpr_
 // 250, 417 / 399, 598 / 520, 864 / 798 (the mean rounded up: 363, 517, 521, 728); one
 // row in 100 of 600 entries 4360 / 656; but one or two entries per row, which idle
 // most of four lanes, 23 qubits 595 / 667 (of the same columns 513 / 666), 670 / 764
-// (three 893 / 917), and 24 or 100 entries in every other row 432 / 595, 1120 /
+// (three 893 / 917, below 2^22 rows equal), and 24 or 100 entries in every other row 432 / 595, 1120 /
 // 1700 (a whole number in the mean).  Other sums stay with
 // the tiles: rows with two short entries (Z + X) run one at a time here, 20-qubit
 // ring 657 / 1290, 0 to 2 each 600 / 900 (and as many as rows, alternately 0 and 2,
@@ -528,7 +528,7 @@ static bool spadd_few(uint64_t nrows, SpAddIn &in, SpFew &f) {
     while (f.lpr_log2 < 6 && double(1u << f.lpr_log2) < need) ++f.lpr_log2;
     f.pieces = mean > 64;
     if (f.pieces ? in.nnz2 == 0 || in.nnz2 > 2 * nrows || in.nnz1 / 64 < nrows + in.nnz2
-                 : in.nnz2 != nrows || in.nnz1 / 3 < nrows || need > 64)
+                 : in.nnz2 != nrows || (in.nnz1 / 3 < nrows && nrows >> 22) || need > 64)
         return false;
     f.rpw_log2 = 6;
     const uint64_t waves = f.pieces ? 65536 : 4096;

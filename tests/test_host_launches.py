@@ -325,11 +325,12 @@ assert names and all("k_apply_{form}" in k for k in names), names
 """)
 
 
-@pytest.mark.parametrize("longer,few", [(1, False), (2, False), (3, True)])
-def test_sums_of_few_strings(run, longer, few):
-    """One entry per row in one matrix and one or two in the other: the staged tiles."""
+@pytest.mark.parametrize("qubits,longer,few", [(22, 1, False), (22, 2, False), (22, 3, True), (21, 1, True)])
+def test_sums_of_few_strings(run, qubits, longer, few):
+    """One entry per row in one matrix and one or two in the other, many rows: the
+    staged tiles."""
     run(f"""
-n = 1 << 20
+n = 1 << {qubits}
 one = (ctypes.c_double * 2)(1.0, 0.0)
 L.check(L.lib.qr_csr_add_fill(n, one, {longer} * n, 64 * GB, 65 * GB, 66 * GB, one, n, 67 * GB, 68 * GB, 69 * GB, 70 * GB,
                               71 * GB, 72 * GB, None))
